@@ -1414,41 +1414,69 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
     extern __shared__ __align__(16) uint8_t dyn[];
     __shared__ uint64_t redu[16];
     __shared__ int32_t bcast[16];
-    // the sublists' prefix sums sit where the planes go: built before each
-    // chunk of 256 entries is fetched, overwritten by the planes after
+    const int G = (int)gridDim.x, lane = (int)threadIdx.x & 63;
+    // Up to 64 sublists (4096 children at 64 each): every wave scans their
+    // counts in registers, and the workgroup's entries are fetched one ahead
+    // of the one being searched, so no barrier stands before the first search.
+    // More: the prefix sums sit where the planes go -- built before each chunk
+    // of 256 entries is fetched, overwritten by the planes after -- and are
+    // built again only when the workgroup has entries past its first chunk.
+    const bool few = groups <= 64;
     int *pre = (int *)dyn;  // [groups + 1]
     __shared__ int red[16], s_carry;
     __shared__ uint32_t s_ent[256];  // the workgroup's next entries, fetched together
-    const int G = (int)gridDim.x;
-    for (int e0 = (int)blockIdx.x;; e0 += 256 * G) {
-        __syncthreads();  // the previous entries' planes are no longer read
-        if (threadIdx.x == 0) s_carry = 0;
-        for (int g0 = 0; g0 < groups; g0 += blockDim.x) {  // exclusive prefix of the counts
-            const int g = g0 + (int)threadIdx.x;
-            const int n = g < groups ? min(gload(ctl + g), cap) : 0;
-            int total;
-            const int ex = block_scan_excl(n, red, &total);
-            if (g < groups) pre[g] = s_carry + ex;
-            __syncthreads();
-            if (threadIdx.x == 0) s_carry += total;
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) pre[groups] = s_carry;
-        __syncthreads();
-        const int count = pre[groups];
-        if (e0 >= count) break;
-        {
-            const int e = e0 + (int)threadIdx.x * G;
-            if (e < count) {
-                int k = 0;  // the last sublist whose entries start at or before e
-                for (int h = STEM_MAX_GROUPS / 2; h > 0; h >>= 1)
-                    if (k + h < groups && pre[k + h] <= e) k += h;
-                s_ent[threadIdx.x] = gload(list + (size_t)k * cap + (e - pre[k]));
+    int incl = 0, count = 0, e = (int)blockIdx.x, j = 0;
+    uint32_t nxt = 0;
+    auto fetch = [&](int q) -> uint32_t {  // entry q of the list (few; q is the same in every lane)
+        const int k = (int)__popcll(__ballot(incl <= q));
+        const int first = k ? __builtin_amdgcn_readlane(incl, k - 1) : 0;
+        return gload(list + (size_t)k * cap + (q - first));
+    };
+    if (few) {
+        incl = wave_scan_i32(lane < groups ? min(gload(ctl + lane), cap) : 0);
+        count = __builtin_amdgcn_readlane(incl, 63);
+        if (e < count) nxt = fetch(e);
+    }
+    for (bool start = true;; start = false, e += G) {
+        uint32_t ent;
+        if (few) {
+            if (e >= count) break;
+            ent = nxt;
+            if (e + G < count) nxt = fetch(e + G);
+        } else {
+            if (!start && e >= count) break;
+            if (start || j == 256) {
+                __syncthreads();  // the previous entries' planes are no longer read
+                if (threadIdx.x == 0) s_carry = 0;
+                for (int g0 = 0; g0 < groups; g0 += blockDim.x) {  // exclusive prefix of the counts
+                    const int g = g0 + (int)threadIdx.x;
+                    const int n = g < groups ? min(gload(ctl + g), cap) : 0;
+                    int total;
+                    const int ex = block_scan_excl(n, red, &total);
+                    if (g < groups) pre[g] = s_carry + ex;
+                    __syncthreads();
+                    if (threadIdx.x == 0) s_carry += total;
+                    __syncthreads();
+                }
+                if (threadIdx.x == 0) pre[groups] = s_carry;
+                __syncthreads();
+                count = pre[groups];
+                if (e >= count) break;
+                const int q = e + (int)threadIdx.x * G;
+                if (q < count) {
+                    int k = 0;  // the last sublist whose entries start at or before q
+                    for (int h = STEM_MAX_GROUPS / 2; h > 0; h >>= 1)
+                        if (k + h < groups && pre[k + h] <= q) k += h;
+                    s_ent[threadIdx.x] = gload(list + (size_t)k * cap + (q - pre[k]));
+                }
+                j = 0;
+                __syncthreads();
             }
+            ent = s_ent[j++];
         }
-        __syncthreads();
-        for (int j = 0; j < 256 && e0 + j * G < count; ++j) {
-            const uint32_t ent = s_ent[j];
+        {
+            // (wave-uniform: the item and the descriptor come by scalar loads)
+            ent = (uint32_t)__builtin_amdgcn_readfirstlane((int)ent);
             const int2 it = items[ent >> 4];
             const int c = (int)(ent & 15u);
             const DevJob &J = jobs[it.x];
