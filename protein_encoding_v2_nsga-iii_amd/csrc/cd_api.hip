@@ -90,6 +90,9 @@ int build_tables(const cd_tables &t, HostTables &h) {
 // Das-Dennis simplex lattice in the order of combinationRepetition
 // (sorting.cuh:1285-1354): multisets of H objectives in lexicographic order,
 // coordinate = H-fold float sum of 1/H over the objective's multiplicity.
+// Rows of REF_STRIDE floats: the coordinates, then the sum of their squares
+// in objective order (perp_dist's divisor, rounded term by term as on the
+// device: no contraction), then 0.
 std::vector<float> das_dennis(int H) {
     std::vector<float> out;
     std::vector<int> x(H, 0);
@@ -98,6 +101,10 @@ std::vector<float> das_dennis(int H) {
         float v[6] = {0, 0, 0, 0, 0, 0};
         for (int i = 0; i < H; ++i) v[x[i]] += step;
         out.insert(out.end(), v, v + 6);
+        float den = 0.f;
+        for (float w : v) den += w * w;
+        out.push_back(den);
+        out.push_back(0.f);
         int i = H - 1;
         while (i >= 0 && x[i] == 5) --i;
         if (i < 0) break;
@@ -170,7 +177,7 @@ Layout layout(int L, int m, int N, int P, int R, int W, int n_dom, int n_asc, bo
     }
     for (int b = 0; b < (sel_only ? 1 : 2); ++b) o.obj[b] = s.add((size_t)P * 6 * 4);
     if (sel_only) o.obj[1] = o.obj[0];
-    o.ref = s.add((size_t)R * 6 * 4);
+    o.ref = s.add((size_t)R * cd::REF_STRIDE * 4);
     o.front = s.add((size_t)P * 4);
     o.np = s.add((size_t)P * 4);
     o.dom = s.add((size_t)P * W * 8);
@@ -398,6 +405,7 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
     if (!sel_only) {  // the tuned shapes of this kind of job, if any
         cd_job *self = J;
         cd::Shapes sh;
+        J->shapes = cdhost::untuned_shapes(&self, 1);
         if (cdhost::cached_shapes(cdhost::work_signature(&self, 1), &sh)) J->shapes = sh;
     } else {
         J->shapes.dom_rows = cd::DOM_ROWS;
@@ -422,7 +430,8 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
     if (e == hipSuccess && J->lds > 48 * 1024) e = cd::set_design_lds_limit(J->lds);
     if (e == hipSuccess && cd::stem_list_lds(J->stem_lds) > 48 * 1024)
         e = cd::set_stem_lds_limit(cd::stem_list_lds(J->stem_lds));
-    if (e == hipSuccess && cd::niche_lds_bytes(J->P) > 48 * 1024) e = cd::set_niche_lds_limit(cd::niche_lds_bytes(J->P));
+    if (e == hipSuccess && cd::niche_lds_need(J->P, J->R) > cd::NICHE_LDS_PLAIN)
+        e = cd::set_niche_lds_limit(cd::niche_lds_need(J->P, J->R));
     if (e != hipSuccess) {
         (void)hipFreeAsync(J->mem, J->stream);
         (void)hipStreamSynchronize(J->stream);
@@ -471,9 +480,12 @@ hipError_t enqueue_generation(const Launch &w, hipStream_t s, hipEvent_t *ev) {
     if (e == hipSuccess)
         e = cd::launch_dominance(w.jobs, w.dom, w.n_dom, true, w.stem_ctl, sl.groups, w.sh.dom_rows, s);
     if (e == hipSuccess) e = mark(3);
-    if (e == hipSuccess) e = cd::launch_fronts(w.jobs, w.njobs, w.max_pool, w.sh.fronts_threads, s);
+    const bool fused = cd::fuse_fronts(w.max_pool, w.pool);
+    if (e == hipSuccess && !fused) e = cd::launch_fronts(w.jobs, w.njobs, w.max_pool, w.sh.fronts_threads, s);
     if (e == hipSuccess) e = mark(4);
-    if (e == hipSuccess) e = cd::launch_associate(w.jobs, w.asc, w.n_asc, w.sh.assoc_designs, s);
+    if (e == hipSuccess)
+        e = fused ? cd::launch_front_associate(w.jobs, w.asc, w.n_asc, w.sh.assoc_designs, s)
+                  : cd::launch_associate(w.jobs, w.asc, w.n_asc, w.sh.assoc_designs, s);
     if (e == hipSuccess) e = mark(5);
     if (e == hipSuccess) e = cd::launch_niche(w.jobs, w.njobs, w.max_pool, w.max_refs, w.sh.niche_threads, s);
     if (e == hipSuccess) e = mark(6);
@@ -510,6 +522,7 @@ void build_lists(cd_job *const *jobs, int count, const cd::Shapes &sh, WorkLists
         wl.lds = std::max(wl.lds, J->lds);
         wl.stem_lds = std::max(wl.stem_lds, J->stem_lds);
         wl.max_pool = std::max(wl.max_pool, J->P);
+        wl.pool += J->P;
         wl.max_refs = std::max(wl.max_refs, J->R);
         wl.mg = std::max(wl.mg, J->m);
         wl.stem_parts = std::max(wl.stem_parts, J->stem_parts);
@@ -521,8 +534,8 @@ hipError_t set_lds_limits(const WorkLists &wl) {
     if (wl.lds > 48 * 1024) e = cd::set_design_lds_limit(wl.lds);
     if (e == hipSuccess && cd::stem_list_lds(wl.stem_lds) > 48 * 1024)
         e = cd::set_stem_lds_limit(cd::stem_list_lds(wl.stem_lds));
-    if (e == hipSuccess && cd::niche_lds_bytes(wl.max_pool) > 48 * 1024)
-        e = cd::set_niche_lds_limit(cd::niche_lds_bytes(wl.max_pool));
+    const size_t niche = cd::niche_lds_need(wl.max_pool, wl.max_refs);
+    if (e == hipSuccess && niche > cd::NICHE_LDS_PLAIN) e = cd::set_niche_lds_limit(niche);
     return e;
 }
 
@@ -573,7 +586,7 @@ Launch job_launch(cd_job *J) {
     return Launch{J->d_self, 1,          J->d_off,     J->N,          J->d_dom,   J->n_dom,   J->d_asc,
                   J->n_asc,  J->lds,     J->stem_lds,  J->P,          J->R,       J->m,          J->stem_parts,
                   J->d_slist,
-                  J->d_sctl, J->N * J->m, 0,           0,             J->shapes};
+                  J->d_sctl, J->N * J->m, 0,           0,             J->P,          J->shapes};
 }
 
 // Wait for the job's own stream and for the streams of the batches that hold it.
@@ -693,6 +706,23 @@ std::string work_signature(cd_job *const *jobs, int count) {
     return "dev" + std::to_string(dev) + "/jobs" + std::to_string(log2_bucket(count)) + "/children" +
            std::to_string(log2_bucket(children)) + "/codons" + std::to_string(log2_bucket(lm)) + "/pool" +
            std::to_string(log2_bucket(pool));
+}
+
+// The shapes of untuned work.  Association: a wave a design while the waves
+// fit the chip (pool <= 12000 designs in all), eight lanes a design above;
+// few designs a workgroup where a generation is a chain of latencies (4 up to
+// 512 designs, 8 up to FUSED_TOTAL, where k_front_associate runs), more
+// where it is throughput.  Measured, microseconds a generation of batches of
+// the 50..2000-residue mix with 4 / 8 / 16 / 64 designs a workgroup: pool 2048
+// 140.1 / 137.6 / 138.7 / 142.5, pool 8192 206.7 / 204.3 / 202.9 / 205.1, pool
+// 28160 557.5 / 557.1 / 557.7 / 553.6, pool 84480 1244 / 1245 / - / 1226; the
+// 100-residue job (pool 256) 50.4 / 50.9.
+cd::Shapes untuned_shapes(cd_job *const *jobs, int count) {
+    cd::Shapes sh = count == 1 ? cd::SHAPES_JOB : cd::SHAPES_BATCH;
+    int64_t pool = 0;
+    for (int j = 0; j < count; ++j) pool += jobs[j]->P;
+    sh.assoc_designs = pool <= 512 ? 4 : pool <= cd::FUSED_TOTAL ? 8 : pool <= 12000 ? 16 : 64;
+    return sh;
 }
 
 bool cached_shapes(const std::string &sig, cd::Shapes *out) {
@@ -828,10 +858,11 @@ int cd_job_read(cd_job *J, int8_t *genome, float *obj, int8_t *idx, int32_t *pql
         for (int i = 0; i < P; ++i)
             for (int k = 0; k < 3; ++k) pql[i * 3 + k] = t[(size_t)i * 4 + k];
     if (state) {
-        std::memcpy(state, st.ext, sizeof(st.ext));
-        std::memcpy(state + 36, st.ideal, sizeof(st.ideal));
-        std::memcpy(state + 42, st.worst, sizeof(st.worst));
-        std::memcpy(state + 48, st.nadir, sizeof(st.nadir));
+        const cd::SelRes &r = st.res[b];
+        std::memcpy(state, r.ext, sizeof(r.ext));
+        std::memcpy(state + 36, r.ideal, sizeof(r.ideal));
+        std::memcpy(state + 42, r.worst, sizeof(r.worst));
+        std::memcpy(state + 48, r.nadir, sizeof(r.nadir));
     }
     return CD_OK;
 }
@@ -922,7 +953,7 @@ static int run_selection(const float *obj, int32_t P, int32_t N, int32_t H, uint
     if (rc != CD_OK) return rc;
     cd::SelState st{};
     st.gen = gen;
-    if (extremes) std::memcpy(st.ext, extremes, sizeof(st.ext));
+    if (extremes) std::memcpy(st.res[gen & 1u].ext, extremes, sizeof(st.res[0].ext));
     hipError_t e = hipMemcpy(J->h.obj[0], obj, (size_t)P * 24, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(J->h.st, &st, sizeof(st), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = cd::launch_zero_np(J->d_self, 1, J->stream);
@@ -947,7 +978,7 @@ int cd_nds(const float *obj, int32_t P, int32_t N, int32_t *front_of, int32_t *n
     cd::SelState st;
     hipError_t e = hipMemcpy(&st, J->h.st, sizeof(st), hipMemcpyDeviceToHost);
     if (e == hipSuccess && front_of) e = hipMemcpy(front_of, J->h.front_of, (size_t)P * 4, hipMemcpyDeviceToHost);
-    if (n_fronts) *n_fronts = st.last + 1;
+    if (n_fronts) *n_fronts = st.res[1].last + 1;  // (the sort ran as generation 0)
     cd_job_destroy(J);
     if (e != hipSuccess) return fail(CD_E_DEVICE, std::string("nds: ") + hipGetErrorString(e));
     return CD_OK;
@@ -965,15 +996,16 @@ int cd_select(const float *obj, int32_t N, int32_t H, uint32_t gen, uint64_t see
     if (e == hipSuccess && sorted) survivors_of(mask, N, sorted);
     if (e == hipSuccess && front_of) e = hipMemcpy(front_of, J->h.front_of, (size_t)2 * N * 4, hipMemcpyDeviceToHost);
     if (e == hipSuccess) {
-        if (extremes) std::memcpy(extremes, st.ext, sizeof(st.ext));
+        const cd::SelRes &r = st.res[(gen + 1u) & 1u];
+        if (extremes) std::memcpy(extremes, r.ext, sizeof(r.ext));
         if (norm) {
-            std::memcpy(norm, st.ideal, 24);
-            std::memcpy(norm + 6, st.worst, 24);
-            std::memcpy(norm + 12, st.nadir, 24);
+            std::memcpy(norm, r.ideal, 24);
+            std::memcpy(norm + 6, r.worst, 24);
+            std::memcpy(norm + 12, r.nadir, 24);
         }
         if (flags) {
-            flags[0] = st.n_cut;
-            flags[1] = st.hyp;
+            flags[0] = r.n_cut;
+            flags[1] = r.hyp;
         }
     }
     cd_job_destroy(J);
@@ -998,6 +1030,7 @@ int cd_batch_create(cd_job *const *jobs, int32_t count, cd_batch **out) {
         B->jobs.push_back(jobs[j]);
     }
     cd::Shapes sh;
+    B->shapes = cdhost::untuned_shapes(jobs, count);
     if (cdhost::cached_shapes(cdhost::work_signature(jobs, count), &sh)) B->shapes = sh;
     cdhost::WorkLists wl;
     cdhost::build_lists(jobs, count, B->shapes, wl);
@@ -1012,6 +1045,7 @@ int cd_batch_create(cd_job *const *jobs, int32_t count, cd_batch **out) {
     B->lds = wl.lds;
     B->stem_lds = wl.stem_lds;
     B->max_pool = wl.max_pool;
+    B->pool = wl.pool;
     B->max_refs = wl.max_refs;
     B->mg = wl.mg;
     B->stem_parts = wl.stem_parts;
@@ -1047,7 +1081,7 @@ static Launch batch_launch(cd_batch *B) {
     return Launch{B->d_jobs,    (int)B->jobs.size(), B->d_off,      B->n_off,   B->d_dom,
                   B->n_dom,     B->d_asc,            B->n_asc,      B->lds,     B->stem_lds,
                   B->max_pool,  B->max_refs,         B->mg,         B->stem_parts, B->d_slist, B->d_sctl,
-                  B->n_cds,     B->n_small,          B->lds_small,  B->shapes};
+                  B->n_cds,     B->n_small,          B->lds_small,  B->pool,      B->shapes};
 }
 
 int cd_batch_profile(cd_batch *B, int32_t generations, float *kernel_ms) {

@@ -71,6 +71,7 @@ struct cd_batch {
     size_t lds_small = 0;   // their k_design LDS
     size_t lds = 0, stem_lds = 0;
     int max_pool = 0;    // largest pool of the batch's jobs
+    int pool = 0;        // designs of all their pools
     int max_refs = 0;    // most reference points of the batch's jobs
     int mg = 0;          // largest m of the batch's jobs
     int stem_parts = 0;  // largest k_stem workgroups per CDS of the batch's jobs
@@ -116,6 +117,7 @@ struct Launch {
     // apart from the others, which take lds
     int n_small;
     size_t lds_small;
+    int pool;  // designs of all jobs' pools
     cd::Shapes sh;
 };
 
@@ -126,7 +128,7 @@ struct WorkLists {
     std::vector<int2> off, asc;
     std::vector<int4> dom;
     size_t lds = 0, stem_lds = 0;
-    int max_pool = 0, max_refs = 0, mg = 0, stem_parts = 0, n_cds = 0;
+    int max_pool = 0, max_refs = 0, mg = 0, stem_parts = 0, n_cds = 0, pool = 0;
     int n_small = 0;  // children (first in off) of jobs with lds at most shapes.design_split
     size_t lds_small = 0;
 };
@@ -140,6 +142,8 @@ void build_lists(cd_job *const *jobs, int count, const cd::Shapes &shapes, WorkL
 // jobs and served ticks of the same kind start from them.
 std::string work_signature(cd_job *const *jobs, int count);
 bool cached_shapes(const std::string &sig, cd::Shapes *out);
+// the shapes of jobs without tuned ones, by their sizes
+cd::Shapes untuned_shapes(cd_job *const *jobs, int count);
 void store_shapes(const std::string &sig, const cd::Shapes &sh);
 
 // Mutation, evaluation and selection of one generation of every job of `w`;

@@ -28,7 +28,8 @@ struct Shapes {
     int assoc_designs;   // designs per k_associate workgroup: 4, 8 or 16 (a wave each), 32 or 64 (eight lanes each)
     int niche_threads;   // niching workgroup (k_place_niche, or k_place and k_niche above 2048 designs): 256, 512 or 1024 threads
 };
-// Untuned shapes: a lone job, and a batch or served tick.
+// Untuned shapes of a lone job, and of a batch or served tick (assoc_designs
+// by the pool: untuned_shapes).
 constexpr Shapes SHAPES_JOB = {0, 512, 6, 64, 512, 4, 1024};
 constexpr Shapes SHAPES_BATCH = {24 * 1024, 512, 7, 128, 1024, 4, 1024};
 bool shapes_valid(const Shapes &s);
@@ -100,17 +101,36 @@ constexpr int FRONT0_THREADS = 256;
 hipError_t launch_fronts(const DevJob *jobs, int njobs, int max_pool, int threads, hipStream_t s);
 // items: (job, first design), `designs` designs per item: 4, 8 or 16 (a wave each), 32 or 64 (eight lanes each)
 hipError_t launch_associate(const DevJob *jobs, const int2 *items, int n, int designs, hipStream_t s);
+// launch_fronts and launch_associate in one launch, for pools of at most
+// FUSED_POOL designs
+constexpr int FUSED_POOL = 2048;
+// Taken while all jobs' pools together hold at most FUSED_TOTAL designs, 512
+// workgroups of 8: each workgroup repeats the job's settling, which costs
+// nothing while the workgroups run side by side and more than the two launches
+// it saves once they queue.  Microseconds of the fronts and association, fused
+// against apart: pool 1024 19.3 / 20.7, 4096 24.8 / 24.6, 8192 37.0 / 28.1.
+constexpr int FUSED_TOTAL = 4096;
+inline bool fuse_fronts(int max_pool, int pool) { return max_pool <= FUSED_POOL && pool <= FUSED_TOTAL; }
+hipError_t launch_front_associate(const DevJob *jobs, const int2 *items, int n, int designs, hipStream_t s);
 // Pools of at most PLACE_NICHE_POOL designs with at most NICHE_STAGE
 // reference points: k_place_niche (one workgroup of `threads` per job,
-// place_niche_lds_bytes(max_pool) of dynamic LDS).  Otherwise k_levels (one
+// place_niche_lds_bytes(max_pool, max_refs) of dynamic LDS).  Otherwise k_levels (one
 // workgroup per job) when some job has more reference points than
 // NICHE_STAGE (max_refs), then k_place and k_niche (grid: jobs x chunks of
 // `threads` (256, 512 or 1024) designs of the largest pool, max_pool; k_niche
-// takes niche_lds_bytes(max_pool) of dynamic LDS, set_niche_lds_limit above
-// 48 KiB)
+// takes niche_lds_bytes(max_pool) of dynamic LDS)
 constexpr int PLACE_NICHE_POOL = 2048;
-inline size_t place_niche_lds_bytes(int P) { return (size_t)12 * P; }
+// slots of its cut list: every design of the pool, and up to three pads a bucket
+__host__ __device__ inline int place_niche_slots(int P, int R) { return P + 3 * (R < P ? R : P); }
+inline size_t place_niche_lds_bytes(int P, int R) { return (size_t)8 * ((place_niche_slots(P, R) + 3) & ~3); }
 size_t niche_lds_bytes(int P);
+// dynamic LDS of the niching of pools up to P with up to R reference points,
+// and its limit, to be raised above NICHE_LDS_PLAIN (k_place_niche's static
+// arrays take 37 KiB beside it)
+constexpr size_t NICHE_LDS_PLAIN = 24 * 1024;
+inline size_t niche_lds_need(int P, int R) {
+    return P <= PLACE_NICHE_POOL && R <= NICHE_STAGE ? place_niche_lds_bytes(P, R) : niche_lds_bytes(P);
+}
 hipError_t set_niche_lds_limit(size_t bytes);
 hipError_t launch_niche(const DevJob *jobs, int njobs, int max_pool, int max_refs, int threads, hipStream_t s);
 hipError_t launch_init_state(const DevJob *jobs, int njobs, hipStream_t s);

@@ -16,11 +16,15 @@
 //                        132-972)
 //   k_associate          nearest reference line per ranked design and the
 //                        niche counts (sorting.cuh:1105-1180)
+//   k_front_associate    the three above in one launch, for few and small
+//                        pools (fuse_fronts)
 //   [k_levels]           the niche levels, when the reference points do not
 //                        fit in LDS (else k_place settles them)
 //   k_place              level-0 picks, whole buckets, the cut list
 //   k_niche              the cut buckets ranked by priority
 //                        (sorting.cuh:1182-1279); ends the generation
+//   k_place_niche        the two above in one workgroup per job, for pools up
+//                        to 2048
 // Hand-offs between workgroups happen at kernel boundaries; atomics that
 // fold per-job quantities are reduced over the workgroup first (same-address
 // atomics serialise at the device's coherence point).
@@ -1049,6 +1053,19 @@ __device__ void build_planes(const uint8_t *rows, int Ls, int L, const int *dl, 
     }
 }
 
+// The niche arrays the association counts into, cleared from entry i0 on in
+// steps.
+__device__ __forceinline__ void clear_niche(const DevJob &J, int i0, int step) {
+    const int R = J.R;
+    if (i0 >= R) return;
+    const NicheView g = niche_view(J.niche, R);
+    for (int r = i0; r < R; r += step) {
+        gstore((uint64_t *)g.cr + r, (uint64_t)0);
+        gstore(g.fill + r, 0);
+        gstore(g.nearest + r, ~0ull);
+    }
+}
+
 // The index of the c-th survivor (0-based, ascending pool index) in the
 // survivor mask of W words: wave-uniform, every lane of the wave takes part.
 __device__ int survivor_at(const uint64_t *selm, int W, int c, uint64_t first) {
@@ -1261,6 +1278,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             gstore(np + N + c, 0);
         }
         if (c == 0 && tid >= 128 && tid < 128 + ACC_WORDS) gstore((uint32_t *)acc + tid - 128, acc_clear_word(tid - 128));
+        clear_niche(J, c * NT + tid, N * NT);  // (and the association from cleared niche arrays)
     }
     lds_barrier();  // tables, synonym ranges, genome row and records
     // codon codes of the row, four per thread step; the padding positions
@@ -1777,66 +1795,6 @@ __global__ __launch_bounds__(256) void k_dominance(const DevJob *__restrict__ jo
     }
 }
 
-__device__ __forceinline__ float asf(const float *x, const float *ideal, int axis) {  // sorting.cuh:428-449
-    float mx = -FLT_MAX;
-#pragma unroll
-    for (int k = 0; k < NOBJ; ++k) {
-        float t = x[k] - ideal[k];
-        if ((double)t < 0.001) t = 0.f;
-        const float v = t / (k == axis ? 1.f : F_PRECISION);
-        if (v > mx) mx = v;
-    }
-    return mx;
-}
-
-// GaussianElimination and helpers, sorting.cuh:451-599 (E x = 1)
-// Every loop is unrolled so that the matrix stays in registers (the first
-// row below the pivot with a usable entry is added through a flag, not an
-// index).
-__device__ void gauss(const float *E, float *sol) {
-    float AB[NOBJ][NOBJ + 1];
-#pragma unroll
-    for (int r = 0; r < NOBJ; ++r) {
-#pragma unroll
-        for (int c = 0; c < NOBJ; ++c) AB[r][c] = E[r * NOBJ + c];
-        AB[r][NOBJ] = 1.0f;
-    }
-#pragma unroll
-    for (int col = 0; col < NOBJ; ++col) {
-        if (fabsf(AB[col][col]) <= 1e-6f) {
-            bool added = false;
-#pragma unroll
-            for (int row = col + 1; row < NOBJ; ++row)
-                if (!added && fabsf(AB[row][col]) > 1e-6f) {
-#pragma unroll
-                    for (int c = col; c < NOBJ + 1; ++c) AB[col][c] += AB[row][c];
-                    added = true;
-                }
-        }
-#pragma unroll
-        for (int row = col + 1; row < NOBJ; ++row) {
-            const float f = AB[row][col] / AB[col][col];
-#pragma unroll
-            for (int c = col; c < NOBJ + 1; ++c) AB[row][c] -= f * AB[col][c];
-        }
-    }
-#pragma unroll
-    for (int row = NOBJ - 1; row >= 0; --row) {
-        float s = 0.f;
-#pragma unroll
-        for (int c = row + 1; c < NOBJ; ++c) s += AB[row][c];
-        float x = AB[row][NOBJ];
-        if (row != NOBJ - 1) x -= s;
-        x /= AB[row][row];
-        AB[row][NOBJ] = x;
-        AB[row][row] = 1.0f;
-#pragma unroll
-        for (int r = 0; r < row; ++r) AB[r][row] *= x;
-    }
-#pragma unroll
-    for (int r = 0; r < NOBJ; ++r) sol[r] = AB[r][NOBJ];
-}
-
 // (v, id) becomes (ov, oid) when that pair is smaller: a smaller value, or
 // the same value with a smaller index (a NaN value is never taken).  Written
 // without short-circuit evaluation so that it compiles to selects.
@@ -1846,27 +1804,27 @@ __device__ __forceinline__ void argmin_pair(float &v, int &id, float ov, int oid
     id = take ? oid : id;
 }
 
-// argmin_pair over a full wave (DPP row shifts and broadcasts, lane 63 read
-// back), wave-uniform; lanes outside a shifted or masked row contribute
-// (FLT_MAX, 0x7FFFFFFF), the start value of every lane's fold.
+// argmin_pair with the pair a DPP step brings from another lane; lanes
+// outside a shifted or masked row contribute (FLT_MAX, 0x7FFFFFFF), the start
+// value of every lane's fold.
 template <int CTRL, int ROWS>
 __device__ __forceinline__ void argmin_dpp(float &v, int &id) {
     const float ov = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(FLT_MAX), __float_as_int(v), CTRL, ROWS, 0xf, false));
     const int oid = __builtin_amdgcn_update_dpp(0x7FFFFFFF, id, CTRL, ROWS, 0xf, false);
     argmin_pair(v, id, ov, oid);
 }
+// The smallest (value, index) pair of a full wave, wave-uniform: the smallest
+// value first, then the smallest index among the lanes that hold it (one
+// instruction a step each, against eight for the pair's comparison).  Values
+// are never NaN; a value above FLT_MAX counts as FLT_MAX with no index, the
+// start value of every lane's fold.
 __device__ __forceinline__ void wave_argmin(float &v, int &id) {
-    argmin_dpp<0x111, 0xf>(v, id);
-    argmin_dpp<0x112, 0xf>(v, id);
-    argmin_dpp<0x114, 0xf>(v, id);
-    argmin_dpp<0x118, 0xf>(v, id);
-    argmin_dpp<0x142, 0xa>(v, id);
-    argmin_dpp<0x143, 0xc>(v, id);
-    v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-    id = __builtin_amdgcn_readlane(id, 63);
+    const float m = wave_min_f32(v);
+    id = wave_min_i32(v == m ? id : 0x7FFFFFFF);
+    v = m;
 }
 
-// asf() for all six axes of one design.  The clamped differences t[k] are +0
+// The ASF values (sorting.cuh:428-449) of one design for all six axes.  The clamped differences t[k] are +0
 // or at least 0.001 (or NaN, which no comparison takes), and axis a takes the
 // strict running maximum of t[a] and t[k] / F_PRECISION over k != a.  A
 // correctly rounded division by a positive constant is nondecreasing, so the
@@ -1899,34 +1857,43 @@ __device__ __forceinline__ unsigned long long asf_key(float v, int id) {
     return ((unsigned long long)ord_bits(v) << 32) | (uint32_t)id;
 }
 
+__device__ __forceinline__ float lane_of(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
 // Extreme points (findExtremePoints, sorting.cuh:601-683) settled axis by
 // axis against the previous ones, by one wave.  The candidate rows are the
-// previous extremes (0-5) and the first front's ASF minima of the six axes
-// (6-11), with their ASF values for every axis in casf.  Lane t (0-5) keeps
-// the row extreme slot t holds; per axis the slots' values and the first
-// front's minimum (lane 6) are reduced to the smallest (value, index) pair --
-// the serial fold over the slots in order gives the same pair, NaN values
-// never being taken -- and the winner's row goes to the axis's slot.  Returns
-// the row held by slot `lane` (lanes 0-5).
-__device__ int settle_extremes(const float *pv, const int *pid, const float (*casf)[NOBJ], int P) {
+// previous extremes (0-5) and the rows of the first front's ASF minima of the
+// six axes (6-11); lane t (0-11) holds row t's ASF values c[] (never NaN), pv
+// and pid the first front's minimum of lane t - 6's axis (lanes 6-11).  Per
+// axis the smallest value among the rows the slots (lanes 0-5) hold and the
+// first front's minimum wins, ties to the first front, then to the lowest slot
+// -- what the serial fold over (value, index) pairs finds, a slot's index being
+// above every design's -- and its row and ASF values go to the axis's slot.
+// Returns the row held by slot `lane` (lanes 0-5).
+__device__ int settle_extremes(float *c, float pv, int pid) {
     const int lane = threadIdx.x & 63;
-    int cur = lane < NOBJ ? lane : 0;
+    int cur = lane;
 #pragma unroll
     for (int axis = 0; axis < NOBJ; ++axis) {
-        const float c = casf[cur][axis];
-        const bool slot = lane < NOBJ && !isnan(c), first = lane == NOBJ;
-        float v = slot ? c : (first ? pv[axis] : FLT_MAX);
-        int id = slot ? P + lane : (first ? pid[axis] : 0x7FFFFFFF);
-        // the smallest pair of lanes 0-7 (prefix minima within the first row)
-        argmin_dpp<0x111, 0xf>(v, id);
-        argmin_dpp<0x112, 0xf>(v, id);
-        argmin_dpp<0x114, 0xf>(v, id);
-        v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 7));
-        id = __builtin_amdgcn_readlane(id, 7);
-        if (id != 0x7FFFFFFF && v < FLT_MAX) {
-            const int t = id - P;  // an extreme slot won: the row it holds
-            const int held = (t >= 0 && t < NOBJ) ? __builtin_amdgcn_readlane(cur, t) : NOBJ + axis;
-            if (lane == axis) cur = held;
+        const bool slot = lane < NOBJ, first = lane == NOBJ + axis;
+        const float v = slot ? c[axis] : (first ? pv : FLT_MAX);
+        // lanes 0-5 and 6-11 lie in one DPP row: its smallest value in lane 15
+        float m = v;
+        m = fminf(m, dpp_f32<0x111, 0xf>(m, FLT_MAX));
+        m = fminf(m, dpp_f32<0x112, 0xf>(m, FLT_MAX));
+        m = fminf(m, dpp_f32<0x114, 0xf>(m, FLT_MAX));
+        m = fminf(m, dpp_f32<0x118, 0xf>(m, FLT_MAX));
+        m = lane_of(m, 15);
+        if (!(m < FLT_MAX)) continue;
+        const uint64_t at = __ballot(v == m && (slot || (first && pid != 0x7FFFFFFF)));
+        const int win = (at >> (NOBJ + axis)) & 1ull ? NOBJ + axis : (int)__builtin_ctzll(at);
+        const int held = __builtin_amdgcn_readlane(cur, win);
+        if (lane == axis) cur = held;
+#pragma unroll
+        for (int k = axis + 1; k < NOBJ; ++k) {
+            const float o = lane_of(c[k], win);
+            if (lane == axis) c[k] = o;
         }
     }
     return cur;
@@ -1937,9 +1904,6 @@ __device__ int settle_extremes(const float *pv, const int *pid, const float (*ca
 // the pivot row with v_readlane; every element takes the same operations in
 // the same order as the row-by-row elimination, so the solution is the same
 // to the bit.  Returns x[lane] in lanes 0-5.
-__device__ __forceinline__ float lane_of(float v, int l) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
 __device__ float gauss_wave(const float *E) {
     const int lane = threadIdx.x & 63;
     const bool row_lane = lane < NOBJ;
@@ -2066,65 +2030,19 @@ __global__ __launch_bounds__(FRONT0_THREADS) void k_front0(const DevJob *__restr
     if (tid == 0 && s_cnt) atomicAdd(&acc->f0, s_cnt);
 }
 
-// One workgroup per job, after k_front0: the selection up to the niching.
-//  * Further fronts while fewer than N designs are ranked (nonDominatedSorting's
-//    peeling, sorting.cuh:1026-1086).
-//  * The extreme points settled against the previous ones and the nadir point
-//    (updateNadirValue_HYP with the MNDF fallback, sorting.cuh:911-972), each
-//    by one wave.
-//  * The survivors of the fronts before the last one, and cleared niche
-//    arrays for k_associate.
-__global__ __launch_bounds__(1024) void k_fronts(const DevJob *__restrict__ jobs) {
-    const DevJob &J = jobs[blockIdx.x];
-    const int P = J.P, W = J.W, N = J.N, R = J.R;
-    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wid = tid >> 6;
-    // the descriptor fields first, held in scalar registers, then every
-    // load of the set-up at once
-    SelState *st = J.st;
-    const SelAcc *acc = J.acc;
-    const uint64_t *rk = J.ranked;
-    const float *o0 = J.obj[0], *o1 = J.obj[1];
-    asm volatile("" : "+s"(st), "+s"(acc), "+s"(rk), "+s"(o0), "+s"(o1));
-    const uint32_t g0 = gload(&st->gen);
-    __shared__ uint64_t ranked[MAX_W], newm[MAX_W], lastm[MAX_W];
-    __shared__ int s_cnt, s_new;
-    __shared__ float ext[NOBJ * NOBJ], ideal[NOBJ], worst[NOBJ], f0max[NOBJ];
-    __shared__ float pv[NOBJ], crow[2 * NOBJ][NOBJ], casf[2 * NOBJ][NOBJ];
-    __shared__ int pid[NOBJ];
-    if (tid < NOBJ) {
-        ideal[tid] = ord_float(gload(acc->lo + tid));
-        worst[tid] = ord_float(gload(acc->hi + tid));
-        f0max[tid] = ord_float(gload(acc->f0hi + tid));
-        const unsigned long long k = gload(acc->asf + tid);
-        pv[tid] = k == ~0ull ? FLT_MAX : ord_float((uint32_t)(k >> 32));
-        pid[tid] = k == ~0ull ? 0x7FFFFFFF : (int)(uint32_t)k;
-    }
-    if (tid < NOBJ * NOBJ) ext[tid] = gload(st->ext + tid);
-    if (tid == 0) {
-        s_cnt = gload(&acc->f0);
-        s_new = 0;
-    }
-    const float *const obj = (g0 & 1u) ? o0 : o1;  // buffer (gen + 1) & 1
-    for (int w = tid; w < W; w += NT) {
-        const uint64_t f0w = gload(rk + w);
-        ranked[w] = f0w;
-        lastm[w] = f0w;
-        newm[w] = 0;
-    }
-    __syncthreads();
-    // candidate rows of the extremes (below): the current extreme points and
-    // the rows of the first front's ASF minima, loaded now so that the loads
-    // overlap the peeling
-    float crv = 0.f;
-    if (tid < 2 * NOBJ * NOBJ) {
-        const int c = tid / NOBJ, k = tid % NOBJ;
-        if (c < NOBJ)
-            crv = ext[c * NOBJ + k];
-        else if (pid[c - NOBJ] < P)
-            crv = gload(obj + (size_t)pid[c - NOBJ] * NOBJ + k);
-    }
-    int f = 0, last_size = s_cnt;
-    while (s_cnt < N) {
+// Further fronts while fewer than N designs are ranked (nonDominatedSorting's
+// peeling, sorting.cuh:1026-1086), by a whole workgroup.  `ranked` and `lastm`
+// hold the first front's words and *s_cnt its size on entry, `newm` zeros and
+// *s_new zero; on return `ranked` and *s_cnt cover every front, `lastm` is the
+// last one.  Returns its index; last_size its size.  front_of is stored when
+// `store` is set (one workgroup a job).
+__device__ int peel_fronts(const DevJob &J, bool store, uint64_t *ranked, uint64_t *newm, uint64_t *lastm, int *s_cnt,
+                           int *s_new, int &last_size) {
+    const int P = J.P, W = J.W, N = J.N;
+    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63;
+    int f = 0;
+    last_size = *s_cnt;
+    while (*s_cnt < N) {
         ++f;
         // a design joins front f when all its dominators are ranked
         int c = 0;
@@ -2137,20 +2055,20 @@ __global__ __launch_bounds__(1024) void k_fronts(const DevJob *__restrict__ jobs
                 joins = !any;
             }
             const uint64_t b = __ballot(joins);
-            if (joins) gstore(J.front_of + r, f);
+            if (joins && store) gstore(J.front_of + r, f);
             if (lane == 0 && b) newm[r >> 6] = b;
             c += __popcll(b);
         }
-        if (lane == 0) atomicAdd(&s_new, c);
+        if (lane == 0) atomicAdd(s_new, c);
         __syncthreads();
-        if (s_new == 0) {  // a dominance cycle: every remaining design forms the front
+        if (*s_new == 0) {  // a dominance cycle: every remaining design forms the front
             for (int r = tid; r < P; r += NT)
                 if (!((ranked[r >> 6] >> (r & 63)) & 1ull)) {
                     atomicOr((unsigned long long *)&newm[r >> 6], 1ull << (r & 63));
-                    J.front_of[r] = f;
+                    if (store) gstore(J.front_of + r, f);
                 }
             __syncthreads();
-            if (tid == 0) s_new = P - s_cnt;
+            if (tid == 0) *s_new = P - *s_cnt;
             __syncthreads();
         }
         for (int w = tid; w < W; w += NT) {
@@ -2158,80 +2076,155 @@ __global__ __launch_bounds__(1024) void k_fronts(const DevJob *__restrict__ jobs
             ranked[w] |= newm[w];
             newm[w] = 0;
         }
-        last_size = s_new;
+        last_size = *s_new;
         __syncthreads();
         if (tid == 0) {
-            s_cnt += s_new;
-            s_new = 0;
+            *s_cnt += *s_new;
+            *s_new = 0;
         }
         __syncthreads();
     }
+    return f;
+}
+
+// What the extreme points and the nadir are settled from, in LDS.
+struct SettleShared {
+    float ideal[NOBJ], worst[NOBJ], f0max[NOBJ];  // pool extrema, first front's maxima
+    float pv[NOBJ];                               // per axis the first front's smallest ASF value
+    int pid[NOBJ];                                // and its design (0x7FFFFFFF: none)
+    float crow[2 * NOBJ][NOBJ];                   // candidate rows of the extremes
+    float ext[NOBJ * NOBJ], nadir[NOBJ];
+};
+
+// Orders a wave's LDS writes before its own later reads (other lanes' values).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// The extreme points settled against the previous ones (prev: lane i < 36
+// holds value i of them) and the nadir point (updateNadirValue_HYP with the
+// MNDF fallback, sorting.cuh:911-972), by one wave; stored to `out` with the
+// front counts when out is not null.
+__device__ void settle_nadir(SettleShared &S, const float *obj, int P, float prev, SelRes *out, int ranked_n, int f,
+                             int last_size, bool n_cut) {
+    const int lane = threadIdx.x & 63;
+    // the candidate rows: the current extreme points and the rows of the first
+    // front's ASF minima; lane t (0-11) takes row t's ASF values for every axis
+    if (lane < NOBJ * NOBJ) {
+        const int c = lane / NOBJ, k = lane % NOBJ, p = S.pid[c];
+        S.crow[c][k] = prev;
+        S.crow[NOBJ + c][k] = p < P ? gload(obj + (size_t)p * NOBJ + k) : 0.f;
+    }
+    wave_lds_sync();
+    const int row = min(lane, 2 * NOBJ - 1), ax = row >= NOBJ ? row - NOBJ : 0;
+    float a[NOBJ];
+    asf_all(S.crow[row], S.ideal, a);
+    const int held = settle_extremes(a, S.pv[ax], S.pid[ax]);
+    const int mine = __shfl(held, lane < NOBJ * NOBJ ? lane / NOBJ : 0, 64);
+    if (lane < NOBJ * NOBJ) S.ext[lane] = S.crow[mine][lane % NOBJ];
+    wave_lds_sync();
+    const float x = gauss_wave(S.ext);  // x[lane], lanes 0-5
+    float xs[NOBJ];
+#pragma unroll
+    for (int i = 0; i < NOBJ; ++i) xs[i] = lane_of(x, i);
+    // residuals of every extreme and the intercepts (a lane each)
+    bool exc = false;
+    float icpt = 0.f;
+    if (lane < NOBJ) {
+        float res = 0.f;
+#pragma unroll
+        for (int i = 0; i < NOBJ; ++i) res += xs[i] * (S.ext[lane * NOBJ + i] - S.ideal[i]);
+        if (fabsf(res - 1.f) > F_PRECISION || isnan(res) || isinf(res)) exc = true;
+        icpt = 1.f / x;
+        if (icpt <= F_PRECISION || isnan(icpt) || isinf(icpt)) exc = true;
+    }
+    const bool hyp = __ballot(exc) != 0;
+    if (lane < NOBJ) {
+        const float lo = S.ideal[lane], hi = S.f0max[lane];
+        const float nad = hyp ? (((hi - lo) > F_PRECISION) ? hi : S.worst[lane]) : lo + icpt;
+        S.nadir[lane] = nad;
+        if (out) {
+            gstore(&out->ideal[lane], lo);
+            gstore(&out->worst[lane], S.worst[lane]);
+            gstore(&out->nadir[lane], nad);
+        }
+    }
+    if (out) {
+        if (lane < NOBJ * NOBJ) gstore(&out->ext[lane], S.ext[lane]);
+        if (lane == 0) {
+            gstore(&out->hyp, (int32_t)hyp);
+            gstore(&out->ranked, ranked_n);
+            gstore(&out->last, f);
+            gstore(&out->base, (f == 0) ? 0 : ranked_n - last_size);
+            gstore(&out->n_cut, (int32_t)n_cut);
+        }
+    }
+}
+
+// One workgroup per job, after k_front0: the selection up to the niching of
+// jobs that k_front_associate does not take.
+//  * Further fronts while fewer than N designs are ranked.
+//  * The extreme points settled against the previous ones and the nadir point,
+//    by one wave.
+//  * The survivors of the fronts before the last one.
+__global__ __launch_bounds__(1024) void k_fronts(const DevJob *__restrict__ jobs) {
+    const DevJob &J = jobs[blockIdx.x];
+    const int P = J.P, W = J.W, N = J.N;
+    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wid = tid >> 6;
+    // the descriptor fields first, held in scalar registers, then every
+    // load of the set-up at once
+    SelState *st = J.st;
+    const SelAcc *acc = J.acc;
+    const uint64_t *rk = J.ranked;
+    const float *o0 = J.obj[0], *o1 = J.obj[1];
+    asm volatile("" : "+s"(st), "+s"(acc), "+s"(rk), "+s"(o0), "+s"(o1));
+    const uint32_t g0 = gload(&st->gen);
+    __shared__ uint64_t ranked[MAX_W], newm[MAX_W], lastm[MAX_W];
+    __shared__ int s_cnt, s_new;
+    __shared__ SettleShared S;
+    const int ei = min(lane, NOBJ * NOBJ - 1);
+    const float e0 = gload(st->res[0].ext + ei), e1 = gload(st->res[1].ext + ei);
+    if (tid < NOBJ) {
+        S.ideal[tid] = ord_float(gload(acc->lo + tid));
+        S.worst[tid] = ord_float(gload(acc->hi + tid));
+        S.f0max[tid] = ord_float(gload(acc->f0hi + tid));
+        const unsigned long long k = gload(acc->asf + tid);
+        S.pv[tid] = k == ~0ull ? FLT_MAX : ord_float((uint32_t)(k >> 32));
+        S.pid[tid] = k == ~0ull ? 0x7FFFFFFF : (int)(uint32_t)k;
+    }
+    if (tid == 0) {
+        s_cnt = gload(&acc->f0);
+        s_new = 0;
+    }
+    const uint32_t gen = __builtin_amdgcn_readfirstlane(g0);
+    const float *const obj = (gen & 1u) ? o0 : o1;  // buffer (gen + 1) & 1
+    for (int w = tid; w < W; w += NT) {
+        const uint64_t f0w = gload(rk + w);
+        ranked[w] = f0w;
+        lastm[w] = f0w;
+        newm[w] = 0;
+    }
+    __syncthreads();
+    int last_size;
+    const int f = peel_fronts(J, true, ranked, newm, lastm, &s_cnt, &s_new, last_size);
     const int ranked_n = s_cnt;
     const bool n_cut = ranked_n == N;
     // survivors so far: every ranked design when the fronts fill N exactly,
     // else the fronts before the last one
     if (J.selm)
         for (int w = tid; w < W; w += NT) gstore(J.selm + w, n_cut ? ranked[w] : (ranked[w] & ~lastm[w]));
-    if (J.niche && !n_cut) {  // k_associate counts into these
-        const NicheView g = niche_view(J.niche, R);
-        for (int r = tid; r < R; r += NT) {
-            g.cr[r] = make_int2(0, 0);
-            gstore(g.fill + r, 0);
-            gstore(g.nearest + r, ~0ull);
-        }
-    }
-    // the candidate rows of the extremes and their ASF values for every axis
-    if (tid < 2 * NOBJ * NOBJ) crow[tid / NOBJ][tid % NOBJ] = crv;
-    __syncthreads();
-    if (tid < 2 * NOBJ * NOBJ) casf[tid / NOBJ][tid % NOBJ] = asf(crow[tid / NOBJ], ideal, tid % NOBJ);
-    __syncthreads();
-    if (wid == 0) {
-        const int held = settle_extremes(pv, pid, casf, P);
-        const int mine = __shfl(held, lane < NOBJ * NOBJ ? lane / NOBJ : 0, 64);
-        if (lane < NOBJ * NOBJ) ext[lane] = crow[mine][lane % NOBJ];
-    }
-    __syncthreads();
-    if (wid == 0) {
-        const float x = gauss_wave(ext);  // x[lane], lanes 0-5
-        float xs[NOBJ];
-#pragma unroll
-        for (int i = 0; i < NOBJ; ++i) xs[i] = lane_of(x, i);
-        // residuals of every extreme and the intercepts (a lane each)
-        bool exc = false;
-        float icpt = 0.f;
-        if (lane < NOBJ) {
-            float res = 0.f;
-#pragma unroll
-            for (int i = 0; i < NOBJ; ++i) res += xs[i] * (ext[lane * NOBJ + i] - ideal[i]);
-            if (fabsf(res - 1.f) > F_PRECISION || isnan(res) || isinf(res)) exc = true;
-            icpt = 1.f / x;
-            if (icpt <= F_PRECISION || isnan(icpt) || isinf(icpt)) exc = true;
-        }
-        const bool hyp = __ballot(exc) != 0;
-        if (lane < NOBJ) {
-            st->ideal[lane] = ideal[lane];
-            st->worst[lane] = worst[lane];
-            st->nadir[lane] = hyp ? (((f0max[lane] - ideal[lane]) > F_PRECISION) ? f0max[lane] : worst[lane])
-                                  : ideal[lane] + icpt;
-        }
-        if (lane < NOBJ * NOBJ) st->ext[lane] = ext[lane];
-        if (lane == 0) {
-            st->hyp = hyp;
-            st->ranked = ranked_n;
-            st->last = f;
-            st->base = (f == 0) ? 0 : ranked_n - last_size;
-            st->n_cut = n_cut;
-        }
-    }
+    if (wid == 0)
+        settle_nadir(S, obj, P, (gen & 1u) ? e1 : e0, st->res + ((gen + 1u) & 1u), ranked_n, f, last_size, n_cut);
 }
 
-__device__ __forceinline__ float perp_dist(const float *f, const float *w) {  // utils.cuh:1149-1171
-    float num = 0.f, den = 0.f;
+// The squared perpendicular distance of f to a reference line, w its weights
+// and den the sum of their squares (utils.cuh:1149-1171 before its root).
+__device__ __forceinline__ float perp_dist2(const float *f, const float *w, float den) {
+    float num = 0.f;
 #pragma unroll
-    for (int i = 0; i < NOBJ; ++i) {
-        num += w[i] * f[i];
-        den += w[i] * w[i];
-    }
+    for (int i = 0; i < NOBJ; ++i) num += w[i] * f[i];
     const float k = num / den;
     float d = 0.f;
 #pragma unroll
@@ -2239,7 +2232,36 @@ __device__ __forceinline__ float perp_dist(const float *f, const float *w) {  //
         const float t = k * w[i] - f[i];
         d += t * t;
     }
-    return sqrtf(d);
+    return d;
+}
+
+// The nearest of the reference lines r = sub, sub + LPD, ... below R: the
+// smallest distance (the root of perp_dist2), ties to the lowest index, as a
+// sweep that takes every strictly smaller root finds it; best stays FLT_MAX
+// when no root is below it.  The root is taken once, of the line kept: a
+// smaller square has a smaller or equal root, and the roots of two squares
+// can only be equal when the squares are within two parts in 2^23, so a
+// square below the kept one by more than one part in 2^20 replaces it at
+// once and the rare one between compares the roots themselves.
+template <int LPD>
+__device__ __forceinline__ void nearest_line(const float *f, const float *refpts, int R, int sub, float &best, int &br) {
+    float b2 = __builtin_inff();
+    br = 0;
+    for (int r = sub; r < R; r += LPD) {
+        const f32x4 *q = (const f32x4 *)(refpts + (size_t)r * REF_STRIDE);
+        const f32x4 a = gload(q), b = gload(q + 1);
+        const float w[NOBJ] = {a.x, a.y, a.z, a.w, b.x, b.y};
+        const float d2 = perp_dist2(f, w, b.z);
+        bool take = d2 < b2 * 0.99999905f;  // 1 - 2^-20
+        if (d2 < b2 && !take) take = sqrtf(d2) < sqrtf(b2);
+        b2 = take ? d2 : b2;
+        br = take ? r : br;
+    }
+    best = sqrtf(b2);
+    if (!(best < FLT_MAX)) {
+        best = FLT_MAX;
+        br = 0;
+    }
 }
 
 __device__ __forceinline__ uint64_t niche_prio(const DevJob &J, uint32_t gen, int d) {
@@ -2248,58 +2270,30 @@ __device__ __forceinline__ uint64_t niche_prio(const DevJob &J, uint32_t gen, in
     return ((uint64_t)r[0] << 32) | (uint32_t)d;
 }
 
-// Nearest reference line of every ranked design (sorting.cuh:1105-1180):
-// LPD lanes per design (a wave, or eight lanes), D designs a workgroup (item
-// = (job, first design)); the lanes of a design take reference lines
-// r = sub, sub + LPD, ... and keep the smallest distance, ties to the lowest
-// index (the first minimum of a sweep in index order).  The niche arrays are
-// folded in with atomics: designs of the fronts before the last count toward
-// their niche, those of the last front toward its bucket, with the bucket's
-// nearest design as a 64-bit (distance, design) minimum.  A distance is never
-// NaN or above FLT_MAX: the sweep starts at FLT_MAX and takes only smaller
-// values.
-template <int D, int LPD>
-__global__ __launch_bounds__(D * LPD) void k_associate(const DevJob *__restrict__ jobs,
-                                                       const int2 *__restrict__ items) {
-    static_assert(LPD == 64 || LPD == 8, "a wave or eight lanes per design");
-    const int2 it = items[blockIdx.x];
-    const DevJob &J = jobs[it.x];
-    const int sub = (int)threadIdx.x % LPD, R = J.R, P = J.P;
-    const SelState *st = J.st;
-    const float *const refpts = J.refpts;
-    // everything the wave reads before its first store, loaded together: the
-    // selection state, the design's front and objectives (at a clamped index)
-    const int n_cut = gload(&st->n_cut), last = gload(&st->last);
-    const uint32_t gen = gload(&st->gen);
-    float ideal[NOBJ], nadir[NOBJ];
-#pragma unroll
-    for (int k = 0; k < NOBJ; ++k) {
-        ideal[k] = gload(&st->ideal[k]);
-        nadir[k] = gload(&st->nadir[k]);
-    }
-    const int d = it.y + (int)threadIdx.x / LPD, dc = min(d, P - 1);
-    // the row in 8-byte words (rows are 24 bytes), each feeding two objectives,
-    // so that the loads stay ahead of the per-objective branches
-    const f32x2 *o2 = (const f32x2 *)(pool_obj(J, gen) + (size_t)dc * NOBJ);
-    const f32x2 x01 = gload(o2), x23 = gload(o2 + 1), x45 = gload(o2 + 2);
-    const int fr = gload(J.front_of + dc);
-    const float x[NOBJ] = {x01.x, x01.y, x23.x, x23.y, x45.x, x45.y};
-    float f[NOBJ];
+// A design's row normalised by the ideal and nadir points (a zero range maps to 0).
+__device__ __forceinline__ void normalise_row(const float *x, const float *ideal, const float *nadir, float *f) {
 #pragma unroll
     for (int k = 0; k < NOBJ; ++k) {
         const float den = nadir[k] - ideal[k];
         f[k] = (den == 0.f) ? 0.f : (x[k] - ideal[k]) / den;
     }
-    if (n_cut || d >= P || fr < 0) return;  // no niching, or no ranked design (all the design's lanes)
-    float best = FLT_MAX;
-    int br = 0;
-    for (int r = sub; r < R; r += LPD) {
-        const float dd = perp_dist(f, refpts + (size_t)r * NOBJ);
-        if (dd < best) {
-            best = dd;
-            br = r;
-        }
-    }
+}
+
+// Association of one ranked design d (row x) by its LPD lanes (sub 0 .. LPD -
+// 1), every lane of the wave or none of a design's lanes taking part:
+// its nearest reference line (sorting.cuh:1105-1180), ties to the lowest
+// index (the first minimum of a sweep in index order).  The niche arrays are
+// folded in with atomics: designs of the fronts before the last count toward
+// their niche, those of the last front toward its bucket, with the bucket's
+// nearest design as a 64-bit (distance, design) minimum.  A distance is never
+// NaN or above FLT_MAX.
+template <int LPD>
+__device__ __forceinline__ void associate_design(const DevJob &J, uint32_t gen, int d, int sub, const float *f,
+                                                 bool is_last) {
+    const int R = J.R;
+    float best;
+    int br;
+    nearest_line<LPD>(f, J.refpts, R, sub, best, br);
     bool writer;
     if (LPD == 64) {
         wave_argmin(best, br);  // (every lane of the wave is here: one design a wave)
@@ -2315,17 +2309,208 @@ __global__ __launch_bounds__(D * LPD) void k_associate(const DevJob *__restrict_
         writer = sub == 7;
     }
     if (writer) {
-        J.ref_of[d] = br;
-        J.dist[d] = best;
+        gstore(J.ref_of + d, br);
         const NicheView g = niche_view(J.niche, R);
-        if (fr < last) {
+        if (!is_last) {
             atomicAdd(&g.cr[br].x, 1);
         } else {
             atomicAdd(&g.cr[br].y, 1);
             atomicMin(g.nearest + br, asf_key(best, d));
-            J.prio[d] = (uint32_t)(niche_prio(J, gen, d) >> 32);
+            gstore(J.prio + d, (uint32_t)(niche_prio(J, gen, d) >> 32));
         }
     }
+}
+
+// Nearest reference line of every ranked design: LPD lanes per design (a
+// wave, or eight lanes), D designs a workgroup (item = (job, first design)).
+template <int D, int LPD>
+__global__ __launch_bounds__(D * LPD) void k_associate(const DevJob *__restrict__ jobs,
+                                                       const int2 *__restrict__ items) {
+    static_assert(LPD == 64 || LPD == 8, "a wave or eight lanes per design");
+    const int2 it = items[blockIdx.x];
+    const DevJob &J = jobs[it.x];
+    const int sub = (int)threadIdx.x % LPD, P = J.P;
+    const SelState *st = J.st;
+    // everything the wave reads before its first store, loaded together: the
+    // selection's result, the design's front and objectives (at a clamped index)
+    const uint32_t gen = __builtin_amdgcn_readfirstlane(gload(&st->gen));
+    const SelRes *res = st->res + ((gen + 1u) & 1u);
+    const int n_cut = gload(&res->n_cut), last = gload(&res->last);
+    float ideal[NOBJ], nadir[NOBJ];
+#pragma unroll
+    for (int k = 0; k < NOBJ; ++k) {
+        ideal[k] = gload(&res->ideal[k]);
+        nadir[k] = gload(&res->nadir[k]);
+    }
+    const int d = it.y + (int)threadIdx.x / LPD, dc = min(d, P - 1);
+    // the row in 8-byte words (rows are 24 bytes), each feeding two objectives,
+    // so that the loads stay ahead of the per-objective branches
+    const f32x2 *o2 = (const f32x2 *)(pool_obj(J, gen) + (size_t)dc * NOBJ);
+    const f32x2 x01 = gload(o2), x23 = gload(o2 + 1), x45 = gload(o2 + 2);
+    const int fr = gload(J.front_of + dc);
+    const float x[NOBJ] = {x01.x, x01.y, x23.x, x23.y, x45.x, x45.y};
+    float f[NOBJ];
+    normalise_row(x, ideal, nadir, f);
+    if (n_cut || d >= P || fr < 0) return;  // no niching, or no ranked design (all the design's lanes)
+    associate_design<LPD>(J, gen, d, sub, f, fr == last);
+}
+
+// k_front0, k_fronts and k_associate in one launch, for pools of at most
+// FUSED_POOL designs: D designs a workgroup as in k_associate, and every
+// workgroup of a job settles the job's selection itself -- the first front
+// from the dominator counts, its maxima and ASF minima, further fronts, the
+// extreme points and the nadir -- instead of reading it from two kernels
+// before.  The settling is a few microseconds of dependent steps whichever
+// workgroup runs it, so doing it side by side costs no time while the
+// workgroups fit the chip, and the two launches and their load rounds go.
+// The workgroup of the job's first designs stores the result (SelState::res
+// of the other parity than the one read, front_of, the survivors so far).
+// Measured for the 100-residue job (pool 256, 4 designs a workgroup): 53.7 ->
+// 50.4 us a generation; 1237-residue job (pool 1554, 8): 94.8 -> 93.4; 500-
+// residue job (pool 2048, 8): 78.8 -> 78.2.  Of its 11.4 us there, the first
+// front takes 2.7, its reductions 2.3, the extremes and the nadir 3.3, the
+// association 1.7.
+template <int D, int LPD>
+__global__ __launch_bounds__(D * LPD) void k_front_associate(const DevJob *__restrict__ jobs,
+                                                             const int2 *__restrict__ items) {
+    constexpr int NT = D * LPD, NW = NT / 64, MW = FUSED_POOL / 64;
+    __shared__ uint64_t ranked[MW], newm[MW], lastm[MW];
+    __shared__ int s_cnt, s_new;
+    __shared__ SettleShared S;
+    __shared__ float red_m[NW][NOBJ], red_v[NW][NOBJ];
+    __shared__ int red_i[NW][NOBJ], red_c[NW];
+    const int2 it = items[blockIdx.x];
+    const DevJob &J = jobs[it.x];
+    // the descriptor fields held in scalar registers, then the loads that
+    // wait for nothing else
+    SelState *st = J.st;
+    const SelAcc *acc = J.acc;
+    const int32_t *np = J.np;
+    const float *o0 = J.obj[0], *o1 = J.obj[1];
+    int32_t *front_of = J.front_of;
+    int P = J.P, W = J.W, N = J.N;
+    asm volatile("" : "+s"(st), "+s"(acc), "+s"(np), "+s"(o0), "+s"(o1), "+s"(front_of), "+s"(P), "+s"(W), "+s"(N));
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, sub = tid % LPD;
+    const bool first = it.y == 0;  // the workgroup that stores the job's selection
+    const uint32_t g0 = gload(&st->gen);
+    float ideal[NOBJ];
+#pragma unroll
+    for (int k = 0; k < NOBJ; ++k) ideal[k] = ord_float(gload(acc->lo + k));
+    const uint32_t hi = gload(acc->hi + min(lane, NOBJ - 1));
+    const int ei = min(lane, NOBJ * NOBJ - 1);
+    const float e0 = gload(st->res[0].ext + ei), e1 = gload(st->res[1].ext + ei);
+    const uint32_t gen = __builtin_amdgcn_readfirstlane(g0);
+    const float *const obj = (gen & 1u) ? o0 : o1;  // buffer (gen + 1) & 1
+    const f32x2 *const rows = (const f32x2 *)obj;
+    const int d = it.y + tid / LPD, dc = min(d, P - 1);
+    const f32x2 x01 = gload(rows + 3 * dc), x23 = gload(rows + 3 * dc + 1), x45 = gload(rows + 3 * dc + 2);
+    // the first front: its words, size, maxima (updateNadirValue_MNDF,
+    // sorting.cuh:685-884) and per-axis ASF minima, ties to the lowest index
+    // (findExtremePoints, sorting.cuh:601-683); a wave without one skips
+    float fm[NOBJ], bv[NOBJ];
+    int bi[NOBJ], cnt = 0;
+#pragma unroll
+    for (int k = 0; k < NOBJ; ++k) {
+        fm[k] = -FLT_MAX;
+        bv[k] = FLT_MAX;
+        bi[k] = 0x7FFFFFFF;
+    }
+    for (int c0 = 0; c0 < P; c0 += 2 * NT) {  // two designs a thread and round
+        int v[2];
+        f32x2 r[2][3];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int qc = min(c0 + u * NT + tid, P - 1);
+            v[u] = gload(np + qc);
+#pragma unroll
+            for (int h = 0; h < 3; ++h) r[u][h] = gload(rows + 3 * qc + h);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int q = c0 + u * NT + tid, w0 = (c0 + u * NT) / 64 + wid;  // a wave's designs are word w0
+            const bool f0 = q < P && v[u] == 0;
+            const uint64_t b = __ballot(f0);
+            if (first && q < P) gstore(front_of + q, f0 ? 0 : -1);
+            if (lane == 0 && w0 < W) {
+                ranked[w0] = b;
+                lastm[w0] = b;
+                newm[w0] = 0;
+            }
+            if (!b) continue;
+            cnt += (int)__popcll(b);
+            const float x[NOBJ] = {r[u][0].x, r[u][0].y, r[u][1].x, r[u][1].y, r[u][2].x, r[u][2].y};
+            float a[NOBJ];
+            asf_all(x, ideal, a);
+#pragma unroll
+            for (int k = 0; k < NOBJ; ++k) {
+                fm[k] = fmaxf(fm[k], f0 ? x[k] : -FLT_MAX);
+                const bool less = f0 && a[k] < bv[k];  // (designs rise: ties keep the first)
+                bv[k] = less ? a[k] : bv[k];
+                bi[k] = less ? q : bi[k];
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NOBJ; ++k) {
+        fm[k] = wave_max_f32(fm[k]);
+        wave_argmin(bv[k], bi[k]);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < NOBJ; ++k) {
+            red_m[wid][k] = fm[k];
+            red_v[wid][k] = bv[k];
+            red_i[wid][k] = bi[k];
+        }
+        red_c[wid] = cnt;
+    }
+    lds_barrier();
+    if (tid < NOBJ) {
+        float m = -FLT_MAX, v = FLT_MAX;
+        int id = 0x7FFFFFFF;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            m = fmaxf(m, red_m[w][tid]);
+            argmin_pair(v, id, red_v[w][tid], red_i[w][tid]);
+        }
+        S.f0max[tid] = m;
+        S.pv[tid] = v;
+        S.pid[tid] = id;
+        S.worst[tid] = ord_float(hi);
+        float lo = ideal[0];
+#pragma unroll
+        for (int k = 1; k < NOBJ; ++k) lo = tid == k ? ideal[k] : lo;
+        S.ideal[tid] = lo;
+    }
+    if (tid == 64) {  // (another wave than the reductions': NW is at least 4)
+        int c = 0;
+        for (int w = 0; w < NW; ++w) c += red_c[w];
+        s_cnt = c;
+        s_new = 0;
+    }
+    lds_barrier();
+    int last_size;
+    const int f = peel_fronts(J, first, ranked, newm, lastm, &s_cnt, &s_new, last_size);
+    const int ranked_n = s_cnt;
+    const bool n_cut = ranked_n == N;
+    // survivors so far: every ranked design when the fronts fill N exactly,
+    // else the fronts before the last one
+    if (first)
+        for (int w = tid; w < W; w += NT) gstore(J.selm + w, n_cut ? ranked[w] : (ranked[w] & ~lastm[w]));
+    else if (n_cut)
+        return;  // no niching
+    if (wid == 0)
+        settle_nadir(S, obj, P, (gen & 1u) ? e1 : e0, first ? st->res + ((gen + 1u) & 1u) : nullptr, ranked_n, f,
+                     last_size, n_cut);
+    if (n_cut) return;
+    lds_barrier();
+    const float x[NOBJ] = {x01.x, x01.y, x23.x, x23.y, x45.x, x45.y};
+    float nadir[NOBJ], fn[NOBJ];
+#pragma unroll
+    for (int k = 0; k < NOBJ; ++k) nadir[k] = S.nadir[k];
+    normalise_row(x, ideal, nadir, fn);
+    if (d >= P || !((ranked[d >> 6] >> (d & 63)) & 1ull)) return;  // no ranked design (all the design's lanes)
+    associate_design<LPD>(J, gen, d, sub, fn, (lastm[d >> 6] >> (d & 63)) & 1ull);
 }
 
 // The levels of referenceBasedSorting (sorting.cuh:1182-1279) in closed form,
@@ -2336,23 +2521,41 @@ __global__ __launch_bounds__(D * LPD) void k_associate(const DevJob *__restrict_
 // first eligible reference points in index order take one more.  Per
 // reference point: its picks, its level-0 pick (an empty niche takes its
 // nearest design, ties to the lowest index), and, for a bucket only part of
-// whose rest is taken (a cut bucket), its offset in the cut list.  Returns
-// the cut list's size.
-__device__ __forceinline__ int niche_levels(const DevJob &J, const int2 *cr, const unsigned long long *nearest,
-                                            int *kp, int *lvl0, int *coff) {
+// whose rest is taken (a cut bucket), its offset in the cut list, a multiple
+// of ALIGN (a power of two).  Returns the cut list's size.
+template <int ALIGN>
+__device__ __forceinline__ int niche_levels(const DevJob &J, int base, const int2 *cr,
+                                            const unsigned long long *nearest, int *kp, int *lvl0, int *coff) {
     const int P = J.P, N = J.N, R = J.R, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __shared__ int s_ncut;
     if (wid == 0) {
-        const int need = N - J.st->base;
+        const int need = N - base;
         // up to 256 reference points: four a lane, in registers
         const bool small = R <= 256;
         int2 rc[4];
+        unsigned long long nr[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const int r = lane + 64 * k;
-            rc[k] = small && r < R ? cr[r] : make_int2(0, 0);
+            const int r = min(lane + 64 * k, R - 1);
+            const bool in = small && lane + 64 * k < R;
+            rc[k] = cr[r];
+            nr[k] = nearest[r];
+            rc[k].x = in ? rc[k].x : 0;
+            rc[k].y = in ? rc[k].y : 0;
         }
-        int lo = -1, clo = 0, hi = P;  // C(lo) < need; C(hi) >= need or hi = P
+        // the bucket taken whole last bounds the final level: with hi its last
+        // level, C(hi) is every design of the last front, at least `need`
+        int top = 0;
+        if (small) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) top = max(top, rc[k].y ? rc[k].x + rc[k].y : 0);
+        } else {
+            for (int r = lane; r < R; r += 64) {
+                const int2 c = cr[r];
+                top = max(top, c.y ? c.x + c.y : 0);
+            }
+        }
+        int lo = -1, clo = 0, hi = min(P, max(wave_max_nonneg(top) - 1, 0));  // C(lo) < need; C(hi) >= need or hi = P
         while (hi - lo > 1) {
             const int mid = lo + ((hi - lo) >> 1);
             int acc = 0;
@@ -2375,9 +2578,9 @@ __device__ __forceinline__ int niche_levels(const DevJob &J, const int2 *cr, con
         }
         const int istar = hi, need_final = need - clo;
         int carry = 0, cut_carry = 0;
-        for (int r0 = 0; r0 < R; r0 += 64) {
+        // 64 reference points r = r0 + lane with their counts and nearest design
+        auto settle = [&](int r0, int2 c, unsigned long long near) {
             const int r = r0 + lane;
-            const int2 c = r < R ? cr[r] : make_int2(0, 0);
             const bool e = r < R && c.x <= istar && istar < c.x + c.y;
             const uint64_t eb = __ballot(e);
             const int ex = carry + (int)__popcll(eb & ((1ull << lane) - 1ull));
@@ -2386,17 +2589,28 @@ __device__ __forceinline__ int niche_levels(const DevJob &J, const int2 *cr, con
             // lowest index (the reference's fallback to the lowest index, for a
             // NaN distance or none below FLT_MAX, never applies: every distance
             // is at most FLT_MAX and none is NaN)
-            const int l0 = (r < R && k > 0 && c.x == 0) ? (int)(uint32_t)nearest[r] : -1;
+            const int l0 = (r < R && k > 0 && c.x == 0) ? (int)(uint32_t)near : -1;
             const int h = l0 >= 0 ? 1 : 0;
             const int cut = (r < R && k - h > 0 && k - h < c.y - h) ? c.y : 0;
-            const int incl = wave_scan_i32(cut);  // inclusive prefix of the cut sizes over the wave
+            const int room = (cut + ALIGN - 1) & ~(ALIGN - 1);
+            const int incl = wave_scan_i32(room);  // inclusive prefix of the cut sizes over the wave
             if (r < R) {
                 kp[r] = k;
                 lvl0[r] = l0;
-                coff[r] = cut ? cut_carry + incl - cut : -1;
+                coff[r] = cut ? cut_carry + incl - room : -1;
             }
             carry += (int)__popcll(eb);
             cut_carry += __builtin_amdgcn_readlane(incl, 63);
+        };
+        if (small) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (64 * k < R) settle(64 * k, rc[k], nr[k]);
+        } else {
+            for (int r0 = 0; r0 < R; r0 += 64) {
+                const int r = min(r0 + lane, R - 1);
+                settle(r0, cr[r], nearest[r]);
+            }
         }
         if (lane == 0) s_ncut = cut_carry;
     }
@@ -2408,9 +2622,10 @@ __device__ __forceinline__ int niche_levels(const DevJob &J, const int2 *cr, con
 // NICHE_STAGE): one workgroup per job, on the arrays in global memory.
 __global__ __launch_bounds__(256) void k_levels(const DevJob *__restrict__ jobs) {
     const DevJob &J = jobs[blockIdx.x];
-    if (J.st->n_cut || J.R <= NICHE_STAGE) return;
+    const SelRes &res = J.st->res[(J.st->gen + 1u) & 1u];
+    if (res.n_cut || J.R <= NICHE_STAGE) return;
     const NicheView g = niche_view(J.niche, J.R);
-    const int ncut = niche_levels(J, g.cr, g.nearest, g.kp, g.lvl0, g.coff);
+    const int ncut = niche_levels<1>(J, res.base, g.cr, g.nearest, g.kp, g.lvl0, g.coff);
     if (threadIdx.x == 0) J.acc->ncut = ncut;
 }
 
@@ -2426,7 +2641,7 @@ __global__ __launch_bounds__(256) void k_levels(const DevJob *__restrict__ jobs)
 // one atomic (when R fits).
 __global__ __launch_bounds__(1024) void k_place(const DevJob *__restrict__ jobs) {
     const DevJob &J = jobs[blockIdx.x];
-    const SelState *st = J.st;
+    const SelRes *const st = J.st->res + ((J.st->gen + 1u) & 1u);
     const int P = J.P, R = J.R, NT = blockDim.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int d0 = blockIdx.y * NT;
     if (d0 >= P) return;
@@ -2449,7 +2664,7 @@ __global__ __launch_bounds__(1024) void k_place(const DevJob *__restrict__ jobs)
             l_cnt[r] = 0;
         }
         __syncthreads();
-        const int ncut = niche_levels(J, s_cr, s_near, s_kp, s_l0, s_co);
+        const int ncut = niche_levels<1>(J, st->base, s_cr, s_near, s_kp, s_l0, s_co);
         if (blockIdx.y == 0) {
             for (int r = tid; r < R; r += NT) {
                 gstore(g.kp + r, s_kp[r]);
@@ -2505,8 +2720,8 @@ __global__ __launch_bounds__(1024) void k_niche(const DevJob *__restrict__ jobs)
     const int R = J.R, NT = blockDim.x, tid = threadIdx.x;
     const int s0 = blockIdx.y * NT;
     if (blockIdx.y == 0 && tid == 0) st->gen = st->gen + 1u;
-    if (st->n_cut || s0 >= J.acc->ncut) return;
-    const int ncut = J.acc->ncut;
+    const int ncut = J.acc->ncut;  // 0 where the fronts filled N exactly
+    if (s0 >= ncut) return;
     const NicheView g = niche_view(J.niche, R);
     __shared__ int s_a, s_b;
     const int s = s0 + tid, sc = min(s, ncut - 1);
@@ -2540,12 +2755,18 @@ __global__ __launch_bounds__(1024) void k_niche(const DevJob *__restrict__ jobs)
 // PLACE_NICHE_POOL designs whose niche arrays fit in LDS (R <= NICHE_STAGE):
 // the levels settled in LDS, the designs of the last front placed (designs
 // d = tid, tid + NT, ...), the cut buckets' keys (priority, design) and
-// buckets kept in LDS (dynamic, 12 bytes a design of the pool) instead of the
+// buckets kept in LDS (dynamic, place_niche_lds_bytes) instead of the
 // global cut list, and the cut designs ranked within their buckets after one
 // barrier instead of a kernel boundary.  The same selection as k_place then
 // k_niche: a design is selected when it is its niche's level-0 pick, when
 // the rest of its bucket is taken whole, or when fewer than kk of the rest of
 // its cut bucket have a smaller key.  Ends the generation, as k_niche does.
+// The buckets' priorities are ranked four to an LDS read (the lanes of one
+// bucket read the same words), and the picks are folded in LDS and stored
+// once: with 64-bit keys read one at a time and an atomic on the survivor
+// mask per pick, the ranking of the 500-residue job's 1335 cut designs (44
+// buckets of up to 63) took 3.1 us, now 2.1, and a pool of 2048 with buckets
+// of hundreds 20.7 us in all.
 __global__ __launch_bounds__(1024) void k_place_niche(const DevJob *__restrict__ jobs) {
     extern __shared__ __align__(16) uint8_t dyn[];
     const DevJob &J = jobs[blockIdx.x];
@@ -2555,25 +2776,39 @@ __global__ __launch_bounds__(1024) void k_place_niche(const DevJob *__restrict__
     int32_t *niche = J.niche;
     const int32_t *front_of = J.front_of, *ref_of = J.ref_of;
     const uint32_t *prio = J.prio;
-    int P = J.P, R = J.R;
-    asm volatile("" : "+s"(st), "+s"(niche), "+s"(front_of), "+s"(ref_of), "+s"(prio), "+s"(P), "+s"(R));
-    const int NT = blockDim.x, tid = threadIdx.x, lane = tid & 63;
-    const int n_cut = gload(&st->n_cut), last = gload(&st->last);
-    int fo = gload(front_of + min(tid, P - 1)), rf = gload(ref_of + min(tid, P - 1));
-    uint32_t pr = gload(prio + min(tid, P - 1));
+    uint64_t *selm = J.selm;
+    int P = J.P, R = J.R, W = J.W;
+    asm volatile("" : "+s"(st), "+s"(niche), "+s"(front_of), "+s"(ref_of), "+s"(prio), "+s"(selm), "+s"(P), "+s"(R), "+s"(W));
+    const int NT = blockDim.x, tid = threadIdx.x;
+    // (both halves of the selection's results, the counter choosing one)
+    const uint32_t g0 = gload(&st->gen);
+    const int nc0 = gload(&st->res[0].n_cut), la0 = gload(&st->res[0].last), ba0 = gload(&st->res[0].base);
+    const int nc1 = gload(&st->res[1].n_cut), la1 = gload(&st->res[1].last), ba1 = gload(&st->res[1].base);
+    int fo[2], rf[2];
+    uint32_t pr[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int dc = min(tid + u * NT, P - 1);
+        fo[u] = gload(front_of + dc);
+        rf[u] = gload(ref_of + dc);
+        pr[u] = gload(prio + dc);
+    }
+    const uint64_t sm = gload(selm + min(tid, W - 1));
     // and the reference points' counts and nearest designs (first chunk)
     const NicheView g = niche_view(niche, R);
     const int rc0 = min(tid, R - 1);
     const uint64_t cr0 = gload((const uint64_t *)g.cr + rc0);  // int2 (x low, y high)
     const unsigned long long nn0 = gload(g.nearest + rc0);
-    if (tid == 0) st->gen = st->gen + 1u;  // (nothing here reads the generation count)
-    if (n_cut) return;
-    uint64_t *keys = (uint64_t *)dyn;          // [P] keys of the cut buckets' designs, bucket by bucket
-    int32_t *kbuck = (int32_t *)(keys + P);    // [P] the bucket of each key
+    const bool h1 = ((g0 + 1u) & 1u) != 0;
+    const int n_cut = h1 ? nc1 : nc0, last = h1 ? la1 : la0, base = h1 ? ba1 : ba0;
+    // the cut buckets' designs, bucket by bucket, each bucket in whole 16-byte
+    // words: priorities (pads hold ~0), and (bucket << 16 | design) (pads ~0)
+    uint32_t *const kpri = (uint32_t *)dyn, *const kwho = kpri + place_niche_slots(P, R);
     __shared__ int2 s_cr[NICHE_STAGE];
     __shared__ unsigned long long s_near[NICHE_STAGE];
     __shared__ int s_kp[NICHE_STAGE], s_l0[NICHE_STAGE], s_co[NICHE_STAGE], l_cnt[NICHE_STAGE];
     __shared__ uint32_t s_pl0[NICHE_STAGE];  // priority of each bucket's level-0 pick
+    __shared__ uint32_t s_sel[PLACE_NICHE_POOL / 32];  // the last front's picks, folded here and stored once
     if (tid < R) {
         s_cr[tid] = make_int2((int)(uint32_t)cr0, (int)(uint32_t)(cr0 >> 32));
         s_near[tid] = nn0;
@@ -2584,54 +2819,72 @@ __global__ __launch_bounds__(1024) void k_place_niche(const DevJob *__restrict__
         s_near[r] = gload(g.nearest + r);
         l_cnt[r] = 0;
     }
+    if (tid < PLACE_NICHE_POOL / 32) s_sel[tid] = 0u;
     __syncthreads();
-    const int ncut = niche_levels(J, s_cr, s_near, s_kp, s_l0, s_co);
+    if (tid == 0) gstore(&st->gen, g0 + 1u);  // (every thread has read the count)
+    if (n_cut) return;
+    const int ncut = niche_levels<4>(J, base, s_cr, s_near, s_kp, s_l0, s_co);  // (with the pads)
     for (int r = tid; r < R; r += NT) {
-        gstore(g.kp + r, s_kp[r]);
-        gstore(g.lvl0 + r, s_l0[r]);
-        gstore(g.coff + r, s_co[r]);
+        const int co = s_co[r], nr = s_cr[r].y;
+        if (co >= 0)
+            for (int i = nr; i & 3; ++i) kpri[co + i] = kwho[co + i] = ~0u;
     }
-    if (tid == 0) J.acc->ncut = ncut;
     // place the designs of the last front
-    for (int d0 = 0; d0 < P; d0 += NT) {
-        const int d = d0 + tid;
-        if (d0) {  // (the first designs' rows were loaded before the levels)
-            const int dc = min(d, P - 1);
-            fo = gload(front_of + dc);
-            rf = gload(ref_of + dc);
-            pr = gload(prio + dc);
-        }
-        const bool mine = d < P && fo == last;
-        bool sel = false;
-        if (mine) {
-            const int l0 = s_l0[rf], co = s_co[rf];
-            sel = d == l0;
-            if (sel) s_pl0[rf] = pr;  // (the level-0 pick is a last-front design of its bucket)
-            if (co >= 0) {
-                const int slot = co + atomicAdd(&l_cnt[rf], 1);
-                keys[slot] = ((uint64_t)pr << 32) | (uint32_t)d;
-                kbuck[slot] = rf;
-            } else if (!sel) {  // not cut: the rest of the bucket is taken whole, or nothing of it
-                sel = s_kp[rf] - (l0 >= 0 ? 1 : 0) > 0;
+    for (int d0 = 0; d0 < P; d0 += 2 * NT) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int d = d0 + u * NT + tid;
+            if (d0) {  // (the first designs' rows were loaded before the levels)
+                const int dc = min(d, P - 1);
+                fo[u] = gload(front_of + dc);
+                rf[u] = gload(ref_of + dc);
+                pr[u] = gload(prio + dc);
             }
+            if (d >= P || fo[u] != last) continue;
+            const int r = rf[u], l0 = s_l0[r], co = s_co[r], kr = s_kp[r];
+            bool sel = d == l0;
+            if (sel) s_pl0[r] = pr[u];  // (the level-0 pick is a last-front design of its bucket)
+            if (co >= 0) {
+                const int slot = co + atomicAdd(&l_cnt[r], 1);
+                kpri[slot] = pr[u];
+                kwho[slot] = ((uint32_t)r << 16) | (uint32_t)d;
+            } else if (!sel) {  // not cut: the rest of the bucket is taken whole, or nothing of it
+                sel = kr - (l0 >= 0 ? 1 : 0) > 0;
+            }
+            if (sel) atomicOr(&s_sel[d >> 5], 1u << (d & 31));
         }
-        const uint64_t b = __ballot(sel);  // a wave's 64 designs are one word of the mask
-        if (lane == 0 && b) atomicOr((unsigned long long *)J.selm + ((d0 + (tid & ~63)) >> 6), b);
     }
     __syncthreads();  // the cut buckets' keys are complete
-    // rank the designs of the cut buckets
+    // rank the designs of the cut buckets: the smaller priorities of a bucket
+    // counted four to an LDS read (the lanes of one bucket read the same
+    // words); equal priorities, one pair in 2^32, go by the design
     for (int sl = tid; sl < ncut; sl += NT) {
-        const uint64_t my = keys[sl];
-        const int r = kbuck[sl], d = (int)(uint32_t)my, l0 = s_l0[r];
-        if (d == l0) continue;
+        const uint32_t who = kwho[sl], my = kpri[sl];
+        if (who == ~0u) continue;
+        const int r = (int)(who >> 16), d = (int)(who & 0xFFFFu), l0 = s_l0[r];
         const int kk = s_kp[r] - (l0 >= 0 ? 1 : 0), off = s_co[r], nr = s_cr[r].y;
-        int rank = 0;
+        const uint32_t pl0 = s_pl0[r];
+        const u32x4 *kq = (const u32x4 *)(kpri + off);
+        int rank = 0, same = 0;
 #pragma unroll 4
-        for (int u = 0; u < nr; ++u) rank += (int)(keys[off + u] < my);
+        for (int i = 0; i < nr; i += 4) {
+            const u32x4 k = kq[i >> 2];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                rank += (int)(k[v] < my);
+                same += (int)(k[v] == my);
+            }
+        }
+        if (same > 1)
+            for (int i = 0; i < nr; ++i) rank += (int)(kpri[off + i] == my && kwho[off + i] < who);
+        if (d == l0) continue;
         // the level-0 pick of the bucket is not part of the rest
-        if (l0 >= 0 && ((((uint64_t)s_pl0[r]) << 32) | (uint32_t)l0) < my) --rank;
-        if (rank < kk) atomicOr((unsigned long long *)J.selm + (d >> 6), 1ull << (d & 63));
+        if (l0 >= 0 && (pl0 < my || (pl0 == my && l0 < d))) --rank;
+        if (rank < kk) atomicOr(&s_sel[d >> 5], 1u << (d & 31));
     }
+    __syncthreads();  // the picks are complete
+    // (pools of at most PLACE_NICHE_POOL designs: at most 32 words)
+    if (tid < W) gstore(selm + tid, sm | (uint64_t)s_sel[2 * tid] | ((uint64_t)s_sel[2 * tid + 1] << 32));
 }
 
 // Initial state after k_design<INIT>: the first N designs survive, extreme points
@@ -2644,13 +2897,23 @@ __global__ void k_init_state(const DevJob *__restrict__ jobs) {
         J.selm[w] = n >= 64 ? ~0ull : (n > 0 ? (1ull << n) - 1ull : 0ull);
     }
     for (int i = threadIdx.x; i < J.P; i += blockDim.x) J.front_of[i] = -1;
+    // (a job initialised again keeps the points of its last selection until
+    // the next one)
+    const uint32_t from = st->gen & 1u;
+    if (threadIdx.x < NOBJ && from) {
+        st->res[0].ideal[threadIdx.x] = st->res[1].ideal[threadIdx.x];
+        st->res[0].worst[threadIdx.x] = st->res[1].worst[threadIdx.x];
+        st->res[0].nadir[threadIdx.x] = st->res[1].nadir[threadIdx.x];
+    }
+    __syncthreads();
     if (threadIdx.x < NOBJ * NOBJ) {
         const int e = threadIdx.x / NOBJ, k = threadIdx.x % NOBJ;
-        st->ext[threadIdx.x] = (e < J.N) ? J.obj[0][(size_t)e * NOBJ + k] : 0.f;
+        st->res[0].ext[threadIdx.x] = (e < J.N) ? J.obj[0][(size_t)e * NOBJ + k] : 0.f;
     }
     if (threadIdx.x == 0) {
+        SelRes &r = st->res[0];
+        r.n_cut = r.hyp = r.ranked = r.last = r.base = 0;
         st->gen = 0;
-        st->n_cut = st->hyp = st->ranked = st->last = st->base = 0;
         st->cds_scanned = 0;
     }
 }
@@ -2662,6 +2925,7 @@ __global__ void k_zero_np(const DevJob *__restrict__ jobs) {
     const DevJob &J = jobs[blockIdx.x];
     for (int i = threadIdx.x; i < J.P; i += blockDim.x) J.np[i] = 0;
     if (threadIdx.x < ACC_WORDS) ((uint32_t *)J.acc)[threadIdx.x] = acc_clear_word(threadIdx.x);
+    if (J.niche) clear_niche(J, threadIdx.x, blockDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2761,6 +3025,18 @@ hipError_t launch_associate(const DevJob *jobs, const int2 *items, int n, int de
     }
     return hipGetLastError();
 }
+hipError_t launch_front_associate(const DevJob *jobs, const int2 *items, int n, int designs, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    switch (designs) {
+    case 4: hipLaunchKernelGGL((k_front_associate<4, 64>), dim3(n), dim3(256), 0, s, jobs, items); break;
+    case 8: hipLaunchKernelGGL((k_front_associate<8, 64>), dim3(n), dim3(512), 0, s, jobs, items); break;
+    case 16: hipLaunchKernelGGL((k_front_associate<16, 64>), dim3(n), dim3(1024), 0, s, jobs, items); break;
+    case 32: hipLaunchKernelGGL((k_front_associate<32, 8>), dim3(n), dim3(256), 0, s, jobs, items); break;
+    case 64: hipLaunchKernelGGL((k_front_associate<64, 8>), dim3(n), dim3(512), 0, s, jobs, items); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
 bool shapes_valid(const Shapes &h) {
     return h.design_split >= 0 && (h.design_threads == 256 || h.design_threads == 512) && h.stem_waves >= 5 &&
            h.stem_waves <= 8 &&
@@ -2790,7 +3066,10 @@ static size_t g_design_lds = 0, g_stem_lds = 0, g_niche_lds = 0;
 
 hipError_t set_niche_lds_limit(size_t bytes) {
     return raise_lds_limit(g_niche_lds, bytes, [](int b) {
-        return hipFuncSetAttribute((const void *)k_niche, hipFuncAttributeMaxDynamicSharedMemorySize, b);
+        const hipError_t e = hipFuncSetAttribute((const void *)k_niche, hipFuncAttributeMaxDynamicSharedMemorySize, b);
+        return e != hipSuccess ? e
+                               : hipFuncSetAttribute((const void *)k_place_niche,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, b);
     });
 }
 hipError_t launch_niche(const DevJob *jobs, int njobs, int max_pool, int max_refs, int threads, hipStream_t s) {
@@ -2802,7 +3081,7 @@ hipError_t launch_niche(const DevJob *jobs, int njobs, int max_pool, int max_ref
         if (e != hipSuccess) return e;
     }
     if (max_pool <= PLACE_NICHE_POOL && max_refs <= NICHE_STAGE) {  // one workgroup per job
-        hipLaunchKernelGGL(k_place_niche, dim3(njobs), dim3(threads), place_niche_lds_bytes(max_pool), s, jobs);
+        hipLaunchKernelGGL(k_place_niche, dim3(njobs), dim3(threads), place_niche_lds_bytes(max_pool, max_refs), s, jobs);
         return hipGetLastError();
     }
     const dim3 grid(njobs, (max_pool + threads - 1) / threads);

@@ -40,18 +40,27 @@ struct CdsStat {
 static_assert(sizeof(CdsStat) == 64, "CdsStat records move as four 16-byte words");
 
 // Selection state of one job (the reference keeps it in __device__ globals,
-// common.cuh:46-59).
-struct SelState {
-    uint32_t gen;      // generations completed
+// common.cuh:46-59).  What one selection hands on -- to the niching, to the
+// next selection (its extreme points) and to the caller -- is kept twice: the
+// selection of generation g reads the extremes of res[g & 1] and writes
+// res[(g + 1) & 1], so several workgroups may settle the same selection side
+// by side while one of them stores it.  Between generations res[gen & 1]
+// holds the latest selection.
+struct SelRes {
     int32_t n_cut;     // fronts filled N exactly (no niching)
     int32_t hyp;       // hyperplane exception (MNDF nadir)
     int32_t ranked;    // designs ranked
     int32_t last;      // index of the last (cut) front
     int32_t base;      // designs in fronts before the last
-    uint32_t pad;
-    unsigned long long cds_scanned;  // CDS whose objectives were recomputed (cumulative)
+    int32_t pad;
     float ext[NOBJ * NOBJ];
     float ideal[NOBJ], worst[NOBJ], nadir[NOBJ];
+};
+struct SelState {
+    uint32_t gen;      // generations completed
+    uint32_t pad;
+    unsigned long long cds_scanned;  // CDS whose objectives were recomputed (cumulative)
+    SelRes res[2];
 };
 
 // Per-generation accumulators of the selection, filled with atomics by the
@@ -106,6 +115,7 @@ __host__ __device__ inline NicheView niche_view(int32_t *base, int R) {
     v.nearest = (unsigned long long *)(base + 6 * R);
     return v;
 }
+constexpr int REF_STRIDE = 8;    // floats per reference point (two 16-byte words)
 constexpr int NICHE_STAGE = 1024;  // reference points whose niche arrays fit in a workgroup's LDS
 
 // Device view of one job.  Pools ping-pong on generation parity: generation
@@ -128,7 +138,7 @@ struct DevJob {
     const int64_t *lw6;    // [64] 2^40-scaled log weights by code
     const int64_t *cpfx6;  // [64*64] 2^40-scaled pair scores by codes (0 where either is a stop)
     const float *cps6;     // [64*64] pair scores by codes (0 where either is a stop)
-    const float *refpts;   // [R*6]
+    const float *refpts;   // [R][REF_STRIDE]: the point's six weights, the sum of their squares, 0
     int8_t *genome[2];     // [P][m][Ls] synonym indices, CDS rows padded with zeros to Ls
     float *obj[2];         // [P][6]
     int8_t *oidx[2];       // [P][12]

@@ -248,7 +248,7 @@ void collect_loop(cd_server *S) {
 hipError_t rebuild(cd_server *S, const std::vector<Entry *> &res) {
     std::vector<cd_job *> jobs;
     for (Entry *E : res) jobs.push_back(E->job);
-    cd::Shapes sh = cd::SHAPES_BATCH;  // the tuned shapes of this kind of resident set, if any
+    cd::Shapes sh = cdhost::untuned_shapes(jobs.data(), (int)jobs.size());  // or the tuned shapes of this kind of resident set, if any
     (void)cdhost::cached_shapes(cdhost::work_signature(jobs.data(), (int)jobs.size()), &sh);
     cdhost::WorkLists wl;
     cdhost::build_lists(jobs.data(), (int)jobs.size(), sh, wl);
@@ -268,7 +268,7 @@ hipError_t rebuild(cd_server *S, const std::vector<Entry *> &res) {
     const cdhost::Launch L{S->d_jobs,   (int)wl.descs.size(), S->d_off,      (int)wl.off.size(), S->d_dom,
                            (int)wl.dom.size(), S->d_asc,      (int)wl.asc.size(), wl.lds,         wl.stem_lds,
                            wl.max_pool,  wl.max_refs,        wl.mg,               wl.stem_parts,      S->d_slist,     S->d_sctl,
-                           wl.n_cds,     wl.n_small,          wl.lds_small,       sh};
+                           wl.n_cds,     wl.n_small,          wl.lds_small,       wl.pool,           sh};
     if (S->gexec) (void)hipGraphExecDestroy(S->gexec);
     if (S->graph) (void)hipGraphDestroy(S->graph);
     S->gexec = nullptr;
