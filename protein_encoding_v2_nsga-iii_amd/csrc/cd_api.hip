@@ -45,6 +45,7 @@ char translate(const uint8_t *c3) {  // codes A0 C1 G2 U3 -> index in U C A G or
 struct HostTables {
     uint8_t code[64];        // code of each codon of the table
     int64_t lw6[64];         // 2^40-scaled log weights
+    uint64_t syn6[64];       // synonym words (DevJob::lw6)
     int64_t cpfx6[64 * 64];  // 2^40-scaled pair scores, 0 where either codon is a stop
     float cps6[64 * 64];     // pair scores, 0 where either codon is a stop
     uint64_t stop6;          // bit per code: the table's last three codons
@@ -68,6 +69,12 @@ int build_tables(const cd_tables &t, HostTables &h) {
         seen |= 1ull << h.code[g];
     }
     if (seen != ~0ull) return fail(CD_E_INVALID, "codon table lists a codon twice");
+    for (int a = 0; a < 21; ++a)
+        for (int j = 0; j < SYN_NUM[a]; ++j) {
+            uint64_t v = ((uint64_t)SYN_NUM[a] << 40) | ((uint64_t)j << 44);
+            for (int i = 0; i < SYN_NUM[a]; ++i) v |= (uint64_t)h.code[SYN_START[a] + i] << (i < 5 ? 6 * i : 32);
+            h.syn6[h.code[SYN_START[a] + j]] = v;
+        }
     h.stop6 = 0;
     for (int g = 61; g < 64; ++g) h.stop6 |= 1ull << h.code[g];
     for (int g = 0; g < 64; ++g) {
@@ -159,7 +166,7 @@ Layout layout(int L, int m, int N, int P, int R, int W, int n_dom, int n_asc, bo
     if (!sel_only) {
         o.pos = s.add(2 * (size_t)cd::row_stride(L));
         o.code = s.add(64);
-        o.lw6 = s.add(64 * 8);
+        o.lw6 = s.add(128 * 8);
         o.cpfx6 = s.add(64 * 64 * 8);
         o.cps6 = s.add(64 * 64 * 4);
         for (int b = 0; b < 2; ++b) {
@@ -232,7 +239,7 @@ int validate(const cd_job_desc *d) {
         if ((d->aa[k] == 20) != (k == d->L - 1)) return fail(CD_E_INVALID, "the stop (20) must be exactly the last codon");
     }
     if (3LL * d->L >= (1 << 20)) return fail(CD_E_INVALID, "sequence too long for stem positions");
-    if (cd::design_lds_bytes(d->L, d->m) > cd::LDS_BYTES || cd::stem_list_lds(cd::stem_lds_bytes(d->L)) > cd::LDS_BYTES)
+    if (cd::design_bytes_accepted(d->L, d->m) > cd::LDS_BYTES || cd::stem_list_lds(cd::stem_lds_bytes(d->L)) > cd::LDS_BYTES)
         return fail(CD_E_INVALID, "m*L too large for one workgroup's LDS (160 KiB)");
     return CD_OK;
 }
@@ -355,6 +362,7 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
         }
         up.add(o.code, t.code, 64);
         up.add(o.lw6, t.lw6, 64);
+        up.add(o.lw6 + 64 * 8, t.syn6, 64);
         up.add(o.cpfx6, t.cpfx6, 64 * 64);
         up.add(o.cps6, t.cps6, 64 * 64);
         h.pos = (const uint8_t *)(base + o.pos);
@@ -447,8 +455,10 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
 // the stem of every changed CDS, objective 5.
 // Initialisation and evaluation of the designs of `items` (offspring
 // generations go through enqueue_generation).
-hipError_t enqueue_designs(const Launch &w, int mode, const int2 *items, int n_items, hipStream_t s) {
-    hipError_t e = cd::launch_design(mode, w.jobs, items, n_items, w.lds, s);
+// fresh: an initialisation of a pool that has not been written before.
+hipError_t enqueue_designs(const Launch &w, int mode, const int2 *items, int n_items, hipStream_t s, bool fresh = false) {
+    hipError_t e = cd::launch_design(mode, w.jobs, items, n_items, w.lds, s, nullptr, nullptr, cd::StemList{0, 0, 0},
+                                     fresh ? 1 : 0);
     if (e == hipSuccess) e = cd::launch_stem(mode, w.jobs, items, n_items, w.mg, w.stem_parts, w.stem_lds, s);
     if (e == hipSuccess) e = cd::launch_stem_finish(mode, w.jobs, items, n_items, s);
     return e;
@@ -635,7 +645,7 @@ int tune_shapes(const cd::Shapes &start, int njobs, int gens, hipStream_t s, App
         unsigned phases;  // bit k: phase k of the generation profile
     };
     const std::vector<Param> params = {
-        {&cd::Shapes::design_split, {0, 20 * 1024, 24 * 1024, 29 * 1024}, 0x3u},
+        {&cd::Shapes::design_split, {0, 6000, 8500, 11000}, 0x3u},
         {&cd::Shapes::design_threads, {256, 512}, 0x1u},
         {&cd::Shapes::stem_waves, {5, 6, 7, 8}, 0x2u},
         {&cd::Shapes::dom_rows, {64, 128, 256}, 0x4u},
@@ -721,6 +731,22 @@ cd::Shapes untuned_shapes(cd_job *const *jobs, int count) {
     cd::Shapes sh = count == 1 ? cd::SHAPES_JOB : cd::SHAPES_BATCH;
     int64_t pool = 0;
     for (int j = 0; j < count; ++j) pool += jobs[j]->P;
+    // k_design in one launch, 512 threads a child while the workgroups are
+    // resident together -- three a CU -- and longer the more codons a child has.
+    // Microseconds with 256 / 512 threads: 2004 codons, 700 children 20.7 /
+    // 19.8, 900 24.3 / 25.3; 6190 codons, 900 35.3 / 33.2, 2048 49.7 / 53.9;
+    // 20008 codons, 1200 77.8 / 68.8, 2048 98.9 / 92.1; up to 700 codons equal
+    // below 768 children and 256 faster above.  Launch classes by LDS do not pay
+    // any more (a second launch's tail against a few more resident workgroups):
+    // ticks of 24 / 48 / 64 jobs 454 / 797 / 1004 us in one launch, 478 / 790 /
+    // 971 split at 8500 bytes, the other way round for other mixes.
+    int64_t children = 0, codons = 0;
+    for (int j = 0; j < count; ++j) {
+        children += jobs[j]->N;
+        codons += (int64_t)jobs[j]->N * jobs[j]->L * jobs[j]->m;
+    }
+    sh.design_split = 0;
+    sh.design_threads = children <= 640 + codons / children / 16 ? 512 : 256;
     sh.assoc_designs = pool <= 512 ? 4 : pool <= cd::FUSED_TOTAL ? 8 : pool <= 12000 ? 16 : 64;
     return sh;
 }
@@ -762,7 +788,7 @@ int cd_job_create(const cd_job_desc *desc, cd_job **out) {
 int cd_job_init(cd_job *J) {
     if (!J || J->selection_only) return fail(CD_E_INVALID, "null job");
     // the offspring work list doubles as the (job, design) list of the init launch
-    HIPCHK(enqueue_designs(job_launch(J), cd::MODE_INIT, J->d_off, J->N, J->stream));
+    HIPCHK(enqueue_designs(job_launch(J), cd::MODE_INIT, J->d_off, J->N, J->stream, !J->inited));
     HIPCHK(cd::launch_init_state(J->d_self, 1, J->stream));
     J->inited = true;
     return CD_OK;
@@ -835,13 +861,16 @@ int cd_job_read(cd_job *J, int8_t *genome, float *obj, int8_t *idx, int32_t *pql
     cd::SelState st;
     HIPCHK(read_state(J, st));
     const int b = (int)(st.gen & 1u), P = J->P;
-    const size_t rows = (size_t)P * J->m, L = J->L, Ls = J->h.Ls;
+    const size_t rows = (size_t)P * J->m, L = J->L;
     hipStream_t s = J->stream;
     std::unique_lock<std::mutex> stage(g_rows.mu, std::defer_lock);
-    if (genome) {  // the padded rows in one transfer, compacted below
+    if (genome) {
+        // packed synonym indices, made on the device in the other buffer (the
+        // next generation writes every row of it), in one transfer
         stage.lock();
-        HIPCHK(g_rows.reserve(rows * Ls));
-        HIPCHK(hipMemcpyAsync(g_rows.p, J->h.genome[b], rows * Ls, hipMemcpyDeviceToHost, s));
+        HIPCHK(g_rows.reserve(rows * L));
+        HIPCHK(cd::launch_export(J->d_self, J->h.genome[b], J->h.genome[b ^ 1], (int)rows, (int)L, s));
+        HIPCHK(hipMemcpyAsync(g_rows.p, J->h.genome[b ^ 1], rows * L, hipMemcpyDeviceToHost, s));
     }
     if (obj) HIPCHK(hipMemcpyAsync(obj, J->h.obj[b], (size_t)P * 6 * 4, hipMemcpyDeviceToHost, s));
     if (idx) HIPCHK(hipMemcpyAsync(idx, J->h.oidx[b], (size_t)P * 12, hipMemcpyDeviceToHost, s));
@@ -851,8 +880,7 @@ int cd_job_read(cd_job *J, int8_t *genome, float *obj, int8_t *idx, int32_t *pql
     if (sorted) HIPCHK(hipMemcpyAsync(mask.data(), J->h.selm, (size_t)J->W * 8, hipMemcpyDeviceToHost, s));
     if (front_of) HIPCHK(hipMemcpyAsync(front_of, J->h.front_of, (size_t)P * 4, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    if (genome)  // CDS rows of L codons from rows of stride Ls
-        for (size_t r = 0; r < rows; ++r) std::memcpy(genome + r * L, g_rows.p + r * Ls, L);
+    if (genome) std::memcpy(genome, g_rows.p, rows * L);
     if (sorted) survivors_of(mask, J->N, sorted);
     if (pql)
         for (int i = 0; i < P; ++i)

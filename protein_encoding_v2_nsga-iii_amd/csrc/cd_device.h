@@ -218,6 +218,18 @@ __device__ __forceinline__ float wave_max_f32(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// Lane l's v (l wave-uniform).
+__device__ __forceinline__ float lane_of(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// Orders a wave's LDS writes before its own later reads (other lanes' values).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Largest v >= 0 over a full wave, wave-uniform: DPP row shifts 1, 2, 4, 8
 // leave each row's maximum in its lane 15, the row broadcasts of lanes 15
 // and 31 carry it across rows, and lane 63 ends with the wave's maximum.

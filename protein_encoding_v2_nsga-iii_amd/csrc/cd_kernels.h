@@ -28,13 +28,20 @@ struct Shapes {
     int assoc_designs;   // designs per k_associate workgroup: 4, 8 or 16 (a wave each), 32 or 64 (eight lanes each)
     int niche_threads;   // niching workgroup (k_place_niche, or k_place and k_niche above 2048 designs): 256, 512 or 1024 threads
 };
-// Untuned shapes of a lone job, and of a batch or served tick (assoc_designs
-// by the pool: untuned_shapes).
+// Untuned shapes of a lone job, and of a batch or served tick (the k_design
+// and k_associate fields by the work's sizes: untuned_shapes).
 constexpr Shapes SHAPES_JOB = {0, 512, 6, 64, 512, 4, 1024};
-constexpr Shapes SHAPES_BATCH = {24 * 1024, 512, 7, 128, 1024, 4, 1024};
+constexpr Shapes SHAPES_BATCH = {0, 256, 7, 128, 1024, 4, 1024};
 bool shapes_valid(const Shapes &s);
+// More children than this in a launch of 256-thread workgroups (seven a CU
+// are resident at 68 VGPRs) and k_design is throughput-bound: it then takes
+// the build for eight waves per SIMD, which spills a few registers (64-job
+// mix 426 -> 397 us, 4096 children of 12008 codons 98.3 -> 98.3; 1024 children of
+// 2004 codons 25.1 -> 26.1).
+constexpr int DESIGN_MANY = 2048;
 
 size_t design_lds_bytes(int L, int m);
+size_t design_bytes_accepted(int L, int m);  // at most LDS_BYTES for a job to be accepted
 size_t stem_lds_bytes(int L);
 size_t cds_plane_bytes(int L);  // one CDS's two bit planes in the job's plane buffer
 int stem_parts_of(int L);  // k_stem workgroups per CDS of L codons (1 .. STEM_PARTS)
@@ -75,6 +82,10 @@ inline size_t stem_list_entries(int n_items, int mg) {
 hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n, size_t lds, hipStream_t s,
                          uint32_t *stem_list = nullptr, int32_t *stem_ctl = nullptr, StemList sl = StemList{0, 0, 0},
                          int item_base = 0, int threads = 256);
+// (MODE_INIT: item_base 1 when the pool has not been written before)
+// the packed synonym indices of a pool's rows [rows][L] from its code rows
+// (stride row_stride(L)), to dst (room for rows * row_stride(L) bytes)
+hipError_t launch_export(const DevJob *job, const int8_t *src, int8_t *dst, int rows, int L, hipStream_t s);
 // initialisation and evaluation: parts workgroups per (item, CDS c < mg),
 // parts the largest stem_parts_of of the jobs: stem of each CDS k_design marked
 hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, int parts, size_t lds,

@@ -43,30 +43,23 @@ namespace cd {
 
 __host__ __device__ constexpr int align16(int x) { return (x + 15) & ~15; }
 
-// k_design's dynamic LDS: log weights by codon code lw6 [64] (int64), the
-// code of every codon of the table [64], per position the first codon and
-// the number of synonyms of its amino acid [Ls] each, then the design's CDS
-// rows (stride Ls = row_stride(L)): synonym indices syn [m][Ls] and codon
-// codes cd6 [m][Ls], then the CDS statistics [m].  Rows are 16-byte aligned,
-// so the genome moves between HBM and LDS in 16-byte words and four codes
-// share a 32-bit word in the Hamming sums.
-// After the genome row is stored, the syn area stages the forward bit planes
-// of the changed CDS (plane_stage_bytes each), so its stride per CDS is the
-// larger of the two.
-constexpr int DL_LW6 = 0, DL_CODE = 512, DL_POS = 576;
-static_assert(DL_POS % 16 == 0, "design LDS rows are 16-byte aligned");
+// k_design's dynamic LDS: log weights by codon code lw6 [64] (int64) and
+// synonym words by code [64] (u64), then the design's code rows [m][Ls]
+// (stride Ls = row_stride(L)), then the CDS statistics [m].  Rows are 16-byte
+// aligned, so the genome moves between HBM and LDS in 16-byte words and four
+// codes share a 32-bit word in the sums.  Holding the pool as codes instead of
+// synonym indices halves this (no index rows, no per-position synonym ranges)
+// and saves the conversion of every codon of every child: 1.4 us a workgroup.
+constexpr int DL_SYN = 512, DL_ROWS = 1024;
 
-// forward planes of one CDS staged in LDS: scan_words(3L) words and one zero
-// word past them (the reverse-complement windows read one word ahead)
+size_t design_lds_bytes(int L, int m) { return DL_ROWS + (size_t)m * (row_stride(L) + sizeof(CdsStat)) + 16; }
+
+// Jobs are accepted up to this size: 160 KiB for m synonym and code rows, the
+// synonym ranges and the statistics of a design.
 __host__ __device__ inline int plane_stage_bytes(int L) { return align16((scan_words(3 * L) + 1) * 8); }
-__host__ __device__ inline int syn_stride(int L) {
+size_t design_bytes_accepted(int L, int m) {
     const int a = row_stride(L), b = plane_stage_bytes(L);
-    return a > b ? a : b;
-}
-
-size_t design_lds_bytes(int L, int m) {
-    const size_t Ls = row_stride(L), SA = syn_stride(L);
-    return (size_t)DL_POS + 2 * Ls + (size_t)m * (SA + Ls) + align16(m * (int)sizeof(CdsStat)) + 16;
+    return (size_t)576 + 2 * a + (size_t)m * ((a > b ? a : b) + a) + align16(m * (int)sizeof(CdsStat)) + 16;
 }
 
 // one CDS's bit planes: the sequence and its reverse complement, each
@@ -84,14 +77,8 @@ struct DesignShared {
     float pobj[NOBJ];
     int32_t pidx[2 * NOBJ];
     int32_t ppql[4];
-    int32_t dirty[MAX_M];
+    int32_t dirty[MAX_M];  // CDS the operator changed
     int32_t hd[MAX_M * (MAX_M - 1) / 2];
-    int64_t red[8 * NW];
-    int32_t red32[8 * NW];
-    uint64_t redu[16];
-    int32_t misc[16];
-    int32_t slw[NW * 11];  // mut_sl: per wave, first [4], last [4], full [3]
-    int32_t dlist[MAX_M];  // the changed CDS, in order
     uint16_t hitq[NW][HITQ];  // per wave: codons that passed an operator's test, awaiting their work
 };
 
@@ -114,16 +101,6 @@ __device__ __forceinline__ void gstore_stat(CdsStat *p, const CdsStat &s) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) gstore(q + i, v.w[i]);
 }
-
-// k_design's LDS tables and the per-position synonym ranges.
-struct DesignLds {
-    const int64_t *lw6;    // [64] log weights by code
-    const uint8_t *code;   // [64] code of each codon of the table
-    const uint8_t *pbase;  // [Ls] first codon of position k's amino acid
-    const uint8_t *pnum;   // [Ls] synonyms of position k's amino acid
-    uint64_t stop6;        // stop codes
-    int Ls;                // row stride
-};
 
 // Facts of codons given by their codes (first base << 4 | second << 2 | third).
 // Third base C (1) or G (2).
@@ -346,16 +323,19 @@ __host__ __device__ inline int stem_parts(int n) {
 }
 
 // ---------------------------------------------------------------------------
-// Evaluation of the CDS flagged dirty, then objectives 0-4
-// (calMinimumCAI/CBP/HSC/HD, calMaximumGC3, utils.cuh:271-626), on codon
-// codes.  A changed CDS is marked for k_stem (pad = 1); its stem fields keep
-// the parent's stem, which seeds the scan (have_parent), or are cleared.  Up
-// to four changed CDS share one pass over the positions; the sums are wave
-// sums (DPP) added over the waves by one thread per value, which also
-// computes the CDS's values (CAI, CPB, HSC quotient, GC3 fraction) kept in
-// its record.  Hamming distances take four codons per 32-bit word of two code
-// rows, a wave per pair: every pair without a parent, only the pairs of a
-// changed CDS with one (sh.hd holds the parent's distances on entry).
+// Evaluation of a design's code rows in LDS (calMinimumCAI/CBP/HSC/HD,
+// calMaximumGC3, utils.cuh:271-626), in three kinds of task, one wave a task
+// and no barrier between them:
+//   sums of one CDS        CAI and CPB sums, hidden stops, GC3 codons, then the
+//                          CDS's values; four codons to a 32-bit word
+//   planes of one CDS      its bit planes for the stem search
+//   Hamming distance of one pair of CDS
+// With the whole workgroup on one CDS at a time (a barrier and a cross-wave
+// sum after each) the reductions cost about as much as the sums.  With the
+// code rows, the tasks and the operators' synonym words the offspring launch
+// went from 608 to 395 us on the 64-job mix (42 240 children), 161 to 98 us for
+// 4096 children of 12 008 codons, 32 to 23 us for 1024 of 2004; the remaining
+// bound is VALU issue, about a quarter of it the operators' Philox draws.
 // ---------------------------------------------------------------------------
 // Per-CDS values of the sums: CAI, CPB, the HSC quotient and the GC3 fraction.
 __device__ __forceinline__ void cds_values(CdsStat &s, int L) {
@@ -365,195 +345,271 @@ __device__ __forceinline__ void cds_values(CdsStat &s, int L) {
     s.ov[3] = (float)s.gc3 / (float)L;
 }
 
-// The pick-th (0-based) set bit of a candidate mask.
-__device__ __forceinline__ int nth_bit(uint32_t mask, uint32_t pick) {
-    for (uint32_t q = 0; q < pick; ++q) mask &= mask - 1u;
-    return __builtin_ctz(mask);
+// Bytes of v (each below 64) that are stop codes: UAA, UAG, UGA are 48, 50
+// and 56 (the job's table keeps the standard code), the bytes whose bits 5
+// and 4 are set, 2 and 0 clear, and 3 and 1 not both set.
+__device__ __forceinline__ int stops4(uint32_t v) {
+    const uint32_t t = v ^ 0x30303030u;
+    const uint32_t z = (t & 0x35353535u) | (t & (t >> 2) & 0x02020202u);  // 0 in a stop's byte
+    return 4 - __popc((z + 0x7F7F7F7Fu) & 0x80808080u);
 }
 
+// Sums of the CDS in row w (nwd words): a word's four codons and their four
+// junctions a step.  Padding codons are code 0: they add the log weight and
+// the pair score of code 0, taken off at the end, and no GC3; their junctions
+// are masked off, and a stop scores no pairs.
+__device__ __forceinline__ void task_sums(const DevJob &J, const int64_t *lw6, const uint32_t *w, int L, int nwd,
+                                          CdsStat *rec, bool have_parent) {
+    const int lane = threadIdx.x & 63, n4 = (L + 3) >> 2;
+    const int64_t *const pair6 = J.cpfx6;
+    int64_t cai = 0, cpb = 0;
+    uint32_t hg = 0;  // hidden stops in the high half, GC3 codons in the low half (both below 2^16)
+#pragma unroll 1
+    for (int q = lane; q < n4; q += 64) {
+        const uint32_t a = w[q], nx = q + 1 < nwd ? w[q + 1] : 0u;
+        const uint32_t b = __builtin_amdgcn_alignbit(nx, a, 8);  // the codons one further on
+        const uint32_t e = ((a & 0x003F003Fu) << 9) | ((b & 0x003F003Fu) << 3);  // byte offsets of pairs 0 and 2
+        const uint32_t o = (((a >> 8) & 0x003F003Fu) << 9) | (((b >> 8) & 0x003F003Fu) << 3);  // of 1 and 3
+        const char *const pb = (const char *)pair6;
+        const int64_t p0 = gload((const int64_t *)(pb + (e & 0xFFFFu))), p1 = gload((const int64_t *)(pb + (o & 0xFFFFu)));
+        const int64_t p2 = gload((const int64_t *)(pb + (e >> 16))), p3 = gload((const int64_t *)(pb + (o >> 16)));
+        cai += (lw6[a & 63u] + lw6[(a >> 8) & 63u]) + (lw6[(a >> 16) & 63u] + lw6[a >> 24]);
+        const uint32_t gc = (a ^ (a >> 1)) & 0x01010101u;  // third base C (1) or G (2)
+        // junctions a|b: a[1] a[2] b[0] and a[2] b[0] b[1]
+        // (countRightSideHSC, utils.cuh:138-161); the last codon has none
+        const int left = L - 1 - 4 * q;
+        const uint32_t keep = left >= 4 ? ~0u : (1u << (8 * max(left, 0))) - 1u;
+        const uint32_t j1 = ((a & 0x0F0F0F0Fu) << 2) | ((b >> 4) & 0x03030303u);
+        const uint32_t j2 = ((a & 0x03030303u) << 4) | ((b >> 2) & 0x0F0F0F0Fu);
+        hg += ((uint32_t)(stops4(j1 & keep) + stops4(j2 & keep)) << 16) + (uint32_t)__popc(gc);
+        cpb += (p0 + p1) + (p2 + p3);
+    }
+    cai = wave_sum_i64(cai);
+    cpb = wave_sum_i64(cpb);
+    hg = (uint32_t)wave_sum_i32((int)hg);
+    const int pads = 4 * n4 - L;
+    CdsStat s = *rec;
+    if (!have_parent) s.l = s.p = s.q = 0;
+    s.cai = cai - pads * lw6[0];
+    s.cpb = cpb - pads * gload(pair6);
+    s.hsc = (int)(hg >> 16);
+    s.gc3 = (int)(hg & 0xFFFFu);
+    s.pad = 1;
+    s.key = 0;
+    cds_values(s, L);
+    if (lane == 0) *rec = s;
+}
+
+// Twelve bits of four codons (three to a byte, bytes in order) packed in a row.
+__device__ __forceinline__ uint32_t pack12(uint32_t x) {
+    const uint32_t t = x | (x >> 5);
+    return (t & 0x3Fu) | ((t >> 10) & 0xFC0u);
+}
+
+// Bit planes of the CDS in row w into the job's plane buffer (sp, then rp):
+// bit p of the sequence plane is position p, of the reverse-complement plane
+// position n-1-p complemented; positions past n are zero; a word is (low bits,
+// high bits) of 32 positions.  A lane builds 32 codons (three words) of one
+// plane from eight words of codes; the reverse complement is the codons read
+// backwards, each with its bases reversed and complemented.
+__device__ __forceinline__ void task_planes(const uint32_t *w, int L, int nwd, uint2 *sp) {
+    const int n = 3 * L, W = scan_words(n), ng = (W + 2) / 3, lane = threadIdx.x & 63;
+    uint2 *const rp = sp + W;
+    for (int i = lane; i < 2 * ng; i += 64) {
+        const bool rev = i >= ng;
+        const int g = rev ? i - ng : i;
+        uint32_t lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {  // codons 32g + 4t .. 32g + 4t + 3 of the plane's sequence
+            const int u = 8 * g + t;
+            uint32_t l, h;
+            if (!rev) {
+                const uint32_t d = u < nwd ? w[u] : 0u;  // (the row's padding codes are 0)
+                // per byte the three bases' low (high) bits in position order
+                l = ((d >> 4) & 0x01010101u) | ((d >> 1) & 0x02020202u) | ((d << 2) & 0x04040404u);
+                h = ((d >> 5) & 0x01010101u) | ((d >> 2) & 0x02020202u) | ((d << 1) & 0x04040404u);
+            } else {
+                const int k = L - 4 - 4 * u;  // the four codons from k on, backwards; those below 0 are past the end
+                const int wi = k >> 2;
+                const uint32_t x0 = wi >= 0 ? w[wi] : 0u, x1 = wi >= -1 && wi + 1 < nwd ? w[wi + 1] : 0u;
+                const uint32_t d = __builtin_bswap32(__builtin_amdgcn_alignbit(x1, x0, 8 * (k & 3)));
+                const uint32_t keep = k >= 0 ? 0x07070707u : k <= -4 ? 0u : 0x07070707u & ((1u << (8 * (k + 4))) - 1u);
+                l = (~((d & 0x01010101u) | ((d >> 1) & 0x02020202u) | ((d >> 2) & 0x04040404u))) & keep;
+                h = (~(((d >> 1) & 0x01010101u) | ((d >> 2) & 0x02020202u) | ((d >> 3) & 0x04040404u))) & keep;
+            }
+            const uint32_t l12 = pack12(l), h12 = pack12(h);
+            const int b = 12 * t, q = b >> 5, o = b & 31;  // compile-time after unrolling
+            lo[q] |= l12 << o;
+            hi[q] |= h12 << o;
+            if (o > 20) {
+                lo[q + 1] |= l12 >> (32 - o);
+                hi[q + 1] |= h12 >> (32 - o);
+            }
+        }
+        uint2 *const out = rev ? rp : sp;
+#pragma unroll
+        for (int v = 0; v < 3; ++v)
+            if (3 * g + v < W) gstore((uint64_t *)(out + 3 * g + v), (uint64_t)lo[v] | ((uint64_t)hi[v] << 32));
+    }
+}
+
+// Hamming distance of the CDS in rows a and b (nv 16-byte words; the padding
+// codes are 0 in every CDS and add nothing), wave-uniform.
+__device__ __forceinline__ int task_pair(const uint32_t *a, const uint32_t *b, int nv) {
+    const u32x4 *a4 = (const u32x4 *)a, *b4 = (const u32x4 *)b;
+    int acc = 0;
+    for (int q = threadIdx.x & 63; q < nv; q += 64) {
+        const u32x4 x = a4[q] ^ b4[q];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc += code_mismatch4(x[v]);
+    }
+    return wave_sum_i32(acc);
+}
+
+// The tasks of a design whose CDS in dmask changed (all of them without a
+// parent): wave wid of nw takes every nw-th.  The pairs are those of the one
+// changed CDS, or every pair when more changed (sh.hd holds the parent's
+// distances on entry).
 template <class SH>
-__device__ void evaluate(const DevJob &J, const DesignLds &D, const uint8_t *cd6, CdsStat *cst, bool have_parent,
-                         SH &sh, float *obj, int32_t *oidx) {
-    const int L = J.L, m = J.m, n = 3 * L, Ls = D.Ls;
-    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wid = tid >> 6, nw = NT >> 6;
-    uint32_t dmask = 0;  // the same in every thread
-    for (int c = 0; c < m; ++c) dmask |= (uint32_t)(sh.dirty[c] != 0) << c;
-    {
-        uint32_t left = dmask;
-        while (left) {
-            int cs[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                cs[u] = left ? __builtin_ctz(left) : -1;
-                left &= left - 1u;
+__device__ __forceinline__ void design_tasks(const DevJob &J, const int64_t *lw6, const uint32_t *rows, uint32_t dmask, bool have_parent,
+                             CdsStat *cst, SH &sh, uint2 *planes, int wid, int nw) {
+    const int L = J.L, m = J.m, nwd = J.Ls >> 2, lane = threadIdx.x & 63, PW = 2 * scan_words(3 * L);
+    const int nd = __popc(dmask), npair = nd == 1 ? m - 1 : (nd ? m * (m - 1) / 2 : 0);
+    uint32_t left = dmask;  // the CDS of task t, for t rising
+    int t0 = 0;
+    int i = 0, j = 0, p0 = -1;  // the last pair enumerated
+    for (int t = wid; t < 2 * nd + npair; t += nw) {
+        if (t < 2 * nd) {
+            const int r = t < nd ? t : t - nd;
+            if (r < t0) {
+                left = dmask;
+                t0 = 0;
             }
-            // one CDS at a time (its sums reduced over the wave into LDS before
-            // the next), four codons a thread per round: the pair scores of all
-            // four (global table, one dependent load each) are fetched together
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (cs[u] < 0) continue;
-                const uint8_t *g = cd6 + cs[u] * Ls;
-                int64_t cai = 0, cpb = 0;
-                int hsc = 0, gcn = 0;
-                for (int k0 = tid; k0 < L; k0 += 4 * NT) {
-                    int64_t ps[4];
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int k = k0 + v * NT;
-                        const bool pair = k < L - 2;
-                        const int kk = pair ? k : 0;  // an index inside the row either way
-                        ps[v] = pair ? gload(J.cpfx6 + g[kk] * 64 + g[kk + 1]) : 0;
-                    }
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int k = k0 + v * NT;
-                        if (k >= L) break;
-                        const int a = g[k];
-                        cai += D.lw6[a];
-                        gcn += code_gc3(a);
-                        if (k < L - 1) hsc += code_hidden(D.stop6, a, g[k + 1]);
-                        cpb += ps[v];
-                    }
-                }
-                cai = wave_sum_i64(cai);
-                cpb = wave_sum_i64(cpb);
-                hsc = wave_sum_i32(hsc);
-                gcn = wave_sum_i32(gcn);
-                if (lane == 0) {
-                    sh.red[wid * 8 + 2 * u] = cai;
-                    sh.red[wid * 8 + 2 * u + 1] = cpb;
-                    sh.red32[wid * 8 + 2 * u] = hsc;
-                    sh.red32[wid * 8 + 2 * u + 1] = gcn;
-                }
-            }
-            lds_barrier();
-            if (tid < 4) {
-                const int c = tid == 0 ? cs[0] : tid == 1 ? cs[1] : tid == 2 ? cs[2] : cs[3];
-                if (c >= 0) {
-                    int64_t a = 0, b = 0;
-                    int h = 0, g = 0;
-                    for (int w = 0; w < nw; ++w) {
-                        a += sh.red[w * 8 + 2 * tid];
-                        b += sh.red[w * 8 + 2 * tid + 1];
-                        h += sh.red32[w * 8 + 2 * tid];
-                        g += sh.red32[w * 8 + 2 * tid + 1];
-                    }
-                    CdsStat s = cst[c];
-                    if (!have_parent) s.l = s.p = s.q = 0;
-                    s.cai = a;
-                    s.cpb = b;
-                    s.hsc = h;
-                    s.gc3 = g;
-                    s.pad = 1;
-                    s.key = 0;
-                    cds_values(s, L);
-                    cst[c] = s;
-                }
-            }
-            lds_barrier();
+            for (; t0 < r; ++t0) left &= left - 1u;
+            const int c = __builtin_ctz(left);
+            if (t < nd)
+                task_sums(J, lw6, rows + c * nwd, L, nwd, cst + c, have_parent);
+            else
+                task_planes(rows + c * nwd, L, nwd, planes + (size_t)c * PW);
+            continue;
         }
-    }
-    // pairwise Hamming distances, pairs (i, j), i < j, in lexicographic order,
-    // a wave each (pair p on wave p mod nw): every pair without a parent,
-    // those with a changed CDS otherwise; the rows' padding codes are 0 in
-    // every CDS and add nothing
-    {
-        const int npair = m * (m - 1) / 2, nwd = Ls >> 2;
-        const uint32_t *w6 = (const uint32_t *)cd6;
-        int i = 0, j = 1;  // pair wid
-        for (int t = 0; t < wid && t < npair; ++t)
-            if (++j == m) {
-                ++i;
-                j = i + 1;
-            }
-        for (int p = wid; p < npair; p += nw) {
-            if (!have_parent || ((dmask >> i) & 1u) || ((dmask >> j) & 1u)) {
-                int acc = 0;
-                for (int q = lane; q < nwd; q += 64) acc += code_mismatch4(w6[i * nwd + q] ^ w6[j * nwd + q]);
-                acc = wave_sum_i32(acc);
-                if (lane == 0) sh.hd[p] = acc;
-            }
-            for (int t = 0; t < nw; ++t)  // the pair nw further on
-                if (++j == m) {
+        const int p = t - 2 * nd;  // pair p of the list
+        int a, b, q;
+        if (nd == 1) {
+            const int c = __builtin_ctz(dmask), o = p < c ? p : p + 1;
+            a = min(c, o);
+            b = max(c, o);
+            q = a * (2 * m - a - 1) / 2 + b - a - 1;
+        } else {
+            for (; p0 < p; ++p0)  // pairs (i, j), i < j, in lexicographic order
+                if (p0 < 0)
+                    j = 1;
+                else if (++j == m) {
                     ++i;
                     j = i + 1;
                 }
+            a = i;
+            b = j;
+            q = p;
+        }
+        const int d = task_pair(rows + a * nwd, rows + b * nwd, nwd >> 2);
+        if (lane == 0) sh.hd[q] = d;
+    }
+}
+
+// Largest v of lanes 0-15 (one DPP row), and the last lane below m holding it.
+__device__ __forceinline__ int last_max16(float v, int m) {
+    float x = v;
+    x = fmaxf(x, dpp_f32<0x111, 0xf>(x, -FLT_MAX));
+    x = fmaxf(x, dpp_f32<0x112, 0xf>(x, -FLT_MAX));
+    x = fmaxf(x, dpp_f32<0x114, 0xf>(x, -FLT_MAX));
+    x = fmaxf(x, dpp_f32<0x118, 0xf>(x, -FLT_MAX));
+    x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 15));
+    const uint64_t at = __ballot(v == x && (int)(threadIdx.x & 63) < m);
+    return 63 - (int)__builtin_clzll(at);
+}
+
+// Objectives 0-4 of the design and their indices, by one wave, stored to
+// oobj and oidx (entry 10, the stem's CDS, is left to the stem search): each
+// is the largest of the CDS's (pairs') values, ties to the last CDS (pair) --
+// a serial sweep that takes every value at least as large as the one it holds
+// (utils.cuh:271-626).  The values are finite, and all zeros of one objective
+// have one sign.  The smallest distance is the largest negated quotient:
+// distinct distances below 2^24 have distinct quotients.
+template <class SH>
+__device__ __forceinline__ void design_objectives(const DevJob &J, const CdsStat *cst, const SH &sh, float *oobj, int8_t *oidx) {
+    const int m = J.m, n = 3 * J.L, lane = threadIdx.x & 63, npair = m * (m - 1) / 2;
+    const float gc3_ref = J.gc3_ref;
+    const bool cl = lane < m;
+    const CdsStat &sc = cst[cl ? lane : 0];
+    const float v0 = sc.ov[0], v1 = sc.ov[1], v2 = sc.ov[2], v3 = sc.ov[3];
+    const float k0 = cl ? -v0 : -FLT_MAX, k1 = cl ? -v1 : -FLT_MAX, k2 = cl ? -v2 : -FLT_MAX;
+    const float k4 = cl ? fabsf(v3 - gc3_ref) : -FLT_MAX;
+    int dist = 0x7FFFFFFF, pair = 0;
+    for (int q = lane; q < npair; q += 64) {  // at most two a lane; ties to the later pair
+        const int d = sh.hd[q];
+        if (d <= dist) {
+            dist = d;
+            pair = q;
         }
     }
-    lds_barrier();
-    // The objectives (calMinimumCAI .. calMaximumGC3, utils.cuh:271-626): each
-    // is the largest of the CDS's (pairs') values, ties to the last CDS (pair)
-    // -- a serial sweep that takes every value at least as large as the one it
-    // holds.  One lane per CDS (pair) and the largest (value bits, index) key
-    // over the wave give the same choice (the values are finite).
-    if (wid == 0) {
-        const float gc3_ref = J.gc3_ref;
-        const bool cl = lane < m;
-        const int c = cl ? lane : 0;
-        auto key = [](bool ok, float v, int i) -> uint64_t {
-            return ok ? ((uint64_t)ord_bits(v) << 32) | (uint32_t)i : 0ull;
-        };
-        const CdsStat &sc = cst[c];
-        const uint64_t k_cai = wave_max_u64(key(cl, -sc.ov[0], lane));
-        const uint64_t k_cpb = wave_max_u64(key(cl, -sc.ov[1], lane));
-        const uint64_t k_hsc = wave_max_u64(key(cl, -sc.ov[2], lane));
-        const uint64_t k_gc = wave_max_u64(key(cl, fabsf(sc.ov[3] - gc3_ref), lane));
-        const int npair = m * (m - 1) / 2;
-        uint64_t kh = 0;
-        for (int q = lane; q < npair; q += 64) {
-            const uint64_t k = key(true, -((float)sh.hd[q] / (float)n), q);
-            kh = k > kh ? k : kh;
-        }
-        kh = wave_max_u64(kh);
-        if (lane < 2 * NOBJ) oidx[lane] = 0;
-        if (lane == 0) {
-            const int ca = (int)(uint32_t)k_cai, cb = (int)(uint32_t)k_cpb, ch = (int)(uint32_t)k_hsc;
-            const int cg = (int)(uint32_t)k_gc, qh = (int)(uint32_t)kh;
-            int i = 0, j = 1;  // pair qh
-            for (int t = 0; t < qh; ++t)
-                if (++j == m) {
-                    ++i;
-                    j = i + 1;
-                }
-            oidx[0] = ca;
-            oidx[2] = cb;
-            oidx[4] = ch;
-            oidx[6] = i;
-            oidx[7] = j;
-            oidx[8] = cg;
-            oidx[9] = (cst[cg].ov[3] - gc3_ref) < 0 ? GC_UP : GC_DOWN;
-            obj[0] = -cst[ca].ov[0];
-            obj[1] = -cst[cb].ov[1];
-            obj[2] = -cst[ch].ov[2];
-            obj[3] = -((float)sh.hd[qh] / (float)n);
-            obj[4] = fabsf(cst[cg].ov[3] - gc3_ref);
-        }
+    const int dmin = wave_min_i32(dist);
+    const int qh = wave_max_i32(dist == dmin ? pair : -1);
+    const int c0 = last_max16(k0, m), c1 = last_max16(k1, m), c2 = last_max16(k2, m), c4 = last_max16(k4, m);
+    int i = 0, r = qh;  // pair qh of the lexicographic order
+    while (r >= m - 1 - i) {
+        r -= m - 1 - i;
+        ++i;
     }
-    lds_barrier();
+    const int j = i + 1 + r;
+    const float dev = lane_of(v3, c4) - gc3_ref;
+    if (lane < 2 * NOBJ && lane != 10) {
+        const int v = lane == 0 ? c0 : lane == 2 ? c1 : lane == 4 ? c2 : lane == 6 ? i : lane == 7 ? j
+                      : lane == 8 ? c4 : lane == 9 ? (dev < 0 ? GC_UP : GC_DOWN) : 0;
+        gstore(oidx + lane, (int8_t)v);
+    }
+    if (lane < NOBJ - 1) {
+        const float o0 = -lane_of(v0, c0), o1 = -lane_of(v1, c1), o2 = -lane_of(v2, c2);
+        const float o3 = -((float)dmin / (float)n), o4 = fabsf(dev);
+        gstore(oobj + lane, lane == 0 ? o0 : lane == 1 ? o1 : lane == 2 ? o2 : lane == 3 ? o3 : o4);
+    }
 }
 
 // ---------------------------------------------------------------------------
-// Mutation operators (include/mutation.cuh) on the synonym indices (syn) and
-// codon codes (cd6) in LDS.  Each thread owns whole codons; operators that
-// read neighbours only touch codons of the other parity or of other CDS, as
-// in the reference.  Draws: the i-th slot an operator visits in CDS c takes
-// words 2(i&1) (the mutation test) and 2(i&1)+1 (the choice, or the
-// shuffle) of Philox(gen, child, c*L + (i >> 1), TAG_MUT), so one call serves
-// two slots and a thread takes the two slots of one call.
+// Mutation operators (include/mutation.cuh) on the code rows in LDS.  A
+// codon's code names its amino acid, so one table word per code (SynWord)
+// holds its synonyms' codes, their number and its own place among them.  Each
+// thread owns whole codons; operators that read neighbours only touch codons
+// of the other parity or of other CDS, as in the reference.  Draws: the i-th
+// slot an operator visits in CDS c takes words 2(i&1) (the mutation test) and
+// 2(i&1)+1 (the choice, or the shuffle) of Philox(gen, child, c*L + (i >> 1),
+// TAG_MUT), so one call serves two slots and a thread takes the two slots of
+// one call.
 // ---------------------------------------------------------------------------
 
 struct MutArgs {
     const DevJob *J;
-    const DesignLds *D;
-    uint8_t *syn, *cd6;
+    const uint64_t *syn;  // [64] synonym words by code
+    uint8_t *rows;        // [m][Ls] codes
+    int Ls;
     uint32_t gen, child;
 };
 
-__device__ __forceinline__ void set_syn(const MutArgs &A, int c, int k, int s) {
-    const int i = c * A.D->Ls + k;
-    A.syn[i] = (uint8_t)s;
-    A.cd6[i] = A.D->code[A.D->pbase[k] + s];
+// A code's synonym word (J.syn6): codes of synonyms 0-4 in six-bit fields of
+// the low half, of synonym 5 in bits 0-5 of the high half, their number in
+// bits 8-10 and the code's own index in bits 12-14 of it.
+struct SynWord {
+    uint32_t lo, hi;
+    __device__ __forceinline__ explicit SynWord(uint64_t v) : lo((uint32_t)v), hi((uint32_t)(v >> 32)) {}
+    __device__ __forceinline__ int num() const { return (int)((hi >> 8) & 7u); }
+    __device__ __forceinline__ int own() const { return (int)((hi >> 12) & 7u); }
+    __device__ __forceinline__ int code(int j) const { return (int)((j < 5 ? lo >> (6 * j) : hi) & 63u); }
+};
+
+// The pick-th (0-based) set bit of a candidate mask.
+__device__ __forceinline__ int nth_bit(uint32_t mask, uint32_t pick) {
+    for (uint32_t q = 0; q < pick; ++q) mask &= mask - 1u;
+    return __builtin_ctz(mask);
 }
 
 __device__ __forceinline__ void pair_draws(const MutArgs &A, int c, int q, uint32_t r[4]) {
@@ -593,9 +649,9 @@ __device__ __forceinline__ void hits_by_wave(int npairs, uint16_t *seg, Test tes
 
 // mutationRandom, mutation.cuh:16-63: every codon of every CDS; a thread
 // takes codons 2q and 2q+1 of CDS c for its (c, q) pairs
-__device__ void mut_random(const MutArgs &A, int32_t *dirty) {
+__device__ __forceinline__ void mut_random(const MutArgs &A, int32_t *dirty) {
     const DevJob &J = *A.J;
-    const int L = J.L, Ls = A.D->Ls, hL = (L + 1) >> 1, total = J.m * hL;
+    const int L = J.L, Ls = A.Ls, hL = (L + 1) >> 1, total = J.m * hL;
     int c = (int)((unsigned)threadIdx.x / (unsigned)hL), q = (int)threadIdx.x - c * hL;
     for (int t = threadIdx.x; t < total; t += blockDim.x) {
         uint32_t r[4];
@@ -603,13 +659,14 @@ __device__ void mut_random(const MutArgs &A, int32_t *dirty) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = 2 * q + h;
-            if (k >= L) break;
-            const int ns = A.D->pnum[k];
-            if (!bern(r[2 * h], J.thr_pm) || ns == 1) continue;
-            const int cur = A.syn[c * Ls + k];
+            if (k >= L || !bern(r[2 * h], J.thr_pm)) continue;
+            uint8_t *at = A.rows + c * Ls + k;
+            const SynWord e(A.syn[*at]);
+            const int ns = e.num(), cur = e.own();
+            if (ns == 1) continue;
             int nw = (int)uniform_int(r[2 * h + 1], (uint32_t)(ns - 1));
             if (nw >= cur) ++nw;
-            set_syn(A, c, k, nw);
+            *at = (uint8_t)e.code(nw);
             dirty[c] = 1;
         }
         q += blockDim.x;
@@ -621,21 +678,21 @@ __device__ void mut_random(const MutArgs &A, int32_t *dirty) {
 }
 
 // mutationCAI with SELECT_UPPER_RANDOM, mutation.cuh:65-142
-__device__ void mut_cai(const MutArgs &A, int cds, int32_t *dirty) {
+__device__ __forceinline__ void mut_cai(const MutArgs &A, int cds, int32_t *dirty) {
     const DevJob &J = *A.J;
-    const int L = J.L, Ls = A.D->Ls;
+    const int L = J.L;
+    uint8_t *const row = A.rows + cds * A.Ls;
     for (int q = threadIdx.x; 2 * q < L; q += blockDim.x) {
         uint32_t r[4];
         pair_draws(A, cds, q, r);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = 2 * q + h;
-            if (k >= L) break;
-            const int ns = A.D->pnum[k];
-            if (!bern(r[2 * h], J.thr_pm) || ns == 1) continue;
-            const int cur = A.syn[cds * Ls + k];
+            if (k >= L || !bern(r[2 * h], J.thr_pm)) continue;
+            const SynWord e(A.syn[row[k]]);
+            const int ns = e.num(), cur = e.own();
             if (cur != ns - 1) {
-                set_syn(A, cds, k, cur + 1 + (int)uniform_int(r[2 * h + 1], (uint32_t)(ns - 1 - cur)));
+                row[k] = (uint8_t)e.code(cur + 1 + (int)uniform_int(r[2 * h + 1], (uint32_t)(ns - 1 - cur)));
                 dirty[cds] = 1;
             }
         }
@@ -645,12 +702,12 @@ __device__ void mut_cai(const MutArgs &A, int cds, int32_t *dirty) {
 // mutationCBP with SELECT_UPPER_RANDOM, mutation.cuh:144-262: the codons
 // k = 2i + parity below L-1; a thread takes i = 2q, 2q+1 (k = 4q + parity,
 // 4q + parity + 2)
-__device__ void mut_cbp(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg) {
+__device__ __forceinline__ void mut_cbp(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg) {
     const DevJob &J = *A.J;
-    const int L = J.L, Ls = A.D->Ls, parity = (int)(A.gen & 1u);
-    const uint64_t thr = J.thr_2pm;
+    const int L = J.L, parity = (int)(A.gen & 1u);
+    const uint64_t thr = J.thr_2pm, stop6 = J.stop6;
     const float *const cps6 = J.cps6;
-    const uint8_t *row = A.cd6 + cds * Ls;
+    uint8_t *const row = A.rows + cds * A.Ls;
     const int npairs = L - 1 - parity > 0 ? (L - 1 - parity + 3) >> 2 : 0;  // 4q + parity < L - 1
     auto test = [&](int q) -> uint32_t {
         uint32_t r[4];
@@ -659,26 +716,25 @@ __device__ void mut_cbp(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = 4 * q + parity + 2 * h;
-            if (k < L - 1 && bern(r[2 * h], thr) && A.D->pnum[k] > 1) hm |= 1u << h;
+            if (k < L - 1 && bern(r[2 * h], thr)) hm |= 1u << h;
         }
         return hm;
     };
     auto work = [&](int slot) {
         const int q = slot >> 1, h = slot & 1, k = 4 * q + parity + 2 * h;
-        uint32_t r[4];
-        pair_draws(A, cds, q, r);
-        const int ns = A.D->pnum[k];
-        const int base = A.D->pbase[k], cur = A.syn[cds * Ls + k];
+        const SynWord e(A.syn[row[k]]);
         const int left = (k > 0) ? (int)row[k - 1] : 0;
         const int right = row[k + 1];
+        const int ns = e.num(), cur = e.own();
+        if (ns == 1) return;
         // every synonym's score, the pair-score loads issued together (a
         // missing neighbour adds nothing; stop codes score 0 in the table)
-        const bool hl = k > 0, hr = !((A.D->stop6 >> right) & 1u);
+        const bool hl = k > 0, hr = !((stop6 >> right) & 1u);
         const float *rowl = cps6 + left * 64, *colr = cps6 + right;
         float sc[MAX_SYN];
 #pragma unroll
         for (int j = 0; j < MAX_SYN; ++j) {
-            const int g = A.D->code[base + (j < ns ? j : 0)];
+            const int g = j < ns ? e.code(j) : e.code(0);
             const float a = gload(rowl + g), b = gload(colr + g * 64);
             float v = 0.f;
             v += hl ? a : 0.f;
@@ -693,7 +749,9 @@ __device__ void mut_cbp(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg
         for (int j = 0; j < MAX_SYN; ++j)
             if (j < ns && j != cur && sc[j] > curv) cand |= 1u << j;
         if (cand) {
-            set_syn(A, cds, k, nth_bit(cand, uniform_int(r[2 * h + 1], (uint32_t)__popc(cand))));
+            uint32_t r[4];
+            pair_draws(A, cds, q, r);
+            row[k] = (uint8_t)e.code(nth_bit(cand, uniform_int(h ? r[3] : r[1], (uint32_t)__popc(cand))));
             dirty[cds] = 1;
         }
     };
@@ -702,12 +760,12 @@ __device__ void mut_cbp(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg
 
 // mutationHSC with SELECT_UPPER_RANDOM, mutation.cuh:264-388: the codons
 // k = 2i + parity below L, two per thread as in mut_cbp
-__device__ void mut_hsc(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg) {
+__device__ __forceinline__ void mut_hsc(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg) {
     const DevJob &J = *A.J;
-    const int L = J.L, Ls = A.D->Ls, parity = (int)(A.gen & 1u);
+    const int L = J.L, parity = (int)(A.gen & 1u);
     const uint64_t thr = J.thr_2pm;
-    const uint8_t *row = A.cd6 + cds * Ls;
-    const uint64_t stop6 = A.D->stop6;
+    uint8_t *const row = A.rows + cds * A.Ls;
+    const uint64_t stop6 = J.stop6;
     const int npairs = L - parity > 0 ? (L - parity + 3) >> 2 : 0;  // 4q + parity < L
     auto test = [&](int q) -> uint32_t {
         uint32_t r[4];
@@ -716,31 +774,30 @@ __device__ void mut_hsc(const MutArgs &A, int cds, int32_t *dirty, uint16_t *seg
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = 4 * q + parity + 2 * h;
-            if (k < L && bern(r[2 * h], thr) && A.D->pnum[k] > 1) hm |= 1u << h;
+            if (k < L && bern(r[2 * h], thr)) hm |= 1u << h;
         }
         return hm;
     };
     auto work = [&](int slot) {
         const int q = slot >> 1, h = slot & 1, k = 4 * q + parity + 2 * h;
-        uint32_t r[4];
-        pair_draws(A, cds, q, r);
-        const int ns = A.D->pnum[k];
-        const int base = A.D->pbase[k], cur = A.syn[cds * Ls + k];
+        const SynWord e(A.syn[row[k]]);
         const int left = (k > 0) ? (int)row[k - 1] : -1;
         const int right = (k < L - 1) ? (int)row[k + 1] : -1;
-        auto count = [&](int j) -> int {
-            const int g = A.D->code[base + j];
+        const int ns = e.num(), cur = e.own();
+        auto count = [&](int g) -> int {
             int v = 0;
             if (left >= 0) v += code_hidden(stop6, left, g);
             if (right >= 0) v += code_hidden(stop6, g, right);
             return v;
         };
-        const int curv = count(cur);
+        const int curv = count(row[k]);
         uint32_t cand = 0;
         for (int j = 0; j < ns; ++j)
-            if (j != cur && count(j) > curv) cand |= 1u << j;
+            if (j != cur && count(e.code(j)) > curv) cand |= 1u << j;
         if (cand) {
-            set_syn(A, cds, k, nth_bit(cand, uniform_int(r[2 * h + 1], (uint32_t)__popc(cand))));
+            uint32_t r[4];
+            pair_draws(A, cds, q, r);
+            row[k] = (uint8_t)e.code(nth_bit(cand, uniform_int(h ? r[3] : r[1], (uint32_t)__popc(cand))));
             dirty[cds] = 1;
         }
     };
@@ -770,28 +827,28 @@ __device__ __forceinline__ uint32_t shuffle(uint32_t x, int n) {
 __device__ __forceinline__ int perm_at(uint32_t perm, int j) { return (int)((perm >> (4 * j)) & 0xFu); }
 
 // mutationHD, mutation.cuh:390-534: codons of cds1, scored against all CDS
-__device__ void mut_hd(const MutArgs &A, int cds1, int cds2, int32_t *dirty, uint16_t *seg) {
+__device__ __forceinline__ void mut_hd(const MutArgs &A, int cds1, int cds2, int32_t *dirty, uint16_t *seg) {
     const DevJob &J = *A.J;
-    const int L = J.L, m = J.m, Ls = A.D->Ls;
+    const int L = J.L, m = J.m, Ls = A.Ls;
     const uint64_t thr = J.thr_pm;
+    uint8_t *const row = A.rows + cds1 * Ls;
     auto test = [&](int q) -> uint32_t {
         uint32_t r[4];
         pair_draws(A, cds1, q, r);
         uint32_t hm = 0;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int k = 2 * q + h;
-            if (k < L && bern(r[2 * h], thr) && A.D->pnum[k] > 1) hm |= 1u << h;
-        }
+        for (int h = 0; h < 2; ++h)
+            if (2 * q + h < L && bern(r[2 * h], thr)) hm |= 1u << h;
         return hm;
     };
     auto work = [&](int k) {
+        const SynWord e(A.syn[row[k]]);
+        const int ns = e.num(), cur = e.own();
+        if (ns == 1) return;
         uint32_t r[4];
         pair_draws(A, cds1, k >> 1, r);
-        const int ns = A.D->pnum[k];
-        const uint32_t order = shuffle(r[2 * (k & 1) + 1], ns);
-        const int base = A.D->pbase[k], cur = A.syn[cds1 * Ls + k];
-        const int g2 = A.cd6[cds2 * Ls + k];
+        const uint32_t order = shuffle((k & 1) ? r[3] : r[1], ns);
+        const int g2 = A.rows[cds2 * Ls + k];
         // every candidate's codes (the synonyms in shuffled order, slot
         // MAX_SYN the current codon) first, then the smallest distance
         // to the other CDS's codons at k (only cds1's codons change here,
@@ -799,13 +856,13 @@ __device__ void mut_hd(const MutArgs &A, int cds1, int cds2, int32_t *dirty, uin
         int gc[MAX_SYN + 1], mn[MAX_SYN + 1], pr[MAX_SYN + 1];
 #pragma unroll
         for (int j = 0; j <= MAX_SYN; ++j) {
-            gc[j] = A.D->code[base + (j == MAX_SYN ? cur : perm_at(order, j < ns ? j : ns - 1))];
+            gc[j] = e.code(j == MAX_SYN ? cur : perm_at(order, j < ns ? j : ns - 1));
             mn[j] = 127;
             pr[j] = code_mismatch(gc[j], g2);
         }
         for (int o = 0; o < m; ++o) {
             if (o == cds1) continue;
-            const int oc = A.cd6[o * Ls + k];
+            const int oc = A.rows[o * Ls + k];
 #pragma unroll
             for (int j = 0; j <= MAX_SYN; ++j) mn[j] = min(mn[j], code_mismatch(gc[j], oc));
         }
@@ -825,7 +882,7 @@ __device__ void mut_hd(const MutArgs &A, int cds1, int cds2, int32_t *dirty, uin
             }
         }
         if (best_mhd != -1 || best_pair != -1) {
-            set_syn(A, cds1, k, best);
+            row[k] = (uint8_t)e.code(best);
             dirty[cds1] = 1;
         }
     };
@@ -833,34 +890,35 @@ __device__ void mut_hd(const MutArgs &A, int cds1, int cds2, int32_t *dirty, uin
 }
 
 // mutationGC3, mutation.cuh:536-653 (probability = the parent's GC3 deviation)
-__device__ void mut_gc3(const MutArgs &A, int cds, int dir, float dev, int32_t *dirty, uint16_t *seg) {
+__device__ __forceinline__ void mut_gc3(const MutArgs &A, int cds, int dir, float dev, int32_t *dirty, uint16_t *seg) {
     const DevJob &J = *A.J;
-    const int L = J.L, Ls = A.D->Ls;
+    const int L = J.L;
     const uint64_t thr = bern_threshold(dev);
+    uint8_t *const row = A.rows + cds * A.Ls;
     auto test = [&](int q) -> uint32_t {
         uint32_t r[4];
         pair_draws(A, cds, q, r);
         uint32_t hm = 0;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int k = 2 * q + h;
-            if (k < L && bern(r[2 * h], thr) && A.D->pnum[k] > 1) hm |= 1u << h;
-        }
+        for (int h = 0; h < 2; ++h)
+            if (2 * q + h < L && bern(r[2 * h], thr)) hm |= 1u << h;
         return hm;
     };
     auto work = [&](int k) {
+        const int g = row[k];
+        const SynWord e(A.syn[g]);
+        const int ns = e.num(), cur = e.own();
+        if (ns == 1) return;
         uint32_t r[4];
         pair_draws(A, cds, k >> 1, r);
-        const int ns = A.D->pnum[k];
-        const uint32_t order = shuffle(r[2 * (k & 1) + 1], ns);
-        const int base = A.D->pbase[k], cur = A.syn[cds * Ls + k];
-        const int curg = code_gc3(A.D->code[base + cur]);
+        const uint32_t order = shuffle((k & 1) ? r[3] : r[1], ns);
+        const int curg = code_gc3(g);
         for (int j = 0; j < ns; ++j) {
             const int sh = perm_at(order, j);
             if (sh == cur) continue;
-            const int ng = code_gc3(A.D->code[base + sh]);
+            const int ng = code_gc3(e.code(sh));
             if ((dir == GC_UP && ng > curg) || (dir == GC_DOWN && ng < curg)) {
-                set_syn(A, cds, k, sh);
+                row[k] = (uint8_t)e.code(sh);
                 dirty[cds] = 1;
                 break;
             }
@@ -869,17 +927,19 @@ __device__ void mut_gc3(const MutArgs &A, int cds, int dir, float dev, int32_t *
     hits_by_wave((L + 1) >> 1, seg, test, work);
 }
 
-// mutationSL, mutation.cuh:775-969.  The accept test of the reference
-// (mutation.cuh:843,896,947) compares the parent's SL objective with the
-// integer quotient l_new / ((n-4)/2); it only needs to know whether the CDS
-// still has any stem and whether it is one full-length hairpin, which two
-// O(n) workgroup checks over the CDS's codes decide.
+// mutationSL, mutation.cuh:775-969, by one wave.  The accept test of the
+// reference (mutation.cuh:843,896,947) compares the parent's SL objective with
+// the integer quotient l_new / ((n-4)/2); it only needs to know whether the
+// CDS still has any stem and whether it is one full-length hairpin.  The first
+// and last 64 bases nearly always decide both: a complementary pair more than
+// the loop apart is a stem, one mismatch rules a full hairpin out.  The rest
+// of the CDS is read only when they do not.
 template <class SH>
-__device__ void mut_sl(const MutArgs &A, SH &sh, int32_t *dirty) {
+__device__ __forceinline__ void mut_sl(const MutArgs &A, SH &sh, int32_t *dirty) {
     const DevJob &J = *A.J;
-    const int L = J.L, n = 3 * L, Ls = A.D->Ls, tid = threadIdx.x, NT = blockDim.x;
+    const int L = J.L, n = 3 * L, lane = threadIdx.x & 63;
     const int cds = sh.pidx[10];
-    const uint8_t *row = A.cd6 + cds * Ls;
+    uint8_t *const row = A.rows + cds * A.Ls;
     const int P0 = sh.ppql[0], Lst = sh.ppql[2];
     const int l_idx = P0 / 3, r_idx = (P0 + Lst - 1) / 3;
     const int mid = (r_idx + l_idx) / 2;
@@ -889,10 +949,7 @@ __device__ void mut_sl(const MutArgs &A, SH &sh, int32_t *dirty) {
     const int den = J.den_sl;
     const float parent_sl = sh.pobj[5];
     const int trials = (odd ? 1 : 0) + 2 * half;
-    const int lane = tid & 63, wid = tid >> 6, nw = NT >> 6;
-    int *ctl = sh.misc + 11;  // [0] changed, [1] saved, [2] terminate, [3] cur_L
-    if (tid == 0) ctl[3] = Lst;
-    lds_barrier();
+    int cur_l = Lst;
     for (int t = 0; t < trials; ++t) {
         int pos;
         if (odd && t == 0) {
@@ -901,155 +958,86 @@ __device__ void mut_sl(const MutArgs &A, SH &sh, int32_t *dirty) {
             const int u = t - (odd ? 1 : 0);
             pos = (u & 1) ? r_st0 + (u >> 1) : l_st0 - (u >> 1);
         }
-        if (tid == 0) {
-            uint32_t r[4];
-            philox(A.gen, A.child, (uint32_t)t, TAG_SL, J.seed, r);
-            const int ns = A.D->pnum[pos];
-            ctl[0] = 0;
-            ctl[1] = A.syn[cds * Ls + pos];
-            if (bern(r[0], J.thr_pm) && ns > 1) {
-                const int cur = A.syn[cds * Ls + pos];
-                int nw = (int)uniform_int(r[1], (uint32_t)(ns - 1));
-                if (nw == cur) ++nw;  // mutation.cuh:827 compares with ==
-                set_syn(A, cds, pos, nw);
-                ctl[0] = 1;
-            }
+        uint32_t r[4];
+        philox(A.gen, A.child, (uint32_t)t, TAG_SL, J.seed, r);
+        const int saved = row[pos];
+        const SynWord e(A.syn[saved]);
+        const int ns = e.num();
+        const bool changed = bern(r[0], J.thr_pm) && ns > 1;
+        if (changed) {
+            int nw = (int)uniform_int(r[1], (uint32_t)(ns - 1));
+            if (nw == e.own()) ++nw;  // mutation.cuh:827 compares with ==
+            if (lane == 0) row[pos] = (uint8_t)e.code(nw);
         }
-        lds_barrier();
-        // first and last position of each base seen by this thread (positions
-        // rise, so the first hit is the first); kept in registers, one per base
-        int f[4] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF}, l4[4] = {-1, -1, -1, -1};
-        int okA = 1, okB = 1, okC = 1;
-        for (int i = tid; i < n; i += NT) {
-            const int b = code_base(row, i);
+        wave_lds_sync();
+        // the first and last 64 bases
+        const int lc = min(lane, n - 1);
+        const int f = code_base(row, lc), b = code_base(row, n - 1 - lc);
+        bool any = false;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (b == q) {
-                    f[q] = min(f[q], i);
-                    l4[q] = i;
-                }
+        for (int a = 0; a < 4; ++a) {
+            const uint64_t F = __ballot(f == a), B = __ballot(b == (a ^ 3));
+            if (F && B && n - 1 - (int)__builtin_ctzll(B) - (int)__builtin_ctzll(F) > MIN_HAIRPIN) any = true;
         }
-        for (int i = tid; i < den; i += NT) {
-            okA &= ((code_base(row, i) ^ code_base(row, n - 1 - i)) == 3);
+        // the full hairpin's pairs (i, n-1-i), and for odd n (i, n-2-i) or (1+i, n-1-i)
+        auto pairs_hold = [&](int i) -> int {
+            const int x = code_base(row, i), y = code_base(row, n - 1 - i);
+            int ok = (x ^ y) == 3 ? 1 : 0;
             if (n & 1) {
-                okB &= ((code_base(row, i) ^ code_base(row, n - 2 - i)) == 3);
-                okC &= ((code_base(row, 1 + i) ^ code_base(row, n - 1 - i)) == 3);
+                ok |= ((x ^ code_base(row, n - 2 - i)) == 3) ? 2 : 0;
+                ok |= ((code_base(row, 1 + i) ^ y) == 3) ? 4 : 0;
             }
-        }
-        // wave minima, maxima and conjunctions (DPP, ballots), combined over
-        // the waves by thread 0
-        const bool allA = __ballot(!okA) == 0, allB = __ballot(!okB) == 0, allC = __ballot(!okC) == 0;
+            return ok;
+        };
+        int full = 0;
+        {
+            const int ok = lane < den ? pairs_hold(lane) : 7;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            f[q] = wave_min_i32(f[q]);
-            l4[q] = wave_max_i32(l4[q]);
+            for (int q = 0; q < 3; ++q) full |= __ballot(!((ok >> q) & 1)) == 0 ? 1 << q : 0;
         }
-        if (lane == 0) {
-            int *w = sh.slw + wid * 11;
+        if (!any) {  // every base
+            int first[4] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF}, last[4] = {-1, -1, -1, -1};
+            for (int i = lane; i < n; i += 64) {
+                const int x = code_base(row, i);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (x == q) {
+                        first[q] = min(first[q], i);
+                        last[q] = i;
+                    }
+            }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                w[q] = f[q];
-                w[4 + q] = l4[q];
+                first[q] = wave_min_i32(first[q]);
+                last[q] = wave_max_i32(last[q]);
             }
-            w[8] = allA;
-            w[9] = allB;
-            w[10] = allC;
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                if (first[a] != 0x7FFFFFFF && last[a ^ 3] >= 0 && last[a ^ 3] - first[a] > MIN_HAIRPIN) any = true;
         }
-        lds_barrier();
-        if (tid == 0) {
-            int first[4] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF}, last[4] = {-1, -1, -1, -1};
-            int full[3] = {1, 1, 1};
-            for (int w = 0; w < nw; ++w) {
-                const int *v = sh.slw + w * 11;
+        if (full && den > 64) {  // every pair
+            int ok = 7;
+            for (int i = lane; i < den; i += 64) ok &= pairs_hold(i);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    first[q] = min(first[q], v[q]);
-                    last[q] = max(last[q], v[4 + q]);
-                }
-#pragma unroll
-                for (int q = 0; q < 3; ++q) full[q] &= v[8 + q];
-            }
-            bool any = false;
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const int b = a ^ 3;
-                if (first[a] != 0x7FFFFFFF && last[b] >= 0 && last[b] - first[a] > MIN_HAIRPIN) any = true;
-            }
-            bool is_full = false;
-            if (den > 0) {
-                if (full[0] && (n - 1 - 2 * (den - 1)) > MIN_HAIRPIN) is_full = true;
-                if ((n & 1) && (full[1] || full[2]) && (n - 2 - 2 * (den - 1)) > MIN_HAIRPIN) is_full = true;
-            }
-            if (any) ctl[3] = is_full ? den : 0;
-            const float rhs = (float)(den > 0 ? ctl[3] / den : 0);
-            ctl[2] = parent_sl > rhs;
-            if (!ctl[2] && ctl[0]) set_syn(A, cds, pos, ctl[1]);
-            if (ctl[2] && ctl[0]) dirty[cds] = 1;
+            for (int q = 0; q < 3; ++q)
+                if (__ballot(!((ok >> q) & 1))) full &= ~(1 << q);
         }
-        lds_barrier();
-        if (ctl[2]) break;
-    }
-}
-
-// Bit planes of the changed CDS into the job's plane buffer: bit p of the
-// sequence plane is position p, of the reverse-complement plane position
-// n-1-p complemented; positions past n are zero; a word is (low bits, high
-// bits) of 32 positions.  The forward words are built 32 codons (three words)
-// per lane from the codes, four codons per 32-bit step, and staged in LDS
-// (stage + c * stride for CDS c); the reverse-complement word j is the
-// forward window of bits n-32-32j .. n-1-32j, bit-reversed and inverted.
-// rows: the CDS's code rows (stride Ls); dl: the changed CDS, nd of them.
-__device__ void build_planes(const uint8_t *rows, int Ls, int L, const int *dl, int nd, uint2 *stage, int stride,
-                             uint2 *gbase) {
-    const int n = 3 * L, W = scan_words(n), ng = (W + 2) / 3, tid = threadIdx.x, NT = blockDim.x;
-    const int nwd = Ls >> 2;
-    for (int i = tid; i < nd * ng; i += NT) {
-        const int e = i / ng, g = i - e * ng, c = dl[e];
-        const uint32_t *row = (const uint32_t *)(rows + c * Ls);
-        uint32_t lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {  // codons 32g + 4t .. 32g + 4t + 3 (zero past the row)
-            const int q = 8 * g + t;
-            const uint32_t d = q < nwd ? row[q] : 0u;
-            // per byte the three bases' low (high) bits in position order
-            const uint32_t l = ((d >> 4) & 0x01010101u) | ((d >> 1) & 0x02020202u) | ((d << 2) & 0x04040404u);
-            const uint32_t h = ((d >> 5) & 0x01010101u) | ((d >> 2) & 0x02020202u) | ((d << 1) & 0x04040404u);
-            const uint32_t l12 = (l & 7u) | ((l >> 5) & 0x38u) | ((l >> 10) & 0x1C0u) | ((l >> 15) & 0xE00u);
-            const uint32_t h12 = (h & 7u) | ((h >> 5) & 0x38u) | ((h >> 10) & 0x1C0u) | ((h >> 15) & 0xE00u);
-            const int b = 12 * t, w = b >> 5, o = b & 31;  // compile-time after unrolling
-            lo[w] |= l12 << o;
-            hi[w] |= h12 << o;
-            if (o > 20) {
-                lo[w + 1] |= l12 >> (32 - o);
-                hi[w + 1] |= h12 >> (32 - o);
-            }
+        bool is_full = false;
+        if (den > 0) {
+            if ((full & 1) && (n - 1 - 2 * (den - 1)) > MIN_HAIRPIN) is_full = true;
+            if ((n & 1) && (full & 6) && (n - 2 - 2 * (den - 1)) > MIN_HAIRPIN) is_full = true;
         }
-        uint2 *st = stage + (size_t)e * stride;
-#pragma unroll
-        for (int u = 0; u < 3; ++u)
-            if (3 * g + u < W) st[3 * g + u] = make_uint2(lo[u], hi[u]);
-        if (g == 0) st[W] = make_uint2(0u, 0u);
-    }
-    lds_barrier();
-    for (int i = tid; i < nd * W; i += NT) {
-        const int e = i / W, j = i - e * W, c = dl[e];
-        const uint2 *st = stage + (size_t)e * stride;
-        uint2 *sp = gbase + (size_t)c * 2 * W, *rp = sp + W;
-        gstore((uint64_t *)(sp + j), (uint64_t)st[j].x | ((uint64_t)st[j].y << 32));
-        const int s0 = n - 32 - 32 * j;  // first bit of the forward window
-        uint32_t wl = 0, wh = 0;
-        if (s0 >= 0) {
-            const uint2 a = st[s0 >> 5], b = st[(s0 >> 5) + 1];
-            wl = __builtin_amdgcn_alignbit(b.x, a.x, (uint32_t)(s0 & 31));
-            wh = __builtin_amdgcn_alignbit(b.y, a.y, (uint32_t)(s0 & 31));
-        } else if (s0 > -32) {
-            wl = st[0].x << (-s0);
-            wh = st[0].y << (-s0);
+        if (any) cur_l = is_full ? den : 0;
+        const float rhs = (float)(den > 0 ? cur_l / den : 0);
+        const bool done = parent_sl > rhs;
+        if (changed) {
+            if (done)
+                dirty[cds] = 1;
+            else if (lane == 0)
+                row[pos] = (uint8_t)saved;
         }
-        const int cnt = n - 32 * j;  // positions of word j below n
-        const uint32_t mask = cnt >= 32 ? ~0u : (cnt <= 0 ? 0u : (1u << cnt) - 1u);
-        const uint32_t rl = ~__builtin_bitreverse32(wl) & mask, rh = ~__builtin_bitreverse32(wh) & mask;
-        gstore((uint64_t *)(rp + j), (uint64_t)rl | ((uint64_t)rh << 32));
+        wave_lds_sync();
+        if (done) break;
     }
 }
 
@@ -1068,7 +1056,7 @@ __device__ __forceinline__ void clear_niche(const DevJob &J, int i0, int step) {
 
 // The index of the c-th survivor (0-based, ascending pool index) in the
 // survivor mask of W words: wave-uniform, every lane of the wave takes part.
-__device__ int survivor_at(const uint64_t *selm, int W, int c, uint64_t first) {
+__device__ __forceinline__ int survivor_at(const uint64_t *selm, int W, int c, uint64_t first) {
     const int lane = threadIdx.x & 63;
     int base = 0;
     uint64_t x = lane < W ? first : 0ull;  // (word `lane` of the mask, loaded by the caller)
@@ -1108,13 +1096,15 @@ __device__ int survivor_at(const uint64_t *selm, int W, int c, uint64_t first) {
 // k_design: one workgroup per design.
 //   INIT       random genome (design 0: best-CAI codons), genPopulation,
 //              utils.cuh:1047-1104, then evaluation into buffer 0
-//   EVAL       evaluation of genome[0][d] into buffer 0
+//   EVAL       evaluation of genome[0][d] (synonym indices) into buffer 0
 //   OFFSPRING  survivor copy, mutation, evaluation (mutationKernel)
-// A design's genome row is m CDS rows of stride Ls; it moves between HBM and
-// LDS in 16-byte words.
+// A design's genome row is m CDS rows of codon codes, of stride Ls; it moves
+// between HBM and LDS in 16-byte words.  item_base of INIT: 1 when the pool
+// has not been written yet (rows N .. 2N-1 are then set to every codon's first
+// synonym).
 // ---------------------------------------------------------------------------
-template <int MODE, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_design(const DevJob *__restrict__ jobs, const int2 *__restrict__ items,
+template <int MODE, int NT, int WAVES>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_design(const DevJob *__restrict__ jobs, const int2 *__restrict__ items,
                                                 uint32_t *__restrict__ stem_list, int32_t *stem_ctl, int stem_group,
                                                 int stem_cap, int item_base) {
     extern __shared__ __align__(16) uint8_t dyn[];
@@ -1122,23 +1112,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     const int2 it = items[blockIdx.x];
     const DevJob &J = jobs[it.x];
     const int L = J.L, m = J.m, Ls = J.Ls, N = J.N;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G16 = (m * Ls) >> 4;  // 16-byte words of a design row
-    const int SA = syn_stride(L);
-    uint8_t *pbase = dyn + DL_POS;
-    uint8_t *pnum = pbase + Ls;
-    uint8_t *syn = pnum + Ls;       // rows at stride Ls; the planes' stage afterwards (stride SA)
-    uint8_t *cd6 = syn + m * SA;
-    CdsStat *cst = (CdsStat *)(cd6 + m * Ls);
+    const int64_t *lw6 = (const int64_t *)dyn;
+    const uint64_t *syn6 = (const uint64_t *)(dyn + DL_SYN);
+    uint8_t *rows = dyn + DL_ROWS;
+    CdsStat *cst = (CdsStat *)(rows + m * Ls);
     const int npair = m * (m - 1) / 2;
-    const DesignLds D{(const int64_t *)(dyn + DL_LW6), dyn + DL_CODE, pbase, pnum, J.stop6, Ls};
 
     // The descriptor fields of the staging phase, read before its stores (a
     // store through a pool pointer could alias the descriptor as far as the
     // compiler knows, and would make every later field a reload).
-    const uint8_t *const pos = J.pos;
-    const int64_t *const lw6 = J.lw6;
-    const uint8_t *const ctab = J.code;
     int8_t *const genome0 = J.genome[0], *const genome1 = J.genome[1];
     float *const obj0 = J.obj[0], *const obj1 = J.obj[1];
     int8_t *const oidx0 = J.oidx[0], *const oidx1 = J.oidx[1];
@@ -1147,36 +1131,25 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     int32_t *const hdp0 = J.hdp[0], *const hdp1 = J.hdp[1];
     int32_t *const np = J.np;
     SelAcc *const acc = J.acc;
-    // stage the tables and the synonym ranges (rows pbase and pnum, as the
-    // job keeps them: padding positions have one synonym at codon 0)
     // Every load of the set-up is issued before the first LDS store (a store
-    // under a branch would wait for its own load first): the tables, the
-    // first words of the synonym ranges, the generation counter and the first
-    // words of the survivor mask.
-    const int npw = (2 * Ls) >> 4;  // 16-byte words of the rows pbase and pnum
-    const uint8_t *p_pos = pos, *p_code = ctab;
-    const int64_t *p_lw = lw6;
+    // under a branch would wait for its own load first): the two tables (the
+    // log weights, then the synonym words: 128 8-byte words together), the
+    // generation counter and the first words of the survivor mask.
+    const int64_t *p_tab = J.lw6;
     const uint64_t *p_sel = J.selm;
     const SelState *p_st = J.st;
     int W = J.W;
-    asm volatile("" : "+s"(p_pos), "+s"(p_code), "+s"(p_lw), "+s"(p_sel), "+s"(p_st), "+s"(W));
-    int64_t v_lw = gload(p_lw + (tid & 63));
-    uint32_t v_code = gload(p_code + (tid & 63));
-    u32x4 v_pos = gload((const u32x4 *)p_pos + min(tid, npw - 1));
+    asm volatile("" : "+s"(p_tab), "+s"(p_sel), "+s"(p_st), "+s"(W));
+    int64_t v_tab = gload(p_tab + (tid & 127));
     uint32_t g0 = 0;
     uint64_t sel0 = 0;
     if (MODE == 2) {
         g0 = gload(&p_st->gen);
-        sel0 = gload(p_sel + min(tid & 63, W - 1));
+        sel0 = gload(p_sel + min(lane, W - 1));
     }
     // (taken here, so that no load is moved into the branches below)
-    asm volatile("" : "+v"(v_lw), "+v"(v_code), "+v"(v_pos), "+v"(sel0));
-    if (tid < 64)
-        ((int64_t *)(dyn + DL_LW6))[tid] = v_lw;
-    else if (tid < 128)
-        dyn[DL_CODE + tid - 64] = (uint8_t)v_code;
-    if (tid < npw) ((u32x4 *)pbase)[tid] = v_pos;
-    for (int i = tid + NT; i < npw; i += NT) ((u32x4 *)pbase)[i] = gload((const u32x4 *)pos + i);
+    asm volatile("" : "+v"(v_tab), "+v"(sel0));
+    if (tid < 128) ((int64_t *)dyn)[tid] = v_tab;
     if (tid < MAX_M) sh.dirty[tid] = (MODE != 2);
     uint32_t gen = 0;
     int dst = 0, out_slot = it.y, src = 0, parent = 0;
@@ -1187,28 +1160,45 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
         out_slot = N + it.y;
         parent = survivor_at(p_sel, W, it.y, sel0);
     }
-    u32x4 *syn4 = (u32x4 *)syn;
+    u32x4 *rows4 = (u32x4 *)rows;
     if (MODE == 0) {
-        // positions take their synonym counts from the job's rows (the LDS
-        // copy above is not yet visible to every thread)
         const int d = it.y;
+        const uint8_t *const pos = J.pos, *const ctab = J.code;
+        uint8_t *const base = (uint8_t *)genome0 + (size_t)(N + d) * m * Ls;
         for (int c = 0; c < m; ++c)
             for (int k = tid; k < Ls; k += NT) {
-                int s = 0;
-                if (k >= L) {
-                    s = 0;
-                } else if (d == 0) {
-                    s = (int)gload(pos + Ls + k) - 1;
-                } else {
-                    uint32_t r[4];
-                    philox(0u, (uint32_t)d, (uint32_t)(c * L + k), TAG_INIT, J.seed, r);
-                    s = (int)uniform_int(r[0], (uint32_t)gload(pos + Ls + k));
+                int v = 0, first = 0;
+                if (k < L) {
+                    const int g = (int)gload(pos + k), ns = (int)gload(pos + Ls + k);
+                    int s = ns - 1;
+                    if (d != 0) {
+                        uint32_t r[4];
+                        philox(0u, (uint32_t)d, (uint32_t)(c * L + k), TAG_INIT, J.seed, r);
+                        s = (int)uniform_int(r[0], (uint32_t)ns);
+                    }
+                    v = (int)gload(ctab + g + s);
+                    first = (int)gload(ctab + g);
                 }
-                syn[c * Ls + k] = (uint8_t)s;
+                rows[c * Ls + k] = (uint8_t)v;
+                if (item_base && N + d < J.P) gstore(base + c * Ls + k, (uint8_t)first);
             }
     } else if (MODE == 1) {
-        const u32x4 *sg = (const u32x4 *)(genome0 + (size_t)it.y * m * Ls);
-        for (int i = tid; i < G16; i += NT) syn4[i] = gload(sg + i);
+        // synonym indices to codes, four a word; the padding positions are
+        // forced to code 0
+        const uint8_t *const pos = J.pos, *const ctab = J.code;
+        const uint32_t *sg = (const uint32_t *)(genome0 + (size_t)it.y * m * Ls);
+        const int nwd = Ls >> 2;
+        uint32_t *c4 = (uint32_t *)rows;
+        for (int c = 0; c < m; ++c)
+            for (int q = tid; q < nwd; q += NT) {
+                const int left = L - 4 * q;  // positions of the word below L
+                const uint32_t keep = left >= 4 ? ~0u : (left <= 0 ? 0u : (1u << (8 * left)) - 1u);
+                const uint32_t g = (gload(sg + c * nwd + q) & keep) + gload((const uint32_t *)pos + q);  // bytewise
+                uint32_t code = 0;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) code |= (uint32_t)gload(ctab + ((g >> (8 * b)) & 0x3Fu)) << (8 * b);
+                c4[c * nwd + q] = code & keep;
+            }
     } else {
         const int c = it.y;
         // the survivor copy (copySolution, utils.cuh:1106-1147): every load
@@ -1247,7 +1237,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             for (int u = 0; u < 4; ++u)
                 if (i0 + u * NT < G16) {
                     gstore(sg + i0 + u * NT, v[u]);
-                    syn4[i0 + u * NT] = v[u];
+                    rows4[i0 + u * NT] = v[u];
                 }
         }
         if (tid < 16) {
@@ -1277,93 +1267,94 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             gstore(np + c, 0);
             gstore(np + N + c, 0);
         }
-        if (c == 0 && tid >= 128 && tid < 128 + ACC_WORDS) gstore((uint32_t *)acc + tid - 128, acc_clear_word(tid - 128));
+        if (c == 0 && tid < ACC_WORDS) gstore((uint32_t *)acc + tid, acc_clear_word(tid));
         clear_niche(J, c * NT + tid, N * NT);  // (and the association from cleared niche arrays)
     }
-    lds_barrier();  // tables, synonym ranges, genome row and records
-    // codon codes of the row, four per thread step; the padding positions
-    // are forced to synonym 0 and code 0 (the table reads stay below 64: a
-    // padding position reads codon 0)
-    {
-        const int nwd = Ls >> 2;
-        const uint32_t *pb4 = (const uint32_t *)pbase;
-        uint32_t *s4 = (uint32_t *)syn, *c4 = (uint32_t *)cd6;
-        for (int c = 0; c < m; ++c)
-            for (int q = tid; q < nwd; q += NT) {
-                const int left = L - 4 * q;  // positions of the word below L
-                const uint32_t keep = left >= 4 ? ~0u : (left <= 0 ? 0u : (1u << (8 * left)) - 1u);
-                const uint32_t s = s4[c * nwd + q] & keep;
-                const uint32_t g = s + pb4[q];  // bytewise: synonyms < 6, first codons < 64
-                uint32_t code = 0;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) code |= (uint32_t)D.code[(g >> (8 * b)) & 0xFFu] << (8 * b);
-                s4[c * nwd + q] = s;
-                c4[c * nwd + q] = code & keep;
-            }
-    }
-    lds_barrier();
+    lds_barrier();  // tables, genome row and records
     if (MODE == 2) {
         const int c = it.y;
         uint32_t r[4];
         philox(gen, (uint32_t)c, 0u, TAG_TYPE, J.seed, r);
         const int type = (int)uniform_int(r[0], (uint32_t)(NOBJ + 1));  // main.cu:172-178
-        const MutArgs A{&J, &D, syn, cd6, gen, (uint32_t)c};
+        const MutArgs A{&J, syn6, rows, Ls, gen, (uint32_t)c};
         switch (type) {  // main.cu:181-211
         case 0: mut_random(A, sh.dirty); break;
         case 1: mut_cai(A, sh.pidx[0], sh.dirty); break;
-        case 2: mut_cbp(A, sh.pidx[2], sh.dirty, sh.hitq[tid >> 6]); break;
-        case 3: mut_hsc(A, sh.pidx[4], sh.dirty, sh.hitq[tid >> 6]); break;
-        case 4: mut_hd(A, sh.pidx[6], sh.pidx[7], sh.dirty, sh.hitq[tid >> 6]); break;
+        case 2: mut_cbp(A, sh.pidx[2], sh.dirty, sh.hitq[wid]); break;
+        case 3: mut_hsc(A, sh.pidx[4], sh.dirty, sh.hitq[wid]); break;
+        case 4: mut_hd(A, sh.pidx[6], sh.pidx[7], sh.dirty, sh.hitq[wid]); break;
         case 5:
             if (sh.pidx[9] == GC_UP || sh.pidx[9] == GC_DOWN)
-                mut_gc3(A, sh.pidx[8], sh.pidx[9], sh.pobj[4], sh.dirty, sh.hitq[tid >> 6]);
+                mut_gc3(A, sh.pidx[8], sh.pidx[9], sh.pobj[4], sh.dirty, sh.hitq[wid]);
             break;
-        default: mut_sl(A, sh, sh.dirty); break;
+        default:
+            if (wid == 0) mut_sl(A, sh, sh.dirty);
+            break;
         }
         lds_barrier();
     }
-
-    float *oobj = (dst ? obj1 : obj0) + (size_t)out_slot * NOBJ;
-    __shared__ float s_obj[NOBJ];
-    __shared__ int32_t s_idx[2 * NOBJ];
+    const uint32_t dmask = (uint32_t)__ballot(lane < m && sh.dirty[min(lane, MAX_M - 1)] != 0);
     // the design's genome row is final: its stores drain during the evaluation
-    u32x4 *og = (u32x4 *)((dst ? genome1 : genome0) + (size_t)out_slot * m * Ls);
-    for (int i = tid; i < G16; i += NT) gstore(og + i, syn4[i]);
-    evaluate(J, D, cd6, cst, MODE == 2, sh, s_obj, s_idx);
-    {  // planes of the changed CDS for k_stem, staged where the syn rows were
-        int nd = 0;
-        for (int c = 0; c < m; ++c) {
-            if (tid == 0 && sh.dirty[c]) sh.dlist[nd] = c;
-            nd += sh.dirty[c] != 0;
-        }
-        lds_barrier();  // the syn rows are stored and the list is written
-        build_planes(cd6, Ls, L, sh.dlist, nd, (uint2 *)syn, SA / 8,
-                     J.planes + (size_t)out_slot * m * 2 * scan_words(3 * L));
+    if (MODE != 1) {
+        u32x4 *og = (u32x4 *)((dst ? genome1 : genome0) + (size_t)out_slot * m * Ls);
+        for (int i = tid; i < G16; i += NT) gstore(og + i, rows4[i]);
     }
-    if (tid < NOBJ - 1) gstore(oobj + tid, s_obj[tid]);  // objective 5: k_stem_finish
-    if (tid < 2 * NOBJ && tid != 10) gstore((dst ? oidx1 : oidx0) + (size_t)out_slot * 2 * NOBJ + tid, (int8_t)s_idx[tid]);
-    if (tid < m) gstore_stat((dst ? cst1 : cst0) + (size_t)out_slot * m + tid, cst[tid]);
-    if (tid < npair) gstore((dst ? hdp1 : hdp0) + (size_t)out_slot * npair + tid, sh.hd[tid]);
-    // CDS evaluated (k_stem scans the same ones); the unchanged CDS's longest
-    // stem.  The first lane of the last wave does this: a wave's wait for the
-    // list atomic's result also waits for the wave's earlier stores, and the
-    // rows, planes and records go to the first waves first.
-    if (tid == NT - 64) {
-        unsigned long long nd = 0;
-        int lmax = 0;
-        for (int c = 0; c < m; ++c) {
-            nd += sh.dirty[c] != 0;
-            if (!sh.dirty[c]) lmax = max(lmax, cst[c].l);
-        }
-        gstore(J.stem_max + out_slot, lmax);  // (k_dominance counts the offspring's changed CDS)
-        if (MODE == MODE_OFFSPRING && nd) {  // the changed CDS for k_stem_list, in the child's sublist
+    design_tasks(J, lw6, (const uint32_t *)rows, dmask, MODE == 2, cst, sh,
+                 J.planes + (size_t)out_slot * m * 2 * scan_words(3 * L), wid, NT / 64);
+    lds_barrier();
+    if (wid == 0)
+        design_objectives(J, cst, sh, (dst ? obj1 : obj0) + (size_t)out_slot * NOBJ,
+                          (dst ? oidx1 : oidx0) + (size_t)out_slot * 2 * NOBJ);
+    if (tid >= NT - 128) {  // the records, by the wave(s) before the last lane's work below
+        const int t = tid - (NT - 128);
+        if (t < m) gstore_stat((dst ? cst1 : cst0) + (size_t)out_slot * m + t, cst[t]);
+        if (t < npair) gstore((dst ? hdp1 : hdp0) + (size_t)out_slot * npair + t, sh.hd[t]);
+    }
+    // the unchanged CDS's longest stem; the changed CDS for k_stem_list
+    if (wid == NT / 64 - 1) {
+        const int l = lane < m && !((dmask >> lane) & 1u) ? cst[lane].l : 0;
+        const int lmax = wave_max_nonneg(l);
+        if (lane == 0) gstore(J.stem_max + out_slot, lmax);  // (k_dominance counts the offspring's changed CDS)
+        if (MODE == MODE_OFFSPRING && dmask) {  // in the child's sublist
             const int item = item_base + (int)blockIdx.x, k = item / stem_group;
-            int e = atomicAdd(stem_ctl + k, (int)nd);
-            for (int c = 0; c < m; ++c)
-                if (sh.dirty[c] && e < stem_cap)
-                    gstore(stem_list + (size_t)k * stem_cap + e++, ((uint32_t)item << 4) | (uint32_t)c);
+            int e = 0;
+            if (lane == 0) e = atomicAdd(stem_ctl + k, (int)__popc(dmask));
+            e = __builtin_amdgcn_readfirstlane(e) + (int)__popc(dmask & ((1u << (lane & 31)) - 1u));
+            if (lane < m && ((dmask >> lane) & 1u) && e < stem_cap)
+                gstore(stem_list + (size_t)k * stem_cap + e, ((uint32_t)item << 4) | (uint32_t)lane);
         }
     }
+}
+
+// Codon codes of `rows` pool rows (stride Ls) to synonym indices, rows packed
+// at L bytes: what a caller reads.  A thread converts 16 consecutive output
+// bytes; a code no row holds yet (0 in an unwritten row is not one: see INIT)
+// does not occur.
+__global__ __launch_bounds__(256) void k_export(const DevJob *__restrict__ jobs, const uint8_t *__restrict__ src,
+                                                uint8_t *__restrict__ dst, int rows) {
+    __shared__ uint8_t own[64];
+    const DevJob &J = jobs[0];
+    const uint32_t L = (uint32_t)J.L, Ls = (uint32_t)J.Ls;
+    const uint64_t *syn = (const uint64_t *)(J.lw6 + 64);
+    if (threadIdx.x < 64) own[threadIdx.x] = (uint8_t)SynWord(gload(syn + threadIdx.x)).own();
+    __syncthreads();
+    const uint64_t total = (uint64_t)rows * L;
+    const uint64_t o0 = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 16;
+    if (o0 >= total) return;
+    uint64_t r = o0 / L;
+    uint32_t k = (uint32_t)(o0 - r * L);
+    const uint8_t *p = src + r * Ls + k;
+    u32x4 v = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        if (o0 + i < total) v[i >> 2] |= (uint32_t)own[gload(p) & 63] << (8 * (i & 3));
+        ++p;
+        if (++k == L) {
+            k = 0;
+            p += Ls - L;
+        }
+    }
+    gstore((u32x4 *)(dst + o0), v);  // (the buffer holds at least 15 bytes past the packed rows, or they fill it)
 }
 
 // Buffer and slot of the design an evaluation work item refers to: children
@@ -1857,10 +1848,6 @@ __device__ __forceinline__ unsigned long long asf_key(float v, int id) {
     return ((unsigned long long)ord_bits(v) << 32) | (uint32_t)id;
 }
 
-__device__ __forceinline__ float lane_of(float v, int l) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
 // Extreme points (findExtremePoints, sorting.cuh:601-683) settled axis by
 // axis against the previous ones, by one wave.  The candidate rows are the
 // previous extremes (0-5) and the rows of the first front's ASF minima of the
@@ -2095,13 +2082,6 @@ struct SettleShared {
     float crow[2 * NOBJ][NOBJ];                   // candidate rows of the extremes
     float ext[NOBJ * NOBJ], nadir[NOBJ];
 };
-
-// Orders a wave's LDS writes before its own later reads (other lanes' values).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
 
 // The extreme points settled against the previous ones (prev: lane i < 36
 // holds value i of them) and the nadir point (updateNadirValue_HYP with the
@@ -2935,21 +2915,30 @@ hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n,
                          uint32_t *stem_list, int32_t *stem_ctl, StemList sl, int item_base, int threads) {
     if (n <= 0) return hipSuccess;
     switch (mode) {
-    case 0: hipLaunchKernelGGL((k_design<0, 256>), dim3(n), dim3(256), lds, s, jobs, items, nullptr, nullptr, 1, 0, 0); break;
-    case 1: hipLaunchKernelGGL((k_design<1, 256>), dim3(n), dim3(256), lds, s, jobs, items, nullptr, nullptr, 1, 0, 0); break;
+    case 0: hipLaunchKernelGGL((k_design<0, 256, 6>), dim3(n), dim3(256), lds, s, jobs, items, nullptr, nullptr, 1, 0, item_base); break;
+    case 1: hipLaunchKernelGGL((k_design<1, 256, 6>), dim3(n), dim3(256), lds, s, jobs, items, nullptr, nullptr, 1, 0, 0); break;
     default:
         if (!stem_list || !stem_ctl || sl.cap <= 0 || sl.group <= 0 || sl.groups > STEM_MAX_GROUPS || item_base < 0)
             return hipErrorInvalidValue;
-        if (threads == 256)
-            hipLaunchKernelGGL((k_design<2, 256>), dim3(n), dim3(256), lds, s, jobs, items, stem_list, stem_ctl,
+        if (threads == 256 && n > DESIGN_MANY)
+            hipLaunchKernelGGL((k_design<2, 256, 8>), dim3(n), dim3(256), lds, s, jobs, items, stem_list, stem_ctl,
+                               sl.group, sl.cap, item_base);
+        else if (threads == 256)
+            hipLaunchKernelGGL((k_design<2, 256, 6>), dim3(n), dim3(256), lds, s, jobs, items, stem_list, stem_ctl,
                                sl.group, sl.cap, item_base);
         else if (threads == 512)
-            hipLaunchKernelGGL((k_design<2, 512>), dim3(n), dim3(512), lds, s, jobs, items, stem_list, stem_ctl,
+            hipLaunchKernelGGL((k_design<2, 512, 6>), dim3(n), dim3(512), lds, s, jobs, items, stem_list, stem_ctl,
                                sl.group, sl.cap, item_base);
         else
             return hipErrorInvalidValue;
         break;
     }
+    return hipGetLastError();
+}
+hipError_t launch_export(const DevJob *job, const int8_t *src, int8_t *dst, int rows, int L, hipStream_t s) {
+    const size_t n = ((size_t)rows * L + 4095) / 4096;
+    if (!n) return hipSuccess;
+    hipLaunchKernelGGL(k_export, dim3((unsigned)n), dim3(256), 0, s, job, (const uint8_t *)src, (uint8_t *)dst, rows);
     return hipGetLastError();
 }
 int stem_parts_of(int L) { return stem_parts(3 * L); }
@@ -3102,8 +3091,9 @@ hipError_t launch_zero_np(const DevJob *jobs, int njobs, hipStream_t s) {
 
 hipError_t set_design_lds_limit(size_t bytes) {
     return raise_lds_limit(g_design_lds, bytes, [](int b) {
-        const void *fns[] = {(const void *)k_design<0, 256>, (const void *)k_design<1, 256>,
-                             (const void *)k_design<2, 256>, (const void *)k_design<2, 512>};
+        const void *fns[] = {(const void *)k_design<0, 256, 6>, (const void *)k_design<1, 256, 6>,
+                             (const void *)k_design<2, 256, 6>,
+                             (const void *)k_design<2, 256, 8>, (const void *)k_design<2, 512, 6>};
         for (const void *f : fns) {
             const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, b);
             if (e != hipSuccess) return e;

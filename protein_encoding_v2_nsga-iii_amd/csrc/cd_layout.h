@@ -135,11 +135,14 @@ struct DevJob {
     const uint8_t *pos;    // [2][Ls]: per position the first codon of its amino acid, then its synonym count
                            // (padding positions: codon 0, one synonym)
     const uint8_t *code;   // [64] code of each codon of the table
-    const int64_t *lw6;    // [64] 2^40-scaled log weights by code
+    const int64_t *lw6;    // [64] 2^40-scaled log weights by code, then [64] synonym words by code: the codes of
+                           // synonyms 0-4 in bits 0-29, of synonym 5 in bits 32-37, their number in bits 40-42, the
+                           // code's own index in bits 44-46
     const int64_t *cpfx6;  // [64*64] 2^40-scaled pair scores by codes (0 where either is a stop)
     const float *cps6;     // [64*64] pair scores by codes (0 where either is a stop)
     const float *refpts;   // [R][REF_STRIDE]: the point's six weights, the sum of their squares, 0
-    int8_t *genome[2];     // [P][m][Ls] synonym indices, CDS rows padded with zeros to Ls
+    int8_t *genome[2];     // [P][m][Ls] codon codes, CDS rows padded with zeros to Ls (a job that only evaluates
+                           // holds the synonym indices it was given)
     float *obj[2];         // [P][6]
     int8_t *oidx[2];       // [P][12]
     int32_t *pql[2];       // [P][4] (p, q, l, 0)
