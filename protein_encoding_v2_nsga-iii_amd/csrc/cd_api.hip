@@ -179,7 +179,7 @@ Layout layout(int L, int m, int N, int P, int R, int W, int n_dom, int n_asc, bo
         o.off = s.add((size_t)N * sizeof(int2));
         o.planes = s.add((size_t)P * m * cd::cds_plane_bytes(L));
         o.stem_max = s.add((size_t)P * 4);
-        o.slist = s.add(cd::stem_list_entries(N, m) * 4);
+        o.slist = s.add(cd::stem_list_entries(N, m) * sizeof(uint2));
         o.sctl = s.add((size_t)cd::STEM_MAX_GROUPS * 4);
     }
     for (int b = 0; b < (sel_only ? 1 : 2); ++b) o.obj[b] = s.add((size_t)P * 6 * 4);
@@ -382,11 +382,10 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
         for (int c = 0; c < J->N; ++c) off[c] = make_int2(0, c);
         up.add(o.off, off.data(), off.size());
         J->d_off = (int2 *)(base + o.off);
-        J->d_slist = (uint32_t *)(base + o.slist);  // the counts in d_sctl start at zero with the cleared allocation
+        J->d_slist = (uint2 *)(base + o.slist);  // the counts in d_sctl start at zero with the cleared allocation
         J->d_sctl = (int32_t *)(base + o.sctl);
         J->lds = cd::design_lds_bytes(J->L, J->m);
         J->stem_lds = cd::stem_lds_bytes(J->L);
-        J->stem_parts = cd::stem_parts_of(J->L);
     }
     const auto ref = das_dennis(d->H);
     up.add(o.ref, ref.data(), ref.size());
@@ -459,7 +458,7 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
 hipError_t enqueue_designs(const Launch &w, int mode, const int2 *items, int n_items, hipStream_t s, bool fresh = false) {
     hipError_t e = cd::launch_design(mode, w.jobs, items, n_items, w.lds, s, nullptr, nullptr, cd::StemList{0, 0, 0},
                                      fresh ? 1 : 0);
-    if (e == hipSuccess) e = cd::launch_stem(mode, w.jobs, items, n_items, w.mg, w.stem_parts, w.stem_lds, s);
+    if (e == hipSuccess) e = cd::launch_stem(mode, w.jobs, items, n_items, w.mg, w.stem_lds, s);
     if (e == hipSuccess) e = cd::launch_stem_finish(mode, w.jobs, items, n_items, s);
     return e;
 }
@@ -474,7 +473,7 @@ hipError_t enqueue_generation(const Launch &w, hipStream_t s, hipEvent_t *ev) {
     // dominance, fronts, association, niching
     auto mark = [&](int k) { return ev ? hipEventRecord(ev[k], s) : hipSuccess; };
     hipError_t e = mark(0);
-    const cd::StemList sl = cd::stem_list_geom(w.n_off, w.mg);
+    const cd::StemList sl = cd::stem_list_plan(w.n_off, w.mg);
     if (e == hipSuccess) {
         const int ns = w.n_small > 0 && w.n_small < w.n_off ? w.n_small : 0;
         if (ns)
@@ -485,7 +484,7 @@ hipError_t enqueue_generation(const Launch &w, hipStream_t s, hipEvent_t *ev) {
     }
     if (e == hipSuccess) e = mark(1);
     if (e == hipSuccess)
-        e = cd::launch_stem_list(w.jobs, w.off, w.stem_list, w.stem_ctl, sl, w.sh.stem_waves, w.stem_lds, s);
+        e = cd::launch_stem_list(w.jobs, w.off, w.n_off, w.mg, w.stem_list, w.stem_ctl, sl, w.sh.stem_waves, w.stem_lds, s);
     if (e == hipSuccess) e = mark(2);
     if (e == hipSuccess)
         e = cd::launch_dominance(w.jobs, w.dom, w.n_dom, true, w.stem_ctl, sl.groups, w.sh.dom_rows, s);
@@ -535,7 +534,6 @@ void build_lists(cd_job *const *jobs, int count, const cd::Shapes &sh, WorkLists
         wl.pool += J->P;
         wl.max_refs = std::max(wl.max_refs, J->R);
         wl.mg = std::max(wl.mg, J->m);
-        wl.stem_parts = std::max(wl.stem_parts, J->stem_parts);
     }
 }
 
@@ -594,7 +592,7 @@ int step_graphs(StepGraphs &G, hipStream_t s, const Launch &w, int generations) 
 
 Launch job_launch(cd_job *J) {
     return Launch{J->d_self, 1,          J->d_off,     J->N,          J->d_dom,   J->n_dom,   J->d_asc,
-                  J->n_asc,  J->lds,     J->stem_lds,  J->P,          J->R,       J->m,          J->stem_parts,
+                  J->n_asc,  J->lds,     J->stem_lds,  J->P,          J->R,       J->m,
                   J->d_slist,
                   J->d_sctl, J->N * J->m, 0,           0,             J->P,          J->shapes};
 }
@@ -1076,7 +1074,6 @@ int cd_batch_create(cd_job *const *jobs, int32_t count, cd_batch **out) {
     B->pool = wl.pool;
     B->max_refs = wl.max_refs;
     B->mg = wl.mg;
-    B->stem_parts = wl.stem_parts;
     B->n_cds = wl.n_cds;
     B->n_small = wl.n_small;
     B->lds_small = wl.lds_small;
@@ -1087,7 +1084,7 @@ int cd_batch_create(cd_job *const *jobs, int32_t count, cd_batch **out) {
     if (e == hipSuccess) e = hipMalloc(&B->d_off, sizeof(int2) * wl.off.size());
     if (e == hipSuccess) e = hipMalloc(&B->d_dom, sizeof(int4) * cap_dom);
     if (e == hipSuccess) e = hipMalloc(&B->d_asc, sizeof(int2) * cap_asc);
-    if (e == hipSuccess) e = hipMalloc(&B->d_slist, sizeof(uint32_t) * cd::stem_list_entries((int)wl.off.size(), wl.mg));
+    if (e == hipSuccess) e = hipMalloc(&B->d_slist, sizeof(uint2) * cd::stem_list_entries((int)wl.off.size(), wl.mg));
     if (e == hipSuccess) e = hipMalloc(&B->d_sctl, sizeof(int32_t) * cd::STEM_MAX_GROUPS);
     if (e == hipSuccess) e = hipMemset(B->d_sctl, 0, sizeof(int32_t) * cd::STEM_MAX_GROUPS);
     if (e == hipSuccess) e = hipMemcpy(B->d_jobs, wl.descs.data(), sizeof(cd::DevJob) * count, hipMemcpyHostToDevice);
@@ -1108,7 +1105,7 @@ int cd_batch_create(cd_job *const *jobs, int32_t count, cd_batch **out) {
 static Launch batch_launch(cd_batch *B) {
     return Launch{B->d_jobs,    (int)B->jobs.size(), B->d_off,      B->n_off,   B->d_dom,
                   B->n_dom,     B->d_asc,            B->n_asc,      B->lds,     B->stem_lds,
-                  B->max_pool,  B->max_refs,         B->mg,         B->stem_parts, B->d_slist, B->d_sctl,
+                  B->max_pool,  B->max_refs,         B->mg,         B->d_slist, B->d_sctl,
                   B->n_cds,     B->n_small,          B->lds_small,  B->pool,      B->shapes};
 }
 

@@ -46,12 +46,11 @@ struct cd_job {
     int2 *d_off = nullptr;
     int4 *d_dom = nullptr;        // domination tiles: the 64 x 64 blocks (b, w), b <= w
     int2 *d_asc = nullptr;        // association groups, room for the smallest group (4 designs)
-    uint32_t *d_slist = nullptr;  // changed CDS of a generation (stem_list_entries) for k_stem_list
+    uint2 *d_slist = nullptr;  // changed CDS of a generation (stem_list_entries) for k_stem_list
     int32_t *d_sctl = nullptr;    // its counts (STEM_MAX_GROUPS), zero between generations (k_dominance clears them)
     int n_dom = 0, n_asc = 0;
     cd::Shapes shapes = cd::SHAPES_JOB;  // launch shapes of its generations (the lists above follow them)
     size_t lds = 0, stem_lds = 0;
-    int stem_parts = 1;  // k_stem workgroups per CDS (initialisation and evaluation)
     StepGraphs graphs;
     bool inited = false;
     bool selection_only = false;
@@ -64,7 +63,7 @@ struct cd_batch {
     int2 *d_off = nullptr;
     int4 *d_dom = nullptr;  // the domination tiles of every job
     int2 *d_asc = nullptr;  // room for 4-design groups
-    uint32_t *d_slist = nullptr;  // changed CDS of a generation (stem_list_entries)
+    uint2 *d_slist = nullptr;  // changed CDS of a generation (stem_list_entries)
     int32_t *d_sctl = nullptr;
     int n_off = 0, n_dom = 0, n_asc = 0, n_cds = 0;
     int n_small = 0;        // children first in d_off whose k_design fits six per CU
@@ -74,7 +73,6 @@ struct cd_batch {
     int pool = 0;        // designs of all their pools
     int max_refs = 0;    // most reference points of the batch's jobs
     int mg = 0;          // largest m of the batch's jobs
-    int stem_parts = 0;  // largest k_stem workgroups per CDS of the batch's jobs
     hipStream_t stream = nullptr;
     StepGraphs graphs;
 };
@@ -108,8 +106,7 @@ struct Launch {
     int max_pool;    // largest pool
     int max_refs;    // most reference points
     int mg;          // largest m
-    int stem_parts;  // largest k_stem workgroups per CDS (initialisation and evaluation)
-    uint32_t *stem_list;  // changed CDS of a generation, in sublists of consecutive children (stem_list_entries)
+    uint2 *stem_list;  // changed CDS of a generation, in sublists of consecutive children (stem_list_entries)
     int32_t *stem_ctl;    // their counts, zero between generations (k_dominance clears them)
     int n_cds;            // CDS of all children: sum of N * m
     // the first n_small children (0: none apart) are of jobs whose k_design
@@ -128,7 +125,7 @@ struct WorkLists {
     std::vector<int2> off, asc;
     std::vector<int4> dom;
     size_t lds = 0, stem_lds = 0;
-    int max_pool = 0, max_refs = 0, mg = 0, stem_parts = 0, n_cds = 0, pool = 0;
+    int max_pool = 0, max_refs = 0, mg = 0, n_cds = 0, pool = 0;
     int n_small = 0;  // children (first in off) of jobs with lds at most shapes.design_split
     size_t lds_small = 0;
 };

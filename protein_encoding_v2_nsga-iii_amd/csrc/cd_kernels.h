@@ -13,7 +13,18 @@ enum DesignMode { MODE_INIT = 0, MODE_EVAL = 1, MODE_OFFSPRING = 2 };
 constexpr size_t LDS_BYTES = 160 * 1024;  // per workgroup on gfx950
 constexpr int DOM_ROWS = 64;               // tile rows per k_dominance workgroup of the standalone sort and selection
 constexpr int ASSOC_DESIGNS = 4;           // designs per k_associate workgroup (a wave each), the smallest shape
-constexpr int STEM_PARTS = 4;              // most k_stem workgroups per CDS (contiguous tile ranges)
+// The stem kernels' shapes by the CDS of a launch (designs x the largest m).
+// Few: the latency of a search counts, 256 threads and 2048 chains each; many:
+// the searches resident per CU do, which the LDS bounds: 128 and 1024.
+// Listed offspring, 256 x 2048 against 128 x 1024: 1024 children of 2004
+// codons 67.7, 69.3 us a generation, 4096 of 12008 (32768 CDS) 240, 247, the
+// 64-job mix (42 240 children) 887, 833.  Chains, 256 threads, 512 / 1024 /
+// 2048 / 4096: 251 / 242 / 238 / 245 us on the 4096 children.
+constexpr int STEM_FEW = 2048;    // initialisation and evaluation
+constexpr int STEM_MANY = 65536;  // offspring
+// Offspring launches up to this size have no list of the changed CDS (the
+// figures stand at k_stem_each).
+constexpr int STEM_EACH = 16384;
 constexpr int STEM_CUS = 256;              // compute units of an MI355X: k_stem_list runs a resident grid
 
 // Launch shapes of one generation's kernels.  Every shape gives the same
@@ -22,7 +33,7 @@ constexpr int STEM_CUS = 256;              // compute units of an MI355X: k_stem
 struct Shapes {
     int design_split;    // k_design LDS bytes up to which children launch apart from the rest (0: one launch)
     int design_threads;  // k_design workgroup of the other children (a lone job: all): 256 or 512 threads
-    int stem_waves;      // k_stem_list waves per SIMD (workgroups per CU): 5, 6, 7 or 8
+    int stem_waves;      // k_stem_list waves per SIMD, at most: 5, 6, 7 or 8
     int dom_rows;        // k_dominance tile rows per workgroup (dom_rows / 64 tiles of 64 x 64): 64, 128 or 256
     int fronts_threads;  // k_fronts workgroup: 256, 512 or 1024 threads
     int assoc_designs;   // designs per k_associate workgroup: 4, 8 or 16 (a wave each), 32 or 64 (eight lanes each)
@@ -30,8 +41,8 @@ struct Shapes {
 };
 // Untuned shapes of a lone job, and of a batch or served tick (the k_design
 // and k_associate fields by the work's sizes: untuned_shapes).
-constexpr Shapes SHAPES_JOB = {0, 512, 6, 64, 512, 4, 1024};
-constexpr Shapes SHAPES_BATCH = {0, 256, 7, 128, 1024, 4, 1024};
+constexpr Shapes SHAPES_JOB = {0, 512, 8, 64, 512, 4, 1024};
+constexpr Shapes SHAPES_BATCH = {0, 256, 8, 128, 1024, 4, 1024};
 bool shapes_valid(const Shapes &s);
 // More children than this in a launch of 256-thread workgroups (seven a CU
 // are resident at 68 VGPRs) and k_design is throughput-bound: it then takes
@@ -44,7 +55,6 @@ size_t design_lds_bytes(int L, int m);
 size_t design_bytes_accepted(int L, int m);  // at most LDS_BYTES for a job to be accepted
 size_t stem_lds_bytes(int L);
 size_t cds_plane_bytes(int L);  // one CDS's two bit planes in the job's plane buffer
-int stem_parts_of(int L);  // k_stem workgroups per CDS of L codons (1 .. STEM_PARTS)
 hipError_t set_design_lds_limit(size_t bytes);
 hipError_t set_stem_lds_limit(size_t bytes);
 
@@ -65,10 +75,20 @@ inline StemList stem_list_geom(int n_items, int mg) {
     g.cap = g.group * mg;
     return g;
 }
+// The list of a generation's launches; cap 0: none, k_stem_each takes every CDS.
+inline StemList stem_list_plan(int n_items, int mg) {
+    StemList g = stem_list_geom(n_items, mg);
+    if ((int64_t)n_items * mg <= STEM_EACH) g.cap = 0;
+    return g;
+}
 // k_stem_list's dynamic LDS holds the sublists' prefix sums (at most this
 // many bytes) before it holds a CDS's planes and tables
 constexpr size_t STEM_PRE_BYTES = 4 * (STEM_MAX_GROUPS + 1);
-inline size_t stem_list_lds(size_t stem_lds) { return stem_lds > STEM_PRE_BYTES ? stem_lds : STEM_PRE_BYTES; }
+// (and beside them the search's chain heads and the queues of four waves)
+inline size_t stem_list_lds(size_t stem_lds) {
+    const size_t b = stem_lds + 4 * (2048 + 1408);
+    return b > STEM_PRE_BYTES ? b : STEM_PRE_BYTES;
+}
 inline size_t stem_list_entries(int n_items, int mg) {
     const StemList g = stem_list_geom(n_items, mg);
     return (size_t)g.groups * g.cap;
@@ -80,22 +100,21 @@ inline size_t stem_list_entries(int n_items, int mg) {
 // children list k_stem_list reads.  threads: the offspring mode's workgroup,
 // 256 or 512 (initialisation and evaluation take 256).
 hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n, size_t lds, hipStream_t s,
-                         uint32_t *stem_list = nullptr, int32_t *stem_ctl = nullptr, StemList sl = StemList{0, 0, 0},
+                         uint2 *stem_list = nullptr, int32_t *stem_ctl = nullptr, StemList sl = StemList{0, 0, 0},
                          int item_base = 0, int threads = 256);
 // (MODE_INIT: item_base 1 when the pool has not been written before)
 // the packed synonym indices of a pool's rows [rows][L] from its code rows
 // (stride row_stride(L)), to dst (room for rows * row_stride(L) bytes)
 hipError_t launch_export(const DevJob *job, const int8_t *src, int8_t *dst, int rows, int L, hipStream_t s);
-// initialisation and evaluation: parts workgroups per (item, CDS c < mg),
-// parts the largest stem_parts_of of the jobs: stem of each CDS k_design marked
-hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, int parts, size_t lds,
-                       hipStream_t s);
+// initialisation and evaluation: a workgroup per (item, CDS c < mg): stem of
+// each CDS of the items' designs
+hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s);
 // offspring generations: stem of each CDS the offspring k_design listed
-// (items and sl as given to it), on as many workgroups as are resident at
-// once (STEM_CUS x the workgroups per CU that `waves`, 5 to 8, and the LDS
-// allow), at most the entries there can be; launch_dominance with the same
-// stem_ctl and sl.groups clears the counts
-hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, const uint32_t *stem_list,
+// (the n items and sl as given to it), on as many workgroups as are resident at
+// once (STEM_CUS x what `waves`, 5 to 8 waves per SIMD, and the LDS allow), at
+// most the entries there can be; launch_dominance with the same stem_ctl and
+// sl.groups clears the counts
+hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, const uint2 *stem_list,
                             const int32_t *stem_ctl, StemList sl, int waves, size_t lds, hipStream_t s);
 // one thread per item: objective 5, clears the marks
 hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s);

@@ -37,6 +37,7 @@
 #include "cd_kernels.h"
 #include "cd_qgram.h"
 #include "cd_scan.h"
+#include "cd_seek.h"
 #include "cd_tile.h"
 
 namespace cd {
@@ -52,7 +53,11 @@ __host__ __device__ constexpr int align16(int x) { return (x + 15) & ~15; }
 // and saves the conversion of every codon of every child: 1.4 us a workgroup.
 constexpr int DL_SYN = 512, DL_ROWS = 1024;
 
-size_t design_lds_bytes(int L, int m) { return DL_ROWS + (size_t)m * (row_stride(L) + sizeof(CdsStat)) + 16; }
+// The change masks of the CDS (sk_mask_words(L) words each) follow the
+// statistics.
+size_t design_lds_bytes(int L, int m) {
+    return DL_ROWS + (size_t)m * (row_stride(L) + sizeof(CdsStat) + 4 * sk_mask_words(L)) + 16;
+}
 
 // Jobs are accepted up to this size: 160 KiB for m synonym and code rows, the
 // synonym ranges and the statistics of a design.
@@ -63,12 +68,24 @@ size_t design_bytes_accepted(int L, int m) {
 }
 
 // one CDS's bit planes: the sequence and its reverse complement, each
-// scan_words(3L) words of (low bits, high bits) of the nucleotide codes
-size_t cds_plane_bytes(int L) { return (size_t)2 * scan_words(3 * L) * sizeof(uint2); }
+// scan_words(3L) words of (low bits, high bits) of the nucleotide codes, then
+// its change mask (bit k: codon k changed) in whole 8-byte words
+__host__ __device__ inline int plane_words(int L) { return 2 * scan_words(3 * L) + ((sk_mask_words(L) + 1) >> 1); }
+size_t cds_plane_bytes(int L) { return (size_t)plane_words(L) * sizeof(uint2); }
 
-// dynamic LDS of k_stem: the bit planes of one CDS, then the q-gram search's
-// index and hit queue
-size_t stem_lds_bytes(int L) { return cds_plane_bytes(L) + qg_lds_bytes(3 * L); }
+// An entry of k_stem_list's list: CDS and child below; the buffer the child is
+// in and its job above.
+__device__ __forceinline__ uint64_t stem_entry(uint32_t job, uint32_t child, uint32_t c, uint32_t buf) {
+    return (uint64_t)((child << 4) | c) | ((uint64_t)((job << 1) | buf) << 32);
+}
+
+// dynamic LDS of the stem kernels: a CDS's planes and change mask, then the
+// word search's index (the launchers add the waves' queues)
+__host__ __device__ inline int stem_index_at(int L) { return align16(plane_words(L) * (int)sizeof(uint2)); }
+size_t stem_lds_bytes(int L) { return (size_t)stem_index_at(L) + sk_lds_bytes(3 * L, 0, 0); }
+static size_t seek_more_bytes(int heads, int threads) {
+    return (size_t)sk_lds_bytes(0, heads, threads / 64) - sk_lds_bytes(0, 0, 0);
+}
 
 constexpr int HITQ = 192;  // a wave's queue of hits: a full batch of 64 and one step's 128
 // k_design's static LDS for a workgroup of NW waves.
@@ -121,28 +138,29 @@ __device__ __forceinline__ int code_base(const uint8_t *row, int p) {
 }
 // ---------------------------------------------------------------------------
 // Longest stem of one CDS held as bit planes in LDS (calMaximumSL,
-// utils.cuh:712-888; the planes are built by k_design).  A changed CDS of an
-// offspring generation is searched by q-grams (cd_qgram.h) from its parent's
-// stem; the initial population, and a CDS the search cannot decide, by tiles
-// (cd_tile.h): the lanes of the `parts` workgroups of the CDS split its tiles
-// into contiguous ranges.  Each workgroup takes the maximum key (longest, then
-// smallest p, then smallest q).  A CDS with no run of 4 and no seed of 4 is
-// scanned exactly along its anti-diagonals (cd_scan.h).
+// utils.cuh:712-888; the planes are built by k_design): word searches
+// (cd_seek.h) at a known or guessed length, lower guesses after a fruitless
+// one, and the tiles (cd_tile.h) for a CDS whose stems are all shorter than 5
+// or that the search gives up on.  A CDS with no run of 4 and no seed of 4 is
+// scanned exactly along its anti-diagonals (cd_scan.h).  Each search takes
+// the maximum key (longest, then smallest p, then smallest q).
 // ---------------------------------------------------------------------------
-// The seed (wave 0): the longest run of pairs (i - k, j + k), k < 64, that
+// The seed: the longest run of pairs (i - k, j + k), k < 64, that
 // still pair in the child, with (i, j) = (p + l - 1, q) the parent's
 // innermost pair.  Each such run is a stem of the child (its pairs lie on one
 // anti-diagonal and enclose at least the parent's loop), so its length bounds
-// the longest stem from below.
+// the longest stem from below.  intact: every pair of the parent's stem still
+// pairs.
 __device__ __forceinline__ int plane_base(const uint2 *sp, int p) {
     const uint2 w = sp[p >> 5];
     const int b = p & 31;
     return (int)(((w.x >> b) & 1u) | (((w.y >> b) & 1u) << 1));
 }
-__device__ __forceinline__ int stem_seed(const uint2 *sp, int n, int l, int p, int q, int lane) {
+__device__ __forceinline__ int stem_seed(const uint2 *sp, int n, int l, int p, int q, int lane, bool &intact) {
     const int i = p + l - 1, j = q;
     const bool pair = l > 0 && lane <= i && j + lane < n && ((plane_base(sp, i - lane) ^ plane_base(sp, j + lane)) == 3);
     uint64_t m = __ballot(pair);
+    intact = l > 0 && l <= 64 && (~m & (~0ull >> (64 - l))) == 0;
     int run = 0;
     while (m) {  // each round removes the last pair of every run
         ++run;
@@ -151,101 +169,27 @@ __device__ __forceinline__ int stem_seed(const uint2 *sp, int n, int l, int p, i
     return run;
 }
 
-// q-gram search (cd_qgram.h) of a CDS for the runs of at least K.  The
-// workgroup builds the index of s in LDS (head, then the links); lane t walks
-// the lookups of the chunks t, t + NT, ... of 8 rc positions.  In rounds,
-// each wave walks until its segment of the hit queue could overflow or its
-// lanes are done, appending the hits of each step by ballot, and then the
-// whole workgroup measures the queued hits.  ctl[4..15]: per wave, the hits
-// queued, whether lanes have lookups left, whether one ran out of budget.
-// Sets *best to the workgroup's maximum key and returns whether every lookup
-// finished.
-__device__ __forceinline__ bool stem_qgram(int n, const uint2 *sp, const uint2 *rp, int K, uint16_t *head, int32_t *ctl,
-                           uint64_t *redu, uint64_t &best) {
-    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wid = tid >> 6, nw = NT >> 6;
-    const int st = qg_stride(K), NI = qg_index_count(n, st);
-    uint16_t *next = head + QG_CODES;
-    uint32_t *queue = (uint32_t *)((uint8_t *)next + qg_link_bytes(n));
-    uint4 *h4 = (uint4 *)head;
-    // two empty heads (QG_NIL) per word; made here rather than kept in
-    // registers across the search loop and the tile fallback's call
-    uint32_t nil2;
-    asm volatile("v_mov_b32 %0, -1" : "=v"(nil2));
-    __syncthreads();  // an earlier search's index and queue are no longer read
-    for (int i = tid; i < QG_CODES / 8; i += NT) h4[i] = make_uint4(nil2, nil2, nil2, nil2);
-    __syncthreads();
-    for (int k = tid; k < NI; k += NT) qg_insert(sp, st, k, head, next);
-    __syncthreads();
-    const int xe = n - QG_Q + 1, nch = (xe + 7) >> 3;
-    QgLane ln;
-    qg_lane_start(ln, rp, head, tid, nch, xe);
-    int budget = qg_budget(8 * ((nch + NT - 1) / NT));
-    uint32_t *seg = queue + wid * QG_SEG;
-    uint64_t b = 0;
-    bool over = false;
-    for (;;) {
-        int cnt = 0;  // the same in every lane of the wave
-        while (cnt <= QG_SEG - 64) {
-            const bool live = !qg_lane_done(ln, nch) && budget > 0 && !qg_chunk_done(ln);
-            if (!__any(live)) {
-                // every lane of the wave has walked its chunk: the lanes with
-                // chunks left load their next ones together (a wave's steps
-                // then only read chain entries)
-                const bool adv = !qg_lane_done(ln, nch) && budget > 0;
-                if (!__any(adv)) break;
-                if (adv) qg_lane_next(ln, rp, head, nch, NT, xe);
-                continue;
-            }
-            int a = 0, x = 0;
-            const bool hit = live && qg_walk_step(ln, next, n, st, budget, a, x);
-            const uint64_t bal = __ballot(hit);
-            const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-            if (hit) seg[cnt + rank] = qg_pack(a, x);
-            cnt += __popcll(bal);
-        }
-        const bool left = !qg_lane_done(ln, nch);
-        const bool rem = __any(left), out = __any(left && budget <= 0);
-        if (lane == 0) {
-            ctl[4 + wid] = cnt;
-            ctl[8 + wid] = rem;
-            ctl[12 + wid] = out;
-        }
-        __syncthreads();
-        int total = 0, more = 0;
-        for (int w = 0; w < nw; ++w) {
-            total += ctl[4 + w];
-            more |= ctl[8 + w];
-            over |= ctl[12 + w] != 0;
-        }
-        for (int h = tid; h < total; h += NT) {  // hit h: wave w's entry h minus the counts before it
-            int w = 0, r = h;
-            while (r >= ctl[4 + w]) r -= ctl[4 + w++];
-            const uint32_t v = queue[w * QG_SEG + r];
-            qg_measure(sp, rp, n, (int)(v >> 16), (int)(v & 0xFFFFu), K, b);
-        }
-        __syncthreads();  // the counts and the queue are read before the next round writes them
-        if (!more || over) break;
-    }
-    best = block_max_u64(b, redu);
-    return !over;
-}
-
-// The tiled scan of share `part` of `parts` of a CDS with a stem of `seed`
-// known (0: none), and its exact scan when there is neither a seed of 4 nor
-// a run of 4; returns the workgroup's maximum key.
-__device__ __forceinline__ uint64_t stem_tiles(int n, const uint2 *sp, const uint2 *rp, int seed, int part, int parts,
-                                               uint64_t *redu) {
+// The tiled scan of a CDS with a stem of `seed` known (0: none) by a
+// workgroup, and its exact scan when there is neither a seed of 4 nor a run of
+// 4; returns the workgroup's maximum key.  Out of line, for the search's rare
+// fallback: inlined, its registers would raise the pressure of the search
+// path.  The LDS pointers keep their address space, so the scan's loads stay
+// LDS loads.
+typedef __attribute__((address_space(3))) uint2 lds_uint2;
+typedef __attribute__((address_space(3))) uint64_t lds_uint64;
+__device__ __noinline__ uint64_t stem_tiles(int n, const lds_uint2 *planes, int seed, lds_uint64 *lds_redu) {
     const int tid = threadIdx.x, NT = blockDim.x;
+    const uint2 *sp = (const uint2 *)planes, *rp = sp + scan_words(n);
+    uint64_t *redu = (uint64_t *)lds_redu;
     // Every lane's K is a length some stem of this CDS has, so the wave may
     // share the largest after each step.  Trip counts are the same for every
     // lane, so every lane takes part in the exchanges.
     int K = max(seed, TILE_MIN_RUN);
     uint64_t best = 0;
     {
-        const int TT = 2 * tile_prefix(n, tile_blocks(n)), T = parts * NT, L = part * NT + tid;
-        const int t0 = (int)((int64_t)L * TT / T), t1 = (int)((int64_t)(L + 1) * TT / T);
-        const int trips = (TT + T - 1) / T;
+        const int TT = 2 * tile_prefix(n, tile_blocks(n));
+        const int t0 = (int)((int64_t)tid * TT / NT), t1 = (int)((int64_t)(tid + 1) * TT / NT);
+        const int trips = (TT + NT - 1) / NT;
         TileCursor cur;
         for (int j = 0; j < trips; ++j) {
             if (t0 + j < t1) {
@@ -257,16 +201,14 @@ __device__ __forceinline__ uint64_t stem_tiles(int n, const uint2 *sp, const uin
     }
     best = block_max_u64(best, redu);
     // With a seed of 4 or more the longest stem is at least 4 long, so the
-    // share holding it measures it; a share without a flag holds nothing
-    // longer.  Without one, a share with no run of 4 is scanned exactly.
+    // tiles measured it; without one and with no run of 4, the exact scan.
     if (seed < TILE_MIN_RUN && (int)(best >> 40) < TILE_MIN_RUN) {
         best = 0;
         K = 1;
-        const int stride = parts * NT, S0 = MIN_HAIRPIN + 1 + part * NT + tid;
-        const int Sw = MIN_HAIRPIN + 1 + part * NT + (tid & ~63), last = 2 * n - 3;
-        const int trips = Sw <= last ? (last - Sw) / stride + 1 : 0;
+        const int S0 = MIN_HAIRPIN + 1 + tid, Sw = MIN_HAIRPIN + 1 + (tid & ~63), last = 2 * n - 3;
+        const int trips = Sw <= last ? (last - Sw) / NT + 1 : 0;
         for (int j = 0; j < trips; ++j) {
-            const int S = S0 + j * stride;
+            const int S = S0 + j * NT;
             if (S <= last) scan_diagonal(sp, rp, n, S, MIN_HAIRPIN, K, best);
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) K = max(K, __shfl_xor(K, o, 64));
@@ -276,50 +218,196 @@ __device__ __forceinline__ uint64_t stem_tiles(int n, const uint2 *sp, const uin
     return best;
 }
 
-// The whole CDS's tiled scan out of line, for the offspring search's rare
-// fallback: inlined, its registers would raise the pressure of the search
-// path.  The LDS pointers keep their address space, so the scan's loads stay
-// LDS loads.
-typedef __attribute__((address_space(3))) uint2 lds_uint2;
-typedef __attribute__((address_space(3))) uint64_t lds_uint64;
-__device__ __noinline__ uint64_t stem_tiles_whole(int n, const lds_uint2 *planes, int seed, lds_uint64 *redu) {
-    const uint2 *sp = (const uint2 *)planes;
-    return stem_tiles(n, sp, sp + scan_words(n), seed, 0, 1, (uint64_t *)redu);
+// LDS of the word search (cd_seek.h).
+struct SeekLds {
+    uint32_t *bits, *head;
+    uint16_t *next;
+    uint32_t *match;         // match, cand, list: the wave's own
+    uint16_t *cand, *list;
+    const uint32_t *chg;     // the CDS's change mask (offspring)
+};
+template <int HEADS>
+__device__ __forceinline__ SeekLds seek_lds(uint8_t *base, int n, int wid, const uint32_t *chg) {
+    SeekLds S;
+    S.bits = (uint32_t *)base;
+    S.head = S.bits + SK_BITWORDS;
+    S.next = (uint16_t *)(S.head + HEADS);
+    S.match = (uint32_t *)((uint8_t *)S.next + sk_link_bytes(n) + wid * (SK_MATCH * 4 + (SK_CAND + SK_LIST) * 2));
+    S.cand = (uint16_t *)(S.match + SK_MATCH);
+    S.list = S.cand + SK_CAND;
+    S.chg = chg;
+    return S;
+}
+// Empties the bitmap and the chains (the next barrier makes it visible).
+template <int NT, int HEADS>
+__device__ __forceinline__ void seek_clear(const SeekLds &S) {
+    u32x4 *b = (u32x4 *)S.bits;
+    const u32x4 zero = {0u, 0u, 0u, 0u}, nil = {SK_NIL, SK_NIL, SK_NIL, SK_NIL};
+#pragma unroll
+    for (int i = 0; i < SK_BITWORDS / 4; i += NT)
+        if (SK_BITWORDS / 4 % NT == 0 || i + (int)threadIdx.x < SK_BITWORDS / 4) b[i + threadIdx.x] = zero;
+#pragma unroll
+    for (int i = 0; i < HEADS / 4; i += NT)
+        if (HEADS / 4 % NT == 0 || i + (int)threadIdx.x < HEADS / 4) b[SK_BITWORDS / 4 + i + threadIdx.x] = nil;
 }
 
-// Longest stem of a changed CDS of an offspring generation (one workgroup),
-// seeded by its parent's record: q-gram searches for the runs of at least
-// the seed when that is 7 or more (exact), else for the runs of at least a
-// guess (exact when one is found), then of at least 7; the tiles follow a
-// fruitless guess of 7, a search out of budget, or a CDS the search does not
-// take.
-__device__ __forceinline__ uint64_t stem_child(int n, const uint2 *planes, int pl, int pp, int pq, int32_t *bcast,
-                                               uint64_t *redu, uint16_t *qhead) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const uint2 *sp = planes, *rp = planes + scan_words(n);
-    if (wid == 0) {
-        const int seed = stem_seed(sp, n, pl, pp, pq, lane);
-        if (lane == 0) {
-            bcast[0] = seed;
-            bcast[2] = pl;
+// Lanes of `bal` below the calling one.
+__device__ __forceinline__ int lanes_below(uint64_t bal) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+}
+
+// One search of a workgroup of NT threads at K (cd_seek.h), the index emptied
+// before and planes and index ready behind a barrier.  Every wave looks up its
+// chunks of 8 positions, 64 chunks a step (of the changed part only the chunks
+// near a changed codon, gathered first), queues the positions whose words are
+// indexed, walks their chains 64 positions at a time and queues the matches,
+// which are measured 64 at a time: the lanes stay busy whatever share of the
+// lookups, positions and chain entries passes, and no barrier stands between.
+// best: the lane's largest key.  Returns false in a wave that ran out of
+// budget.
+template <int NT, int HEADS>
+__device__ __forceinline__ bool seek_run(const SeekLds &S, const uint2 *sp, const uint2 *rp, int n, int L, int K,
+                                         bool changed, uint64_t &best) {
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int Q = sk_word(n, K), st = sk_stride(n, K), NI = sk_count(n, K);
+    const uint32_t mask = (1u << Q) - 1u;
+    for (int k = tid; k < NI; k += NT) sk_insert(rp, st, mask, k, S.bits, S.head, HEADS, S.next);
+    lds_barrier();
+    const int xe = sk_positions(n, K, changed), nch = (xe + 7) >> 3;
+    // (the same in every lane) chain steps left; positions, matches and chunks queued
+    int steps = sk_budget(n), cnt = 0, nm = 0, listed = 0;
+    int c0 = wid * 64;
+    for (bool last = false; !last;) {
+        int ch = nch;  // the lane's chunk of this step
+        if (changed) {
+            while (listed < 64 && c0 < nch) {
+                const int c = c0 + lane;
+                const bool act = c < nch && sk_chunk_changed(S.chg, L, K, c);
+                const uint64_t bal = __ballot(act);
+                if (act) S.list[listed + lanes_below(bal)] = (uint16_t)c;
+                listed += (int)__popcll(bal);
+                c0 += NT;
+            }
+            wave_lds_sync();
+            const int take = min(listed, 64);
+            listed -= take;
+            if (lane < take) ch = S.list[listed + lane];
+            last = listed == 0 && c0 >= nch;
+        } else {
+            ch = min(c0 + lane, nch);
+            c0 += NT;
+            last = c0 >= nch;
+        }
+        uint32_t hit = ch < nch ? sk_chunk_lookup(sp, S.bits, mask, ch, xe) : 0u;
+        // queue the lane's positions: all together when they fit (a step has
+        // some twenty), else in two halves
+        uint32_t rest = 0u;
+        int mine = __popc(hit), incl = wave_scan_i32(mine), got = __builtin_amdgcn_readlane(incl, 63);
+        const bool halves = cnt + got > SK_CAND;
+        if (halves) {
+            rest = hit & 0xF0u;
+            hit &= 0x0Fu;
+            mine = __popc(hit);
+            incl = wave_scan_i32(mine);
+            got = __builtin_amdgcn_readlane(incl, 63);
+        }
+        for (bool more = true; more;) {
+            int at = cnt + incl - mine;
+            while (hit) {
+                S.cand[at++] = (uint16_t)(8 * ch + __builtin_ctz(hit));
+                hit &= hit - 1u;
+            }
+            cnt += got;
+            wave_lds_sync();
+            more = __any(rest != 0u);
+            const bool drain = last && !more;
+            while (cnt >= 64 || (drain && cnt > 0)) {
+                const int take = min(cnt, 64);
+                cnt -= take;
+                const int a = lane < take ? (int)S.cand[cnt + lane] : 0;
+                const uint32_t w = sk_number_at(sp, a, mask);
+                uint32_t e = lane < take ? S.head[sk_chain(w, HEADS)] : SK_NIL;
+                while (__any(e != SK_NIL)) {
+                    if (--steps < 0) return false;
+                    int ma = a, mb = 0;
+                    bool ok = false;
+                    if (e != SK_NIL) {
+                        mb = st * (int)e;
+                        const uint32_t v = sk_number_at(rp, mb, mask);
+                        e = S.next[e];
+                        ok = v == w && sk_half(n, Q, changed, ma, mb);
+                    }
+                    const uint64_t bal = __ballot(ok);
+                    if (ok) S.match[nm + lanes_below(bal)] = qg_pack(ma, mb);
+                    nm += (int)__popcll(bal);
+                    if (nm >= 64) {
+                        wave_lds_sync();
+                        nm -= 64;
+                        const uint32_t v = S.match[nm + lane];
+                        qg_measure(sp, rp, n, (int)(v >> 16), (int)(v & 0xFFFFu), K, best);
+                    }
+                }
+            }
+            if (more) {  // the second half
+                hit = rest;
+                rest = 0u;
+                mine = __popc(hit);
+                incl = wave_scan_i32(mine);
+                got = __builtin_amdgcn_readlane(incl, 63);
+            }
         }
     }
-    __syncthreads();
-    const int seed = bcast[0];
-    for (int K = qg_first_k(n, seed, bcast[2]); K;) {
-        uint64_t qbest;
-        if (!stem_qgram(n, sp, rp, K, qhead, bcast, redu, qbest)) break;
-        if (seed >= QG_KMIN || (int)(qbest >> 40) >= K) return qbest;
-        K = qg_next_k(K);
+    if (nm > 0) {
+        wave_lds_sync();
+        if (lane < nm) {
+            const uint32_t v = S.match[lane];
+            qg_measure(sp, rp, n, (int)(v >> 16), (int)(v & 0xFFFFu), K, best);
+        }
     }
-    return stem_tiles_whole(n, (const lds_uint2 *)planes, seed, (lds_uint64 *)redu);
+    return true;
 }
 
-// Workgroups of k_stem per CDS of n bases: about three tiles per lane or
-// more, at most STEM_PARTS.
-__host__ __device__ inline int stem_parts(int n) {
-    const int TT = 2 * tile_prefix(n, tile_blocks(n)), p = TT / (3 * 256);
-    return p < 1 ? 1 : (p > STEM_PARTS ? STEM_PARTS : p);
+// The search(es) of one CDS by a workgroup of NT threads: planes in LDS at sp
+// and rp, the index emptied, all behind a barrier.  parent: whether (pl, pp,
+// pq) is the longest stem of the CDS's parent, from which it differs in the
+// codons of S.chg.  Returns the workgroup's largest key; every thread holds it.
+template <int NT, int HEADS>
+__device__ __forceinline__ uint64_t seek_cds(const SeekLds &S, const uint2 *sp, const uint2 *rp, int n, int L,
+                                             bool parent, int pl, int pp, int pq, uint64_t *redu, int32_t *flag) {
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    bool intact = false;
+    const int seed = parent ? stem_seed(sp, n, pl, pp, pq, lane, intact) : 0;  // every wave itself
+    intact = intact && sk_takes(n, pl);
+    int K = intact ? pl : parent ? sk_first_k(n, seed, pl) : sk_blind_k(n);
+    bool fresh = true;
+    while (K && sk_takes(n, K)) {
+        if (!fresh) {
+            lds_barrier();  // the search before has read the index
+            seek_clear<NT, HEADS>(S);
+            lds_barrier();
+        }
+        fresh = false;
+        uint64_t best = intact && lane == 0 ? scan_key(pl, pp, pq) : 0ull;
+        const bool ok = seek_run<NT, HEADS>(S, sp, rp, n, L, K, intact, best);
+        best = wave_max_u64(best);
+        if (lane == 0) {
+            redu[wid] = best;
+            flag[wid] = ok;
+        }
+        lds_barrier();
+        bool all = true;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) {
+            best = redu[w] > best ? redu[w] : best;
+            all &= flag[w] != 0;
+        }
+        if (!all) break;  // out of budget
+        if ((int)(best >> 40) >= K) return best;
+        K = sk_next_k(K, seed);
+        lds_barrier();  // redu and flag are read
+    }
+    lds_barrier();
+    return stem_tiles(n, (const lds_uint2 *)sp, seed, (lds_uint64 *)redu);
 }
 
 // ---------------------------------------------------------------------------
@@ -411,8 +499,9 @@ __device__ __forceinline__ uint32_t pack12(uint32_t x) {
 // position n-1-p complemented; positions past n are zero; a word is (low bits,
 // high bits) of 32 positions.  A lane builds 32 codons (three words) of one
 // plane from eight words of codes; the reverse complement is the codons read
-// backwards, each with its bases reversed and complemented.
-__device__ __forceinline__ void task_planes(const uint32_t *w, int L, int nwd, uint2 *sp) {
+// backwards, each with its bases reversed and complemented.  The change mask
+// follows the planes.
+__device__ __forceinline__ void task_planes(const uint32_t *w, int L, int nwd, const uint32_t *chg, uint2 *sp) {
     const int n = 3 * L, W = scan_words(n), ng = (W + 2) / 3, lane = threadIdx.x & 63;
     uint2 *const rp = sp + W;
     for (int i = lane; i < 2 * ng; i += 64) {
@@ -451,6 +540,8 @@ __device__ __forceinline__ void task_planes(const uint32_t *w, int L, int nwd, u
         for (int v = 0; v < 3; ++v)
             if (3 * g + v < W) gstore((uint64_t *)(out + 3 * g + v), (uint64_t)lo[v] | ((uint64_t)hi[v] << 32));
     }
+    uint32_t *const mk = (uint32_t *)(sp + 2 * W);
+    for (int i = lane; i < sk_mask_words(L); i += 64) gstore(mk + i, chg[i]);
 }
 
 // Hamming distance of the CDS in rows a and b (nv 16-byte words; the padding
@@ -472,8 +563,8 @@ __device__ __forceinline__ int task_pair(const uint32_t *a, const uint32_t *b, i
 // distances on entry).
 template <class SH>
 __device__ __forceinline__ void design_tasks(const DevJob &J, const int64_t *lw6, const uint32_t *rows, uint32_t dmask, bool have_parent,
-                             CdsStat *cst, SH &sh, uint2 *planes, int wid, int nw) {
-    const int L = J.L, m = J.m, nwd = J.Ls >> 2, lane = threadIdx.x & 63, PW = 2 * scan_words(3 * L);
+                             const uint32_t *chg, CdsStat *cst, SH &sh, uint2 *planes, int wid, int nw) {
+    const int L = J.L, m = J.m, nwd = J.Ls >> 2, lane = threadIdx.x & 63, PW = plane_words(L);
     const int nd = __popc(dmask), npair = nd == 1 ? m - 1 : (nd ? m * (m - 1) / 2 : 0);
     uint32_t left = dmask;  // the CDS of task t, for t rising
     int t0 = 0;
@@ -490,7 +581,7 @@ __device__ __forceinline__ void design_tasks(const DevJob &J, const int64_t *lw6
             if (t < nd)
                 task_sums(J, lw6, rows + c * nwd, L, nwd, cst + c, have_parent);
             else
-                task_planes(rows + c * nwd, L, nwd, planes + (size_t)c * PW);
+                task_planes(rows + c * nwd, L, nwd, chg + c * sk_mask_words(L), planes + (size_t)c * PW);
             continue;
         }
         const int p = t - 2 * nd;  // pair p of the list
@@ -591,7 +682,8 @@ struct MutArgs {
     const DevJob *J;
     const uint64_t *syn;  // [64] synonym words by code
     uint8_t *rows;        // [m][Ls] codes
-    int Ls;
+    uint32_t *chg;        // [m][sk_mask_words(L)] changed codons
+    int Ls, CW;
     uint32_t gen, child;
 };
 
@@ -605,6 +697,12 @@ struct SynWord {
     __device__ __forceinline__ int own() const { return (int)((hi >> 12) & 7u); }
     __device__ __forceinline__ int code(int j) const { return (int)((j < 5 ? lo >> (6 * j) : hi) & 63u); }
 };
+
+// Codon k of CDS c becomes `code`.
+__device__ __forceinline__ void set_code(const MutArgs &A, int c, int k, int code) {
+    A.rows[c * A.Ls + k] = (uint8_t)code;
+    atomicOr(A.chg + c * A.CW + (k >> 5), 1u << (k & 31));
+}
 
 // The pick-th (0-based) set bit of a candidate mask.
 __device__ __forceinline__ int nth_bit(uint32_t mask, uint32_t pick) {
@@ -660,13 +758,12 @@ __device__ __forceinline__ void mut_random(const MutArgs &A, int32_t *dirty) {
         for (int h = 0; h < 2; ++h) {
             const int k = 2 * q + h;
             if (k >= L || !bern(r[2 * h], J.thr_pm)) continue;
-            uint8_t *at = A.rows + c * Ls + k;
-            const SynWord e(A.syn[*at]);
+            const SynWord e(A.syn[A.rows[c * Ls + k]]);
             const int ns = e.num(), cur = e.own();
             if (ns == 1) continue;
             int nw = (int)uniform_int(r[2 * h + 1], (uint32_t)(ns - 1));
             if (nw >= cur) ++nw;
-            *at = (uint8_t)e.code(nw);
+            set_code(A, c, k, e.code(nw));
             dirty[c] = 1;
         }
         q += blockDim.x;
@@ -681,7 +778,7 @@ __device__ __forceinline__ void mut_random(const MutArgs &A, int32_t *dirty) {
 __device__ __forceinline__ void mut_cai(const MutArgs &A, int cds, int32_t *dirty) {
     const DevJob &J = *A.J;
     const int L = J.L;
-    uint8_t *const row = A.rows + cds * A.Ls;
+    const uint8_t *const row = A.rows + cds * A.Ls;
     for (int q = threadIdx.x; 2 * q < L; q += blockDim.x) {
         uint32_t r[4];
         pair_draws(A, cds, q, r);
@@ -692,7 +789,7 @@ __device__ __forceinline__ void mut_cai(const MutArgs &A, int cds, int32_t *dirt
             const SynWord e(A.syn[row[k]]);
             const int ns = e.num(), cur = e.own();
             if (cur != ns - 1) {
-                row[k] = (uint8_t)e.code(cur + 1 + (int)uniform_int(r[2 * h + 1], (uint32_t)(ns - 1 - cur)));
+                set_code(A, cds, k, e.code(cur + 1 + (int)uniform_int(r[2 * h + 1], (uint32_t)(ns - 1 - cur))));
                 dirty[cds] = 1;
             }
         }
@@ -707,7 +804,7 @@ __device__ __forceinline__ void mut_cbp(const MutArgs &A, int cds, int32_t *dirt
     const int L = J.L, parity = (int)(A.gen & 1u);
     const uint64_t thr = J.thr_2pm, stop6 = J.stop6;
     const float *const cps6 = J.cps6;
-    uint8_t *const row = A.rows + cds * A.Ls;
+    const uint8_t *const row = A.rows + cds * A.Ls;
     const int npairs = L - 1 - parity > 0 ? (L - 1 - parity + 3) >> 2 : 0;  // 4q + parity < L - 1
     auto test = [&](int q) -> uint32_t {
         uint32_t r[4];
@@ -751,7 +848,7 @@ __device__ __forceinline__ void mut_cbp(const MutArgs &A, int cds, int32_t *dirt
         if (cand) {
             uint32_t r[4];
             pair_draws(A, cds, q, r);
-            row[k] = (uint8_t)e.code(nth_bit(cand, uniform_int(h ? r[3] : r[1], (uint32_t)__popc(cand))));
+            set_code(A, cds, k, e.code(nth_bit(cand, uniform_int(h ? r[3] : r[1], (uint32_t)__popc(cand)))));
             dirty[cds] = 1;
         }
     };
@@ -764,7 +861,7 @@ __device__ __forceinline__ void mut_hsc(const MutArgs &A, int cds, int32_t *dirt
     const DevJob &J = *A.J;
     const int L = J.L, parity = (int)(A.gen & 1u);
     const uint64_t thr = J.thr_2pm;
-    uint8_t *const row = A.rows + cds * A.Ls;
+    const uint8_t *const row = A.rows + cds * A.Ls;
     const uint64_t stop6 = J.stop6;
     const int npairs = L - parity > 0 ? (L - parity + 3) >> 2 : 0;  // 4q + parity < L
     auto test = [&](int q) -> uint32_t {
@@ -797,7 +894,7 @@ __device__ __forceinline__ void mut_hsc(const MutArgs &A, int cds, int32_t *dirt
         if (cand) {
             uint32_t r[4];
             pair_draws(A, cds, q, r);
-            row[k] = (uint8_t)e.code(nth_bit(cand, uniform_int(h ? r[3] : r[1], (uint32_t)__popc(cand))));
+            set_code(A, cds, k, e.code(nth_bit(cand, uniform_int(h ? r[3] : r[1], (uint32_t)__popc(cand)))));
             dirty[cds] = 1;
         }
     };
@@ -831,7 +928,7 @@ __device__ __forceinline__ void mut_hd(const MutArgs &A, int cds1, int cds2, int
     const DevJob &J = *A.J;
     const int L = J.L, m = J.m, Ls = A.Ls;
     const uint64_t thr = J.thr_pm;
-    uint8_t *const row = A.rows + cds1 * Ls;
+    const uint8_t *const row = A.rows + cds1 * Ls;
     auto test = [&](int q) -> uint32_t {
         uint32_t r[4];
         pair_draws(A, cds1, q, r);
@@ -882,7 +979,7 @@ __device__ __forceinline__ void mut_hd(const MutArgs &A, int cds1, int cds2, int
             }
         }
         if (best_mhd != -1 || best_pair != -1) {
-            row[k] = (uint8_t)e.code(best);
+            set_code(A, cds1, k, e.code(best));
             dirty[cds1] = 1;
         }
     };
@@ -894,7 +991,7 @@ __device__ __forceinline__ void mut_gc3(const MutArgs &A, int cds, int dir, floa
     const DevJob &J = *A.J;
     const int L = J.L;
     const uint64_t thr = bern_threshold(dev);
-    uint8_t *const row = A.rows + cds * A.Ls;
+    const uint8_t *const row = A.rows + cds * A.Ls;
     auto test = [&](int q) -> uint32_t {
         uint32_t r[4];
         pair_draws(A, cds, q, r);
@@ -918,7 +1015,7 @@ __device__ __forceinline__ void mut_gc3(const MutArgs &A, int cds, int dir, floa
             if (sh == cur) continue;
             const int ng = code_gc3(e.code(sh));
             if ((dir == GC_UP && ng > curg) || (dir == GC_DOWN && ng < curg)) {
-                row[k] = (uint8_t)e.code(sh);
+                set_code(A, cds, k, e.code(sh));
                 dirty[cds] = 1;
                 break;
             }
@@ -939,7 +1036,7 @@ __device__ __forceinline__ void mut_sl(const MutArgs &A, SH &sh, int32_t *dirty)
     const DevJob &J = *A.J;
     const int L = J.L, n = 3 * L, lane = threadIdx.x & 63;
     const int cds = sh.pidx[10];
-    uint8_t *const row = A.rows + cds * A.Ls;
+    const uint8_t *const row = A.rows + cds * A.Ls;
     const int P0 = sh.ppql[0], Lst = sh.ppql[2];
     const int l_idx = P0 / 3, r_idx = (P0 + Lst - 1) / 3;
     const int mid = (r_idx + l_idx) / 2;
@@ -967,7 +1064,7 @@ __device__ __forceinline__ void mut_sl(const MutArgs &A, SH &sh, int32_t *dirty)
         if (changed) {
             int nw = (int)uniform_int(r[1], (uint32_t)(ns - 1));
             if (nw == e.own()) ++nw;  // mutation.cuh:827 compares with ==
-            if (lane == 0) row[pos] = (uint8_t)e.code(nw);
+            if (lane == 0) set_code(A, cds, pos, e.code(nw));  // (a codon put back stays marked)
         }
         wave_lds_sync();
         // the first and last 64 bases
@@ -1034,7 +1131,7 @@ __device__ __forceinline__ void mut_sl(const MutArgs &A, SH &sh, int32_t *dirty)
             if (done)
                 dirty[cds] = 1;
             else if (lane == 0)
-                row[pos] = (uint8_t)saved;
+                A.rows[cds * A.Ls + pos] = (uint8_t)saved;
         }
         wave_lds_sync();
         if (done) break;
@@ -1105,7 +1202,7 @@ __device__ __forceinline__ int survivor_at(const uint64_t *selm, int W, int c, u
 // ---------------------------------------------------------------------------
 template <int MODE, int NT, int WAVES>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_design(const DevJob *__restrict__ jobs, const int2 *__restrict__ items,
-                                                uint32_t *__restrict__ stem_list, int32_t *stem_ctl, int stem_group,
+                                                uint2 *__restrict__ stem_list, int32_t *stem_ctl, int stem_group,
                                                 int stem_cap, int item_base) {
     extern __shared__ __align__(16) uint8_t dyn[];
     __shared__ DesignShared<NT / 64> sh;
@@ -1118,7 +1215,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
     const uint64_t *syn6 = (const uint64_t *)(dyn + DL_SYN);
     uint8_t *rows = dyn + DL_ROWS;
     CdsStat *cst = (CdsStat *)(rows + m * Ls);
-    const int npair = m * (m - 1) / 2;
+    uint32_t *const chg = (uint32_t *)(cst + m);
+    const int CW = sk_mask_words(L), npair = m * (m - 1) / 2;
 
     // The descriptor fields of the staging phase, read before its stores (a
     // store through a pool pointer could alias the descriptor as far as the
@@ -1151,6 +1249,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
     asm volatile("" : "+v"(v_tab), "+v"(sel0));
     if (tid < 128) ((int64_t *)dyn)[tid] = v_tab;
     if (tid < MAX_M) sh.dirty[tid] = (MODE != 2);
+    for (int i = tid; i < m * CW; i += NT) chg[i] = 0u;
     uint32_t gen = 0;
     int dst = 0, out_slot = it.y, src = 0, parent = 0;
     if (MODE == 2) {
@@ -1276,7 +1375,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
         uint32_t r[4];
         philox(gen, (uint32_t)c, 0u, TAG_TYPE, J.seed, r);
         const int type = (int)uniform_int(r[0], (uint32_t)(NOBJ + 1));  // main.cu:172-178
-        const MutArgs A{&J, syn6, rows, Ls, gen, (uint32_t)c};
+        const MutArgs A{&J, syn6, rows, chg, Ls, CW, gen, (uint32_t)c};
         switch (type) {  // main.cu:181-211
         case 0: mut_random(A, sh.dirty); break;
         case 1: mut_cai(A, sh.pidx[0], sh.dirty); break;
@@ -1299,8 +1398,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
         u32x4 *og = (u32x4 *)((dst ? genome1 : genome0) + (size_t)out_slot * m * Ls);
         for (int i = tid; i < G16; i += NT) gstore(og + i, rows4[i]);
     }
-    design_tasks(J, lw6, (const uint32_t *)rows, dmask, MODE == 2, cst, sh,
-                 J.planes + (size_t)out_slot * m * 2 * scan_words(3 * L), wid, NT / 64);
+    design_tasks(J, lw6, (const uint32_t *)rows, dmask, MODE == 2, chg, cst, sh,
+                 J.planes + (size_t)out_slot * m * plane_words(L), wid, NT / 64);
     lds_barrier();
     if (wid == 0)
         design_objectives(J, cst, sh, (dst ? obj1 : obj0) + (size_t)out_slot * NOBJ,
@@ -1315,13 +1414,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
         const int l = lane < m && !((dmask >> lane) & 1u) ? cst[lane].l : 0;
         const int lmax = wave_max_nonneg(l);
         if (lane == 0) gstore(J.stem_max + out_slot, lmax);  // (k_dominance counts the offspring's changed CDS)
-        if (MODE == MODE_OFFSPRING && dmask) {  // in the child's sublist
+        if (MODE == MODE_OFFSPRING && dmask && stem_cap) {  // in the child's sublist
             const int item = item_base + (int)blockIdx.x, k = item / stem_group;
             int e = 0;
             if (lane == 0) e = atomicAdd(stem_ctl + k, (int)__popc(dmask));
             e = __builtin_amdgcn_readfirstlane(e) + (int)__popc(dmask & ((1u << (lane & 31)) - 1u));
             if (lane < m && ((dmask >> lane) & 1u) && e < stem_cap)
-                gstore(stem_list + (size_t)k * stem_cap + e, ((uint32_t)item << 4) | (uint32_t)lane);
+                gstore((uint64_t *)(stem_list + (size_t)k * stem_cap + e),
+                       stem_entry((uint32_t)it.x, (uint32_t)it.y, (uint32_t)lane, (uint32_t)dst));
         }
     }
 }
@@ -1370,76 +1470,149 @@ __device__ __forceinline__ void item_slot(const DevJob &J, int mode, int y, int 
 }
 
 // ---------------------------------------------------------------------------
-// k_stem (initialisation and evaluation): up to STEM_PARTS workgroups per
-// (work item, CDS); blockIdx.x = part * nic + item * mg + c with mg the
-// largest m of the jobs launched and nic = items * mg.  Part-major order keeps
-// the workgroups that do work consecutive, so the round-robin placement of
-// workgroups on the XCDs spreads them over all eight (a CDS-major order with
-// unused parts would leave the working ones on the XCDs of one residue
-// class).  CDS not marked by k_design (pad 0) are skipped.  Each part folds
-// its best key into the record with an atomic maximum; k_stem_finish decodes
-// it.
+// k_stem (initialisation and evaluation): one workgroup per (work item, CDS),
+// blockIdx.x = item * mg + c with mg the largest m of the jobs launched: a
+// word search at a guessed length (sk_blind_k).  k_stem_finish decodes the key.
+// 128 threads and 1024 chains a CDS where there are many, 256 and 2048 where the
+// latency of one counts (STEM_FEW).  8192 CDS of 1503 bases: 24.7 us; by the tiles
+// of the match matrix 216.
 // ---------------------------------------------------------------------------
-// Six waves per SIMD (at most 80 VGPRs) keep ~1500 workgroups resident at
-// once on 256 CUs.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_stem(const DevJob *__restrict__ jobs, const int2 *__restrict__ items, int mode,
-                                              int mg, int nic) {
+template <int NT, int HEADS>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_stem(const DevJob *__restrict__ jobs, const int2 *__restrict__ items, int mode,
+                                              int mg) {
     extern __shared__ __align__(16) uint8_t dyn[];
     __shared__ uint64_t redu[16];
-    const int part = (int)(blockIdx.x / (unsigned)nic), ic = (int)(blockIdx.x % (unsigned)nic);
-    const int2 it = items[ic / mg];
-    const int c = ic % mg;
+    __shared__ int32_t flag[NT / 64];
+    const int2 it = items[blockIdx.x / (unsigned)mg];
+    const int c = (int)(blockIdx.x % (unsigned)mg);
     const DevJob &J = jobs[it.x];
-    const int L = J.L, m = J.m, n = 3 * L, parts = stem_parts(n);
-    if (c >= m || part >= parts) return;
+    const int L = J.L, m = J.m, n = 3 * L, wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (c >= m) return;
     int buf, slot;
     item_slot(J, mode, it.y, buf, slot);
     CdsStat *cs = J.cst[buf] + (size_t)slot * m + c;
-    if (cs->pad == 0) return;  // same word for every thread; k_stem never writes it
     uint64_t *planes = (uint64_t *)dyn;  // the CDS's planes as k_design left them
     const int nwords = 2 * scan_words(n);
-    const uint64_t *gp = (const uint64_t *)(J.planes + ((size_t)slot * m + c) * nwords);
-    for (int i = threadIdx.x; i < nwords; i += blockDim.x) planes[i] = gload(gp + i);
-    __syncthreads();
+    const uint64_t *gp = (const uint64_t *)(J.planes + ((size_t)slot * m + c) * plane_words(L));
+    for (int i = threadIdx.x; i < nwords; i += NT) planes[i] = gload(gp + i);
+    const SeekLds S = seek_lds<HEADS>(dyn + stem_index_at(L), n, wid, nullptr);
+    seek_clear<NT, HEADS>(S);
+    lds_barrier();
     const uint2 *sp = (const uint2 *)planes;
-    const uint64_t key = stem_tiles(n, sp, sp + scan_words(n), 0, part, parts, redu);
-    if (threadIdx.x == 0 && key) atomicMax((unsigned long long *)&cs->key, (unsigned long long)key);
+    const uint64_t key = seek_cds<NT, HEADS>(S, sp, sp + scan_words(n), n, L, false, 0, 0, 0, redu, flag);
+    if (threadIdx.x == 0) gstore(&cs->key, key);
 }
 
 // ---------------------------------------------------------------------------
-// k_stem_list (offspring generations): the changed CDS k_design listed,
-// entry (item << 4) | c, in `groups` sublists of cap entries with their
-// counts in ctl; the entries are numbered sublist by sublist (a prefix sum
-// of the counts), which keeps the children list's order, and gridDim.x
-// workgroups take them round-robin, one workgroup per CDS.  The parent's stem seeds the
-// q-gram search (stem_child).  Each entry's key goes into the CDS record and
-// its length into the design's longest stem (stem_max) with atomic maxima.
-// k_dominance clears ctl[0] for the next generation.
+// The stem of child `child`'s CDS c (offspring generations): the parent's stem
+// (it stands in the child's record) and the change mask decide the search
+// (seek_cds).  The key goes into the CDS record and the length into the
+// design's longest stem (stem_max) with an atomic maximum.  buf: the buffer
+// the child is in, or -1: take it from the generation counter, and leave a
+// CDS that did not change alone.
 // ---------------------------------------------------------------------------
-template <int WAVES>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_stem_list(
-    const DevJob *__restrict__ jobs, const int2 *__restrict__ items, const uint32_t *__restrict__ list,
-    const int32_t *__restrict__ ctl, int groups, int cap) {
+template <int NT, int HEADS>
+__device__ __forceinline__ void stem_child(const DevJob &J, int child, int c, int buf, uint8_t *dyn, uint64_t *redu, int32_t *flag) {
+    // The descriptor fields first, held in scalar registers; then the record
+    // (of both buffers while the counter is on its way), the planes and the
+    // mask, loaded together.  The child sits at slot N + child of the next
+    // buffer, (gen + 1) & 1.
+    const SelState *p_st = J.st;
+    CdsStat *cs0 = J.cst[0], *cs1 = J.cst[1];
+    const uint2 *p_pl = J.planes;
+    int32_t *p_sm = J.stem_max;
+    int L = J.L, m = J.m, N = J.N;
+    asm volatile("" : "+s"(p_st), "+s"(cs0), "+s"(cs1), "+s"(p_pl), "+s"(p_sm), "+s"(L), "+s"(m), "+s"(N));
+    if (buf < 0 && c >= m) return;
+    const int n = 3 * L, slot = N + child, tid = (int)threadIdx.x;
+    const size_t rec = (size_t)slot * m + c;
+    const int nwords = plane_words(L), pw = 2 * scan_words(n);
+    const uint64_t *gp = (const uint64_t *)(p_pl + rec * nwords);
+    CdsStat *cs = (buf > 0 ? cs1 : cs0) + rec;
+    const int32_t *r0 = (const int32_t *)cs;
+    int pl = gload(r0 + 6), pp = gload(r0 + 7), pq = gload(r0 + 8), fresh = 1;  // CdsStat::l, p, q
+    uint32_t gen = 0;
+    int l1 = 0, p1 = 0, q1 = 0, f1 = 0;
+    if (buf < 0) {
+        gen = gload(&p_st->gen);
+        const int32_t *r1 = (const int32_t *)(cs1 + rec);
+        fresh = gload(r0 + 9);  // CdsStat::pad
+        l1 = gload(r1 + 6), p1 = gload(r1 + 7), q1 = gload(r1 + 8), f1 = gload(r1 + 9);
+    }
+    const uint64_t v0 = gload(gp + min(tid, nwords - 1)), v1 = gload(gp + min(tid + NT, nwords - 1));
+    if (buf < 0 && !(__builtin_amdgcn_readfirstlane(gen) & 1u)) {
+        cs = cs1 + rec;
+        pl = l1, pp = p1, pq = q1, fresh = f1;
+    }
+    if (__builtin_amdgcn_readfirstlane(fresh) == 0) return;
+    uint64_t *planes = (uint64_t *)dyn;  // the CDS's planes and change mask as k_design left them
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const SeekLds S = seek_lds<HEADS>(dyn + stem_index_at(L), n, wid, (const uint32_t *)(planes + pw));
+    if (buf >= 0) lds_barrier();  // the previous entry's LDS is no longer read
+    seek_clear<NT, HEADS>(S);
+    if (tid < nwords) planes[tid] = v0;
+    if (tid + NT < nwords) planes[tid + NT] = v1;
+    for (int i = tid + 2 * NT; i < nwords; i += NT) planes[i] = gload(gp + i);
+    lds_barrier();
+    const uint2 *sp = (const uint2 *)planes;
+    const uint64_t key = seek_cds<NT, HEADS>(S, sp, sp + scan_words(n), n, L, true, pl, pp, pq, redu, flag);
+    if (tid == 0) {
+        gstore(&cs->key, key);
+        if (key) atomicMax(&p_sm[slot], (int)(key >> 40));
+    }
+}
+
+// k_stem_each: a workgroup per CDS of the children, for small launches: the
+// unchanged CDS leave after their record, and k_design does not wait for the
+// list's counters at its end.  Against the list: 128 children of 202 codons
+// 39.2 -> 38.2 us a generation, 777 of 6190 75.2 -> 74.2, 1024 of 2004
+// 67.7 -> 62.0 (k_design 25.8 -> 21.1); 4096 of 12008 (32768 CDS) 240.0 ->
+// 241.7; the 64-job mix 835 -> 1208, mostly empty workgroups.
+template <int NT, int HEADS>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_stem_each(
+    const DevJob *__restrict__ jobs, const int2 *__restrict__ items, int mg) {
     extern __shared__ __align__(16) uint8_t dyn[];
     __shared__ uint64_t redu[16];
-    __shared__ int32_t bcast[16];
+    __shared__ int32_t flag[NT / 64];
+    const int2 it = items[blockIdx.x / (unsigned)mg];
+    stem_child<NT, HEADS>(jobs[it.x], it.y, (int)(blockIdx.x % (unsigned)mg), -1, dyn, redu, flag);
+}
+
+// ---------------------------------------------------------------------------
+// k_stem_list (offspring generations): the changed CDS k_design listed
+// (stem_entry), in `groups` sublists of cap entries with their counts in ctl;
+// the entries are numbered sublist by sublist (a prefix sum of the counts),
+// which keeps the children list's order, and gridDim.x workgroups of NT threads
+// take them round-robin, one CDS a workgroup at a time (stem_child).
+// k_dominance clears ctl for the next generation.
+// Bound by the searches resident per CU (LDS) and their chain of lookups: the
+// scans of the tiles that this search replaced took 502 us on the 64-job mix
+// (now 326), 130 us for 4096 children of 12 008 codons (69), 32 us for 777 of
+// 6190 (21).
+// ---------------------------------------------------------------------------
+template <int NT, int HEADS>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_stem_list(
+    const DevJob *__restrict__ jobs, const uint2 *__restrict__ list, const int32_t *__restrict__ ctl, int groups, int cap) {
+    extern __shared__ __align__(16) uint8_t dyn[];
+    __shared__ uint64_t redu[16];
+    __shared__ int32_t flag[NT / 64];
     const int G = (int)gridDim.x, lane = (int)threadIdx.x & 63;
     // Up to 64 sublists (4096 children at 64 each): every wave scans their
     // counts in registers, and the workgroup's entries are fetched one ahead
     // of the one being searched, so no barrier stands before the first search.
     // More: the prefix sums sit where the planes go -- built before each chunk
-    // of 256 entries is fetched, overwritten by the planes after -- and are
+    // of 64 entries is fetched, overwritten by the planes after -- and are
     // built again only when the workgroup has entries past its first chunk.
     const bool few = groups <= 64;
     int *pre = (int *)dyn;  // [groups + 1]
     __shared__ int red[16], s_carry;
-    __shared__ uint32_t s_ent[256];  // the workgroup's next entries, fetched together
+    __shared__ uint64_t s_ent[64];  // the workgroup's next entries, fetched together
     int incl = 0, count = 0, e = (int)blockIdx.x, j = 0;
-    uint32_t nxt = 0;
-    auto fetch = [&](int q) -> uint32_t {  // entry q of the list (few; q is the same in every lane)
+    uint64_t nxt = 0;
+    auto fetch = [&](int q) -> uint64_t {  // entry q of the list (few; q is the same in every lane)
         const int k = (int)__popcll(__ballot(incl <= q));
         const int first = k ? __builtin_amdgcn_readlane(incl, k - 1) : 0;
-        return gload(list + (size_t)k * cap + (q - first));
+        return gload((const uint64_t *)(list + (size_t)k * cap + (q - first)));
     };
     if (few) {
         incl = wave_scan_i32(lane < groups ? min(gload(ctl + lane), cap) : 0);
@@ -1447,14 +1620,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
         if (e < count) nxt = fetch(e);
     }
     for (bool start = true;; start = false, e += G) {
-        uint32_t ent;
+        uint64_t ent;
         if (few) {
             if (e >= count) break;
             ent = nxt;
             if (e + G < count) nxt = fetch(e + G);
         } else {
             if (!start && e >= count) break;
-            if (start || j == 256) {
+            if (start || j == 64) {
                 __syncthreads();  // the previous entries' planes are no longer read
                 if (threadIdx.x == 0) s_carry = 0;
                 for (int g0 = 0; g0 < groups; g0 += blockDim.x) {  // exclusive prefix of the counts
@@ -1472,11 +1645,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
                 count = pre[groups];
                 if (e >= count) break;
                 const int q = e + (int)threadIdx.x * G;
-                if (q < count) {
+                if (threadIdx.x < 64 && q < count) {
                     int k = 0;  // the last sublist whose entries start at or before q
                     for (int h = STEM_MAX_GROUPS / 2; h > 0; h >>= 1)
                         if (k + h < groups && pre[k + h] <= q) k += h;
-                    s_ent[threadIdx.x] = gload(list + (size_t)k * cap + (q - pre[k]));
+                    s_ent[threadIdx.x] = gload((const uint64_t *)(list + (size_t)k * cap + (q - pre[k])));
                 }
                 j = 0;
                 __syncthreads();
@@ -1484,44 +1657,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
             ent = s_ent[j++];
         }
         {
-            // (wave-uniform: the item and the descriptor come by scalar loads)
-            ent = (uint32_t)__builtin_amdgcn_readfirstlane((int)ent);
-            const int2 it = items[ent >> 4];
-            const int c = (int)(ent & 15u);
-            const DevJob &J = jobs[it.x];
-            // The descriptor fields first, held in scalar registers; then the
-            // generation counter, the planes and the parent's stem from both
-            // record buffers, loaded together (only the choice of record
-            // waits for the counter).  The child sits at slot N + child of
-            // the next buffer, (gen + 1) & 1.
-            const SelState *p_st = J.st;
-            CdsStat *cs0 = J.cst[0], *cs1 = J.cst[1];
-            const uint2 *p_pl = J.planes;
-            int32_t *p_sm = J.stem_max;
-            int L = J.L, m = J.m, N = J.N;
-            asm volatile("" : "+s"(p_st), "+s"(cs0), "+s"(cs1), "+s"(p_pl), "+s"(p_sm), "+s"(L), "+s"(m), "+s"(N));
-            const int n = 3 * L, slot = N + it.y, tid = (int)threadIdx.x;
-            const size_t rec = (size_t)slot * m + c;
-            const int nwords = 2 * scan_words(n);
-            const uint64_t *gp = (const uint64_t *)(p_pl + rec * nwords);
-            const uint32_t g0 = gload(&p_st->gen);
-            const int32_t *r0 = (const int32_t *)(cs0 + rec), *r1 = (const int32_t *)(cs1 + rec);
-            const int l0 = gload(r0 + 6), p0 = gload(r0 + 7), q0 = gload(r0 + 8);  // CdsStat::l, p, q
-            const int l1 = gload(r1 + 6), p1 = gload(r1 + 7), q1 = gload(r1 + 8);
-            const uint64_t v0 = gload(gp + min(tid, nwords - 1));
-            uint64_t *planes = (uint64_t *)dyn;  // the CDS's planes as k_design left them
-            __syncthreads();  // the previous entry's LDS is no longer read
-            if (tid < nwords) planes[tid] = v0;
-            for (int i = tid + (int)blockDim.x; i < nwords; i += blockDim.x) planes[i] = gload(gp + i);
-            const bool b1 = ((__builtin_amdgcn_readfirstlane(g0) + 1u) & 1u) != 0;
-            CdsStat *cs = (b1 ? cs1 : cs0) + rec;
-            __syncthreads();
-            const uint64_t key = stem_child(n, (const uint2 *)planes, b1 ? l1 : l0, b1 ? p1 : p0, b1 ? q1 : q0, bcast,
-                                            redu, (uint16_t *)(planes + nwords));
-            if (tid == 0 && key) {
-                atomicMax((unsigned long long *)&cs->key, (unsigned long long)key);
-                atomicMax(&p_sm[slot], (int)(key >> 40));
-            }
+            // (wave-uniform: the descriptor comes by scalar loads)
+            const uint32_t ex = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)ent);
+            const uint32_t ey = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(ent >> 32));
+            stem_child<NT, HEADS>(jobs[ey >> 1], (int)(ex >> 4), (int)(ex & 15u), (int)(ey & 1u), dyn, redu, flag);
         }
     }
 }
@@ -2912,13 +3051,13 @@ __global__ void k_zero_np(const DevJob *__restrict__ jobs) {
 // Launchers
 // ---------------------------------------------------------------------------
 hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n, size_t lds, hipStream_t s,
-                         uint32_t *stem_list, int32_t *stem_ctl, StemList sl, int item_base, int threads) {
+                         uint2 *stem_list, int32_t *stem_ctl, StemList sl, int item_base, int threads) {
     if (n <= 0) return hipSuccess;
     switch (mode) {
     case 0: hipLaunchKernelGGL((k_design<0, 256, 6>), dim3(n), dim3(256), lds, s, jobs, items, nullptr, nullptr, 1, 0, item_base); break;
     case 1: hipLaunchKernelGGL((k_design<1, 256, 6>), dim3(n), dim3(256), lds, s, jobs, items, nullptr, nullptr, 1, 0, 0); break;
     default:
-        if (!stem_list || !stem_ctl || sl.cap <= 0 || sl.group <= 0 || sl.groups > STEM_MAX_GROUPS || item_base < 0)
+        if (!stem_list || !stem_ctl || sl.cap < 0 || sl.group <= 0 || sl.groups > STEM_MAX_GROUPS || item_base < 0)
             return hipErrorInvalidValue;
         if (threads == 256 && n > DESIGN_MANY)
             hipLaunchKernelGGL((k_design<2, 256, 8>), dim3(n), dim3(256), lds, s, jobs, items, stem_list, stem_ctl,
@@ -2941,40 +3080,37 @@ hipError_t launch_export(const DevJob *job, const int8_t *src, int8_t *dst, int 
     hipLaunchKernelGGL(k_export, dim3((unsigned)n), dim3(256), 0, s, job, (const uint8_t *)src, (uint8_t *)dst, rows);
     return hipGetLastError();
 }
-int stem_parts_of(int L) { return stem_parts(3 * L); }
-
-hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, int parts, size_t lds,
-                       hipStream_t s) {
+hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    if (parts < 1 || parts > STEM_PARTS) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_stem, dim3(n * mg * parts), dim3(256), lds, s, jobs, items, mode, mg, n * mg);
+    if ((int64_t)n * mg <= STEM_FEW)
+        hipLaunchKernelGGL((k_stem<256, 2048>), dim3(n * mg), dim3(256), lds + seek_more_bytes(2048, 256), s, jobs, items, mode, mg);
+    else
+        hipLaunchKernelGGL((k_stem<128, 1024>), dim3(n * mg), dim3(128), lds + seek_more_bytes(1024, 128), s, jobs, items, mode, mg);
     return hipGetLastError();
 }
-hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, const uint32_t *stem_list,
+hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, const uint2 *stem_list,
                             const int32_t *stem_ctl, StemList sl, int waves, size_t lds, hipStream_t s) {
-    if (sl.cap <= 0 || sl.groups <= 0) return hipSuccess;
-    if (sl.groups > STEM_MAX_GROUPS) return hipErrorInvalidValue;
-    const int capacity = sl.groups * sl.cap;
-    if (lds < 4 * ((size_t)sl.groups + 1)) lds = 4 * ((size_t)sl.groups + 1);  // the prefix sums share the planes' LDS
-    if (!stem_list || !stem_ctl || waves < 5 || waves > 8) return hipErrorInvalidValue;
-    // workgroups take the entries round-robin, so every one should be
-    // resident from the start: per CU, the waves per SIMD or what the
-    // registers and the LDS (dynamic and static) hold, as the runtime counts it
-    const void *fn = waves == 5   ? (const void *)k_stem_list<5>
-                     : waves == 6 ? (const void *)k_stem_list<6>
-                     : waves == 7 ? (const void *)k_stem_list<7>
-                                  : (const void *)k_stem_list<8>;
-    int fit = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, fn, 256, lds) != hipSuccess || fit < 1) fit = 1;
-    const int per_cu = fit < waves ? fit : waves;
-    const int grid = capacity < STEM_CUS * per_cu ? capacity : STEM_CUS * per_cu;
-    switch (waves) {
-    case 5: hipLaunchKernelGGL(k_stem_list<5>, dim3(grid), dim3(256), lds, s, jobs, items, stem_list, stem_ctl, sl.groups, sl.cap); break;
-    case 6: hipLaunchKernelGGL(k_stem_list<6>, dim3(grid), dim3(256), lds, s, jobs, items, stem_list, stem_ctl, sl.groups, sl.cap); break;
-    case 7: hipLaunchKernelGGL(k_stem_list<7>, dim3(grid), dim3(256), lds, s, jobs, items, stem_list, stem_ctl, sl.groups, sl.cap); break;
-    default: hipLaunchKernelGGL(k_stem_list<8>, dim3(grid), dim3(256), lds, s, jobs, items, stem_list, stem_ctl, sl.groups, sl.cap); break;
+    if (n <= 0) return hipSuccess;
+    if (!stem_list || !stem_ctl || waves < 5 || waves > 8 || sl.groups > STEM_MAX_GROUPS) return hipErrorInvalidValue;
+    if (sl.cap == 0) {
+        hipLaunchKernelGGL((k_stem_each<256, 2048>), dim3(n * mg), dim3(256), lds + seek_more_bytes(2048, 256), s, jobs, items, mg);
+        return hipGetLastError();
     }
-    return hipGetLastError();
+    const int capacity = sl.groups * sl.cap;
+    // workgroups take the entries round-robin, so every one should be
+    // resident from the start: per CU, `waves` waves per SIMD or what the
+    // registers and the LDS (dynamic and static) hold, as the runtime counts it
+    auto go = [&](auto kern, int heads, int threads) -> hipError_t {
+        size_t bytes = lds + seek_more_bytes(heads, threads);
+        if (bytes < 4 * ((size_t)sl.groups + 1)) bytes = 4 * ((size_t)sl.groups + 1);  // the prefix sums share the planes' LDS
+        int fit = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, (const void *)kern, threads, bytes) != hipSuccess || fit < 1) fit = 1;
+        const int most = waves * 256 / threads, per_cu = fit < most ? fit : most;
+        const int grid = capacity < STEM_CUS * per_cu ? capacity : STEM_CUS * per_cu;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), bytes, s, jobs, stem_list, stem_ctl, sl.groups, sl.cap);
+        return hipGetLastError();
+    };
+    return (int64_t)n * mg <= STEM_MANY ? go(k_stem_list<256, 2048>, 2048, 256) : go(k_stem_list<128, 1024>, 1024, 128);
 }
 hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
@@ -3103,8 +3239,9 @@ hipError_t set_design_lds_limit(size_t bytes) {
 }
 hipError_t set_stem_lds_limit(size_t bytes) {
     return raise_lds_limit(g_stem_lds, bytes, [](int b) {
-        const void *fns[] = {(const void *)k_stem, (const void *)k_stem_list<5>, (const void *)k_stem_list<6>,
-                             (const void *)k_stem_list<7>, (const void *)k_stem_list<8>};
+        const void *fns[] = {(const void *)k_stem<128, 1024>,      (const void *)k_stem<256, 2048>,
+                             (const void *)k_stem_each<256, 2048>, (const void *)k_stem_list<128, 1024>,
+                             (const void *)k_stem_list<256, 2048>};
         for (const void *f : fns) {
             const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, b);
             if (e != hipSuccess) return e;

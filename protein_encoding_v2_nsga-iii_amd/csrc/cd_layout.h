@@ -34,7 +34,7 @@ struct CdsStat {
     int32_t gc3;  // codons whose third base is G or C
     int32_t l, p, q;  // longest stem and its position (canonical tie rule)
     int32_t pad;      // 1 while the stem fields await k_stem
-    uint64_t key;     // best stem key of the parts of k_stem (atomic max), valid while pad is 1
+    uint64_t key;     // longest stem as k_stem found it, valid while pad is 1
     float ov[4];      // the CDS's CAI, CPB, HSC quotient and GC3 fraction, from the sums above
 };
 static_assert(sizeof(CdsStat) == 64, "CdsStat records move as four 16-byte words");

@@ -104,7 +104,7 @@ struct cd_server {
     cd::DevJob *d_jobs = nullptr;
     int2 *d_off = nullptr, *d_asc = nullptr;
     int4 *d_dom = nullptr;
-    uint32_t *d_slist = nullptr;  // changed CDS of a tick (stem_list_entries)
+    uint2 *d_slist = nullptr;  // changed CDS of a tick (stem_list_entries)
     int32_t *d_sctl = nullptr;    // their counts (STEM_MAX_GROUPS), zero between ticks
     size_t cap_jobs = 0, cap_off = 0, cap_dom = 0, cap_asc = 0, cap_slist = 0;
     hipGraph_t graph = nullptr;
@@ -267,7 +267,7 @@ hipError_t rebuild(cd_server *S, const std::vector<Entry *> &res) {
     if (e != hipSuccess) return e;
     const cdhost::Launch L{S->d_jobs,   (int)wl.descs.size(), S->d_off,      (int)wl.off.size(), S->d_dom,
                            (int)wl.dom.size(), S->d_asc,      (int)wl.asc.size(), wl.lds,         wl.stem_lds,
-                           wl.max_pool,  wl.max_refs,        wl.mg,               wl.stem_parts,      S->d_slist,     S->d_sctl,
+                           wl.max_pool,  wl.max_refs,        wl.mg,               S->d_slist,     S->d_sctl,
                            wl.n_cds,     wl.n_small,          wl.lds_small,       wl.pool,           sh};
     if (S->gexec) (void)hipGraphExecDestroy(S->gexec);
     if (S->graph) (void)hipGraphDestroy(S->graph);
