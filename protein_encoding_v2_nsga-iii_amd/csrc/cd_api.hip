@@ -150,57 +150,79 @@ struct Sizes {
 
 namespace {
 
-// Lay out every device buffer of a job in one allocation.
+// What a descriptor is set up for: a job, one evaluation of P designs, or one
+// selection from P objective vectors (a sort is the first part of one).
+enum class Use { Job, Evaluate, Select };
+
+// Lay out every device buffer of a job in one allocation.  The regions the
+// host fills come first, `head` bytes in all, and go up in one transfer; what
+// a single evaluation (obj, oidx, pql) or selection (st, selm, front) gives
+// back lies together and comes down in one.
 struct Layout {
     size_t pos, code, lw6, cpfx6, cps6, ref, genome[2], obj[2], oidx[2], pql[2], cst[2], hdp[2], planes, stem_max, slist,
         sctl,
         front,
         np, dom,
         ref_of, dist, niche, st, acc, ranked, selm, prio, cutl, cutr, self, off, domi, asc;
-    size_t total;
+    size_t head, total;
 };
 
-Layout layout(int L, int m, int N, int P, int R, int W, int n_dom, int n_asc, bool sel_only) {
+Layout layout(int L, int m, int N, int P, int R, int W, int n_dom, int n_asc, Use use) {
     Sizes s;
     Layout o{};
-    if (!sel_only) {
+    o.self = s.add(sizeof(cd::DevJob));
+    if (use != Use::Select) {
         o.pos = s.add(2 * (size_t)cd::row_stride(L));
         o.code = s.add(64);
         o.lw6 = s.add(128 * 8);
         o.cpfx6 = s.add(64 * 64 * 8);
         o.cps6 = s.add(64 * 64 * 4);
-        for (int b = 0; b < 2; ++b) {
-            o.genome[b] = s.add((size_t)P * m * cd::row_stride(L));
+        o.off = s.add((size_t)(use == Use::Job ? N : P) * sizeof(int2));
+    }
+    if (use != Use::Evaluate) {
+        o.ref = s.add((size_t)R * cd::REF_STRIDE * 4);
+        o.domi = s.add((size_t)n_dom * sizeof(int4));
+        o.asc = s.add((size_t)n_asc * sizeof(int2));
+    }
+    if (use == Use::Select) {
+        o.obj[0] = o.obj[1] = s.add((size_t)P * 6 * 4);
+        o.st = s.add(sizeof(cd::SelState));
+        o.head = s.total;
+        o.selm = s.add((size_t)W * 8);
+        o.front = s.add((size_t)P * 4);
+    } else {
+        o.head = s.total;
+        for (int b = 0; b < (use == Use::Job ? 2 : 1); ++b) {
+            o.obj[b] = s.add((size_t)P * 6 * 4);
             o.oidx[b] = s.add((size_t)P * 12);
             o.pql[b] = s.add((size_t)P * 16);
+            // (an evaluation reads packed rows, in whole words)
+            o.genome[b] = s.add(use == Use::Job ? (size_t)P * m * cd::row_stride(L) : (size_t)P * m * L + 8);
             o.cst[b] = s.add((size_t)P * m * sizeof(cd::CdsStat));
             o.hdp[b] = s.add((size_t)P * (m * (m - 1) / 2) * 4);
         }
-        o.off = s.add((size_t)N * sizeof(int2));
         o.planes = s.add((size_t)P * m * cd::cds_plane_bytes(L));
         o.stem_max = s.add((size_t)P * 4);
+    }
+    if (use == Use::Job) {
         o.slist = s.add(cd::stem_list_entries(N, m) * sizeof(uint2));
         o.sctl = s.add((size_t)cd::STEM_MAX_GROUPS * 4);
+        o.st = s.add(sizeof(cd::SelState));
+        o.selm = s.add((size_t)W * 8);
+        o.front = s.add((size_t)P * 4);
     }
-    for (int b = 0; b < (sel_only ? 1 : 2); ++b) o.obj[b] = s.add((size_t)P * 6 * 4);
-    if (sel_only) o.obj[1] = o.obj[0];
-    o.ref = s.add((size_t)R * cd::REF_STRIDE * 4);
-    o.front = s.add((size_t)P * 4);
-    o.np = s.add((size_t)P * 4);
-    o.dom = s.add((size_t)P * W * 8);
-    o.ref_of = s.add((size_t)P * 4);
-    o.dist = s.add((size_t)P * 4);
-    o.niche = s.add((size_t)cd::NICHE_INTS * R * 4);
-    o.st = s.add(sizeof(cd::SelState));
-    o.acc = s.add(sizeof(cd::SelAcc));
-    o.ranked = s.add((size_t)W * 8);
-    o.selm = s.add((size_t)W * 8);
-    o.prio = s.add((size_t)P * 4);
-    o.cutl = s.add((size_t)P * 8);
-    o.cutr = s.add((size_t)P * 4);
-    o.self = s.add(sizeof(cd::DevJob));
-    o.domi = s.add((size_t)n_dom * sizeof(int4));
-    o.asc = s.add((size_t)n_asc * sizeof(int2));
+    if (use != Use::Evaluate) {
+        o.np = s.add((size_t)P * 4);
+        o.dom = s.add((size_t)P * W * 8);
+        o.ref_of = s.add((size_t)P * 4);
+        o.dist = s.add((size_t)P * 4);
+        o.niche = s.add((size_t)cd::NICHE_INTS * R * 4);
+        o.acc = s.add(sizeof(cd::SelAcc));
+        o.ranked = s.add((size_t)W * 8);
+        o.prio = s.add((size_t)P * 4);
+        o.cutl = s.add((size_t)P * 8);
+        o.cutr = s.add((size_t)P * 4);
+    }
     o.total = s.total;
     return o;
 }
@@ -285,39 +307,137 @@ hipError_t keep_pool_memory() {
     return e;
 }
 
-// Regions of a job's allocation to upload at creation; the rest of the
-// allocation is zero (cleared on the device).
-struct Upload {
-    std::vector<char> bytes;
-    std::vector<std::pair<size_t, std::pair<size_t, size_t>>> parts;  // (device offset, (host offset, size))
-    template <class T>
-    void add(size_t dev_off, const T *src, size_t count) {
-        const size_t at = bytes.size(), n = count * sizeof(T);
-        bytes.resize(at + n);
-        std::memcpy(bytes.data() + at, src, n);
-        parts.push_back({dev_off, {at, n}});
-    }
-};
-
-int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out) {
-    cd_job *J = new cd_job();
-    J->selection_only = sel_only;
-    J->L = sel_only ? 0 : d->L;
-    J->m = sel_only ? 0 : d->m;
+// The sizes of a descriptor's job (J->N, H, L, m, R, P, W), its layout and its
+// tables.
+int size_job(cd_job *J, const cd_job_desc *d, Use use, int P, Layout &o, HostTables &t) {
+    J->selection_only = use == Use::Select;
+    J->L = use == Use::Select ? 0 : d->L;
+    J->m = use == Use::Select ? 0 : d->m;
     J->N = d->N;
     J->H = d->H;
     J->R = (int)n_ref(d->H);
-    J->P = P_override > 0 ? P_override : 2 * d->N;
-    J->W = (J->P + 63) / 64;
+    J->P = P;
+    J->W = (P + 63) / 64;
     work_counts(J->P, J->W, &J->n_dom, &J->n_asc);
-    Layout o = layout(J->L, J->m, J->N, J->P, J->R, J->W, J->n_dom, J->n_asc, sel_only);
-    HostTables t;
-    if (!sel_only) {
-        const int rc = build_tables(d->tables, t);
-        if (rc != CD_OK) {
-            delete J;
-            return rc;
+    o = layout(J->L, J->m, J->N, J->P, J->R, J->W, J->n_dom, J->n_asc, use);
+    return use == Use::Select ? CD_OK : build_tables(d->tables, t);
+}
+
+// The descriptor and work lists of J in an allocation at base, and the image
+// of its first o.head bytes (cleared by the caller).
+void describe_job(cd_job *J, const cd_job_desc *d, Use use, const Layout &o, const HostTables &t, char *base, char *image) {
+    auto put = [&](size_t at, const void *src, size_t bytes) { std::memcpy(image + at, src, bytes); };
+    const bool designs = use != Use::Select, select = use != Use::Evaluate;
+    cd::DevJob &h = J->h;
+    h.L = J->L;
+    h.m = J->m;
+    h.N = J->N;
+    h.P = J->P;
+    h.R = J->R;
+    h.W = J->W;
+    h.den_sl = designs ? (3 * J->L - 4) / 2 : 1;
+    h.Ls = designs ? cd::row_stride(J->L) : 0;
+    h.seed = d->seed;
+    h.thr_pm = bern_threshold_host(d->Pm);
+    h.thr_2pm = bern_threshold_host(d->Pm * 2.0f);
+    h.gc3_ref = d->tables.gc3_ref;
+    for (int b = 0; b < 2; ++b) h.obj[b] = (float *)(base + o.obj[use == Use::Job ? b : 0]);
+    if (designs) {
+        // per position the first codon of its amino acid and its synonym count
+        uint8_t *pos = (uint8_t *)image + o.pos;
+        for (int k = 0; k < h.Ls; ++k) {
+            const int a = k < J->L ? d->aa[k] : -1;
+            pos[k] = a >= 0 ? (uint8_t)SYN_START[a] : 0;
+            pos[h.Ls + k] = a >= 0 ? (uint8_t)SYN_NUM[a] : 1;
         }
+        put(o.code, t.code, 64);
+        put(o.lw6, t.lw6, 64 * 8);
+        put(o.lw6 + 64 * 8, t.syn6, 64 * 8);
+        put(o.cpfx6, t.cpfx6, 64 * 64 * 8);
+        put(o.cps6, t.cps6, 64 * 64 * 4);
+        h.pos = (const uint8_t *)(base + o.pos);
+        h.code = (const uint8_t *)(base + o.code);
+        h.lw6 = (const int64_t *)(base + o.lw6);
+        h.cpfx6 = (const int64_t *)(base + o.cpfx6);
+        h.cps6 = (const float *)(base + o.cps6);
+        h.stop6 = t.stop6;
+        for (int b = 0; b < 2; ++b) {
+            const int u = use == Use::Job ? b : 0;
+            h.genome[b] = (int8_t *)(base + o.genome[u]);
+            h.oidx[b] = (int8_t *)(base + o.oidx[u]);
+            h.pql[b] = (int32_t *)(base + o.pql[u]);
+            h.cst[b] = (cd::CdsStat *)(base + o.cst[u]);
+            h.hdp[b] = (int32_t *)(base + o.hdp[u]);
+        }
+        h.planes = (uint2 *)(base + o.planes);
+        h.stem_max = (int32_t *)(base + o.stem_max);
+        int2 *off = (int2 *)(image + o.off);
+        for (int c = 0, n = use == Use::Job ? J->N : J->P; c < n; ++c) off[c] = make_int2(0, c);
+        J->d_off = (int2 *)(base + o.off);
+        J->lds = cd::design_lds_bytes(J->L, J->m);
+        J->stem_lds = cd::stem_lds_bytes(J->L);
+    }
+    if (use == Use::Job) {
+        J->d_slist = (uint2 *)(base + o.slist);  // the counts in d_sctl start at zero with the cleared allocation
+        J->d_sctl = (int32_t *)(base + o.sctl);
+        // the tuned shapes of this kind of job, if any
+        cd_job *self = J;
+        cd::Shapes sh;
+        J->shapes = cdhost::untuned_shapes(&self, 1);
+        if (cdhost::cached_shapes(cdhost::work_signature(&self, 1), &sh)) J->shapes = sh;
+    } else {
+        J->shapes.dom_rows = cd::DOM_ROWS;
+    }
+    if (select) {
+        const auto ref = das_dennis(d->H);
+        put(o.ref, ref.data(), ref.size() * sizeof(float));
+        h.refpts = (const float *)(base + o.ref);
+        h.front_of = (int32_t *)(base + o.front);
+        h.np = (int32_t *)(base + o.np);
+        h.dom = (uint64_t *)(base + o.dom);
+        h.ref_of = (int32_t *)(base + o.ref_of);
+        h.dist = (float *)(base + o.dist);
+        h.niche = (int32_t *)(base + o.niche);
+        h.st = (cd::SelState *)(base + o.st);
+        h.acc = (cd::SelAcc *)(base + o.acc);
+        h.ranked = (uint64_t *)(base + o.ranked);
+        h.selm = (uint64_t *)(base + o.selm);
+        h.prio = (uint32_t *)(base + o.prio);
+        h.cutl = (uint64_t *)(base + o.cutl);
+        h.cutr = (int32_t *)(base + o.cutr);
+        std::vector<int4> dom;
+        std::vector<int2> asc;
+        job_lists(J->P, J->W, J->shapes, dom, asc);
+        put(o.domi, dom.data(), dom.size() * sizeof(int4));
+        put(o.asc, asc.data(), asc.size() * sizeof(int2));
+        J->n_dom = (int)dom.size();
+        J->n_asc = (int)asc.size();
+        J->d_dom = (int4 *)(base + o.domi);
+        J->d_asc = (int2 *)(base + o.asc);
+    }
+    put(o.self, &h, sizeof(h));
+    J->d_self = (cd::DevJob *)(base + o.self);
+}
+
+// Raise the kernels' dynamic LDS limits to what J's launches take.
+hipError_t job_lds_limits(const cd_job *J, bool select) {
+    hipError_t e = hipSuccess;
+    if (J->lds > 48 * 1024) e = cd::set_design_lds_limit(J->lds);
+    if (e == hipSuccess && cd::stem_list_lds(J->stem_lds) > 48 * 1024)
+        e = cd::set_stem_lds_limit(cd::stem_list_lds(J->stem_lds));
+    if (e == hipSuccess && select && cd::niche_lds_need(J->P, J->R) > cd::NICHE_LDS_PLAIN)
+        e = cd::set_niche_lds_limit(cd::niche_lds_need(J->P, J->R));
+    return e;
+}
+
+int create_job(const cd_job_desc *d, cd_job **out) {
+    cd_job *J = new cd_job();
+    Layout o;
+    HostTables t;
+    const int rc = size_job(J, d, Use::Job, 2 * d->N, o, t);
+    if (rc != CD_OK) {
+        delete J;
+        return rc;
     }
     // the job's own stream does not wait for (or hold up) work on other
     // streams, such as a served tick that is running while this job is
@@ -335,110 +455,12 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
     }
     J->mem_bytes = o.total;
     char *base = (char *)J->mem;
-    Upload up;
-    cd::DevJob &h = J->h;
-    h.L = J->L;
-    h.m = J->m;
-    h.N = J->N;
-    h.P = J->P;
-    h.R = J->R;
-    h.W = J->W;
-    h.den_sl = sel_only ? 1 : (3 * J->L - 4) / 2;
-    h.Ls = sel_only ? 0 : cd::row_stride(J->L);
-    h.seed = d->seed;
-    h.thr_pm = bern_threshold_host(d->Pm);
-    h.thr_2pm = bern_threshold_host(d->Pm * 2.0f);
-    h.gc3_ref = d->tables.gc3_ref;
-    if (!sel_only) {
-        {  // per position the first codon of its amino acid and its synonym count
-            const int Ls = cd::row_stride(J->L);
-            std::vector<uint8_t> pos(2 * (size_t)Ls, 0);
-            for (int k = 0; k < Ls; ++k) {
-                const int a = k < J->L ? d->aa[k] : -1;
-                pos[k] = a >= 0 ? (uint8_t)SYN_START[a] : 0;
-                pos[Ls + k] = a >= 0 ? (uint8_t)SYN_NUM[a] : 1;
-            }
-            up.add(o.pos, pos.data(), pos.size());
-        }
-        up.add(o.code, t.code, 64);
-        up.add(o.lw6, t.lw6, 64);
-        up.add(o.lw6 + 64 * 8, t.syn6, 64);
-        up.add(o.cpfx6, t.cpfx6, 64 * 64);
-        up.add(o.cps6, t.cps6, 64 * 64);
-        h.pos = (const uint8_t *)(base + o.pos);
-        h.code = (const uint8_t *)(base + o.code);
-        h.lw6 = (const int64_t *)(base + o.lw6);
-        h.cpfx6 = (const int64_t *)(base + o.cpfx6);
-        h.cps6 = (const float *)(base + o.cps6);
-        h.stop6 = t.stop6;
-        for (int b = 0; b < 2; ++b) {
-            h.genome[b] = (int8_t *)(base + o.genome[b]);
-            h.oidx[b] = (int8_t *)(base + o.oidx[b]);
-            h.pql[b] = (int32_t *)(base + o.pql[b]);
-            h.cst[b] = (cd::CdsStat *)(base + o.cst[b]);
-            h.hdp[b] = (int32_t *)(base + o.hdp[b]);
-        }
-        std::vector<int2> off(J->N);
-        for (int c = 0; c < J->N; ++c) off[c] = make_int2(0, c);
-        up.add(o.off, off.data(), off.size());
-        J->d_off = (int2 *)(base + o.off);
-        J->d_slist = (uint2 *)(base + o.slist);  // the counts in d_sctl start at zero with the cleared allocation
-        J->d_sctl = (int32_t *)(base + o.sctl);
-        J->lds = cd::design_lds_bytes(J->L, J->m);
-        J->stem_lds = cd::stem_lds_bytes(J->L);
-    }
-    const auto ref = das_dennis(d->H);
-    up.add(o.ref, ref.data(), ref.size());
-    h.refpts = (const float *)(base + o.ref);
-    h.obj[0] = (float *)(base + o.obj[0]);
-    h.obj[1] = (float *)(base + o.obj[1]);
-    h.front_of = (int32_t *)(base + o.front);
-    h.np = (int32_t *)(base + o.np);
-    h.planes = sel_only ? nullptr : (uint2 *)(base + o.planes);
-    h.stem_max = sel_only ? nullptr : (int32_t *)(base + o.stem_max);
-    h.dom = (uint64_t *)(base + o.dom);
-    h.ref_of = (int32_t *)(base + o.ref_of);
-    h.dist = (float *)(base + o.dist);
-    h.niche = (int32_t *)(base + o.niche);
-    h.st = (cd::SelState *)(base + o.st);
-    h.acc = (cd::SelAcc *)(base + o.acc);
-    h.ranked = (uint64_t *)(base + o.ranked);
-    h.selm = (uint64_t *)(base + o.selm);
-    h.prio = (uint32_t *)(base + o.prio);
-    h.cutl = (uint64_t *)(base + o.cutl);
-    h.cutr = (int32_t *)(base + o.cutr);
-    up.add(o.self, &h, 1);
-    J->d_self = (cd::DevJob *)(base + o.self);
-    if (!sel_only) {  // the tuned shapes of this kind of job, if any
-        cd_job *self = J;
-        cd::Shapes sh;
-        J->shapes = cdhost::untuned_shapes(&self, 1);
-        if (cdhost::cached_shapes(cdhost::work_signature(&self, 1), &sh)) J->shapes = sh;
-    } else {
-        J->shapes.dom_rows = cd::DOM_ROWS;
-    }
-    {
-        std::vector<int4> dom;
-        std::vector<int2> asc;
-        job_lists(J->P, J->W, J->shapes, dom, asc);
-        up.add(o.domi, dom.data(), dom.size());
-        up.add(o.asc, asc.data(), asc.size());
-        J->n_dom = (int)dom.size();
-        J->n_asc = (int)asc.size();
-    }
-    J->d_dom = (int4 *)(base + o.domi);
-    J->d_asc = (int2 *)(base + o.asc);
-    e = hipMemsetAsync(J->mem, 0, o.total, J->stream);
-    for (const auto &pt : up.parts)
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(base + pt.first, up.bytes.data() + pt.second.first, pt.second.second,
-                               hipMemcpyHostToDevice, J->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(J->stream);  // the staged bytes are released below
-    if (e == hipSuccess && J->lds > 48 * 1024) e = cd::set_design_lds_limit(J->lds);
-    if (e == hipSuccess && cd::stem_list_lds(J->stem_lds) > 48 * 1024)
-        e = cd::set_stem_lds_limit(cd::stem_list_lds(J->stem_lds));
-    if (e == hipSuccess && cd::niche_lds_need(J->P, J->R) > cd::NICHE_LDS_PLAIN)
-        e = cd::set_niche_lds_limit(cd::niche_lds_need(J->P, J->R));
+    std::vector<char> image(o.head, 0);
+    describe_job(J, d, Use::Job, o, t, base, image.data());
+    e = hipMemsetAsync(base + o.head, 0, o.total - o.head, J->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(base, image.data(), o.head, hipMemcpyHostToDevice, J->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(J->stream);  // the image is released below
+    if (e == hipSuccess) e = job_lds_limits(J, true);
     if (e != hipSuccess) {
         (void)hipFreeAsync(J->mem, J->stream);
         (void)hipStreamSynchronize(J->stream);
@@ -448,6 +470,85 @@ int create_job(const cd_job_desc *d, bool sel_only, int P_override, cd_job **out
     }
     *out = J;
     return CD_OK;
+}
+
+// A stream with a device and a pinned host buffer for the calls that hold
+// nothing from one to the next (cd_eval_batch, cd_nds, cd_select).  A call
+// takes one for its duration -- an idle one of its device, else a new one -- so
+// calls of several threads run side by side; at most SHOTS_IDLE idle ones with
+// buffers of at most SHOT_KEEP bytes are kept, the others are freed with the
+// call.  With them, one transfer each way and one synchronisation an evaluation
+// of 16 designs takes 58 us instead of 271, a selection of 1024 from 2048 104
+// instead of 269; with the chunks below one of 2048 designs of 2004 codons 314
+// instead of 482.
+constexpr size_t EVAL_CHUNK = (size_t)1 << 20;  // bytes of packed rows
+constexpr size_t SHOTS_IDLE = 4, SHOT_KEEP = (size_t)64 << 20;
+struct Shot {
+    int dev = 0;
+    hipStream_t stream = nullptr;
+    char *mem = nullptr, *host = nullptr;
+    size_t mem_cap = 0, host_cap = 0;
+    hipError_t reserve(size_t mem_bytes, size_t host_bytes) {
+        hipError_t e = hipSuccess;
+        if (mem_bytes > mem_cap) {
+            if (mem) (void)hipFreeAsync(mem, stream);
+            mem = nullptr;
+            mem_cap = 0;
+            e = hipMallocAsync((void **)&mem, mem_bytes + mem_bytes / 4, stream);
+            if (e == hipSuccess) mem_cap = mem_bytes + mem_bytes / 4;
+        }
+        if (e == hipSuccess && host_bytes > host_cap) {
+            if (host) (void)hipHostFree(host);
+            host = nullptr;
+            host_cap = 0;
+            e = hipHostMalloc((void **)&host, host_bytes + host_bytes / 4, hipHostMallocDefault);
+            if (e == hipSuccess) host_cap = host_bytes + host_bytes / 4;
+        }
+        return e;
+    }
+    void free() {
+        if (mem) (void)hipFreeAsync(mem, stream);
+        if (stream) {
+            (void)hipStreamSynchronize(stream);
+            (void)hipStreamDestroy(stream);
+        }
+        if (host) (void)hipHostFree(host);
+    }
+};
+struct Shots {
+    std::mutex mu;
+    std::vector<Shot> idle;
+    hipError_t take(Shot &s) {
+        hipError_t e = hipGetDevice(&s.dev);
+        if (e != hipSuccess) return e;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            for (size_t i = idle.size(); i-- > 0;)
+                if (idle[i].dev == s.dev) {
+                    s = idle[i];
+                    idle.erase(idle.begin() + (ptrdiff_t)i);
+                    return hipSuccess;
+                }
+        }
+        e = hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking);
+        if (e == hipSuccess) e = keep_pool_memory();
+        return e;
+    }
+    // ok: the call's work has ended without an error
+    void give(Shot &s, bool ok) {
+        if (ok && s.mem_cap <= SHOT_KEEP && s.host_cap <= SHOT_KEEP) {
+            std::lock_guard<std::mutex> lk(mu);
+            if (idle.size() < SHOTS_IDLE) {
+                idle.push_back(s);
+                return;
+            }
+        }
+        s.free();
+    }
+};
+Shots &shots() {  // (never destroyed: the runtime may be gone by then)
+    static Shots *p = new Shots();
+    return *p;
 }
 
 // Evaluate the designs of `items`: mutation (children) and objectives 0-4,
@@ -773,14 +874,14 @@ int64_t cd_job_device_bytes(int32_t L, int32_t m, int32_t N, int32_t H) {
     const int P = 2 * N, W = (P + 63) / 64;
     int n_dom, n_asc;
     work_counts(P, W, &n_dom, &n_asc);
-    return (int64_t)layout(L, m, N, P, (int)n_ref(H), W, n_dom, n_asc, false).total;
+    return (int64_t)layout(L, m, N, P, (int)n_ref(H), W, n_dom, n_asc, Use::Job).total;
 }
 
 int cd_job_create(const cd_job_desc *desc, cd_job **out) {
     if (!out) return fail(CD_E_INVALID, "null output handle");
     int rc = validate(desc);
     if (rc != CD_OK) return rc;
-    return create_job(desc, false, 0, out);
+    return create_job(desc, out);
 }
 
 int cd_job_init(cd_job *J) {
@@ -926,116 +1027,143 @@ int cd_eval_batch(const cd_job_desc *desc, const int8_t *genome, int32_t count, 
                   int32_t *pql) {
     if (!desc || !genome || count <= 0) return fail(CD_E_INVALID, "bad eval arguments");
     cd_job_desc d = *desc;
-    d.N = (count + 1) / 2;
+    d.N = (int32_t)(((int64_t)count + 1) / 2);
     d.H = 1;
     d.Pm = 0.f;
     int rc = validate(&d);
     if (rc != CD_OK) return rc;
-    cd_job *J = nullptr;
-    rc = create_job(&d, false, 0, &J);
+    cd_job job;
+    cd_job *J = &job;
+    Layout o;
+    HostTables t;
+    rc = size_job(J, &d, Use::Evaluate, count, o, t);
     if (rc != CD_OK) return rc;
-    std::vector<int2> items(count);
-    for (int i = 0; i < count; ++i) items[i] = make_int2(0, i);
-    int2 *d_items = nullptr;
-    hipError_t e = hipMalloc(&d_items, sizeof(int2) * count);
-    if (e == hipSuccess) e = hipMemcpy(d_items, items.data(), sizeof(int2) * count, hipMemcpyHostToDevice);
-    if (e == hipSuccess) {  // CDS rows of L codons into rows of stride Ls (zero pads), one transfer
-        const size_t rows = (size_t)count * J->m, L = J->L, Ls = J->h.Ls;
-        std::lock_guard<std::mutex> lk(g_rows.mu);
-        e = g_rows.reserve(rows * Ls);
-        if (e == hipSuccess) {
-            for (size_t r = 0; r < rows; ++r) {
-                std::memcpy(g_rows.p + r * Ls, genome + r * L, L);
-                std::memset(g_rows.p + r * Ls + L, 0, Ls - L);
-            }
-            e = hipMemcpy(J->h.genome[0], g_rows.p, rows * Ls, hipMemcpyHostToDevice);
-        }
+    const size_t row = (size_t)J->m * J->L, bytes = row * count;
+    const size_t out_bytes = o.genome[0] - o.obj[0];
+    Shot w;
+    hipError_t e = shots().take(w);
+    if (e == hipSuccess) e = w.reserve(o.total, o.head + bytes + 16 + out_bytes);
+    if (e != hipSuccess) {
+        shots().give(w, false);
+        return fail(CD_E_NOMEM, std::string("eval buffers: ") + hipGetErrorString(e));
     }
-    if (e == hipSuccess) e = enqueue_designs(job_launch(J), cd::MODE_EVAL, d_items, count, J->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(J->stream);
-    if (e == hipSuccess && obj) e = hipMemcpy(obj, J->h.obj[0], (size_t)count * 24, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && idx) e = hipMemcpy(idx, J->h.oidx[0], (size_t)count * 12, hipMemcpyDeviceToHost);
-    std::vector<int32_t> t((size_t)count * 4);
-    if (e == hipSuccess && pql) e = hipMemcpy(t.data(), J->h.pql[0], t.size() * 4, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && pql)
-        for (int i = 0; i < count; ++i)
-            for (int k = 0; k < 3; ++k) pql[i * 3 + k] = t[(size_t)i * 4 + k];
-    if (d_items) (void)hipFree(d_items);
-    cd_job_destroy(J);
+    char *const stage = w.host + o.head, *const res = stage + ((bytes + 15) & ~(size_t)15);
+    std::memset(w.host, 0, o.head);
+    describe_job(J, &d, Use::Evaluate, o, t, w.mem, w.host);
+    e = job_lds_limits(J, false);
+    if (e == hipSuccess) e = hipMemcpyAsync(w.mem, w.host, o.head, hipMemcpyHostToDevice, w.stream);
+    // The rows go up packed as the caller holds them (k_design addresses them
+    // bytewise), EVAL_CHUNK bytes at a time, so that the copy into pinned
+    // memory, the transfer and the kernels of successive chunks overlap.
+    const int per = std::max(1, (int)std::min<size_t>(EVAL_CHUNK / row, (size_t)count));
+    for (int i = 0; i < count && e == hipSuccess; i += per) {
+        const int n = std::min(per, count - i);
+        std::memcpy(stage + i * row, genome + i * row, n * row);
+        e = hipMemcpyAsync(w.mem + o.genome[0] + i * row, stage + i * row, n * row, hipMemcpyHostToDevice, w.stream);
+        if (e == hipSuccess) e = cd::launch_design(cd::MODE_EVAL, J->d_self, J->d_off + i, n, J->lds, w.stream);
+        if (e == hipSuccess) e = cd::launch_stem(cd::MODE_EVAL, J->d_self, J->d_off + i, n, J->m, J->stem_lds, w.stream);
+    }
+    if (e == hipSuccess) e = cd::launch_stem_finish(cd::MODE_EVAL, J->d_self, J->d_off, count, w.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(res, w.mem + o.obj[0], out_bytes, hipMemcpyDeviceToHost, w.stream);
+    const hipError_t es = hipStreamSynchronize(w.stream);
+    if (e == hipSuccess) e = es;
+    if (e == hipSuccess) {
+        if (obj) std::memcpy(obj, res, (size_t)count * 24);
+        if (idx) std::memcpy(idx, res + (o.oidx[0] - o.obj[0]), (size_t)count * 12);
+        const int32_t *q = (const int32_t *)(res + (o.pql[0] - o.obj[0]));
+        if (pql)
+            for (int i = 0; i < count; ++i)
+                for (int k = 0; k < 3; ++k) pql[i * 3 + k] = q[(size_t)i * 4 + k];
+    }
+    shots().give(w, e == hipSuccess);
     if (e != hipSuccess) return fail(CD_E_DEVICE, std::string("eval: ") + hipGetErrorString(e));
     return CD_OK;
 }
 
+// One selection (full) or sort of P objective vectors.  On success *st, mask
+// (J.W words) and front (P) hold its state, survivor mask and fronts.
 static int run_selection(const float *obj, int32_t P, int32_t N, int32_t H, uint32_t gen, uint64_t seed,
-                         const float *extremes, bool full, cd_job **out) {
+                         const float *extremes, bool full, cd::SelState *st, std::vector<uint64_t> *mask, int32_t *front) {
     if (!obj || P <= 0 || N <= 0 || N > P || P > 64 * cd::MAX_W || H < 1)
         return fail(CD_E_INVALID, "bad selection arguments");
     cd_job_desc d{};
     d.N = N;
     d.H = H;
     d.seed = seed;
-    cd_job *J = nullptr;
-    int rc = create_job(&d, true, P, &J);
+    cd_job job;
+    cd_job *J = &job;
+    Layout o;
+    HostTables t;
+    int rc = size_job(J, &d, Use::Select, P, o, t);
     if (rc != CD_OK) return rc;
-    cd::SelState st{};
-    st.gen = gen;
-    if (extremes) std::memcpy(st.res[gen & 1u].ext, extremes, sizeof(st.res[0].ext));
-    hipError_t e = hipMemcpy(J->h.obj[0], obj, (size_t)P * 24, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(J->h.st, &st, sizeof(st), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = cd::launch_zero_np(J->d_self, 1, J->stream);
-    const cd::Shapes &sh = J->shapes;
-    if (e == hipSuccess) e = cd::launch_dominance(J->d_self, J->d_dom, J->n_dom, false, nullptr, 0, sh.dom_rows, J->stream);
-    if (e == hipSuccess) e = cd::launch_fronts(J->d_self, 1, J->P, sh.fronts_threads, J->stream);
-    if (e == hipSuccess && full) e = cd::launch_associate(J->d_self, J->d_asc, J->n_asc, sh.assoc_designs, J->stream);
-    if (e == hipSuccess && full) e = cd::launch_niche(J->d_self, 1, J->P, J->R, sh.niche_threads, J->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(J->stream);
+    const size_t out_bytes = o.front + (size_t)P * 4 - o.st;
+    Shot w;
+    hipError_t e = shots().take(w);
+    if (e == hipSuccess) e = w.reserve(o.total, o.head + out_bytes);
     if (e != hipSuccess) {
-        cd_job_destroy(J);
-        return fail(CD_E_DEVICE, std::string("selection: ") + hipGetErrorString(e));
+        shots().give(w, false);
+        return fail(CD_E_NOMEM, std::string("selection buffers: ") + hipGetErrorString(e));
     }
-    *out = J;
+    std::memset(w.host, 0, o.head);
+    describe_job(J, &d, Use::Select, o, t, w.mem, w.host);
+    std::memcpy(w.host + o.obj[0], obj, (size_t)P * 24);
+    cd::SelState *s0 = (cd::SelState *)(w.host + o.st);
+    s0->gen = gen;
+    if (extremes) std::memcpy(s0->res[gen & 1u].ext, extremes, sizeof(s0->res[0].ext));
+    e = job_lds_limits(J, true);
+    if (e == hipSuccess) e = hipMemsetAsync(w.mem + o.head, 0, o.total - o.head, w.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(w.mem, w.host, o.head, hipMemcpyHostToDevice, w.stream);
+    if (e == hipSuccess) e = cd::launch_zero_np(J->d_self, 1, w.stream);
+    const cd::Shapes &sh = J->shapes;
+    if (e == hipSuccess) e = cd::launch_dominance(J->d_self, J->d_dom, J->n_dom, false, nullptr, 0, sh.dom_rows, w.stream);
+    const bool fused = full && cd::fuse_fronts(P, P);
+    if (e == hipSuccess && !fused) e = cd::launch_fronts(J->d_self, 1, P, sh.fronts_threads, w.stream);
+    if (e == hipSuccess && full)
+        e = fused ? cd::launch_front_associate(J->d_self, J->d_asc, J->n_asc, sh.assoc_designs, w.stream)
+                  : cd::launch_associate(J->d_self, J->d_asc, J->n_asc, sh.assoc_designs, w.stream);
+    if (e == hipSuccess && full) e = cd::launch_niche(J->d_self, 1, P, J->R, sh.niche_threads, w.stream);
+    char *const res = w.host + o.head;
+    if (e == hipSuccess) e = hipMemcpyAsync(res, w.mem + o.st, out_bytes, hipMemcpyDeviceToHost, w.stream);
+    const hipError_t es = hipStreamSynchronize(w.stream);
+    if (e == hipSuccess) e = es;
+    if (e == hipSuccess) {
+        std::memcpy(st, res, sizeof(*st));
+        if (mask) {
+            mask->resize(J->W);
+            std::memcpy(mask->data(), res + (o.selm - o.st), (size_t)J->W * 8);
+        }
+        if (front) std::memcpy(front, res + (o.front - o.st), (size_t)P * 4);
+    }
+    shots().give(w, e == hipSuccess);
+    if (e != hipSuccess) return fail(CD_E_DEVICE, std::string("selection: ") + hipGetErrorString(e));
     return CD_OK;
 }
 
 int cd_nds(const float *obj, int32_t P, int32_t N, int32_t *front_of, int32_t *n_fronts) {
-    cd_job *J = nullptr;
-    int rc = run_selection(obj, P, N, 1, 0, 0, nullptr, false, &J);
-    if (rc != CD_OK) return rc;
     cd::SelState st;
-    hipError_t e = hipMemcpy(&st, J->h.st, sizeof(st), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && front_of) e = hipMemcpy(front_of, J->h.front_of, (size_t)P * 4, hipMemcpyDeviceToHost);
-    if (n_fronts) *n_fronts = st.res[1].last + 1;  // (the sort ran as generation 0)
-    cd_job_destroy(J);
-    if (e != hipSuccess) return fail(CD_E_DEVICE, std::string("nds: ") + hipGetErrorString(e));
-    return CD_OK;
+    const int rc = run_selection(obj, P, N, 1, 0, 0, nullptr, false, &st, nullptr, front_of);
+    if (rc == CD_OK && n_fronts) *n_fronts = st.res[1].last + 1;  // (the sort ran as generation 0)
+    return rc;
 }
 
 int cd_select(const float *obj, int32_t N, int32_t H, uint32_t gen, uint64_t seed, float *extremes, int32_t *sorted,
               int32_t *front_of, float *norm, int32_t *flags) {
-    cd_job *J = nullptr;
-    int rc = run_selection(obj, 2 * N, N, H, gen, seed, extremes, true, &J);
-    if (rc != CD_OK) return rc;
     cd::SelState st;
-    hipError_t e = hipMemcpy(&st, J->h.st, sizeof(st), hipMemcpyDeviceToHost);
-    std::vector<uint64_t> mask(J->W);
-    if (e == hipSuccess && sorted) e = hipMemcpy(mask.data(), J->h.selm, (size_t)J->W * 8, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && sorted) survivors_of(mask, N, sorted);
-    if (e == hipSuccess && front_of) e = hipMemcpy(front_of, J->h.front_of, (size_t)2 * N * 4, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) {
-        const cd::SelRes &r = st.res[(gen + 1u) & 1u];
-        if (extremes) std::memcpy(extremes, r.ext, sizeof(r.ext));
-        if (norm) {
-            std::memcpy(norm, r.ideal, 24);
-            std::memcpy(norm + 6, r.worst, 24);
-            std::memcpy(norm + 12, r.nadir, 24);
-        }
-        if (flags) {
-            flags[0] = r.n_cut;
-            flags[1] = r.hyp;
-        }
+    std::vector<uint64_t> mask;
+    const int rc = run_selection(obj, 2 * N, N, H, gen, seed, extremes, true, &st, &mask, front_of);
+    if (rc != CD_OK) return rc;
+    if (sorted) survivors_of(mask, N, sorted);
+    const cd::SelRes &r = st.res[(gen + 1u) & 1u];
+    if (extremes) std::memcpy(extremes, r.ext, sizeof(r.ext));
+    if (norm) {
+        std::memcpy(norm, r.ideal, 24);
+        std::memcpy(norm + 6, r.worst, 24);
+        std::memcpy(norm + 12, r.nadir, 24);
     }
-    cd_job_destroy(J);
-    if (e != hipSuccess) return fail(CD_E_DEVICE, std::string("select: ") + hipGetErrorString(e));
+    if (flags) {
+        flags[0] = r.n_cut;
+        flags[1] = r.hyp;
+    }
     return CD_OK;
 }
 

@@ -1285,14 +1285,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
         // synonym indices to codes, four a word; the padding positions are
         // forced to code 0
         const uint8_t *const pos = J.pos, *const ctab = J.code;
-        const uint32_t *sg = (const uint32_t *)(genome0 + (size_t)it.y * m * Ls);
+        const uint32_t *sg = (const uint32_t *)genome0;  // rows of L bytes, packed; the buffer has a word past them
         const int nwd = Ls >> 2;
         uint32_t *c4 = (uint32_t *)rows;
         for (int c = 0; c < m; ++c)
             for (int q = tid; q < nwd; q += NT) {
                 const int left = L - 4 * q;  // positions of the word below L
                 const uint32_t keep = left >= 4 ? ~0u : (left <= 0 ? 0u : (1u << (8 * left)) - 1u);
-                const uint32_t g = (gload(sg + c * nwd + q) & keep) + gload((const uint32_t *)pos + q);  // bytewise
+                const size_t at = ((size_t)it.y * m + c) * L + (left > 0 ? 4 * q : 0);
+                const uint32_t s0 = gload(sg + (at >> 2)), s1 = gload(sg + (at >> 2) + 1);
+                const uint32_t sw = __builtin_amdgcn_alignbyte(s1, s0, (uint32_t)at & 3u);
+                const uint32_t g = (sw & keep) + gload((const uint32_t *)pos + q);  // bytewise
                 uint32_t code = 0;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) code |= (uint32_t)gload(ctab + ((g >> (8 * b)) & 0x3Fu)) << (8 * b);

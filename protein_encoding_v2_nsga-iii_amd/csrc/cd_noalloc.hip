@@ -1,6 +1,6 @@
 // cd_noalloc.hip -- non-dominated sorting that allocates nothing.
 //
-// cd_nds allocates a job-sized block for its scratch (the domination bit
+// cd_nds may allocate device memory for its scratch (the domination bit
 // matrix, dominator counts, selection state and work list).  Callers that
 // cannot allocate device memory (code under graph capture, tight serving
 // loops) use cd_nds_noalloc instead: the same kernels (k_dominance, k_fronts)
