@@ -67,10 +67,10 @@ size_t design_bytes_accepted(int L, int m) {
     return (size_t)576 + 2 * a + (size_t)m * ((a > b ? a : b) + a) + align16(m * (int)sizeof(CdsStat)) + 16;
 }
 
-// one CDS's bit planes: the sequence and its reverse complement, each
-// scan_words(3L) words of (low bits, high bits) of the nucleotide codes, then
-// its change mask (bit k: codon k changed) in whole 8-byte words
-__host__ __device__ inline int plane_words(int L) { return 2 * scan_words(3 * L) + ((sk_mask_words(L) + 1) >> 1); }
+// one CDS's bit planes as k_design leaves them: the sequence's, scan_words(3L)
+// words of (low bits, high bits) of the nucleotide codes, then the change mask
+// (bit k: codon k changed) in whole 8-byte words
+__host__ __device__ inline int plane_words(int L) { return scan_words(3 * L) + ((sk_mask_words(L) + 1) >> 1); }
 size_t cds_plane_bytes(int L) { return (size_t)plane_words(L) * sizeof(uint2); }
 
 // An entry of k_stem_list's list: CDS and child below; the buffer the child is
@@ -79,9 +79,10 @@ __device__ __forceinline__ uint64_t stem_entry(uint32_t job, uint32_t child, uin
     return (uint64_t)((child << 4) | c) | ((uint64_t)((job << 1) | buf) << 32);
 }
 
-// dynamic LDS of the stem kernels: a CDS's planes and change mask, then the
-// word search's index (the launchers add the waves' queues)
-__host__ __device__ inline int stem_index_at(int L) { return align16(plane_words(L) * (int)sizeof(uint2)); }
+// dynamic LDS of the stem kernels: a CDS's planes, its reverse complement's and
+// the change mask, then the word search's index (the launchers add the chain
+// heads and the waves' queues)
+__host__ __device__ inline int stem_index_at(int L) { return align16((scan_words(3 * L) + plane_words(L)) * (int)sizeof(uint2)); }
 size_t stem_lds_bytes(int L) { return (size_t)stem_index_at(L) + sk_lds_bytes(3 * L, 0, 0); }
 static size_t seek_more_bytes(int heads, int threads) {
     return (size_t)sk_lds_bytes(0, heads, threads / 64) - sk_lds_bytes(0, 0, 0);
@@ -250,6 +251,54 @@ __device__ __forceinline__ void seek_clear(const SeekLds &S) {
     for (int i = 0; i < HEADS / 4; i += NT)
         if (HEADS / 4 % NT == 0 || i + (int)threadIdx.x < HEADS / 4) b[SK_BITWORDS / 4 + i + threadIdx.x] = nil;
 }
+
+// A CDS's planes and change mask from the job's plane buffer g into LDS
+// (planes of the sequence, planes of the reverse complement, mask) by NT
+// threads: the first NT words' loads on construction, the rest and all stores
+// in place().  Bit b of the reverse complement is position n-1-b complemented:
+// a word of it is 32 positions of the sequence turned round.
+template <int NT>
+struct PlaneLoad {
+    const uint64_t *g;
+    int n, W, words;
+    uint64_t fwd, r0, r1, mask;
+    __device__ __forceinline__ int turn_at(int i) const { return max(n - 32 - 32 * i, 0) >> 5; }
+    __device__ __forceinline__ uint64_t turned(int i, uint64_t a, uint64_t b) const {
+        const int e = n - 32 * i, st = e - 32;  // positions st .. e-1
+        uint32_t lo, hi, keep = ~0u;
+        if (st >= 0) {
+            lo = scan_funnel((uint32_t)b, (uint32_t)a, st & 31);
+            hi = scan_funnel((uint32_t)(b >> 32), (uint32_t)(a >> 32), st & 31);
+        } else {
+            keep = e > 0 ? (1u << e) - 1u : 0u;
+            lo = (uint32_t)a << (-st & 31);
+            hi = (uint32_t)(a >> 32) << (-st & 31);
+        }
+        return (uint64_t)(~__builtin_bitreverse32(lo) & keep) | ((uint64_t)(~__builtin_bitreverse32(hi) & keep) << 32);
+    }
+    __device__ __forceinline__ PlaneLoad(const uint64_t *gp, int L) : g(gp), n(3 * L), W(scan_words(n)), words(plane_words(L)) {
+        const int tid = (int)threadIdx.x, i = min(tid, W - 1), t = turn_at(i);
+        fwd = gload(g + i);
+        r0 = gload(g + t);
+        r1 = gload(g + t + 1);
+        mask = gload(g + min(W + tid, words - 1));
+    }
+    __device__ __forceinline__ void place(uint64_t *planes) const {
+        const int tid = (int)threadIdx.x;
+        if (tid < W) {
+            planes[tid] = fwd;
+            planes[W + tid] = turned(tid, r0, r1);
+        }
+        if (W + tid < words) planes[2 * W + tid] = mask;
+        for (int i = tid + NT; i < W; i += NT) {
+            const int t = turn_at(i);
+            const uint64_t f = gload(g + i), a = gload(g + t), b = gload(g + t + 1);
+            planes[i] = f;
+            planes[W + i] = turned(i, a, b);
+        }
+        for (int i = W + tid + NT; i < words; i += NT) planes[W + i] = gload(g + i);
+    }
+};
 
 // Lanes of `bal` below the calling one.
 __device__ __forceinline__ int lanes_below(uint64_t bal) {
@@ -494,53 +543,37 @@ __device__ __forceinline__ uint32_t pack12(uint32_t x) {
     return (t & 0x3Fu) | ((t >> 10) & 0xFC0u);
 }
 
-// Bit planes of the CDS in row w into the job's plane buffer (sp, then rp):
-// bit p of the sequence plane is position p, of the reverse-complement plane
-// position n-1-p complemented; positions past n are zero; a word is (low bits,
-// high bits) of 32 positions.  A lane builds 32 codons (three words) of one
-// plane from eight words of codes; the reverse complement is the codons read
-// backwards, each with its bases reversed and complemented.  The change mask
-// follows the planes.
+// Bit planes of the CDS in row w into the job's plane buffer, then its change
+// mask: bit p is position p, positions past n are zero; a word is (low bits,
+// high bits) of 32 positions.  A lane builds a word from the eleven or twelve
+// codons it meets, which start at any byte; the reverse complement's planes
+// are made from these where they are used (PlaneLoad).  A lane per 32 codons
+// and both planes took a fifth of k_design's vector instructions: 64-job mix
+// 410 -> 379 us, 4096 children of 12 008 codons 106 -> 91, 128 of 202 13.5 ->
+// 11.9, and 2 to 6 us more in the stem kernels of the first two.
 __device__ __forceinline__ void task_planes(const uint32_t *w, int L, int nwd, const uint32_t *chg, uint2 *sp) {
-    const int n = 3 * L, W = scan_words(n), ng = (W + 2) / 3, lane = threadIdx.x & 63;
-    uint2 *const rp = sp + W;
-    for (int i = lane; i < 2 * ng; i += 64) {
-        const bool rev = i >= ng;
-        const int g = rev ? i - ng : i;
-        uint32_t lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+    const int n = 3 * L, W = scan_words(n), lane = threadIdx.x & 63;
+    for (int i = lane; i < W; i += 64) {
+        const uint32_t k0 = 32u * (uint32_t)i / 3u, r = 32u * (uint32_t)i - 3u * k0;
+        const int q = (int)(k0 >> 2);
+        uint32_t d[4];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {  // codons 32g + 4t .. 32g + 4t + 3 of the plane's sequence
-            const int u = 8 * g + t;
-            uint32_t l, h;
-            if (!rev) {
-                const uint32_t d = u < nwd ? w[u] : 0u;  // (the row's padding codes are 0)
-                // per byte the three bases' low (high) bits in position order
-                l = ((d >> 4) & 0x01010101u) | ((d >> 1) & 0x02020202u) | ((d << 2) & 0x04040404u);
-                h = ((d >> 5) & 0x01010101u) | ((d >> 2) & 0x02020202u) | ((d << 1) & 0x04040404u);
-            } else {
-                const int k = L - 4 - 4 * u;  // the four codons from k on, backwards; those below 0 are past the end
-                const int wi = k >> 2;
-                const uint32_t x0 = wi >= 0 ? w[wi] : 0u, x1 = wi >= -1 && wi + 1 < nwd ? w[wi + 1] : 0u;
-                const uint32_t d = __builtin_bswap32(__builtin_amdgcn_alignbit(x1, x0, 8 * (k & 3)));
-                const uint32_t keep = k >= 0 ? 0x07070707u : k <= -4 ? 0u : 0x07070707u & ((1u << (8 * (k + 4))) - 1u);
-                l = (~((d & 0x01010101u) | ((d >> 1) & 0x02020202u) | ((d >> 2) & 0x04040404u))) & keep;
-                h = (~(((d >> 1) & 0x01010101u) | ((d >> 2) & 0x02020202u) | ((d >> 3) & 0x04040404u))) & keep;
-            }
-            const uint32_t l12 = pack12(l), h12 = pack12(h);
-            const int b = 12 * t, q = b >> 5, o = b & 31;  // compile-time after unrolling
-            lo[q] |= l12 << o;
-            hi[q] |= h12 << o;
-            if (o > 20) {
-                lo[q + 1] |= l12 >> (32 - o);
-                hi[q + 1] |= h12 >> (32 - o);
-            }
+        for (int t = 0; t < 4; ++t) d[t] = w[min(q + t, nwd - 1)];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) d[t] = q + t < nwd ? d[t] : 0u;  // (the row's padding codes are 0)
+        uint32_t l[3], h[3];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const uint32_t c = __builtin_amdgcn_alignbyte(d[t + 1], d[t], k0 & 3u);
+            // per byte the three bases' low (high) bits in position order
+            l[t] = pack12(((c >> 4) & 0x01010101u) | ((c >> 1) & 0x02020202u) | ((c << 2) & 0x04040404u));
+            h[t] = pack12(((c >> 5) & 0x01010101u) | ((c >> 2) & 0x02020202u) | ((c << 1) & 0x04040404u));
         }
-        uint2 *const out = rev ? rp : sp;
-#pragma unroll
-        for (int v = 0; v < 3; ++v)
-            if (3 * g + v < W) gstore((uint64_t *)(out + 3 * g + v), (uint64_t)lo[v] | ((uint64_t)hi[v] << 32));
+        const uint32_t lo = __builtin_amdgcn_alignbit(l[2] >> 8, l[0] | (l[1] << 12) | (l[2] << 24), r);
+        const uint32_t hi = __builtin_amdgcn_alignbit(h[2] >> 8, h[0] | (h[1] << 12) | (h[2] << 24), r);
+        gstore((uint64_t *)(sp + i), (uint64_t)lo | ((uint64_t)hi << 32));
     }
-    uint32_t *const mk = (uint32_t *)(sp + 2 * W);
+    uint32_t *const mk = (uint32_t *)(sp + W);
     for (int i = lane; i < sk_mask_words(L); i += 64) gstore(mk + i, chg[i]);
 }
 
@@ -1494,10 +1527,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
     int buf, slot;
     item_slot(J, mode, it.y, buf, slot);
     CdsStat *cs = J.cst[buf] + (size_t)slot * m + c;
-    uint64_t *planes = (uint64_t *)dyn;  // the CDS's planes as k_design left them
-    const int nwords = 2 * scan_words(n);
-    const uint64_t *gp = (const uint64_t *)(J.planes + ((size_t)slot * m + c) * plane_words(L));
-    for (int i = threadIdx.x; i < nwords; i += NT) planes[i] = gload(gp + i);
+    uint64_t *planes = (uint64_t *)dyn;
+    const PlaneLoad<NT> load((const uint64_t *)(J.planes + ((size_t)slot * m + c) * plane_words(L)), L);
+    load.place(planes);
     const SeekLds S = seek_lds<HEADS>(dyn + stem_index_at(L), n, wid, nullptr);
     seek_clear<NT, HEADS>(S);
     lds_barrier();
@@ -1529,8 +1561,6 @@ __device__ __forceinline__ void stem_child(const DevJob &J, int child, int c, in
     if (buf < 0 && c >= m) return;
     const int n = 3 * L, slot = N + child, tid = (int)threadIdx.x;
     const size_t rec = (size_t)slot * m + c;
-    const int nwords = plane_words(L), pw = 2 * scan_words(n);
-    const uint64_t *gp = (const uint64_t *)(p_pl + rec * nwords);
     CdsStat *cs = (buf > 0 ? cs1 : cs0) + rec;
     const int32_t *r0 = (const int32_t *)cs;
     int pl = gload(r0 + 6), pp = gload(r0 + 7), pq = gload(r0 + 8), fresh = 1;  // CdsStat::l, p, q
@@ -1542,20 +1572,18 @@ __device__ __forceinline__ void stem_child(const DevJob &J, int child, int c, in
         fresh = gload(r0 + 9);  // CdsStat::pad
         l1 = gload(r1 + 6), p1 = gload(r1 + 7), q1 = gload(r1 + 8), f1 = gload(r1 + 9);
     }
-    const uint64_t v0 = gload(gp + min(tid, nwords - 1)), v1 = gload(gp + min(tid + NT, nwords - 1));
+    const PlaneLoad<NT> load((const uint64_t *)(p_pl + rec * plane_words(L)), L);
     if (buf < 0 && !(__builtin_amdgcn_readfirstlane(gen) & 1u)) {
         cs = cs1 + rec;
         pl = l1, pp = p1, pq = q1, fresh = f1;
     }
     if (__builtin_amdgcn_readfirstlane(fresh) == 0) return;
-    uint64_t *planes = (uint64_t *)dyn;  // the CDS's planes and change mask as k_design left them
+    uint64_t *planes = (uint64_t *)dyn;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const SeekLds S = seek_lds<HEADS>(dyn + stem_index_at(L), n, wid, (const uint32_t *)(planes + pw));
+    const SeekLds S = seek_lds<HEADS>(dyn + stem_index_at(L), n, wid, (const uint32_t *)(planes + 2 * scan_words(n)));
     if (buf >= 0) lds_barrier();  // the previous entry's LDS is no longer read
     seek_clear<NT, HEADS>(S);
-    if (tid < nwords) planes[tid] = v0;
-    if (tid + NT < nwords) planes[tid + NT] = v1;
-    for (int i = tid + 2 * NT; i < nwords; i += NT) planes[i] = gload(gp + i);
+    load.place(planes);
     lds_barrier();
     const uint2 *sp = (const uint2 *)planes;
     const uint64_t key = seek_cds<NT, HEADS>(S, sp, sp + scan_words(n), n, L, true, pl, pp, pq, redu, flag);

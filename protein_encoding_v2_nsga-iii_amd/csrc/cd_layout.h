@@ -148,7 +148,7 @@ struct DevJob {
     int32_t *pql[2];       // [P][4] (p, q, l, 0)
     CdsStat *cst[2];       // [P][m]
     int32_t *hdp[2];       // [P][m(m-1)/2] Hamming distances of the design's CDS pairs (i < j, lexicographic)
-    uint2 *planes;         // [P][m][2][scan_words(3L)] bit planes (sequence, reverse complement) of the CDS
+    uint2 *planes;         // [P][m] bit planes of the CDS's sequence (scan_words(3L) words), then its change mask,
                            // k_design evaluated, read by k_stem
     int32_t *front_of;     // [P]
     int32_t *np;           // [P] dominator counts
