@@ -266,28 +266,6 @@ int validate(const cd_job_desc *d) {
     return CD_OK;
 }
 
-// Pinned host staging for genome rows, which the device holds at a padded
-// stride Ls: reads copy the padded block in one transfer and drop the pads on
-// the host, writes add them on the host and copy in one transfer (a pitched
-// copy to or from pageable memory runs row by row).  Grown on demand and kept
-// for the life of the process; callers serialise on its lock.
-struct Staging {
-    std::mutex mu;
-    uint8_t *p = nullptr;
-    size_t cap = 0;
-    hipError_t reserve(size_t n) {  // with mu held
-        if (n <= cap) return hipSuccess;
-        if (p) (void)hipHostFree(p);
-        p = nullptr;
-        cap = 0;
-        const size_t c = std::max(n + n / 4, (size_t)1 << 20);
-        hipError_t e = hipHostMalloc((void **)&p, c, hipHostMallocDefault);
-        if (e == hipSuccess) cap = c;
-        return e;
-    }
-};
-Staging g_rows;
-
 // Memory a job frees stays in the device's stream-ordered pool for the next
 // job instead of going back to the system at each synchronisation (set once
 // per device).
@@ -305,6 +283,42 @@ hipError_t keep_pool_memory() {
     if (e == hipSuccess) e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
     if (e == hipSuccess) done[dev] = true;
     return e;
+}
+
+// Streams of jobs that have ended, for the next ones: creating and destroying
+// one costs about 50 us.  At most STREAMS_IDLE are kept, synchronised.
+constexpr size_t STREAMS_IDLE = 16;
+struct Streams {
+    std::mutex mu;
+    std::vector<std::pair<int, hipStream_t>> idle;  // (device, stream)
+    hipError_t take(int *dev, hipStream_t *s) {
+        const hipError_t e = hipGetDevice(dev);
+        if (e != hipSuccess) return e;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            for (size_t i = idle.size(); i-- > 0;)
+                if (idle[i].first == *dev) {
+                    *s = idle[i].second;
+                    idle.erase(idle.begin() + (ptrdiff_t)i);
+                    return hipSuccess;
+                }
+        }
+        return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+    }
+    void give(int dev, hipStream_t s) {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            if (idle.size() < STREAMS_IDLE) {
+                idle.push_back({dev, s});
+                return;
+            }
+        }
+        (void)hipStreamDestroy(s);
+    }
+};
+Streams &streams() {  // (never destroyed: the runtime may be gone by then)
+    static Streams *p = new Streams();
+    return *p;
 }
 
 // The sizes of a descriptor's job (J->N, H, L, m, R, P, W), its layout and its
@@ -445,7 +459,7 @@ int create_job(const cd_job_desc *d, cd_job **out) {
     // The allocation comes from the device's stream-ordered pool: freeing it
     // (cd_job_destroy) does not wait for every stream of the device, which
     // hipFree does, so jobs can come and go while others run.
-    hipError_t e = hipStreamCreateWithFlags(&J->stream, hipStreamNonBlocking);
+    hipError_t e = streams().take(&J->dev, &J->stream);
     if (e == hipSuccess) e = keep_pool_memory();
     if (e == hipSuccess) e = hipMallocAsync(&J->mem, o.total, J->stream);
     if (e != hipSuccess) {
@@ -473,7 +487,8 @@ int create_job(const cd_job_desc *d, cd_job **out) {
 }
 
 // A stream with a device and a pinned host buffer for the calls that hold
-// nothing from one to the next (cd_eval_batch, cd_nds, cd_select).  A call
+// nothing from one to the next (cd_eval_batch, cd_nds, cd_select; cd_job_read
+// takes the pinned buffer and the events).  A call
 // takes one for its duration -- an idle one of its device, else a new one -- so
 // calls of several threads run side by side; at most SHOTS_IDLE idle ones with
 // buffers of at most SHOT_KEEP bytes are kept, the others are freed with the
@@ -481,11 +496,12 @@ int create_job(const cd_job_desc *d, cd_job **out) {
 // of 16 designs takes 58 us instead of 271, a selection of 1024 from 2048 104
 // instead of 269; with the chunks below one of 2048 designs of 2004 codons 314
 // instead of 482.
-constexpr size_t EVAL_CHUNK = (size_t)1 << 20;  // bytes of packed rows
+constexpr size_t EVAL_CHUNK = (size_t)1 << 20, READ_CHUNK = (size_t)4 << 20;  // bytes of packed rows
 constexpr size_t SHOTS_IDLE = 4, SHOT_KEEP = (size_t)64 << 20;
 struct Shot {
     int dev = 0;
     hipStream_t stream = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
     char *mem = nullptr, *host = nullptr;
     size_t mem_cap = 0, host_cap = 0;
     hipError_t reserve(size_t mem_bytes, size_t host_bytes) {
@@ -513,6 +529,8 @@ struct Shot {
             (void)hipStreamDestroy(stream);
         }
         if (host) (void)hipHostFree(host);
+        for (hipEvent_t x : ev)
+            if (x) (void)hipEventDestroy(x);
     }
 };
 struct Shots {
@@ -531,6 +549,8 @@ struct Shots {
                 }
         }
         e = hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking);
+        for (hipEvent_t &x : s.ev)
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
         if (e == hipSuccess) e = keep_pool_memory();
         return e;
     }
@@ -674,20 +694,19 @@ int capture(hipStream_t s, hipGraph_t *g, hipGraphExec_t *ge, const Launch &w, i
     return CD_OK;
 }
 
-// Enqueue `generations` generations as graph launches: blocks of
-// GRAPH_BLOCK, then single generations (each graph captured on first use).
+// Enqueue `generations` generations: blocks of GRAPH_BLOCK as graph launches,
+// the others kernel by kernel.  The first GRAPH_AFTER generations of a graph's
+// life go kernel by kernel too, so that the device has work while the host
+// captures the graph, and short runs need none.
 int step_graphs(StepGraphs &G, hipStream_t s, const Launch &w, int generations) {
     int g = generations;
-    if (g >= GRAPH_BLOCK && !G.exec[1]) {
-        const int rc = capture(s, &G.graph[1], &G.exec[1], w, GRAPH_BLOCK);
+    for (; g > 0 && !G.exec && G.direct < GRAPH_AFTER; --g, ++G.direct) HIPCHK(enqueue_generation(w, s, nullptr));
+    if (g >= GRAPH_BLOCK && !G.exec) {
+        const int rc = capture(s, &G.graph, &G.exec, w, GRAPH_BLOCK);
         if (rc != CD_OK) return rc;
     }
-    for (; g >= GRAPH_BLOCK; g -= GRAPH_BLOCK) HIPCHK(hipGraphLaunch(G.exec[1], s));
-    if (g > 0 && !G.exec[0]) {
-        const int rc = capture(s, &G.graph[0], &G.exec[0], w, 1);
-        if (rc != CD_OK) return rc;
-    }
-    for (; g > 0; --g) HIPCHK(hipGraphLaunch(G.exec[0], s));
+    for (; g >= GRAPH_BLOCK; g -= GRAPH_BLOCK) HIPCHK(hipGraphLaunch(G.exec, s));
+    for (; g > 0; --g) HIPCHK(enqueue_generation(w, s, nullptr));
     return CD_OK;
 }
 
@@ -957,33 +976,49 @@ int cd_job_read(cd_job *J, int8_t *genome, float *obj, int8_t *idx, int32_t *pql
                 float *state) {
     if (!J || J->selection_only) return fail(CD_E_INVALID, "null job");
     if (!J->inited) return fail(CD_E_STATE, "cd_job_read before cd_job_init");
-    cd::SelState st;
-    HIPCHK(read_state(J, st));
-    const int b = (int)(st.gen & 1u), P = J->P;
-    const size_t rows = (size_t)P * J->m, L = J->L;
-    hipStream_t s = J->stream;
-    std::unique_lock<std::mutex> stage(g_rows.mu, std::defer_lock);
-    if (genome) {
-        // packed synonym indices, made on the device in the other buffer (the
-        // next generation writes every row of it), in one transfer
-        stage.lock();
-        HIPCHK(g_rows.reserve(rows * L));
-        HIPCHK(cd::launch_export(J->d_self, J->h.genome[b], J->h.genome[b ^ 1], (int)rows, (int)L, s));
-        HIPCHK(hipMemcpyAsync(g_rows.p, J->h.genome[b ^ 1], rows * L, hipMemcpyDeviceToHost, s));
+    const int P = J->P;
+    const cd::ReadRest at(P, J->W);
+    const size_t total = genome ? (size_t)P * J->m * J->L : 0, chunk = std::min(total, READ_CHUNK);
+    const size_t head = (at.bytes + 255) & ~(size_t)255, room = (chunk + 255) & ~(size_t)255;
+    Shot w;
+    hipError_t e = shots().take(w);
+    if (e == hipSuccess) e = w.reserve(0, head + 2 * room);
+    for (cd_batch *B : J->batches)
+        if (e == hipSuccess) e = hipStreamSynchronize(B->stream);
+    // a chunk is copied out while the next one is on its way
+    uint8_t *const half[2] = {(uint8_t *)w.host + head, (uint8_t *)w.host + head + room};
+    auto send = [&](size_t first, int k, bool rest) {
+        if (e == hipSuccess)
+            e = cd::launch_read(J->d_self, half[k], rest ? w.host : nullptr, at.bytes, first, std::min(chunk, total - first), J->stream);
+        if (e == hipSuccess) e = hipEventRecord(w.ev[k], J->stream);
+    };
+    send(0, 0, true);
+    for (size_t first = 0, k = 0; first < total; first += chunk, k ^= 1) {
+        if (first + chunk < total) send(first + chunk, (int)(k ^ 1), false);
+        if (e == hipSuccess) e = hipEventSynchronize(w.ev[k]);
+        if (e == hipSuccess) std::memcpy(genome + first, half[k], std::min(chunk, total - first));
     }
-    if (obj) HIPCHK(hipMemcpyAsync(obj, J->h.obj[b], (size_t)P * 6 * 4, hipMemcpyDeviceToHost, s));
-    if (idx) HIPCHK(hipMemcpyAsync(idx, J->h.oidx[b], (size_t)P * 12, hipMemcpyDeviceToHost, s));
-    std::vector<int32_t> t(pql ? (size_t)P * 4 : 0);
-    if (pql) HIPCHK(hipMemcpyAsync(t.data(), J->h.pql[b], t.size() * 4, hipMemcpyDeviceToHost, s));
-    std::vector<uint64_t> mask(sorted ? J->W : 0);
-    if (sorted) HIPCHK(hipMemcpyAsync(mask.data(), J->h.selm, (size_t)J->W * 8, hipMemcpyDeviceToHost, s));
-    if (front_of) HIPCHK(hipMemcpyAsync(front_of, J->h.front_of, (size_t)P * 4, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    if (genome) std::memcpy(genome, g_rows.p, rows * L);
-    if (sorted) survivors_of(mask, J->N, sorted);
-    if (pql)
-        for (int i = 0; i < P; ++i)
-            for (int k = 0; k < 3; ++k) pql[i * 3 + k] = t[(size_t)i * 4 + k];
+    const hipError_t es = hipStreamSynchronize(J->stream);
+    if (e == hipSuccess) e = es;
+    cd::SelState st;
+    if (e == hipSuccess) {
+        std::memcpy(&st, w.host, sizeof(st));
+        if (obj) std::memcpy(obj, w.host + at.obj, (size_t)P * 24);
+        if (idx) std::memcpy(idx, w.host + at.idx, (size_t)P * 12);
+        if (front_of) std::memcpy(front_of, w.host + at.front, (size_t)P * 4);
+        if (sorted) {
+            std::vector<uint64_t> mask(J->W);
+            std::memcpy(mask.data(), w.host + at.selm, (size_t)J->W * 8);
+            survivors_of(mask, J->N, sorted);
+        }
+        const int32_t *q = (const int32_t *)(w.host + at.pql);
+        if (pql)
+            for (int i = 0; i < P; ++i)
+                for (int k = 0; k < 3; ++k) pql[i * 3 + k] = q[(size_t)i * 4 + k];
+    }
+    shots().give(w, e == hipSuccess);
+    HIPCHK(e);
+    const int b = (int)(st.gen & 1u);
     if (state) {
         const cd::SelRes &r = st.res[b];
         std::memcpy(state, r.ext, sizeof(r.ext));
@@ -1015,10 +1050,7 @@ int cd_job_destroy(cd_job *J) {
     if (J->stream) (void)hipStreamSynchronize(J->stream);
     J->graphs.reset();
     if (J->mem) (void)hipFreeAsync(J->mem, J->stream);  // back to the pool, after the job's last work
-    if (J->stream) {
-        (void)hipStreamSynchronize(J->stream);
-        (void)hipStreamDestroy(J->stream);
-    }
+    if (J->stream) streams().give(J->dev, J->stream);
     delete J;
     return CD_OK;
 }

@@ -14,21 +14,24 @@
 struct cd_batch;
 
 // One job: tables, pools and selection state in one device allocation.
-// The captured generation graphs of a job or batch: [0] one generation,
-// [1] GRAPH_BLOCK generations back to back.  A long step launches the block
-// graph (consecutive graph launches leave several microseconds between
-// them; the kernels inside one graph follow each other closely).
+// The captured graph of a job or batch: GRAPH_BLOCK generations back to back
+// (consecutive graph launches leave several microseconds between them; the
+// kernels inside one graph follow each other closely).  Before it is captured
+// GRAPH_AFTER generations are enqueued kernel by kernel, 17 us of host time
+// each: less than a generation takes, so the device stays busy during the
+// capture (120 to 250 us).
 constexpr int GRAPH_BLOCK = 8;
+constexpr int GRAPH_AFTER = 16;
 struct StepGraphs {
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    hipGraphExec_t exec[2] = {nullptr, nullptr};
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    int direct = 0;  // generations enqueued before the capture
     void reset() {
-        for (int k = 0; k < 2; ++k) {
-            if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
-            if (graph[k]) (void)hipGraphDestroy(graph[k]);
-            exec[k] = nullptr;
-            graph[k] = nullptr;
-        }
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (graph) (void)hipGraphDestroy(graph);
+        exec = nullptr;
+        graph = nullptr;
+        direct = 0;
     }
 };
 
@@ -42,6 +45,7 @@ struct cd_job {
     int L = 0, m = 0, N = 0, H = 0, R = 0, P = 0, W = 0;
     void *mem = nullptr;
     size_t mem_bytes = 0;
+    int dev = 0;  // the stream's device
     hipStream_t stream = nullptr;
     int2 *d_off = nullptr;
     int4 *d_dom = nullptr;        // domination tiles: the 64 x 64 blocks (b, w), b <= w

@@ -103,9 +103,17 @@ hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n,
                          uint2 *stem_list = nullptr, int32_t *stem_ctl = nullptr, StemList sl = StemList{0, 0, 0},
                          int item_base = 0, int threads = 256);
 // (MODE_INIT: item_base 1 when the pool has not been written before)
-// the packed synonym indices of a pool's rows [rows][L] from its code rows
-// (stride row_stride(L)), to dst (room for rows * row_stride(L) bytes)
-hipError_t launch_export(const DevJob *job, const int8_t *src, int8_t *dst, int rows, int L, hipStream_t s);
+// what a caller reads of a job to pinned host memory: the bytes [first, first +
+// bytes) of the pool's packed synonym indices to rows (first a multiple of 16;
+// room for whole 16-byte words), and, unless rest is null, the arrays of
+// ReadRest one after the other
+struct ReadRest {
+    size_t selm, front, obj, idx, pql, bytes;  // offsets; the selection state comes first
+    ReadRest(int P, int W)
+        : selm(sizeof(SelState)), front(selm + 8 * (size_t)W), obj(front + 4 * (size_t)P), idx(obj + 24 * (size_t)P),
+          pql(idx + 12 * (size_t)P), bytes(pql + 16 * (size_t)P) {}
+};
+hipError_t launch_read(const DevJob *job, uint8_t *rows, void *rest, size_t rest_bytes, size_t first, size_t bytes, hipStream_t s);
 // initialisation and evaluation: a workgroup per (item, CDS c < mg): stem of
 // each CDS of the items' designs
 hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s);

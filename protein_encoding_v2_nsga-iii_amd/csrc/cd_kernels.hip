@@ -1462,35 +1462,58 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
     }
 }
 
-// Codon codes of `rows` pool rows (stride Ls) to synonym indices, rows packed
-// at L bytes: what a caller reads.  A thread converts 16 consecutive output
-// bytes; a code no row holds yet (0 in an unwritten row is not one: see INIT)
-// does not occur.
-__global__ __launch_bounds__(256) void k_export(const DevJob *__restrict__ jobs, const uint8_t *__restrict__ src,
-                                                uint8_t *__restrict__ dst, int rows) {
+// What a caller reads of a job, written straight to the host's pinned memory:
+// the first gblocks workgroups convert `bytes` bytes from byte `first` on (both
+// multiples of 16, or the last) of the pool's packed synonym indices, 16 a
+// thread, to `rows`; the others copy the selection state, survivor mask,
+// fronts, objectives, their indices and stem positions, word by word, to
+// `rest` (ReadRest).  The buffer comes from the generation counter
+// here, so nothing is read back before.  Bound by the link: 200 x 2 CDS of
+// 351 codons with their records in one launch and one wait, 60 us a call;
+// a copy for each array and one for the counter, 186 us.
+__global__ __launch_bounds__(256) void k_read(const DevJob *__restrict__ jobs, uint8_t *__restrict__ rows, uint32_t *__restrict__ rest,
+                                              uint64_t first, uint64_t bytes, uint32_t gblocks) {
     __shared__ uint8_t own[64];
     const DevJob &J = jobs[0];
+    const int b = (int)(gload(&J.st->gen) & 1u);
+    if (blockIdx.x >= gblocks) {
+        const uint32_t P = (uint32_t)J.P, t = (blockIdx.x - gblocks) * 256 + threadIdx.x;
+        const uint32_t ends[6] = {(uint32_t)(sizeof(SelState) / 4), 2u * (uint32_t)J.W, P, 6 * P, 3 * P, 4 * P};
+        const uint32_t *from[6] = {(const uint32_t *)J.st, (const uint32_t *)J.selm, (const uint32_t *)J.front_of,
+                                   (const uint32_t *)(b ? J.obj[1] : J.obj[0]), (const uint32_t *)(b ? J.oidx[1] : J.oidx[0]),
+                                   (const uint32_t *)(b ? J.pql[1] : J.pql[0])};
+        uint32_t at = t;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            if (at < ends[k]) {
+                gstore(rest + t, gload(from[k] + at));
+                return;
+            }
+            at -= ends[k];
+        }
+        return;
+    }
     const uint32_t L = (uint32_t)J.L, Ls = (uint32_t)J.Ls;
+    const uint8_t *const src = (const uint8_t *)(b ? J.genome[1] : J.genome[0]);
     const uint64_t *syn = (const uint64_t *)(J.lw6 + 64);
     if (threadIdx.x < 64) own[threadIdx.x] = (uint8_t)SynWord(gload(syn + threadIdx.x)).own();
     __syncthreads();
-    const uint64_t total = (uint64_t)rows * L;
-    const uint64_t o0 = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 16;
-    if (o0 >= total) return;
-    uint64_t r = o0 / L;
-    uint32_t k = (uint32_t)(o0 - r * L);
+    const uint64_t at = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 16;
+    if (at >= bytes) return;
+    uint64_t r = (first + at) / L;
+    uint32_t k = (uint32_t)(first + at - r * L);
     const uint8_t *p = src + r * Ls + k;
     u32x4 v = {0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        if (o0 + i < total) v[i >> 2] |= (uint32_t)own[gload(p) & 63] << (8 * (i & 3));
+        if (at + i < bytes) v[i >> 2] |= (uint32_t)own[gload(p) & 63] << (8 * (i & 3));
         ++p;
         if (++k == L) {
             k = 0;
             p += Ls - L;
         }
     }
-    gstore((u32x4 *)(dst + o0), v);  // (the buffer holds at least 15 bytes past the packed rows, or they fill it)
+    gstore((u32x4 *)(rows + at), v);  // (room for whole 16-byte words)
 }
 
 // Buffer and slot of the design an evaluation work item refers to: children
@@ -3105,10 +3128,10 @@ hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n,
     }
     return hipGetLastError();
 }
-hipError_t launch_export(const DevJob *job, const int8_t *src, int8_t *dst, int rows, int L, hipStream_t s) {
-    const size_t n = ((size_t)rows * L + 4095) / 4096;
+hipError_t launch_read(const DevJob *job, uint8_t *rows, void *rest, size_t rest_bytes, size_t first, size_t bytes, hipStream_t s) {
+    const size_t g = (bytes + 4095) / 4096, n = g + (rest ? (rest_bytes + 1023) / 1024 : 0);
     if (!n) return hipSuccess;
-    hipLaunchKernelGGL(k_export, dim3((unsigned)n), dim3(256), 0, s, job, (const uint8_t *)src, (uint8_t *)dst, rows);
+    hipLaunchKernelGGL(k_read, dim3((unsigned)n), dim3(256), 0, s, job, rows, (uint32_t *)rest, (uint64_t)first, (uint64_t)bytes, (uint32_t)g);
     return hipGetLastError();
 }
 hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s) {
