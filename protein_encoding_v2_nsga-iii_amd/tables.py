@@ -4,6 +4,7 @@ The genome encoding is the reference's (m CDS copies of one protein, each
 codon a synonym of its amino acid) stored as int8 synonym indices instead of
 ASCII nucleotides (include/utils.cuh:1072-1077, include/info.cuh:9-31).
 """
+import functools
 import json
 import os
 from dataclasses import dataclass
@@ -48,9 +49,16 @@ class Tables:
         return self.codons.encode("ascii")
 
 
+@functools.lru_cache(maxsize=None)
+def _reference_data() -> dict:
+    """The data file beside this module, parsed once (2 ms)."""
+    with open(_DATA) as f:
+        return json.load(f)
+
+
 def reference_tables() -> Tables:
     """The reference's own table (include/info.cuh:7-54)."""
-    d = json.load(open(_DATA))
+    d = _reference_data()
     return Tables(d["codons"], np.asarray(d["weights"], np.float32), np.asarray(d["cps"], np.float32),
                   float(np.float32(d["gc3_ref"])))
 
