@@ -126,6 +126,15 @@ hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg
                             const int32_t *stem_ctl, StemList sl, int waves, size_t lds, hipStream_t s);
 // one thread per item: objective 5, clears the marks
 hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s);
+// a sort of P objective vectors obj [P][6] (device memory) until at least N are
+// ranked: front_of [P], *n_fronts; scratch: dom [W][P], any [W][W], W = (P + 63) / 64
+struct SortArgs {
+    const float *obj;
+    int32_t *front_of, *n_fronts;
+    uint64_t *dom, *any;
+    int P, N, W;
+};
+hipError_t launch_sort(const SortArgs &a, hipStream_t s);
 // items: (job, 64b, w, 0), the 64 x 64 tiles b <= w, rows / 64 (rows: 64, 128 or 256) per workgroup.  finish: the offspring generation, whose children's stem
 // objective (and stem records) k_dominance completes in place of
 // launch_stem_finish; stem_ctl (or null): the ctl_n changed-CDS counts of
