@@ -240,8 +240,8 @@ void work_counts(int P, int W, int *n_dom, int *n_asc) {
 // given shapes.  The tiles are the 64 x 64 blocks (row block b, column block
 // w) with b <= w; k_dominance takes dom_rows / 64 of them per workgroup.
 void job_lists(int P, int W, const cd::Shapes &sh, std::vector<int4> &dom, std::vector<int2> &asc, int j = 0) {
-    for (int b = 0; b < W; ++b)
-        for (int w = b; w < W; ++w) dom.push_back(make_int4(j, 64 * b, w, 0));
+    for (int w = 0; w < W; ++w)
+        for (int b = 0; b <= w; ++b) dom.push_back(make_int4(j, 64 * b, w, 0));
     for (int t = 0; t < (P + sh.assoc_designs - 1) / sh.assoc_designs; ++t)
         asc.push_back(make_int2(j, t * sh.assoc_designs));
 }
