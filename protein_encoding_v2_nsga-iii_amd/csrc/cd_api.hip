@@ -858,13 +858,21 @@ cd::Shapes untuned_shapes(cd_job *const *jobs, int count) {
     // any more (a second launch's tail against a few more resident workgroups):
     // ticks of 24 / 48 / 64 jobs 454 / 797 / 1004 us in one launch, 478 / 790 /
     // 971 split at 8500 bytes, the other way round for other mixes.
-    int64_t children = 0, codons = 0;
+    int64_t children = 0, codons = 0, tiles = 0;
     for (int j = 0; j < count; ++j) {
+        tiles += (int64_t)jobs[j]->W * (jobs[j]->W + 1) / 2;
         children += jobs[j]->N;
         codons += (int64_t)jobs[j]->N * jobs[j]->L * jobs[j]->m;
     }
     sh.design_split = 0;
     sh.design_threads = children <= 640 + codons / children / 16 ? 512 : 256;
+    // Domination tiles a workgroup: one while a tile's latency counts, four when
+    // the chip is full of them.  Microseconds a generation with 64 / 128 / 256
+    // rows: batches of 72 tiles 39.1 / 40.2 / 42.2, 544 56.8 / 57.4 / 59.0, 1056
+    // 64.8 / 65.4 / 64.7, 3168 104 / 103 / 102, 6336 178 / 174 / 173, the 64-job
+    // mix (17 700) 817 / 808 / 802; lone jobs of 1176 tiles 63.6 / 66 / 64, 4186
+    // 87.1 / 88.3 / 88.1, 8256 225 / 222 / 220.5.
+    sh.dom_rows = tiles <= (count > 1 ? 1024 : 6000) ? 64 : 256;
     sh.assoc_designs = pool <= 512 ? 4 : pool <= cd::FUSED_TOTAL ? 8 : pool <= 12000 ? 16 : 64;
     return sh;
 }
