@@ -156,8 +156,8 @@ enum class Use { Job, Evaluate, Select };
 
 // Lay out every device buffer of a job in one allocation.  The regions the
 // host fills come first, `head` bytes in all, and go up in one transfer; what
-// a single evaluation (obj, oidx, pql) or selection (st, selm, front) gives
-// back lies together and comes down in one.
+// a single selection gives back (st, selm, front) lies together and comes down
+// in one.
 struct Layout {
     size_t pos, code, lw6, cpfx6, cps6, ref, genome[2], obj[2], oidx[2], pql[2], cst[2], hdp[2], planes, stem_max, slist,
         sctl,
@@ -193,11 +193,12 @@ Layout layout(int L, int m, int N, int P, int R, int W, int n_dom, int n_asc, Us
     } else {
         o.head = s.total;
         for (int b = 0; b < (use == Use::Job ? 2 : 1); ++b) {
-            o.obj[b] = s.add((size_t)P * 6 * 4);
-            o.oidx[b] = s.add((size_t)P * 12);
-            o.pql[b] = s.add((size_t)P * 16);
-            // (an evaluation reads packed rows, in whole words)
-            o.genome[b] = s.add(use == Use::Job ? (size_t)P * m * cd::row_stride(L) : (size_t)P * m * L + 8);
+            if (use == Use::Job) {  // (an evaluation's rows and results are in pinned memory)
+                o.obj[b] = s.add((size_t)P * 6 * 4);
+                o.oidx[b] = s.add((size_t)P * 12);
+                o.pql[b] = s.add((size_t)P * 16);
+                o.genome[b] = s.add((size_t)P * m * cd::row_stride(L));
+            }
             o.cst[b] = s.add((size_t)P * m * sizeof(cd::CdsStat));
             o.hdp[b] = s.add((size_t)P * (m * (m - 1) / 2) * 4);
         }
@@ -492,10 +493,9 @@ int create_job(const cd_job_desc *d, cd_job **out) {
 // takes one for its duration -- an idle one of its device, else a new one -- so
 // calls of several threads run side by side; at most SHOTS_IDLE idle ones with
 // buffers of at most SHOT_KEEP bytes are kept, the others are freed with the
-// call.  With them, one transfer each way and one synchronisation an evaluation
-// of 16 designs takes 58 us instead of 271, a selection of 1024 from 2048 104
-// instead of 269; with the chunks below one of 2048 designs of 2004 codons 314
-// instead of 482.
+// call.  With them, one launch that fetches the set-up and one synchronisation
+// an evaluation of 16 designs takes 49 us instead of 271, a selection of 1024
+// from 2048 90 instead of 269.
 constexpr size_t EVAL_CHUNK = (size_t)1 << 20, READ_CHUNK = (size_t)4 << 20;  // bytes of packed rows
 constexpr size_t SHOTS_IDLE = 4, SHOT_KEEP = (size_t)64 << 20;
 struct Shot {
@@ -1079,38 +1079,45 @@ int cd_eval_batch(const cd_job_desc *desc, const int8_t *genome, int32_t count, 
     rc = size_job(J, &d, Use::Evaluate, count, o, t);
     if (rc != CD_OK) return rc;
     const size_t row = (size_t)J->m * J->L, bytes = row * count;
-    const size_t out_bytes = o.genome[0] - o.obj[0];
+    // pinned: the image, the packed rows (a word past them is read), the results
+    const size_t r_obj = o.head + a256(bytes + 8), r_idx = r_obj + a256((size_t)count * 24), r_pql = r_idx + a256((size_t)count * 12);
     Shot w;
     hipError_t e = shots().take(w);
-    if (e == hipSuccess) e = w.reserve(o.total, o.head + bytes + 16 + out_bytes);
+    if (e == hipSuccess) e = w.reserve(o.total, r_pql + (size_t)count * 16);
     if (e != hipSuccess) {
         shots().give(w, false);
         return fail(CD_E_NOMEM, std::string("eval buffers: ") + hipGetErrorString(e));
     }
-    char *const stage = w.host + o.head, *const res = stage + ((bytes + 15) & ~(size_t)15);
     std::memset(w.host, 0, o.head);
     describe_job(J, &d, Use::Evaluate, o, t, w.mem, w.host);
+    J->h.genome[0] = (int8_t *)w.host + o.head;
+    J->h.obj[0] = (float *)(w.host + r_obj);
+    J->h.oidx[0] = (int8_t *)w.host + r_idx;
+    J->h.pql[0] = (int32_t *)(w.host + r_pql);
+    std::memcpy(w.host + o.self, &J->h, sizeof(J->h));
     e = job_lds_limits(J, false);
-    if (e == hipSuccess) e = hipMemcpyAsync(w.mem, w.host, o.head, hipMemcpyHostToDevice, w.stream);
-    // The rows go up packed as the caller holds them (k_design addresses them
-    // bytewise), EVAL_CHUNK bytes at a time, so that the copy into pinned
-    // memory, the transfer and the kernels of successive chunks overlap.
+    if (e == hipSuccess) e = cd::launch_fetch(w.mem, w.host, o.head, w.stream);
+    // The rows are copied into pinned memory packed as the caller holds them,
+    // EVAL_CHUNK bytes at a time, and k_design reads them from there bytewise,
+    // each once: the copies overlap the kernel of the chunk before.  The stems
+    // follow in one launch, and the kernels store the results to pinned memory
+    // too.  2048 designs of 2004 codons, 4 MB: 206 us; with transfers by the
+    // copy engine 304, with the stems chunk by chunk 232, with chunks of half the
+    // size 238.
     const int per = std::max(1, (int)std::min<size_t>(EVAL_CHUNK / row, (size_t)count));
     for (int i = 0; i < count && e == hipSuccess; i += per) {
         const int n = std::min(per, count - i);
-        std::memcpy(stage + i * row, genome + i * row, n * row);
-        e = hipMemcpyAsync(w.mem + o.genome[0] + i * row, stage + i * row, n * row, hipMemcpyHostToDevice, w.stream);
-        if (e == hipSuccess) e = cd::launch_design(cd::MODE_EVAL, J->d_self, J->d_off + i, n, J->lds, w.stream);
-        if (e == hipSuccess) e = cd::launch_stem(cd::MODE_EVAL, J->d_self, J->d_off + i, n, J->m, J->stem_lds, w.stream);
+        std::memcpy(w.host + o.head + i * row, genome + i * row, n * row);
+        e = cd::launch_design(cd::MODE_EVAL, J->d_self, J->d_off + i, n, J->lds, w.stream);
     }
+    if (e == hipSuccess) e = cd::launch_stem(cd::MODE_EVAL, J->d_self, J->d_off, count, J->m, J->stem_lds, w.stream);
     if (e == hipSuccess) e = cd::launch_stem_finish(cd::MODE_EVAL, J->d_self, J->d_off, count, w.stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(res, w.mem + o.obj[0], out_bytes, hipMemcpyDeviceToHost, w.stream);
     const hipError_t es = hipStreamSynchronize(w.stream);
     if (e == hipSuccess) e = es;
     if (e == hipSuccess) {
-        if (obj) std::memcpy(obj, res, (size_t)count * 24);
-        if (idx) std::memcpy(idx, res + (o.oidx[0] - o.obj[0]), (size_t)count * 12);
-        const int32_t *q = (const int32_t *)(res + (o.pql[0] - o.obj[0]));
+        if (obj) std::memcpy(obj, w.host + r_obj, (size_t)count * 24);
+        if (idx) std::memcpy(idx, w.host + r_idx, (size_t)count * 12);
+        const int32_t *q = (const int32_t *)(w.host + r_pql);
         if (pql)
             for (int i = 0; i < count; ++i)
                 for (int k = 0; k < 3; ++k) pql[i * 3 + k] = q[(size_t)i * 4 + k];
@@ -1152,7 +1159,7 @@ static int run_selection(const float *obj, int32_t P, int32_t N, int32_t H, uint
     if (extremes) std::memcpy(s0->res[gen & 1u].ext, extremes, sizeof(s0->res[0].ext));
     e = job_lds_limits(J, true);
     if (e == hipSuccess) e = hipMemsetAsync(w.mem + o.head, 0, o.total - o.head, w.stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(w.mem, w.host, o.head, hipMemcpyHostToDevice, w.stream);
+    if (e == hipSuccess) e = cd::launch_fetch(w.mem, w.host, o.head, w.stream);
     if (e == hipSuccess) e = cd::launch_zero_np(J->d_self, 1, w.stream);
     const cd::Shapes &sh = J->shapes;
     if (e == hipSuccess) e = cd::launch_dominance(J->d_self, J->d_dom, J->n_dom, false, nullptr, 0, sh.dom_rows, w.stream);

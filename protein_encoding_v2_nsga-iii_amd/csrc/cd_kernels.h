@@ -103,6 +103,9 @@ hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n,
                          uint2 *stem_list = nullptr, int32_t *stem_ctl = nullptr, StemList sl = StemList{0, 0, 0},
                          int item_base = 0, int threads = 256);
 // (MODE_INIT: item_base 1 when the pool has not been written before)
+// bytes (rounded up to 16) from pinned host memory to the device, both 16-byte
+// aligned
+hipError_t launch_fetch(void *dst, const void *src, size_t bytes, hipStream_t s);
 // what a caller reads of a job to pinned host memory: the bytes [first, first +
 // bytes) of the pool's packed synonym indices to rows (first a multiple of 16;
 // room for whole 16-byte words), and, unless rest is null, the arrays of

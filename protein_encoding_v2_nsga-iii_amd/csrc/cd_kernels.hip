@@ -1318,7 +1318,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
         // synonym indices to codes, four a word; the padding positions are
         // forced to code 0
         const uint8_t *const pos = J.pos, *const ctab = J.code;
-        const uint32_t *sg = (const uint32_t *)genome0;  // rows of L bytes, packed; the buffer has a word past them
+        const uint32_t *sg = (const uint32_t *)genome0;  // rows of L bytes, packed, in the caller's pinned memory; it has a word past them
         const int nwd = Ls >> 2;
         uint32_t *c4 = (uint32_t *)rows;
         for (int c = 0; c < m; ++c)
@@ -1326,7 +1326,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
                 const int left = L - 4 * q;  // positions of the word below L
                 const uint32_t keep = left >= 4 ? ~0u : (left <= 0 ? 0u : (1u << (8 * left)) - 1u);
                 const size_t at = ((size_t)it.y * m + c) * L + (left > 0 ? 4 * q : 0);
-                const uint32_t s0 = gload(sg + (at >> 2)), s1 = gload(sg + (at >> 2) + 1);
+                // (the next word is the next lane's; only the wave's and the
+                // row's last lane read it: the rows come over the link)
+                const uint32_t s0 = gload(sg + (at >> 2));
+                uint32_t s1 = __shfl_down(s0, 1, 64);
+                if (lane == 63 || left <= 4) s1 = gload(sg + (at >> 2) + 1);
                 const uint32_t sw = __builtin_amdgcn_alignbyte(s1, s0, (uint32_t)at & 3u);
                 const uint32_t g = (sw & keep) + gload((const uint32_t *)pos + q);  // bytewise
                 uint32_t code = 0;
@@ -1460,6 +1464,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
                        stem_entry((uint32_t)it.x, (uint32_t)it.y, (uint32_t)lane, (uint32_t)dst));
         }
     }
+}
+
+// `words` 16-byte words from the host's pinned memory to the device: what a call
+// sets up, some 60 KB, where the copy engine's hand-over to the first kernel
+// takes longer than the transfer.
+__global__ __launch_bounds__(256) void k_fetch(u32x4 *__restrict__ dst, const u32x4 *__restrict__ src, uint32_t words) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < words) gstore(dst + i, gload(src + i));
 }
 
 // What a caller reads of a job, written straight to the host's pinned memory:
@@ -3216,6 +3228,12 @@ hipError_t launch_design(int mode, const DevJob *jobs, const int2 *items, int n,
             return hipErrorInvalidValue;
         break;
     }
+    return hipGetLastError();
+}
+hipError_t launch_fetch(void *dst, const void *src, size_t bytes, hipStream_t s) {
+    const uint32_t words = (uint32_t)((bytes + 15) / 16);
+    if (!words) return hipSuccess;
+    hipLaunchKernelGGL(k_fetch, dim3((words + 255) / 256), dim3(256), 0, s, (u32x4 *)dst, (const u32x4 *)src, words);
     return hipGetLastError();
 }
 hipError_t launch_read(const DevJob *job, uint8_t *rows, void *rest, size_t rest_bytes, size_t first, size_t bytes, hipStream_t s) {
