@@ -174,7 +174,7 @@ int cd_batch_destroy(cd_batch *batch);
 typedef struct cd_shapes {
     int32_t design_split;   /* k_design LDS bytes up to which children launch apart (0: one launch) */
     int32_t design_threads; /* k_design workgroup size of the other children (a lone job: all): 256 or 512 */
-    int32_t stem_waves;     /* k_stem_list workgroups per CU: 5 to 8 */
+    int32_t stem_waves;     /* k_stem_list waves per SIMD at most: 5 to 8 */
     int32_t dom_rows;       /* k_dominance tile rows per workgroup (64 x 64 tiles): 64, 128 or 256 */
     int32_t fronts_threads; /* k_fronts workgroup size: 256, 512 or 1024 */
     int32_t assoc_designs;  /* k_associate designs per workgroup: 4, 8 or 16 (a wave each), 32 or 64 (8 lanes each) */

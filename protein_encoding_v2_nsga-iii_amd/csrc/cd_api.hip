@@ -491,12 +491,13 @@ int create_job(const cd_job_desc *d, cd_job **out) {
 // nothing from one to the next (cd_eval_batch, cd_nds, cd_select; cd_job_read
 // takes the pinned buffer and the events).  A call
 // takes one for its duration -- an idle one of its device, else a new one -- so
-// calls of several threads run side by side; at most SHOTS_IDLE idle ones with
-// buffers of at most SHOT_KEEP bytes are kept, the others are freed with the
+// calls of several threads run side by side; at most SHOTS_IDLE idle ones and
+// buffers of at most SHOT_KEEP bytes are kept, the rest is freed with the
 // call.  With them, one launch that fetches the set-up and one synchronisation
 // an evaluation of 16 designs takes 49 us instead of 271, a selection of 1024
 // from 2048 90 instead of 269.
-constexpr size_t EVAL_CHUNK = (size_t)1 << 20, READ_CHUNK = (size_t)4 << 20;  // bytes of packed rows
+constexpr size_t EVAL_CHUNK = (size_t)1 << 20, READ_CHUNK = (size_t)4 << 20,  // bytes of packed rows
+                 EVAL_WINDOW = (size_t)32 << 20;
 constexpr size_t SHOTS_IDLE = 4, SHOT_KEEP = (size_t)64 << 20;
 struct Shot {
     int dev = 0;
@@ -556,7 +557,17 @@ struct Shots {
     }
     // ok: the call's work has ended without an error
     void give(Shot &s, bool ok) {
-        if (ok && s.mem_cap <= SHOT_KEEP && s.host_cap <= SHOT_KEEP) {
+        if (ok) {
+            if (s.mem_cap > SHOT_KEEP) {
+                (void)hipFreeAsync(s.mem, s.stream);
+                s.mem = nullptr;
+                s.mem_cap = 0;
+            }
+            if (s.host_cap > SHOT_KEEP) {
+                (void)hipHostFree(s.host);
+                s.host = nullptr;
+                s.host_cap = 0;
+            }
             std::lock_guard<std::mutex> lk(mu);
             if (idle.size() < SHOTS_IDLE) {
                 idle.push_back(s);
@@ -1063,20 +1074,13 @@ int cd_job_destroy(cd_job *J) {
     return CD_OK;
 }
 
-int cd_eval_batch(const cd_job_desc *desc, const int8_t *genome, int32_t count, float *obj, int8_t *idx,
-                  int32_t *pql) {
-    if (!desc || !genome || count <= 0) return fail(CD_E_INVALID, "bad eval arguments");
-    cd_job_desc d = *desc;
-    d.N = (int32_t)(((int64_t)count + 1) / 2);
-    d.H = 1;
-    d.Pm = 0.f;
-    int rc = validate(&d);
-    if (rc != CD_OK) return rc;
+// One evaluation of `count` designs with a validated description.
+static int evaluate(const cd_job_desc &d, const int8_t *genome, int32_t count, float *obj, int8_t *idx, int32_t *pql) {
     cd_job job;
     cd_job *J = &job;
     Layout o;
     HostTables t;
-    rc = size_job(J, &d, Use::Evaluate, count, o, t);
+    const int rc = size_job(J, &d, Use::Evaluate, count, o, t);
     if (rc != CD_OK) return rc;
     const size_t row = (size_t)J->m * J->L, bytes = row * count;
     // pinned: the image, the packed rows (a word past them is read), the results
@@ -1125,6 +1129,24 @@ int cd_eval_batch(const cd_job_desc *desc, const int8_t *genome, int32_t count, 
     shots().give(w, e == hipSuccess);
     if (e != hipSuccess) return fail(CD_E_DEVICE, std::string("eval: ") + hipGetErrorString(e));
     return CD_OK;
+}
+
+int cd_eval_batch(const cd_job_desc *desc, const int8_t *genome, int32_t count, float *obj, int8_t *idx,
+                  int32_t *pql) {
+    if (!desc || !genome || count <= 0) return fail(CD_E_INVALID, "bad eval arguments");
+    cd_job_desc d = *desc;
+    d.N = (int32_t)(((int64_t)count + 1) / 2);
+    d.H = 1;
+    d.Pm = 0.f;
+    int rc = validate(&d);
+    // EVAL_WINDOW bytes of rows at a time, so that the pinned buffer is one
+    // that is kept
+    const size_t row = rc == CD_OK ? (size_t)d.m * d.L : 1;
+    const int per = std::max(1, (int)std::min<size_t>(EVAL_WINDOW / row, (size_t)count));
+    for (int i = 0; i < count && rc == CD_OK; i += per)
+        rc = evaluate(d, genome + i * row, std::min(per, count - i), obj ? obj + (size_t)i * 6 : nullptr,
+                      idx ? idx + (size_t)i * 12 : nullptr, pql ? pql + (size_t)i * 3 : nullptr);
+    return rc;
 }
 
 // One selection (full) or sort of P objective vectors.  On success *st, mask

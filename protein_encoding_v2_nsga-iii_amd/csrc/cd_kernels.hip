@@ -4,8 +4,8 @@
 //   k_design<OFFSPRING>  one workgroup per child: parent from the survivor
 //                        mask, survivor copy, mutation, objectives 0-4
 //                        (mutationKernel, main.cu:121-240)
-//   k_stem_list          longest stem of each CDS the mutation changed
-//                        (calMaximumSL)
+//   k_stem_each          longest stem of each CDS the mutation changed
+//   (k_stem_list)        (calMaximumSL), for small (large) launches
 //   k_dominance          objective 5 of the children, bit-packed
 //                        eps-domination matrix (sorting.cuh:994-1023), the
 //                        pool's ideal and worst points

@@ -19,6 +19,9 @@
 // number of hits per lookup is about (n / st) / 4096 for sequences without
 // long repeats.  A lookup loop stops at a hit budget, and the caller then
 // scans the tiles instead (a periodic sequence can match itself everywhere).
+//
+// The kernels search by cd_seek.h's words, which measure and pack their matches
+// with qg_measure and qg_pack; the q-gram search's host harness keeps the rest.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -54,3 +54,18 @@ def test_threads(cdp, orc):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_windows(cdp):
+    """More rows than one window: the designs on each side of its end."""
+    print("windows", flush=True)
+    T = cdp.tables
+    L, m, count = 1001, 16, 2200
+    aa, tab = T.synth_protein(L - 1, 9), T.synth_tables(9)
+    pop = T.random_population(aa, m, count, 9)
+    got = cdp.evaluate(aa, tab, pop)
+    per = (32 << 20) // (m * L)
+    assert 0 < per < count
+    for a, b in ((0, 3), (per - 3, per + 3), (count - 3, count)):
+        for x, y in zip(got, cdp.evaluate(aa, tab, pop[a:b])):
+            assert np.array_equal(x[a:b], y)
