@@ -51,16 +51,16 @@ HBM_BYTES_S = 8.0e12            # MI355X HBM3E peak
 VALU_WAVE_INSTR_S = 256 * 2.4e9  # 256 CUs x 4 SIMDs x one wave64 VALU instruction per 4 cycles, 2.4 GHz
 KERNELS = ("offspring", "stem", "dominance", "fronts", "associate", "niche")
 SECTIONS = ("headline", "c3full", "c1", "c2", "cpu")
-DEFAULT_BATCH_SHAPES = dict(design_split=24 * 1024, design_threads=512, stem_waves=7, dom_rows=128,
-                            fronts_threads=1024, assoc_designs=4, niche_threads=1024)
+DEFAULT_BATCH_SHAPES = dict(design_split=0, design_threads=256, stem_waves=8, dom_rows=256,
+                            fronts_threads=1024, assoc_designs=64, niche_threads=1024)
 
 # Hardware counters of the offspring phase of one batched tick at the default
-# workload (both k_design<2> launch classes), from the rocprofv3 --pmc runs
-# summarised in profiles/pmc_batched_mix_64jobs.md: HBM bytes (FETCH_SIZE x
-# its copy-kernel factor + WRITE_SIZE x its factor), VALU wave-instructions,
-# LDS instructions and LDS bank-conflict cycles.
-TICK_COUNTERS = {"hbm_bytes": 736134804, "valu_wave_instr": 244725985, "lds_instr": 24882951,
-                 "lds_conflict_cycles": 6257523}
+# workload, from the rocprofv3 --pmc runs summarised in
+# profiles/pmc_batched_mix_64jobs.md: HBM bytes (FETCH_SIZE x its copy-kernel
+# factor + WRITE_SIZE x its factor), VALU wave-instructions, LDS instructions
+# and LDS bank-conflict cycles.
+TICK_COUNTERS = {"hbm_bytes": 704758481, "valu_wave_instr": 166839218, "lds_instr": 8242560,
+                 "lds_conflict_cycles": 5521106}
 
 
 def log(msg):
@@ -130,7 +130,7 @@ def bench_headline(cdp, args):
         roof = {"bound": "hbm", "achieved": round(rate / 1e9, 2), "peak": HBM_BYTES_S / 1e9, "unit": "GB/s",
                 "frac": round(rate / HBM_BYTES_S, 5),
                 "traffic": TICK_COUNTERS["hbm_bytes"] if TICK_COUNTERS else None,
-                "kernel": "k_design<offspring>: both launch classes of one tick",
+                "kernel": "k_design<offspring> of one tick",
                 "bytes_per_launch": int(nbytes), "ms_per_launch": round(prof[0], 4)}
     else:
         roof = {"bound": "see kernel", "kernel": dominant, "ms_per_launch": round(prof[KERNELS.index(dominant)], 4),
@@ -138,7 +138,7 @@ def bench_headline(cdp, args):
     counters = None
     if TICK_COUNTERS:
         c = TICK_COUNTERS
-        counters = {"kernel": "k_design<offspring> (one tick's two launches)",
+        counters = {"kernel": "k_design<offspring> of one tick",
                     "valu_issue_frac": round(c["valu_wave_instr"] / (prof[0] / 1e3) / VALU_WAVE_INSTR_S, 4),
                     "valu_peak_wave_instr_s": VALU_WAVE_INSTR_S,
                     "lds_bank_conflict_cycles_per_lds_instr": round(c["lds_conflict_cycles"] / c["lds_instr"], 4),
