@@ -203,10 +203,10 @@ int cd_batch_shapes(cd_batch *batch, cd_shapes *get, const cd_shapes *set);
  * (cd_job_device_bytes) fit the budget beside the jobs holding memory and
  * fewer than max_jobs hold memory, and initialises it on its own stream
  * while the resident jobs keep running; a worker thread advances every
- * resident job one generation per tick (one captured hipGraph per resident
- * set); a collecting thread copies a finished job's final pool to host
- * memory and frees its device memory.  Populations, fronts and generator
- * state stay on the device until the job's generation budget is spent.  A
+ * resident job one generation per tick; a collecting thread copies a
+ * finished job's final pool to host memory and frees its device memory.
+ * Populations, fronts and generator state stay on the device until the
+ * job's generation budget is spent.  A
  * job's result is the same alone and in any mix.  Thread-safe: submit, wait
  * and result may be called from any thread. */
 typedef struct cd_server cd_server;

@@ -5,9 +5,8 @@
 //              the budget beside the jobs that hold memory (and a slot is
 //              free), creates each job and enqueues its initialisation on the
 //              job's own stream, and hands it over with an event;
-//   worker     advances every resident job one generation per tick: one
-//              hipGraph captured per resident set (captured again when the set
-//              changes), at most two ticks in flight; a job whose
+//   worker     advances every resident job one generation per tick, at most
+//              two ticks in flight; a job whose
 //              initialisation event has completed joins at the next tick, a
 //              job leaves after the tick that completes its generation budget;
 //   collector  waits for a finished job's last tick, copies its final pool and
@@ -76,12 +75,6 @@ double seconds(Clock::time_point a, Clock::time_point b) { return std::chrono::d
 
 struct cd_server {
     std::mutex mu;
-    // held by the worker while it captures a tick, and by the other threads
-    // around the HIP calls that create, initialise, collect or destroy a job
-    // (stream and event creation, waits and destruction, stream-ordered
-    // allocation): such calls from another thread can end a capture in
-    // progress
-    std::mutex capture_mu;
     std::condition_variable cv_admit, cv_work, cv_collect, cv_done;
     std::thread admitter, worker, collector;
     bool stop = false;
@@ -95,7 +88,7 @@ struct cd_server {
     int64_t ticks = 0, designs = 0;
     double tick_ms = 0.0;  // GPU time of the ticks (events around each launch)
     double busy_s = 0.0;   // worker wall time with jobs resident
-    int64_t rebuilds = 0;  // resident-set changes (lists uploaded, tick captured again)
+    int64_t rebuilds = 0;  // resident-set changes (lists uploaded)
     double rebuild_s = 0.0;
     double launch_s = 0.0;  // worker time launching ticks
     double wait_s = 0.0;    // worker time waiting for the tick two back
@@ -107,10 +100,8 @@ struct cd_server {
     uint2 *d_slist = nullptr;  // changed CDS of a tick (stem_list_entries)
     int32_t *d_sctl = nullptr;    // their counts (STEM_MAX_GROUPS), zero between ticks
     size_t cap_jobs = 0, cap_off = 0, cap_dom = 0, cap_asc = 0, cap_slist = 0;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec = nullptr;
+    cdhost::Launch tick{};  // one tick of the resident set (worker only)
     std::string fatal;        // a device error that stopped the server
-    std::string fatal_stage;  // the step of the tick's capture that failed, if it was one (worker only)
 };
 
 namespace {
@@ -145,7 +136,6 @@ int collect(Entry *E) {
 // Release a job's device memory and end its request.
 void finish(cd_server *S, Entry *E, int state, const std::string &err) {
     {
-        std::lock_guard<std::mutex> cap(S->capture_mu);
         if (E->job) {
             cd_job_destroy(E->job);
             E->job = nullptr;
@@ -203,7 +193,6 @@ void admit_loop(cd_server *S) {
         }
         int rc = CD_OK;
         {
-            std::lock_guard<std::mutex> cap(S->capture_mu);
             rc = cd_job_create(&E->req.desc, &E->job);
             if (rc == CD_OK) rc = cd_job_init(E->job);  // enqueued on the job's own stream
             if (rc == CD_OK && hipEventCreateWithFlags(&E->ready, hipEventDisableTiming) != hipSuccess)
@@ -234,9 +223,6 @@ void collect_loop(cd_server *S) {
         }
         int rc = CD_OK;
         {
-            // E->last was recorded on the tick stream, which the worker may be
-            // capturing: waiting on it then would end the capture
-            std::lock_guard<std::mutex> cap(S->capture_mu);
             if (E->last && hipEventSynchronize(E->last) != hipSuccess) rc = CD_E_DEVICE;
             if (rc == CD_OK) rc = collect(E);
         }
@@ -244,7 +230,10 @@ void collect_loop(cd_server *S) {
     }
 }
 
-// Upload the work lists of `res` and capture one tick's launch sequence.
+// Upload the work lists of `res`: what a tick launches.  A tick's kernels are
+// enqueued one by one, 20 us of host time against 240 a tick: a graph of them
+// would have to be captured for every set, with the other threads' job
+// creation, reads and destruction kept out meanwhile.
 hipError_t rebuild(cd_server *S, const std::vector<Entry *> &res) {
     std::vector<cd_job *> jobs;
     for (Entry *E : res) jobs.push_back(E->job);
@@ -252,7 +241,7 @@ hipError_t rebuild(cd_server *S, const std::vector<Entry *> &res) {
     (void)cdhost::cached_shapes(cdhost::work_signature(jobs.data(), (int)jobs.size()), &sh);
     cdhost::WorkLists wl;
     cdhost::build_lists(jobs.data(), (int)jobs.size(), sh, wl);
-    hipError_t e = hipStreamSynchronize(S->stream);  // no tick in flight reads the old lists or graph
+    hipError_t e = hipStreamSynchronize(S->stream);  // no tick in flight reads the old lists
     if (e == hipSuccess) e = ensure(S->d_jobs, S->cap_jobs, wl.descs.size());
     if (e == hipSuccess) e = ensure(S->d_off, S->cap_off, wl.off.size());
     if (e == hipSuccess) e = ensure(S->d_dom, S->cap_dom, wl.dom.size());
@@ -265,35 +254,11 @@ hipError_t rebuild(cd_server *S, const std::vector<Entry *> &res) {
     if (e == hipSuccess) e = hipMemcpy(S->d_asc, wl.asc.data(), sizeof(int2) * wl.asc.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = cdhost::set_lds_limits(wl);
     if (e != hipSuccess) return e;
-    const cdhost::Launch L{S->d_jobs,   (int)wl.descs.size(), S->d_off,      (int)wl.off.size(), S->d_dom,
-                           (int)wl.dom.size(), S->d_asc,      (int)wl.asc.size(), wl.lds,         wl.stem_lds,
-                           wl.max_pool,  wl.max_refs,        wl.mg,               S->d_slist,     S->d_sctl,
-                           wl.n_cds,     wl.n_small,          wl.lds_small,       wl.pool,           sh};
-    if (S->gexec) (void)hipGraphExecDestroy(S->gexec);
-    if (S->graph) (void)hipGraphDestroy(S->graph);
-    S->gexec = nullptr;
-    S->graph = nullptr;
-    // job creation, initialisation, collection and destruction on the other
-    // threads wait for the capture (capture_mu)
-    std::lock_guard<std::mutex> cap(S->capture_mu);
-    e = hipStreamBeginCapture(S->stream, hipStreamCaptureModeRelaxed);
-    if (e != hipSuccess) {
-        S->fatal_stage = "begin capture";
-        return e;
-    }
-    const hipError_t ec = cdhost::enqueue_generation(L, S->stream, nullptr);
-    e = hipStreamEndCapture(S->stream, &S->graph);
-    if (ec != hipSuccess) {
-        S->fatal_stage = "capture";
-        return ec;
-    }
-    if (e != hipSuccess) {
-        S->fatal_stage = "end capture";
-        return e;
-    }
-    e = hipGraphInstantiate(&S->gexec, S->graph, nullptr, nullptr, 0);
-    if (e != hipSuccess) S->fatal_stage = "graph instantiation";
-    return e;
+    S->tick = cdhost::Launch{S->d_jobs,   (int)wl.descs.size(), S->d_off,      (int)wl.off.size(), S->d_dom,
+                             (int)wl.dom.size(), S->d_asc,      (int)wl.asc.size(), wl.lds,         wl.stem_lds,
+                             wl.max_pool,  wl.max_refs,        wl.mg,               S->d_slist,     S->d_sctl,
+                             wl.n_cds,     wl.n_small,          wl.lds_small,       wl.pool,           sh};
+    return hipSuccess;
 }
 
 void work_loop(cd_server *S) {
@@ -372,12 +337,11 @@ void work_loop(cd_server *S) {
         if (e == hipSuccess) e = retire(slot);  // at most two ticks in flight
         const Clock::time_point w1 = Clock::now();
         if (e == hipSuccess) e = hipEventRecord(ev[slot][0], S->stream);
-        if (e == hipSuccess) e = hipGraphLaunch(S->gexec, S->stream);
+        if (e == hipSuccess) e = cdhost::enqueue_generation(S->tick, S->stream, nullptr);
         if (e == hipSuccess) e = hipEventRecord(ev[slot][1], S->stream);
         const Clock::time_point w2 = Clock::now();
         if (e != hipSuccess) {  // a device error ends every request and the server
-            fail_all(S, std::string("serving loop: ") + (S->fatal_stage.empty() ? "" : S->fatal_stage + ": ") +
-                            hipGetErrorString(e));
+            fail_all(S, std::string("serving loop: ") + hipGetErrorString(e));
             break;
         }
         inflight[slot] = true;
@@ -557,8 +521,6 @@ int cd_server_destroy(cd_server *S) {
         if (E->ready) (void)hipEventDestroy(E->ready);
         if (E->last) (void)hipEventDestroy(E->last);
     }
-    if (S->gexec) (void)hipGraphExecDestroy(S->gexec);
-    if (S->graph) (void)hipGraphDestroy(S->graph);
     if (S->stream) (void)hipStreamDestroy(S->stream);
     if (S->d_jobs) (void)hipFree(S->d_jobs);
     if (S->d_off) (void)hipFree(S->d_off);
