@@ -135,15 +135,13 @@ int collect(Entry *E) {
 
 // Release a job's device memory and end its request.
 void finish(cd_server *S, Entry *E, int state, const std::string &err) {
-    {
-        if (E->job) {
-            cd_job_destroy(E->job);
-            E->job = nullptr;
-        }
-        if (E->ready) (void)hipEventDestroy(E->ready);
-        if (E->last) (void)hipEventDestroy(E->last);
-        E->ready = E->last = nullptr;
+    if (E->job) {
+        cd_job_destroy(E->job);
+        E->job = nullptr;
     }
+    if (E->ready) (void)hipEventDestroy(E->ready);
+    if (E->last) (void)hipEventDestroy(E->last);
+    E->ready = E->last = nullptr;
     std::lock_guard<std::mutex> lk(S->mu);
     E->state = state;
     E->error = err;
@@ -191,14 +189,11 @@ void admit_loop(cd_server *S) {
             S->used += E->req.bytes;
             S->admitted += 1;
         }
-        int rc = CD_OK;
-        {
-            rc = cd_job_create(&E->req.desc, &E->job);
-            if (rc == CD_OK) rc = cd_job_init(E->job);  // enqueued on the job's own stream
-            if (rc == CD_OK && hipEventCreateWithFlags(&E->ready, hipEventDisableTiming) != hipSuccess)
-                rc = CD_E_DEVICE;
-            if (rc == CD_OK && hipEventRecord(E->ready, E->job->stream) != hipSuccess) rc = CD_E_DEVICE;
-        }
+        int rc = cd_job_create(&E->req.desc, &E->job);
+        if (rc == CD_OK) rc = cd_job_init(E->job);  // enqueued on the job's own stream
+        if (rc == CD_OK && hipEventCreateWithFlags(&E->ready, hipEventDisableTiming) != hipSuccess)
+            rc = CD_E_DEVICE;
+        if (rc == CD_OK && hipEventRecord(E->ready, E->job->stream) != hipSuccess) rc = CD_E_DEVICE;
         if (rc != CD_OK) {
             finish(S, E, CD_SERVER_FAILED, cd_last_error());
             continue;
@@ -222,10 +217,8 @@ void collect_loop(cd_server *S) {
             S->done.pop_front();
         }
         int rc = CD_OK;
-        {
-            if (E->last && hipEventSynchronize(E->last) != hipSuccess) rc = CD_E_DEVICE;
-            if (rc == CD_OK) rc = collect(E);
-        }
+        if (E->last && hipEventSynchronize(E->last) != hipSuccess) rc = CD_E_DEVICE;
+        if (rc == CD_OK) rc = collect(E);
         finish(S, E, rc == CD_OK ? CD_SERVER_DONE : CD_SERVER_FAILED, rc == CD_OK ? "" : cd_last_error());
     }
 }
