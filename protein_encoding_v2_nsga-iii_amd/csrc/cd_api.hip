@@ -616,7 +616,7 @@ hipError_t enqueue_generation(const Launch &w, hipStream_t s, hipEvent_t *ev) {
     }
     if (e == hipSuccess) e = mark(1);
     if (e == hipSuccess)
-        e = cd::launch_stem_list(w.jobs, w.off, w.n_off, w.mg, w.stem_list, w.stem_ctl, sl, w.sh.stem_waves, w.stem_lds, s);
+        e = cd::launch_stem_list(w.jobs, w.off, w.n_off, w.mg, w.longest, w.stem_list, w.stem_ctl, sl, w.sh.stem_waves, w.stem_lds, s);
     if (e == hipSuccess) e = mark(2);
     if (e == hipSuccess)
         e = cd::launch_dominance(w.jobs, w.dom, w.n_dom, true, w.stem_ctl, sl.groups, w.sh.dom_rows, s);
@@ -666,6 +666,7 @@ void build_lists(cd_job *const *jobs, int count, const cd::Shapes &sh, WorkLists
         wl.pool += J->P;
         wl.max_refs = std::max(wl.max_refs, J->R);
         wl.mg = std::max(wl.mg, J->m);
+        wl.longest = std::max(wl.longest, J->L);
     }
 }
 
@@ -723,7 +724,7 @@ int step_graphs(StepGraphs &G, hipStream_t s, const Launch &w, int generations) 
 
 Launch job_launch(cd_job *J) {
     return Launch{J->d_self, 1,          J->d_off,     J->N,          J->d_dom,   J->n_dom,   J->d_asc,
-                  J->n_asc,  J->lds,     J->stem_lds,  J->P,          J->R,       J->m,
+                  J->n_asc,  J->lds,     J->stem_lds,  J->P,          J->R,       J->m,   J->L,
                   J->d_slist,
                   J->d_sctl, J->N * J->m, 0,           0,             J->P,          J->shapes};
 }
@@ -1271,6 +1272,7 @@ int cd_batch_create(cd_job *const *jobs, int32_t count, cd_batch **out) {
     B->pool = wl.pool;
     B->max_refs = wl.max_refs;
     B->mg = wl.mg;
+    B->longest = wl.longest;
     B->n_cds = wl.n_cds;
     B->n_small = wl.n_small;
     B->lds_small = wl.lds_small;
@@ -1302,7 +1304,7 @@ int cd_batch_create(cd_job *const *jobs, int32_t count, cd_batch **out) {
 static Launch batch_launch(cd_batch *B) {
     return Launch{B->d_jobs,    (int)B->jobs.size(), B->d_off,      B->n_off,   B->d_dom,
                   B->n_dom,     B->d_asc,            B->n_asc,      B->lds,     B->stem_lds,
-                  B->max_pool,  B->max_refs,         B->mg,         B->d_slist, B->d_sctl,
+                  B->max_pool,  B->max_refs,         B->mg,         B->longest, B->d_slist, B->d_sctl,
                   B->n_cds,     B->n_small,          B->lds_small,  B->pool,      B->shapes};
 }
 

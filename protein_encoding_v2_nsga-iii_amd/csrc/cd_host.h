@@ -77,6 +77,7 @@ struct cd_batch {
     int pool = 0;        // designs of all their pools
     int max_refs = 0;    // most reference points of the batch's jobs
     int mg = 0;          // largest m of the batch's jobs
+    int longest = 0;     // codons of their longest CDS
     hipStream_t stream = nullptr;
     StepGraphs graphs;
 };
@@ -110,6 +111,7 @@ struct Launch {
     int max_pool;    // largest pool
     int max_refs;    // most reference points
     int mg;          // largest m
+    int longest;     // codons of the longest CDS
     uint2 *stem_list;  // changed CDS of a generation, in sublists of consecutive children (stem_list_entries)
     int32_t *stem_ctl;    // their counts, zero between generations (k_dominance clears them)
     int n_cds;            // CDS of all children: sum of N * m
@@ -129,7 +131,7 @@ struct WorkLists {
     std::vector<int2> off, asc;
     std::vector<int4> dom;
     size_t lds = 0, stem_lds = 0;
-    int max_pool = 0, max_refs = 0, mg = 0, n_cds = 0, pool = 0;
+    int max_pool = 0, max_refs = 0, mg = 0, longest = 0, n_cds = 0, pool = 0;
     int n_small = 0;  // children (first in off) of jobs with lds at most shapes.design_split
     size_t lds_small = 0;
 };

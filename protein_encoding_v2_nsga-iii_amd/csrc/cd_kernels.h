@@ -22,6 +22,13 @@ constexpr int ASSOC_DESIGNS = 4;           // designs per k_associate workgroup 
 // 2048 / 4096: 251 / 242 / 238 / 245 us on the 4096 children.
 constexpr int STEM_FEW = 2048;    // initialisation and evaluation
 constexpr int STEM_MANY = 65536;  // offspring
+// Listed offspring of CDS of at most this many codons take the second shape
+// whatever their number: their indexes are small, so twice as many searches
+// reside with it.  5 / 16 jobs of 4 x 1024 CDS, 256 x 2048 against 128 x 1024:
+// 101 codons 122.8 / 111.4 and 245.7 / 211.3 us a generation, 600 141.4 / 138.1
+// and 298.2 / 281.7, 900 147.3 / 140.7 and 333.9 / 308.4, 1300 163.7 / 171.8 and
+// 394.1 / 408.3.
+constexpr int STEM_SHORT = 1024;
 // Offspring launches up to this size have no list of the changed CDS (the
 // figures stand at k_stem_each).
 constexpr int STEM_EACH = 16384;
@@ -123,9 +130,9 @@ hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, i
 // offspring generations: stem of each CDS the offspring k_design listed
 // (the n items and sl as given to it), on as many workgroups as are resident at
 // once (STEM_CUS x what `waves`, 5 to 8 waves per SIMD, and the LDS allow), at
-// most the entries there can be; launch_dominance with the same stem_ctl and
-// sl.groups clears the counts
-hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, const uint2 *stem_list,
+// most the entries there can be; longest: codons of the longest CDS;
+// launch_dominance with the same stem_ctl and sl.groups clears the counts
+hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, int longest, const uint2 *stem_list,
                             const int32_t *stem_ctl, StemList sl, int waves, size_t lds, hipStream_t s);
 // one thread per item: objective 5, clears the marks
 hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s);

@@ -3250,7 +3250,7 @@ hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, i
         hipLaunchKernelGGL((k_stem<128, 1024>), dim3(n * mg), dim3(128), lds + seek_more_bytes(1024, 128), s, jobs, items, mode, mg);
     return hipGetLastError();
 }
-hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, const uint2 *stem_list,
+hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, int longest, const uint2 *stem_list,
                             const int32_t *stem_ctl, StemList sl, int waves, size_t lds, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (!stem_list || !stem_ctl || waves < 5 || waves > 8 || sl.groups > STEM_MAX_GROUPS) return hipErrorInvalidValue;
@@ -3272,7 +3272,8 @@ hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg
         hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), bytes, s, jobs, stem_list, stem_ctl, sl.groups, sl.cap);
         return hipGetLastError();
     };
-    return (int64_t)n * mg <= STEM_MANY ? go(k_stem_list<256, 2048>, 2048, 256) : go(k_stem_list<128, 1024>, 1024, 128);
+    const bool few = (int64_t)n * mg <= STEM_MANY && longest > STEM_SHORT;
+    return few ? go(k_stem_list<256, 2048>, 2048, 256) : go(k_stem_list<128, 1024>, 1024, 128);
 }
 hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;

@@ -249,7 +249,7 @@ hipError_t rebuild(cd_server *S, const std::vector<Entry *> &res) {
     if (e != hipSuccess) return e;
     S->tick = cdhost::Launch{S->d_jobs,   (int)wl.descs.size(), S->d_off,      (int)wl.off.size(), S->d_dom,
                              (int)wl.dom.size(), S->d_asc,      (int)wl.asc.size(), wl.lds,         wl.stem_lds,
-                             wl.max_pool,  wl.max_refs,        wl.mg,               S->d_slist,     S->d_sctl,
+                             wl.max_pool,  wl.max_refs,        wl.mg,  wl.longest,  S->d_slist,     S->d_sctl,
                              wl.n_cds,     wl.n_small,          wl.lds_small,       wl.pool,           sh};
     return hipSuccess;
 }

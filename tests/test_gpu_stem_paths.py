@@ -32,6 +32,21 @@ def test_launch_sizes(cdp, orc, N, m, L):
     generations(cdp, orc, T.synth_protein(L - 1, N), T.synth_tables(N), m, N, 2, N + m)
 
 
+@pytest.mark.parametrize("L", [1024, 1025])
+def test_listed_lengths(cdp, L):
+    """(the children's records against the same designs evaluated anew: the
+    oracle's stems of 16400 such CDS take half a minute)"""
+    print("listed", L, flush=True)
+    T = cdp.tables
+    aa, tab = T.synth_protein(L - 1, L), T.synth_tables(L)
+    j = cdp.Job(aa, tab, 16, 1025, 2, 0.1, L).init()
+    j.step(3)
+    r = j.read()
+    j.close()
+    for a, b in zip(cdp.evaluate(aa, tab, r["genome"]), (r["obj"], r["idx"], r["pql"])):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("L", [32, 64, 65, 1024, 1025])
 def test_lengths(cdp, orc, L):
     print("length", L, flush=True)
