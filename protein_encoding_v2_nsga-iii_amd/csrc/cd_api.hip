@@ -440,8 +440,7 @@ hipError_t job_lds_limits(const cd_job *J, bool select) {
     if (J->lds > 48 * 1024) e = cd::set_design_lds_limit(J->lds);
     if (e == hipSuccess && cd::stem_list_lds(J->stem_lds) > 48 * 1024)
         e = cd::set_stem_lds_limit(cd::stem_list_lds(J->stem_lds));
-    if (e == hipSuccess && select && cd::niche_lds_need(J->P, J->R) > cd::NICHE_LDS_PLAIN)
-        e = cd::set_niche_lds_limit(cd::niche_lds_need(J->P, J->R));
+    if (e == hipSuccess && select) e = cd::set_niche_lds_limit(J->P, J->R);
     return e;
 }
 
@@ -675,8 +674,7 @@ hipError_t set_lds_limits(const WorkLists &wl) {
     if (wl.lds > 48 * 1024) e = cd::set_design_lds_limit(wl.lds);
     if (e == hipSuccess && cd::stem_list_lds(wl.stem_lds) > 48 * 1024)
         e = cd::set_stem_lds_limit(cd::stem_list_lds(wl.stem_lds));
-    const size_t niche = cd::niche_lds_need(wl.max_pool, wl.max_refs);
-    if (e == hipSuccess && niche > cd::NICHE_LDS_PLAIN) e = cd::set_niche_lds_limit(niche);
+    if (e == hipSuccess) e = cd::set_niche_lds_limit(wl.max_pool, wl.max_refs);
     return e;
 }
 

@@ -181,14 +181,16 @@ constexpr int PLACE_NICHE_POOL = 2048;
 __host__ __device__ inline int place_niche_slots(int P, int R) { return P + 3 * (R < P ? R : P); }
 inline size_t place_niche_lds_bytes(int P, int R) { return (size_t)8 * ((place_niche_slots(P, R) + 3) & ~3); }
 size_t niche_lds_bytes(int P);
-// dynamic LDS of the niching of pools up to P with up to R reference points,
-// and its limit, to be raised above NICHE_LDS_PLAIN (k_place_niche's static
-// arrays take 37 KiB beside it)
+// The rule above, and the dynamic LDS of the niching kernel it takes; that
+// kernel's limit is raised above NICHE_LDS_PLAIN.  Of that kernel only:
+// k_place_niche's static arrays take 37 KiB, so it cannot have the 128 KB that
+// k_niche takes for a pool of 16384.
 constexpr size_t NICHE_LDS_PLAIN = 24 * 1024;
+inline bool takes_place_niche(int max_pool, int max_refs) { return max_pool <= PLACE_NICHE_POOL && max_refs <= NICHE_STAGE; }
 inline size_t niche_lds_need(int P, int R) {
-    return P <= PLACE_NICHE_POOL && R <= NICHE_STAGE ? place_niche_lds_bytes(P, R) : niche_lds_bytes(P);
+    return takes_place_niche(P, R) ? place_niche_lds_bytes(P, R) : niche_lds_bytes(P);
 }
-hipError_t set_niche_lds_limit(size_t bytes);
+hipError_t set_niche_lds_limit(int max_pool, int max_refs);
 hipError_t launch_niche(const DevJob *jobs, int njobs, int max_pool, int max_refs, int threads, hipStream_t s);
 hipError_t launch_init_state(const DevJob *jobs, int njobs, hipStream_t s);
 hipError_t launch_zero_np(const DevJob *jobs, int njobs, hipStream_t s);

@@ -3358,14 +3358,15 @@ static hipError_t raise_lds_limit(size_t &held, size_t bytes, F apply) {
     if (e == hipSuccess) held = bytes;
     return e;
 }
-static size_t g_design_lds = 0, g_stem_lds = 0, g_niche_lds = 0;
+static size_t g_design_lds = 0, g_stem_lds = 0, g_niche_lds = 0, g_place_niche_lds = 0;
 
-hipError_t set_niche_lds_limit(size_t bytes) {
-    return raise_lds_limit(g_niche_lds, bytes, [](int b) {
-        const hipError_t e = hipFuncSetAttribute((const void *)k_niche, hipFuncAttributeMaxDynamicSharedMemorySize, b);
-        return e != hipSuccess ? e
-                               : hipFuncSetAttribute((const void *)k_place_niche,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, b);
+hipError_t set_niche_lds_limit(int max_pool, int max_refs) {
+    const size_t bytes = niche_lds_need(max_pool, max_refs);
+    if (bytes <= NICHE_LDS_PLAIN) return hipSuccess;
+    const bool place = takes_place_niche(max_pool, max_refs);
+    const void *const kern = place ? (const void *)k_place_niche : (const void *)k_niche;
+    return raise_lds_limit(place ? g_place_niche_lds : g_niche_lds, bytes, [kern](int b) {
+        return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, b);
     });
 }
 hipError_t launch_niche(const DevJob *jobs, int njobs, int max_pool, int max_refs, int threads, hipStream_t s) {
@@ -3376,7 +3377,7 @@ hipError_t launch_niche(const DevJob *jobs, int njobs, int max_pool, int max_ref
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    if (max_pool <= PLACE_NICHE_POOL && max_refs <= NICHE_STAGE) {  // one workgroup per job
+    if (takes_place_niche(max_pool, max_refs)) {  // one workgroup per job
         hipLaunchKernelGGL(k_place_niche, dim3(njobs), dim3(threads), place_niche_lds_bytes(max_pool, max_refs), s, jobs);
         return hipGetLastError();
     }
