@@ -15,9 +15,12 @@
 // A4 = A2 & A2<<2, ... marks the positions that end a window of k matches,
 // a window of K (the longest stem this lane knows, at least the seed) is
 // assembled from it, and only the run ends carrying such a window are
-// measured exactly.  Every run of length >= K is measured, and K never
-// exceeds the longest stem of the CDS, so the maximum over all lanes is exact
-// including the tie rule (longest, then smallest p, then smallest q).
+// measured exactly.  Of every anti-diagonal the first run of each length >= K
+// that is longer than those before it is measured, and K never exceeds the
+// longest stem of the CDS, so the maximum over all lanes is exact including the
+// tie rule (longest, then smallest p, then smallest q: p rises along an
+// anti-diagonal).  (A repetitive CDS without a run of 4 can hold a run of one or
+// two at every other position.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -100,7 +103,8 @@ __host__ __device__ inline void scan_diagonal(const uint2 *sp, const uint2 *rp, 
     const int ss = i0 & 31, st = t0 & 31;
     const uint2 *ps = sp + (i0 >> 5), *pr = rp + (t0 >> 5);
     ScanWindow win;
-    scan_window(K, win);
+    int Kd = K;  // the window on the rest of this anti-diagonal
+    scan_window(Kd, win);
     // match bits of chunk c from words c and c+1 (the last chunk is masked)
     auto chunk_at = [&](int c) -> uint32_t {
         const uint2 a0 = ps[c], a1 = ps[c + 1], b0 = pr[c], b1 = pr[c + 1];
@@ -133,9 +137,10 @@ __host__ __device__ inline void scan_diagonal(const uint2 *sp, const uint2 *rp, 
             const int ie = i0 + 32 * (c - 1) + k;
             const uint64_t key = scan_key(l, ie - l + 1, S - ie);
             if (key > best) best = key;
-            if (l > K) {
-                K = l;
-                scan_window(K, win);
+            K = l > K ? l : K;
+            if (l >= Kd) {  // (p rises along it: of one length the first run is the best)
+                Kd = l + 1;
+                scan_window(Kd, win);
                 Lp = scan_level(win, Mp, A2p, A4p, A8p);
             }
         }

@@ -17,8 +17,12 @@
 // 7 at K = 7, else 4 (K is at least 4).
 // Diagonals so flagged in a tile are measured exactly from the planes, 64
 // rows at a time: every maximal run meeting the tile whose length is at least W,
-// extended past the tile as far as it goes.  So every run of length
-// >= min(K, 8) is measured, and with K never above the longest stem the
+// extended past the tile as far as it goes -- but for one that starts eight or
+// more rows above the tile: its first window ends above, whichever window that
+// tile looks for, so an earlier tile of the block measures it.  (A repetitive CDS
+// has runs of thousands of pairs: followed again by every tile that they cross,
+// they made its scan cubic in its length: 1500 residues of FK 8.6 ms by one
+// workgroup.)  So every run of length >= min(K, 8) is measured, and with K never above the longest stem the
 // maximum of the keys is exact including the tie rule (longest, then
 // smallest p, then smallest q).  The windows 7 and 8 keep flags rare once K
 // nears the longest stem; the windows 5 and 6 would need longer histories
@@ -91,20 +95,19 @@ __host__ __device__ inline int tile_run_down(const uint2 *X, const uint2 *Y, int
     return cnt;
 }
 
-// Exact measure of diagonal d of half h around rows [ua, uz] (uz - ua < 40):
-// every maximal run of matches that meets [ua, uz], extended inside the valid
-// rows 0 .. (n-6-d)/2, is offered to best (and K) if at least lmin long
-// (4 <= lmin <= 8).  Works on 64 rows of match bits at once: the run through
+// Exact measure of diagonal d of half h around the tile of rows u0 .. u0+31:
+// every maximal run of matches that meets rows u0-lmin+1 .. u0+31 and starts
+// after row u0-8, extended inside the valid rows 0 .. (n-6-d)/2, is offered to
+// best (and K) if at least lmin long (4 <= lmin <= 8).  Works on 64 rows of match bits at once: the run through
 // ua is followed down the diagonal, and runs starting in (ua, uz] are found
 // from their first lmin-window; a run reaching the word's last row is
 // followed up the diagonal.
-__host__ __device__ inline void tile_verify(const uint2 *X, const uint2 *Y, int n, int h, int d, int ua, int uz,
-                                            int lmin, uint64_t &best, int &K) {
+__host__ __device__ inline void tile_verify(const uint2 *X, const uint2 *Y, int n, int h, int d, int u0, int lmin,
+                                            uint64_t &best, int &K) {
     const int hi = n - 6 - d;
     if (hi < 0) return;
     const int umax = hi >> 1;
-    if (ua < 0) ua = 0;
-    if (uz > umax) uz = umax;
+    const int ua = u0 > 0 ? u0 - lmin + 1 : 0, uz = u0 + 31 < umax ? u0 + 31 : umax;
     if (ua > uz) return;
     uint64_t m = (uint64_t)tile_match(X, Y, d, ua) | ((uint64_t)tile_match(X, Y, d, ua + 32) << 32);
     if (umax - ua < 63) m &= (2ull << (umax - ua)) - 1ull;  // rows ua .. umax
@@ -131,8 +134,15 @@ __host__ __device__ inline void tile_verify(const uint2 *X, const uint2 *Y, int 
     const int lim = uz - ua;               // <= 39, so every window tested lies inside the word
     g &= (2ull << lim) - 1ull;
     if (m & 1ull) {  // the run through ua
-        const int down = tile_run_down(X, Y, d, ua - 1), len = run_from(0);
-        offer(ua - down, down + len);
+        int len = 64;
+        if (u0 > 0 && (~tile_match(X, Y, d, u0 - 8) & ((1u << (9 - lmin)) - 1u)) == 0u) {  // from row u0-8 or before
+            if (~m) len = __builtin_ctzll(~m);
+            if (len >= lmin - 1 && K < 8) K = 8;  // (and rows up to u0-1: the run has 8)
+        } else {
+            len = run_from(0);
+            const int down = tile_run_down(X, Y, d, ua - 1);
+            offer(ua - down, down + len);
+        }
         g = clear_to(g, len - 1);
     }
     while (g) {  // runs starting at bit b in (0, lim] and at least lmin long
@@ -258,7 +268,7 @@ __host__ __device__ inline void tile_step(const uint2 *sp, const uint2 *rp, int 
     while (f) {
         const int k = __builtin_ctz(f);
         f &= f - 1u;
-        tile_verify(X, Y, n, c.h, base + k, u0 - W + 1, u0 + 31, W, best, K);
+        tile_verify(X, Y, n, c.h, base + k, u0, W, best, K);
     }
     if (++c.g == tile_groups(n, base)) {  // next block (of the next half after the last)
         c.g = 0;
