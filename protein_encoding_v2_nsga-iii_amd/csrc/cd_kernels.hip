@@ -140,11 +140,12 @@ __device__ __forceinline__ int code_base(const uint8_t *row, int p) {
 // ---------------------------------------------------------------------------
 // Longest stem of one CDS held as bit planes in LDS (calMaximumSL,
 // utils.cuh:712-888; the planes are built by k_design): word searches
-// (cd_seek.h) at a known or guessed length, lower guesses after a fruitless
-// one, and the tiles (cd_tile.h) for a CDS whose stems are all shorter than 5
-// or that the search gives up on.  A CDS with no run of 4 and no seed of 4 is
-// scanned exactly along its anti-diagonals (cd_scan.h).  Each search takes
-// the maximum key (longest, then smallest p, then smallest q).
+// (cd_seek.h) at a known or guessed length, a lower guess after a fruitless
+// one and the length met after one that stopped early, and the tiles (cd_tile.h)
+// for a CDS whose stems are all shorter than 5 or that the searches give up on.
+// A CDS with no run of 4 and no seed of 4 is scanned exactly along its
+// anti-diagonals (cd_scan.h).  Each search takes the maximum key (longest, then
+// smallest p, then smallest q).
 // ---------------------------------------------------------------------------
 // The seed: the longest run of pairs (i - k, j + k), k < 64, that
 // still pair in the child, with (i, j) = (p + l - 1, q) the parent's
@@ -313,7 +314,7 @@ __device__ __forceinline__ int lanes_below(uint64_t bal) {
 // which are measured 64 at a time: the lanes stay busy whatever share of the
 // lookups, positions and chain entries passes, and no barrier stands between.
 // best: the lane's largest key.  Returns false in a wave that ran out of
-// budget.
+// budget or stopped at a far longer stem (sk_stops).
 template <int NT, int HEADS>
 __device__ __forceinline__ bool seek_run(const SeekLds &S, const uint2 *sp, const uint2 *rp, int n, int L, int K,
                                          bool changed, uint64_t &best) {
@@ -394,6 +395,7 @@ __device__ __forceinline__ bool seek_run(const SeekLds &S, const uint2 *sp, cons
                         nm -= 64;
                         const uint32_t v = S.match[nm + lane];
                         qg_measure(sp, rp, n, (int)(v >> 16), (int)(v & 0xFFFFu), K, best);
+                        if (__any(sk_stops(K, best))) return false;
                     }
                 }
             }
@@ -425,7 +427,7 @@ __device__ __forceinline__ uint64_t seek_cds(const SeekLds &S, const uint2 *sp, 
                                              bool parent, int pl, int pp, int pq, uint64_t *redu, int32_t *flag) {
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     bool intact = false;
-    const int seed = parent ? stem_seed(sp, n, pl, pp, pq, lane, intact) : 0;  // every wave itself
+    int seed = parent ? stem_seed(sp, n, pl, pp, pq, lane, intact) : 0;  // every wave itself
     intact = intact && sk_takes(n, pl);
     int K = intact ? pl : parent ? sk_first_k(n, seed, pl) : sk_blind_k(n);
     bool fresh = true;
@@ -450,9 +452,10 @@ __device__ __forceinline__ uint64_t seek_cds(const SeekLds &S, const uint2 *sp, 
             best = redu[w] > best ? redu[w] : best;
             all &= flag[w] != 0;
         }
-        if (!all) break;  // out of budget
-        if ((int)(best >> 40) >= K) return best;
-        K = sk_next_k(K, seed);
+        const int found = (int)(best >> 40);  // (a stem of the CDS, also where the budget ran out)
+        if (all && found >= K) return best;
+        K = sk_after_k(n, K, all, found, seed, parent);
+        seed = max(seed, found);
         lds_barrier();  // redu and flag are read
     }
     lds_barrier();
