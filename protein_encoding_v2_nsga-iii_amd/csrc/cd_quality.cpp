@@ -177,7 +177,9 @@ class Wfg {
                 y[e] = p[1];
                 m += 1 - (to - e);
             }
-            v += area * (p[2] - (i > 0 ? a[3 * (size_t)o[i - 1] + 2] : 0.0));
+            // (an area without bound times no extent would not be a number)
+            const double extent = p[2] - (i > 0 ? a[3 * (size_t)o[i - 1] + 2] : 0.0);
+            if (extent > 0.0) v += area * extent;
         }
         return v;
     }
