@@ -727,6 +727,25 @@ Launch job_launch(cd_job *J) {
                   J->d_sctl, J->N * J->m, 0,           0,             J->P,          J->shapes};
 }
 
+// The calling thread's device is `dev` while it lives: a job is stepped and read
+// whichever device is current, and its kernels, and the events recorded on its
+// stream, have to be of the stream's device.
+class OnDevice {
+  public:
+    explicit OnDevice(int dev) {
+        int now = dev;
+        if (hipGetDevice(&now) == hipSuccess && now != dev && hipSetDevice(dev) == hipSuccess) was_ = now;
+    }
+    ~OnDevice() {
+        if (was_ >= 0) (void)hipSetDevice(was_);
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+
+  private:
+    int was_ = -1;
+};
+
 // Wait for the job's own stream and for the streams of the batches that hold it.
 hipError_t sync_job(cd_job *J) {
     for (cd_batch *B : J->batches) {
@@ -935,6 +954,7 @@ int cd_job_step(cd_job *J, int32_t generations) {
     if (!J->inited) return fail(CD_E_STATE, "cd_job_step before cd_job_init");
     if (!J->batches.empty()) return fail(CD_E_STATE, "the job is held by a batch: advance it through the batch");
     if (generations < 0) return fail(CD_E_INVALID, "negative generation count");
+    const OnDevice on(J->dev);
     return step_graphs(J->graphs, J->stream, job_launch(J), generations);
 }
 
@@ -994,6 +1014,7 @@ int cd_job_read(cd_job *J, int8_t *genome, float *obj, int8_t *idx, int32_t *pql
                 float *state) {
     if (!J || J->selection_only) return fail(CD_E_INVALID, "null job");
     if (!J->inited) return fail(CD_E_STATE, "cd_job_read before cd_job_init");
+    const OnDevice on(J->dev);
     const int P = J->P;
     const cd::ReadRest at(P, J->W);
     const size_t total = genome ? (size_t)P * J->m * J->L : 0, chunk = std::min(total, READ_CHUNK);
@@ -1314,6 +1335,7 @@ int cd_batch_profile(cd_batch *B, int32_t generations, float *kernel_ms) {
 int cd_batch_step(cd_batch *B, int32_t generations) {
     if (!B) return fail(CD_E_INVALID, "null batch");
     if (generations < 0) return fail(CD_E_INVALID, "negative generation count");
+    const OnDevice on(B->jobs[0]->dev);
     return step_graphs(B->graphs, B->stream, batch_launch(B), generations);
 }
 

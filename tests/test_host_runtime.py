@@ -1,0 +1,57 @@
+"""The engine's host code on a stand-in for the HIP runtime (fake_hip.cpp: two
+devices, rules on streams, events and memory, kernels that do nothing), each
+case in a process of its own."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+SETUP = """
+import ctypes as C, importlib, sys
+F = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+F.fake_used.restype = F.fake_host.restype = C.c_size_t
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+cdp = importlib.import_module("protein_encoding_v2_nsga-iii_amd")
+T = cdp.tables
+def job(residues=30, m=2, N=16, seed=1):
+    return cdp.Job(T.synth_protein(residues, seed), T.synth_tables(seed), m, N, 2, 0.1, seed).init()
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    if not shutil.which("g++"):
+        pytest.skip("g++ not available")
+    out = str(tmp_path_factory.mktemp("hip") / "fake_hip.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", os.path.join(HERE, "fake_hip.cpp"), "-o", out],
+                   check=True, capture_output=True)
+    return out
+
+
+def run(fake, code):
+    r = subprocess.run([sys.executable, "-c", SETUP + code, fake, os.path.dirname(HERE)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_another_device_is_current(fake, batched):
+    """A job or batch of device 0 is stepped (by graph and kernel by kernel) and
+    read while device 1 is the thread's, which it stays."""
+    run(fake, f"""
+jobs = [job(seed=1), job(seed=2)]
+work = cdp.Batch(jobs) if {batched} else jobs[0]
+work.step(30)
+F.hipSetDevice(1)
+work.step(11)
+jobs[0].read()
+dev = C.c_int()
+F.hipGetDevice(C.byref(dev))
+assert dev.value == 1 and F.fake_launches(0) > 0 and F.fake_launches(1) == 0
+job(seed=3).read()
+assert F.fake_launches(1) > 0
+""")
