@@ -1089,7 +1089,14 @@ int cd_job_destroy(cd_job *J) {
     if (J->stream) (void)hipStreamSynchronize(J->stream);
     J->graphs.reset();
     if (J->mem) (void)hipFreeAsync(J->mem, J->stream);  // back to the pool, after the job's last work
-    if (J->stream) streams().give(J->dev, J->stream);
+    if (J->stream) {
+        // the memory is free with the call: a server hands its bytes to the next
+        // job, which would otherwise be allocated beside it
+        if (hipStreamSynchronize(J->stream) == hipSuccess)
+            streams().give(J->dev, J->stream);
+        else
+            (void)hipStreamDestroy(J->stream);
+    }
     delete J;
     return CD_OK;
 }

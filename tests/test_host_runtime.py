@@ -55,3 +55,15 @@ assert dev.value == 1 and F.fake_launches(0) > 0 and F.fake_launches(1) == 0
 job(seed=3).read()
 assert F.fake_launches(1) > 0
 """)
+
+
+def test_memory_of_a_closed_job_can_be_had_again(fake):
+    """With the call that ends it, as a server counts it."""
+    run(fake, """
+before = F.fake_used()
+j = job()
+assert F.fake_used() > before
+j.step(3)
+j.close()
+assert F.fake_used() == before
+""")
