@@ -125,7 +125,10 @@ int cd_job_cds_scanned(cd_job *job, int64_t *count);
 int cd_job_destroy(cd_job *job);
 
 /* Evaluate `count` designs [count][m][L] (the six objective reductions of
- * utils.cuh:271-888).  desc->N, H, Pm and seed are ignored. */
+ * utils.cuh:271-888).  desc->N, H, Pm and seed are ignored.  This call, cd_nds,
+ * cd_select and cd_job_read keep up to four idle buffers of at most 64 MiB of
+ * device and of pinned host memory each for the next ones, beside any server's
+ * budget; they are given back when an allocation fails. */
 int cd_eval_batch(const cd_job_desc *desc, const int8_t *genome, int32_t count,
                   float *obj, int8_t *idx, int32_t *pql);
 

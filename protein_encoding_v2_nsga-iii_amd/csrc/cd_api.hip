@@ -322,6 +322,20 @@ Streams &streams() {  // (never destroyed: the runtime may be gone by then)
     return *p;
 }
 
+// `allocate` (a HIP allocation), and once more without the idle buffers of the
+// one-shot calls (Shots) when memory has run out.
+void drop_idle_shots();
+template <class F>
+hipError_t allocated(F allocate) {
+    hipError_t e = allocate();
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();  // (or the next launch would report it)
+    drop_idle_shots();
+    e = allocate();
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 // The sizes of a descriptor's job (J->N, H, L, m, R, P, W), its layout and its
 // tables.
 int size_job(cd_job *J, const cd_job_desc *d, Use use, int P, Layout &o, HostTables &t) {
@@ -461,7 +475,7 @@ int create_job(const cd_job_desc *d, cd_job **out) {
     // hipFree does, so jobs can come and go while others run.
     hipError_t e = streams().take(&J->dev, &J->stream);
     if (e == hipSuccess) e = keep_pool_memory();
-    if (e == hipSuccess) e = hipMallocAsync(&J->mem, o.total, J->stream);
+    if (e == hipSuccess) e = allocated([&] { return hipMallocAsync(&J->mem, o.total, J->stream); });
     if (e != hipSuccess) {
         if (J->stream) (void)hipStreamDestroy(J->stream);
         delete J;
@@ -492,9 +506,10 @@ int create_job(const cd_job_desc *d, cd_job **out) {
 // takes one for its duration -- an idle one of its device, else a new one -- so
 // calls of several threads run side by side; at most SHOTS_IDLE idle ones and
 // buffers of at most SHOT_KEEP bytes are kept, the rest is freed with the
-// call.  With them, one launch that fetches the set-up and one synchronisation
-// an evaluation of 16 designs takes 49 us instead of 271, a selection of 1024
-// from 2048 90 instead of 269.
+// call, and the idle ones too when an allocation fails (allocated).  With them,
+// one launch that fetches the set-up and one synchronisation an evaluation of 16
+// designs takes 49 us, a selection of 1024 from 2048 89; with a job allocated,
+// filled by ten transfers and freed for each, 294 and 288.
 constexpr size_t EVAL_CHUNK = (size_t)1 << 20, READ_CHUNK = (size_t)4 << 20,  // bytes of packed rows
                  EVAL_WINDOW = (size_t)32 << 20;
 constexpr size_t SHOTS_IDLE = 4, SHOT_KEEP = (size_t)64 << 20;
@@ -510,14 +525,14 @@ struct Shot {
             if (mem) (void)hipFreeAsync(mem, stream);
             mem = nullptr;
             mem_cap = 0;
-            e = hipMallocAsync((void **)&mem, mem_bytes + mem_bytes / 4, stream);
+            e = allocated([&] { return hipMallocAsync((void **)&mem, mem_bytes + mem_bytes / 4, stream); });
             if (e == hipSuccess) mem_cap = mem_bytes + mem_bytes / 4;
         }
         if (e == hipSuccess && host_bytes > host_cap) {
             if (host) (void)hipHostFree(host);
             host = nullptr;
             host_cap = 0;
-            e = hipHostMalloc((void **)&host, host_bytes + host_bytes / 4, hipHostMallocDefault);
+            e = allocated([&] { return hipHostMalloc((void **)&host, host_bytes + host_bytes / 4, hipHostMallocDefault); });
             if (e == hipSuccess) host_cap = host_bytes + host_bytes / 4;
         }
         return e;
@@ -575,11 +590,20 @@ struct Shots {
         }
         s.free();
     }
+    void drop_idle() {
+        std::vector<Shot> all;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            all.swap(idle);
+        }
+        for (Shot &s : all) s.free();
+    }
 };
 Shots &shots() {  // (never destroyed: the runtime may be gone by then)
     static Shots *p = new Shots();
     return *p;
 }
+void drop_idle_shots() { shots().drop_idle(); }
 
 // Evaluate the designs of `items`: mutation (children) and objectives 0-4,
 // the stem of every changed CDS, objective 5.

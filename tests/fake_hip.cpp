@@ -4,7 +4,8 @@
 //   * work goes to a stream only while its device is the calling thread's, but
 //     for copies, clears and graph launches; an event is recorded only on a
 //     stream of its own device
-//   * memory freed on a stream can be had again once the stream was waited for
+//   * memory freed on a stream can be had again on it, and elsewhere once the
+//     stream was waited for
 //   * device memory has a limit; every timed interval is shorter than the last
 // Loaded with RTLD_GLOBAL before the engine, its symbols come first.
 #include <cstdint>
@@ -37,8 +38,12 @@ thread_local struct {
     void *stream;
 } config;
 
-int take(void **p, size_t n) {
+int take(void **p, size_t n, Stream *s = nullptr) {
     std::lock_guard<std::mutex> lk(mu);
+    if (s) {  // what was freed on it is its own again
+        used -= s->freed;
+        s->freed = 0;
+    }
     if (used + n > limit) return OUT_OF_MEMORY;
     *p = std::calloc(1, n ? n : 1);
     device[*p] = n;
@@ -80,7 +85,7 @@ int hipGetLastError() {
 }
 
 int hipMalloc(void **p, size_t n) { return take(p, n); }
-int hipMallocAsync(void **p, size_t n, void *s) { return ((Stream *)s)->dev != current ? INVALID_HANDLE : take(p, n); }
+int hipMallocAsync(void **p, size_t n, void *s) { return ((Stream *)s)->dev != current ? INVALID_HANDLE : take(p, n, (Stream *)s); }
 int hipFree(void *p) { return p ? give(p, nullptr) : OK; }
 int hipFreeAsync(void *p, void *s) { return give(p, (Stream *)s); }
 int hipHostMalloc(void **p, size_t n, unsigned) {

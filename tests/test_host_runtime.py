@@ -67,3 +67,25 @@ j.step(3)
 j.close()
 assert F.fake_used() == before
 """)
+
+
+def test_idle_buffers_are_given_back(fake):
+    """What a one-shot call keeps for the next one leaves no job, and no larger
+    call, without memory; and what is kept is bounded."""
+    run(fake, """
+aa, tab = T.synth_protein(300, 1), T.synth_tables(1)
+pop = T.random_population(aa, 2, 4000, 1)
+cdp.evaluate(aa, tab, pop)
+kept = F.fake_used()
+assert 0 < kept <= 64 << 20 and F.fake_host() <= 64 << 20
+need = cdp.device_bytes(301, 2, 500, 2)
+F.fake_limit.argtypes = [C.c_size_t]
+F.fake_limit(need + kept // 2)
+j = job(residues=300, N=500)
+assert F.fake_used() == need
+j.close()
+cdp.evaluate(aa, tab, pop[:1000])
+kept = F.fake_used()
+F.fake_limit(4 * kept)
+cdp.evaluate(aa, tab, pop[:3200])
+""")
