@@ -188,10 +188,12 @@ typedef struct cd_shapes {
  * (HIP events around each kernel) over `gens_per_candidate` ordinary
  * generations of the job or batch -- which therefore advances by
  * *generations_run generations, with exactly the results it would have had
- * in any shape.  The chosen shapes are installed and cached for the device
+ * in any shape.  A shape of a kernel that the work does not launch keeps its
+ * value.  The chosen shapes are installed and cached for the device
  * under a coarse signature of the work (job count, children, codons per
- * child, pool size, in power-of-two buckets); jobs, batches and the
- * server's ticks created later with the same signature start from them. */
+ * child, pool size, in power-of-two buckets, and the kernels it takes); jobs,
+ * batches and the server's ticks created later with the same signature start
+ * from them. */
 int cd_job_tune(cd_job *job, int32_t gens_per_candidate, cd_shapes *chosen, int32_t *generations_run);
 int cd_batch_tune(cd_batch *batch, int32_t gens_per_candidate, cd_shapes *chosen, int32_t *generations_run);
 /* Read (get) and/or install (set) the shapes of a job or batch; either

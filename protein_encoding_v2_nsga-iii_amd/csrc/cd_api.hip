@@ -824,6 +824,13 @@ int tune_shapes(const cd::Shapes &start, int njobs, int gens, hipStream_t s, App
         {&cd::Shapes::assoc_designs, {4, 8, 16, 32, 64}, 0x10u},
         {&cd::Shapes::niche_threads, {256, 512, 1024}, 0x20u},
     };
+    // the parameters of kernels that this work does not launch keep their values:
+    // their candidates differ by chance alone
+    auto used = [](const Param &p, const Launch &w) {
+        if (p.field == &cd::Shapes::stem_waves) return cd::stem_path(w.n_off, w.mg, w.longest) != cd::STEM_PATH_EACH;
+        if (p.field == &cd::Shapes::fronts_threads) return !cd::fuse_fronts(w.max_pool, w.pool);
+        return true;
+    };
     cd::Shapes cur = start;
     *run = 0;
     for (const Param &p : params) {
@@ -843,7 +850,7 @@ int tune_shapes(const cd::Shapes &start, int njobs, int gens, hipStream_t s, App
             double cost = 0.0;
             for (int k = 0; k < CD_PROFILE_KERNELS; ++k)
                 if (p.phases >> k & 1u) cost += ms[k];
-            if (cost < best_cost) {
+            if (cost < best_cost && used(p, w)) {
                 best_cost = cost;
                 best_v = v;
             }
@@ -875,18 +882,27 @@ int log2_bucket(int64_t x) {
 }
 }  // namespace
 
+// (with the kernels that its launches take: within one bucket of sizes they
+// differ, and with them what a shape means)
 std::string work_signature(cd_job *const *jobs, int count) {
-    int64_t children = 0, lm = 0, pool = 0;
+    int64_t children = 0, lm = 0, pool = 0, pools = 0;
+    int mg = 0, longest = 0, refs = 0;
     for (int j = 0; j < count; ++j) {
         children += jobs[j]->N;
         lm = std::max(lm, (int64_t)jobs[j]->L * jobs[j]->m);
         pool = std::max(pool, (int64_t)jobs[j]->P);
+        pools += jobs[j]->P;
+        mg = std::max(mg, jobs[j]->m);
+        longest = std::max(longest, jobs[j]->L);
+        refs = std::max(refs, jobs[j]->R);
     }
+    const int path = (int)cd::stem_path((int)children, mg, longest) + 4 * (int)cd::fuse_fronts((int)pool, (int)pools) +
+                     8 * (int)cd::takes_place_niche((int)pool, refs) + 16 * (int)(children > cd::DESIGN_MANY);
     int dev = 0;
     (void)hipGetDevice(&dev);
     return "dev" + std::to_string(dev) + "/jobs" + std::to_string(log2_bucket(count)) + "/children" +
            std::to_string(log2_bucket(children)) + "/codons" + std::to_string(log2_bucket(lm)) + "/pool" +
-           std::to_string(log2_bucket(pool));
+           std::to_string(log2_bucket(pool)) + "/path" + std::to_string(path);
 }
 
 // The shapes of untuned work.  Association: a wave a design while the waves

@@ -82,6 +82,13 @@ inline StemList stem_list_geom(int n_items, int mg) {
     g.cap = g.group * mg;
     return g;
 }
+// The stem kernel of a generation of n children of up to mg CDS, the longest of
+// `longest` codons.
+enum StemPath { STEM_PATH_EACH = 0, STEM_PATH_FEW = 1, STEM_PATH_MANY = 2 };  // k_stem_each, k_stem_list's two shapes
+inline StemPath stem_path(int n_items, int mg, int longest) {
+    const int64_t cds = (int64_t)n_items * mg;
+    return cds <= STEM_EACH ? STEM_PATH_EACH : cds <= STEM_MANY && longest > STEM_SHORT ? STEM_PATH_FEW : STEM_PATH_MANY;
+}
 // The list of a generation's launches; cap 0: none, k_stem_each takes every CDS.
 inline StemList stem_list_plan(int n_items, int mg) {
     StemList g = stem_list_geom(n_items, mg);

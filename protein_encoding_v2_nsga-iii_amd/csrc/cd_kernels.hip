@@ -3275,8 +3275,7 @@ hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg
         hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), bytes, s, jobs, stem_list, stem_ctl, sl.groups, sl.cap);
         return hipGetLastError();
     };
-    const bool few = (int64_t)n * mg <= STEM_MANY && longest > STEM_SHORT;
-    return few ? go(k_stem_list<256, 2048>, 2048, 256) : go(k_stem_list<128, 1024>, 1024, 128);
+    return stem_path(n, mg, longest) == STEM_PATH_FEW ? go(k_stem_list<256, 2048>, 2048, 256) : go(k_stem_list<128, 1024>, 1024, 128);
 }
 hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;

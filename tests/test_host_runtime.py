@@ -89,3 +89,32 @@ kept = F.fake_used()
 F.fake_limit(4 * kept)
 cdp.evaluate(aa, tab, pop[:3200])
 """)
+
+
+def test_tuner_leaves_unused_shapes_alone(fake):
+    """(every candidate is timed quicker than the one before, so a shape that
+    the launches use ends at its last candidate.)  A pool of 256 with 256 CDS
+    uses neither k_fronts nor k_stem_list; one of 5000 with 40000 both."""
+    run(fake, """
+for N, m, used in ((128, 2, False), (2500, 16, True)):
+    j = job(m=m, N=N)
+    j.shapes(set=dict(j.shapes(), fronts_threads=256, stem_waves=5))
+    got, _ = j.tune(1)
+    assert got["niche_threads"] == 1024 and got["assoc_designs"] == 64
+    assert (got["fronts_threads"], got["stem_waves"]) == ((1024, 8) if used else (256, 5)), got
+""")
+
+
+@pytest.mark.parametrize("tuned,other", [((1024, 2), (1025, 2)), ((1024, 16), (1025, 16)), ((2048, 2), (2049, 2))])
+def test_tuned_shapes_stay_with_their_launches(fake, tuned, other):
+    """Sizes of one power of two on the two sides of a rule of the dispatch: the
+    fused fronts and the one-workgroup niching (pools of 2048), the list of
+    changed CDS (16384), the eight-wave build of k_design (2048 children)."""
+    run(fake, f"""
+untuned = job(m={other[1]}, N={other[0]}).shapes()
+a = job(m={tuned[1]}, N={tuned[0]})
+chosen, _ = a.tune(1)
+assert chosen != untuned
+assert job(m={other[1]}, N={other[0]}).shapes() == untuned
+assert job(m={tuned[1]}, N={tuned[0]}, seed=2).shapes() == chosen
+""")
