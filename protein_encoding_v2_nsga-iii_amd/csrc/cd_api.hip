@@ -163,7 +163,7 @@ struct Layout {
         sctl,
         front,
         np, dom,
-        ref_of, dist, niche, st, acc, ranked, selm, prio, cutl, cutr, self, off, domi, asc;
+        ref_of, niche, st, acc, ranked, selm, prio, cutl, cutr, self, off, domi, asc;
     size_t head, total;
 };
 
@@ -216,7 +216,6 @@ Layout layout(int L, int m, int N, int P, int R, int W, int n_dom, int n_asc, Us
         o.np = s.add((size_t)P * 4);
         o.dom = s.add((size_t)P * W * 8);
         o.ref_of = s.add((size_t)P * 4);
-        o.dist = s.add((size_t)P * 4);
         o.niche = s.add((size_t)cd::NICHE_INTS * R * 4);
         o.acc = s.add(sizeof(cd::SelAcc));
         o.ranked = s.add((size_t)W * 8);
@@ -425,7 +424,6 @@ void describe_job(cd_job *J, const cd_job_desc *d, Use use, const Layout &o, con
         h.np = (int32_t *)(base + o.np);
         h.dom = (uint64_t *)(base + o.dom);
         h.ref_of = (int32_t *)(base + o.ref_of);
-        h.dist = (float *)(base + o.dist);
         h.niche = (int32_t *)(base + o.niche);
         h.st = (cd::SelState *)(base + o.st);
         h.acc = (cd::SelAcc *)(base + o.acc);
@@ -605,16 +603,14 @@ Shots &shots() {  // (never destroyed: the runtime may be gone by then)
 }
 void drop_idle_shots() { shots().drop_idle(); }
 
-// Evaluate the designs of `items`: mutation (children) and objectives 0-4,
-// the stem of every changed CDS, objective 5.
-// Initialisation and evaluation of the designs of `items` (offspring
-// generations go through enqueue_generation).
-// fresh: an initialisation of a pool that has not been written before.
-hipError_t enqueue_designs(const Launch &w, int mode, const int2 *items, int n_items, hipStream_t s, bool fresh = false) {
-    hipError_t e = cd::launch_design(mode, w.jobs, items, n_items, w.lds, s, nullptr, nullptr, cd::StemList{0, 0, 0},
-                                     fresh ? 1 : 0);
-    if (e == hipSuccess) e = cd::launch_stem(mode, w.jobs, items, n_items, w.mg, w.stem_lds, s);
-    if (e == hipSuccess) e = cd::launch_stem_finish(mode, w.jobs, items, n_items, s);
+// Initialisation of the children's work list `w.off` (offspring generations go
+// through enqueue_generation): the designs, the stem of every CDS, objective 5.
+// fresh: the pool has not been written before.
+hipError_t enqueue_init(const Launch &w, hipStream_t s, bool fresh) {
+    hipError_t e = cd::launch_design(cd::MODE_INIT, w.jobs, w.off, w.n_off, w.lds, s, nullptr, nullptr,
+                                     cd::StemList{0, 0, 0}, fresh ? 1 : 0);
+    if (e == hipSuccess) e = cd::launch_stem(w.jobs, w.off, w.n_off, w.mg, w.stem_lds, s);
+    if (e == hipSuccess) e = cd::launch_stem_finish(w.jobs, w.off, w.n_off, s);
     return e;
 }
 
@@ -983,7 +979,7 @@ int cd_job_create(const cd_job_desc *desc, cd_job **out) {
 int cd_job_init(cd_job *J) {
     if (!J || J->selection_only) return fail(CD_E_INVALID, "null job");
     // the offspring work list doubles as the (job, design) list of the init launch
-    HIPCHK(enqueue_designs(job_launch(J), cd::MODE_INIT, J->d_off, J->N, J->stream, !J->inited));
+    HIPCHK(enqueue_init(job_launch(J), J->stream, !J->inited));
     HIPCHK(cd::launch_init_state(J->d_self, 1, J->stream));
     J->inited = true;
     return CD_OK;
@@ -1181,8 +1177,8 @@ static int evaluate(const cd_job_desc &d, const int8_t *genome, int32_t count, f
         std::memcpy(w.host + o.head + i * row, genome + i * row, n * row);
         e = cd::launch_design(cd::MODE_EVAL, J->d_self, J->d_off + i, n, J->lds, w.stream);
     }
-    if (e == hipSuccess) e = cd::launch_stem(cd::MODE_EVAL, J->d_self, J->d_off, count, J->m, J->stem_lds, w.stream);
-    if (e == hipSuccess) e = cd::launch_stem_finish(cd::MODE_EVAL, J->d_self, J->d_off, count, w.stream);
+    if (e == hipSuccess) e = cd::launch_stem(J->d_self, J->d_off, count, J->m, J->stem_lds, w.stream);
+    if (e == hipSuccess) e = cd::launch_stem_finish(J->d_self, J->d_off, count, w.stream);
     const hipError_t es = hipStreamSynchronize(w.stream);
     if (e == hipSuccess) e = es;
     if (e == hipSuccess) {

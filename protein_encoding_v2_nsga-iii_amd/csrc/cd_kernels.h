@@ -133,7 +133,7 @@ struct ReadRest {
 hipError_t launch_read(const DevJob *job, uint8_t *rows, void *rest, size_t rest_bytes, size_t first, size_t bytes, hipStream_t s);
 // initialisation and evaluation: a workgroup per (item, CDS c < mg): stem of
 // each CDS of the items' designs
-hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s);
+hipError_t launch_stem(const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s);
 // offspring generations: stem of each CDS the offspring k_design listed
 // (the n items and sl as given to it), on as many workgroups as are resident at
 // once (STEM_CUS x what `waves`, 5 to 8 waves per SIMD, and the LDS allow), at
@@ -142,7 +142,7 @@ hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, i
 hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, int longest, const uint2 *stem_list,
                             const int32_t *stem_ctl, StemList sl, int waves, size_t lds, hipStream_t s);
 // one thread per item: objective 5, clears the marks
-hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s);
+hipError_t launch_stem_finish(const DevJob *jobs, const int2 *items, int n, hipStream_t s);
 // a sort of P objective vectors obj [P][6] (device memory) until at least N are
 // ranked: front_of [P], *n_fronts; scratch: dom [W][P], any [W][W], W = (P + 63) / 64
 struct SortArgs {

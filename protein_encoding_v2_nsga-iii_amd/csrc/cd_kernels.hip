@@ -1531,18 +1531,6 @@ __global__ __launch_bounds__(256) void k_read(const DevJob *__restrict__ jobs, u
     gstore((u32x4 *)(rows + at), v);  // (room for whole 16-byte words)
 }
 
-// Buffer and slot of the design an evaluation work item refers to: children
-// of the current generation sit at N + child in the next buffer.
-__device__ __forceinline__ void item_slot(const DevJob &J, int mode, int y, int &buf, int &slot) {
-    if (mode == MODE_OFFSPRING) {
-        buf = (int)((J.st->gen + 1u) & 1u);
-        slot = J.N + y;
-    } else {
-        buf = 0;
-        slot = y;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // k_stem (initialisation and evaluation): one workgroup per (work item, CDS),
 // blockIdx.x = item * mg + c with mg the largest m of the jobs launched: a
@@ -1552,8 +1540,7 @@ __device__ __forceinline__ void item_slot(const DevJob &J, int mode, int y, int 
 // of the match matrix 216.
 // ---------------------------------------------------------------------------
 template <int NT, int HEADS>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_stem(const DevJob *__restrict__ jobs, const int2 *__restrict__ items, int mode,
-                                              int mg) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_stem(const DevJob *__restrict__ jobs, const int2 *__restrict__ items, int mg) {
     extern __shared__ __align__(16) uint8_t dyn[];
     __shared__ uint64_t redu[16];
     __shared__ int32_t flag[NT / 64];
@@ -1562,11 +1549,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
     const DevJob &J = jobs[it.x];
     const int L = J.L, m = J.m, n = 3 * L, wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (c >= m) return;
-    int buf, slot;
-    item_slot(J, mode, it.y, buf, slot);
-    CdsStat *cs = J.cst[buf] + (size_t)slot * m + c;
+    const size_t rec = (size_t)it.y * m + c;  // (the designs are in buffer 0)
+    CdsStat *cs = J.cst[0] + rec;
     uint64_t *planes = (uint64_t *)dyn;
-    const PlaneLoad<NT> load((const uint64_t *)(J.planes + ((size_t)slot * m + c) * plane_words(L)), L);
+    const PlaneLoad<NT> load((const uint64_t *)(J.planes + rec * plane_words(L)), L);
     load.place(planes);
     const SeekLds S = seek_lds<HEADS>(dyn + stem_index_at(L), n, wid, nullptr);
     seek_clear<NT, HEADS>(S);
@@ -1782,21 +1768,16 @@ __device__ int stem_finish_at(CdsStat *cst, float *obj, int8_t *oidx, int32_t *p
     gstore(pq + 3, 0);
     return changed;
 }
-__device__ int stem_finish(const DevJob &J, int buf, int slot) {
-    return stem_finish_at(J.cst[buf], J.obj[buf], J.oidx[buf], J.pql[buf], J.m, J.den_sl, slot);
-}
 
-// stem_finish for every work item's design (initialisation and evaluation;
-// the offspring generation leaves it to k_dominance).
+// stem_finish_at for every work item's design (initialisation and evaluation,
+// in buffer 0; the offspring generation leaves it to k_dominance).
 __global__ __launch_bounds__(256) void k_stem_finish(const DevJob *__restrict__ jobs, const int2 *__restrict__ items,
-                                                     int n_items, int mode) {
+                                                     int n_items) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_items) return;
     const int2 it = items[i];
     const DevJob &J = jobs[it.x];
-    int buf, slot;
-    item_slot(J, mode, it.y, buf, slot);
-    stem_finish(J, buf, slot);
+    stem_finish_at(J.cst[0], J.obj[0], J.oidx[0], J.pql[0], J.m, J.den_sl, it.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -2413,8 +2394,7 @@ __global__ __launch_bounds__(1024) void k_fronts(const DevJob *__restrict__ jobs
     const bool n_cut = ranked_n == N;
     // survivors so far: every ranked design when the fronts fill N exactly,
     // else the fronts before the last one
-    if (J.selm)
-        for (int w = tid; w < W; w += NT) gstore(J.selm + w, n_cut ? ranked[w] : (ranked[w] & ~lastm[w]));
+    for (int w = tid; w < W; w += NT) gstore(J.selm + w, n_cut ? ranked[w] : (ranked[w] & ~lastm[w]));
     if (wid == 0)
         settle_nadir(S, obj, P, (gen & 1u) ? e1 : e0, st->res + ((gen + 1u) & 1u), ranked_n, f, last_size, n_cut);
 }
@@ -3203,7 +3183,7 @@ __global__ void k_zero_np(const DevJob *__restrict__ jobs) {
     const DevJob &J = jobs[blockIdx.x];
     for (int i = threadIdx.x; i < J.P; i += blockDim.x) J.np[i] = 0;
     if (threadIdx.x < ACC_WORDS) ((uint32_t *)J.acc)[threadIdx.x] = acc_clear_word(threadIdx.x);
-    if (J.niche) clear_niche(J, threadIdx.x, blockDim.x);
+    clear_niche(J, threadIdx.x, blockDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -3245,12 +3225,12 @@ hipError_t launch_read(const DevJob *job, uint8_t *rows, void *rest, size_t rest
     hipLaunchKernelGGL(k_read, dim3((unsigned)n), dim3(256), 0, s, job, rows, (uint32_t *)rest, (uint64_t)first, (uint64_t)bytes, (uint32_t)g);
     return hipGetLastError();
 }
-hipError_t launch_stem(int mode, const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s) {
+hipError_t launch_stem(const DevJob *jobs, const int2 *items, int n, int mg, size_t lds, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if ((int64_t)n * mg <= STEM_FEW)
-        hipLaunchKernelGGL((k_stem<256, 2048>), dim3(n * mg), dim3(256), lds + seek_more_bytes(2048, 256), s, jobs, items, mode, mg);
+        hipLaunchKernelGGL((k_stem<256, 2048>), dim3(n * mg), dim3(256), lds + seek_more_bytes(2048, 256), s, jobs, items, mg);
     else
-        hipLaunchKernelGGL((k_stem<128, 1024>), dim3(n * mg), dim3(128), lds + seek_more_bytes(1024, 128), s, jobs, items, mode, mg);
+        hipLaunchKernelGGL((k_stem<128, 1024>), dim3(n * mg), dim3(128), lds + seek_more_bytes(1024, 128), s, jobs, items, mg);
     return hipGetLastError();
 }
 hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg, int longest, const uint2 *stem_list,
@@ -3277,9 +3257,9 @@ hipError_t launch_stem_list(const DevJob *jobs, const int2 *items, int n, int mg
     };
     return stem_path(n, mg, longest) == STEM_PATH_FEW ? go(k_stem_list<256, 2048>, 2048, 256) : go(k_stem_list<128, 1024>, 1024, 128);
 }
-hipError_t launch_stem_finish(int mode, const DevJob *jobs, const int2 *items, int n, hipStream_t s) {
+hipError_t launch_stem_finish(const DevJob *jobs, const int2 *items, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_stem_finish, dim3((n + 255) / 256), dim3(256), 0, s, jobs, items, n, mode);
+    hipLaunchKernelGGL(k_stem_finish, dim3((n + 255) / 256), dim3(256), 0, s, jobs, items, n);
     return hipGetLastError();
 }
 hipError_t launch_sort(const SortArgs &a, hipStream_t s) {

@@ -155,12 +155,11 @@ struct DevJob {
     int32_t *stem_max;     // [P] longest stem of the design (k_design: unchanged CDS, k_stem: atomic maximum)
     uint64_t *dom;         // [W][P], word-major: bit b of dom[w * P + j] set when design 64w + b dominates j
     int32_t *ref_of;       // [P]
-    float *dist;           // [P]
-    int32_t *niche;        // NICHE_INTS x R words per reference point (NicheView); null for a sort alone
+    int32_t *niche;        // NICHE_INTS x R words per reference point (NicheView)
     SelState *st;
     SelAcc *acc;
     uint64_t *ranked;      // [W] first front (bit i of word w: design 64w + i)
-    uint64_t *selm;        // [W] survivors: the next generation's parents, in ascending pool index; null for a sort alone
+    uint64_t *selm;        // [W] survivors: the next generation's parents, in ascending pool index
     uint32_t *prio;        // [P] high word of a last-front design's niche priority
     uint64_t *cutl;        // [P] (priority << 32 | design) of the cut buckets' designs, bucket by bucket
     int32_t *cutr;         // [P] the reference point of each cut-list entry
