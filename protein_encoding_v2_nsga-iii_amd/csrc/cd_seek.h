@@ -181,9 +181,12 @@ __host__ __device__ inline bool sk_stops(int K, uint64_t best) { return (int)(be
 // pair.  Initialisation of 64 designs of 1500 residues of FK (stems of 2200): 160
 // us, 8.6 ms when every search that stopped went to the tiles; of 600 of K (none):
 // 86 us, 92 with a guess at every length.
+// The chain ends whatever a search returns: K falls, or grows by half and can
+// only grow from there, because `seed` is then the length met.
 __host__ __device__ inline int sk_after_k(int n, int K, bool all, int found, int seed, bool parent) {
-    if (all) return parent || K >= sk_blind_k(n) ? sk_next_k(K, seed) : 0;
-    return 2 * found >= 3 * K ? found : 0;
+    if (!all) return 2 * found >= 3 * K ? found : 0;
+    const int next = parent || K >= sk_blind_k(n) ? sk_next_k(K, seed) : 0;
+    return next < K ? next : 0;
 }
 
 // LDS of a search on n bases by `waves` waves with `heads` chains: bitmap, chain heads, links, per

@@ -4,7 +4,10 @@
 // where the searches end without a stem.  Reads CDS from stdin, one per line:
 // "sequence" (digits 0-3; initialisation), or "sequence l p q mask" (a child:
 // its parent's longest stem, and 0/1 per codon that changed).  An argument
-// replaces every wave's budget.  Prints "l p q searches tiled".
+// replaces every wave's budget.  Prints "l p q searches tiled".  A line "after n K
+// all found seed parent" prints the length of the next search.
+#include <algorithm>
+#include <cstdio>
 #include <iostream>
 #include <sstream>
 #include <string>
@@ -131,7 +134,14 @@ int main(int argc, char **argv) {
         std::istringstream in(line);
         std::string seq, maskstr;
         int pl = 0, pp = 0, pq = 0;
-        in >> seq >> pl >> pp >> pq >> maskstr;
+        in >> seq;
+        if (seq == "after") {
+            int a[6];
+            for (int &x : a) in >> x;
+            std::printf("%d\n", cd::sk_after_k(a[0], a[1], a[2] != 0, a[3], a[4], a[5] != 0));
+            continue;
+        }
+        in >> pl >> pp >> pq >> maskstr;
         Cds c;
         const int n = c.n = (int)seq.size();
         c.L = n / 3;

@@ -110,3 +110,13 @@ def test_no_stem_two_guesses(orc, harness):
         s = np.resize(u, 1800).astype(np.uint8)
         (g,) = run(harness, [text(s)])
         assert g[:3] == orc.sl(s, 0) and g[3] == 2 and g[4] == 1
+
+
+def test_the_chain_ends(harness):
+    """Whatever a search returns, the next one is shorter, or at least half as
+    long again, or none; and after a longer one none is shorter."""
+    cases = [(n, K, a, f, s, p) for n in (30, 600, 5000) for K in (5, 6, 9, 14) for a in (0, 1)
+             for f in (0, K - 1, K, 2 * K) for s in (0, 4, K - 1, K, K + 1) for p in (0, 1)]
+    for (n, K, a, f, s, p), (k,) in zip(cases, run(harness, ["after %d %d %d %d %d %d" % c for c in cases])):
+        assert k < K or (not a and 2 * k >= 3 * K), (n, K, a, f, s, p, k)
+        assert not (a and s >= K) or k == 0, (n, K, a, f, s, p, k)
