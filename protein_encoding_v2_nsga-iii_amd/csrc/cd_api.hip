@@ -935,8 +935,10 @@ cd::Shapes untuned_shapes(cd_job *const *jobs, int count) {
     // the chip is full of them.  Microseconds a generation with 64 / 128 / 256
     // rows: batches of 72 tiles 39.1 / 40.2 / 42.2, 544 56.8 / 57.4 / 59.0, 1056
     // 64.8 / 65.4 / 64.7, 3168 104 / 103 / 102, 6336 178 / 174 / 173, the 64-job
-    // mix (17 700) 817 / 808 / 802; lone jobs of 1176 tiles 63.6 / 66 / 64, 4186
-    // 87.1 / 88.3 / 88.1, 8256 225 / 222 / 220.5.
+    // mix (17 700) 817 / 808 / 802; lone jobs of 202 codons, 528 tiles 51.3 / 52.7 /
+    // 52.2, 2850 81.5 / 82.2 / 80.1, 4095 88.4 / 89.5 / 89.1, 5253 96.3 / 97.2 / 95.3,
+    // 6105 101.8 / 100.2 / 99.6, 8256 113.2 / 110.6 / 112.1, 12 403 138 / 131 / 131,
+    // 32 896 224 / 209 / 203.
     sh.dom_rows = tiles <= (count > 1 ? 1024 : 6000) ? 64 : 256;
     sh.assoc_designs = pool <= 512 ? 4 : pool <= cd::FUSED_TOTAL ? 8 : pool <= 12000 ? 16 : 64;
     return sh;
@@ -1018,10 +1020,6 @@ int cd_job_sync(cd_job *J) {
     return CD_OK;
 }
 
-// Reads of a job's device state go through its own (non-blocking) stream,
-// never the legacy null stream, so that they neither wait for nor disturb
-// other streams -- for instance a served tick being captured in another
-// thread.
 // The survivors in ascending pool index: the first N set bits of the
 // survivor mask.
 static void survivors_of(const std::vector<uint64_t> &mask, int N, int32_t *out) {
@@ -1031,6 +1029,9 @@ static void survivors_of(const std::vector<uint64_t> &mask, int N, int32_t *out)
     for (; k < N; ++k) out[k] = -1;
 }
 
+// Reads of a job's device state go through its own (non-blocking) stream,
+// never the legacy null stream, so that they do not wait for other streams -- for
+// instance a server's ticks.
 static hipError_t read_state(cd_job *J, cd::SelState &st) {
     hipError_t e = sync_job(J);
     if (e == hipSuccess) e = hipMemcpyAsync(&st, J->h.st, sizeof(st), hipMemcpyDeviceToHost, J->stream);

@@ -13,7 +13,6 @@
 
 struct cd_batch;
 
-// One job: tables, pools and selection state in one device allocation.
 // The captured graph of a job or batch: GRAPH_BLOCK generations back to back
 // (consecutive graph launches leave several microseconds between them; the
 // kernels inside one graph follow each other closely).  Before it is captured
@@ -35,6 +34,7 @@ struct StepGraphs {
     }
 };
 
+// One job: tables, pools and selection state in one device allocation.
 struct cd_job {
     // live batches that hold the job: while any does, the job is advanced
     // only through them (cd_job_step and cd_job_destroy fail) and reads wait
@@ -70,7 +70,7 @@ struct cd_batch {
     uint2 *d_slist = nullptr;  // changed CDS of a generation (stem_list_entries)
     int32_t *d_sctl = nullptr;
     int n_off = 0, n_dom = 0, n_asc = 0, n_cds = 0;
-    int n_small = 0;        // children first in d_off whose k_design fits six per CU
+    int n_small = 0;        // children first in d_off, launched apart (Launch::n_small)
     size_t lds_small = 0;   // their k_design LDS
     size_t lds = 0, stem_lds = 0;
     int max_pool = 0;    // largest pool of the batch's jobs
@@ -115,9 +115,9 @@ struct Launch {
     uint2 *stem_list;  // changed CDS of a generation, in sublists of consecutive children (stem_list_entries)
     int32_t *stem_ctl;    // their counts, zero between generations (k_dominance clears them)
     int n_cds;            // CDS of all children: sum of N * m
-    // the first n_small children (0: none apart) are of jobs whose k_design
-    // LDS, at most lds_small (at most sh.design_split), they are launched
-    // apart from the others, which take lds
+    // the first n_small children (0: none apart) are of jobs whose k_design LDS
+    // is at most sh.design_split; they are launched apart, with lds_small, from
+    // the others, which take lds
     int n_small;
     size_t lds_small;
     int pool;  // designs of all jobs' pools

@@ -54,14 +54,18 @@ bool shapes_valid(const Shapes &s);
 // More children than this in a launch of 256-thread workgroups (seven a CU
 // are resident at 68 VGPRs) and k_design is throughput-bound: it then takes
 // the build for eight waves per SIMD, which spills a few registers (64-job
-// mix 426 -> 397 us, 4096 children of 12008 codons 98.3 -> 98.3; 1024 children of
-// 2004 codons 25.1 -> 26.1).
+// mix 426 -> 397 us).  Microseconds of k_design for six / eight waves a SIMD,
+// children of 202 codons: 1536 of them 15.8 / 16.9, 2100 20.5 / 20.2, 3072 24.6 /
+// 24.3, 4096 29.8 / 28.7, 6000 39.4 / 37.2; of 2004: 1536 21.5 / 22.5, 2100 26.7 /
+// 26.5, 4096 39.2 / 38.2; of 12 008: 2100 64.7 / 67.6, 3072 76.2 / 78.7, 4096 90.4 /
+// 91.0; batches of 50 to 950 residues, 2048 children 23.1 / 23.7, 2560 30.7 / 34.0,
+// 4096 42.2 / 41.4, 8192 74.1 / 69.0.
 constexpr int DESIGN_MANY = 2048;
 
 size_t design_lds_bytes(int L, int m);
 size_t design_bytes_accepted(int L, int m);  // at most LDS_BYTES for a job to be accepted
 size_t stem_lds_bytes(int L);
-size_t cds_plane_bytes(int L);  // one CDS's two bit planes in the job's plane buffer
+size_t cds_plane_bytes(int L);  // one CDS in the job's plane buffer: its sequence's bit planes and its change mask
 hipError_t set_design_lds_limit(size_t bytes);
 hipError_t set_stem_lds_limit(size_t bytes);
 

@@ -723,7 +723,7 @@ struct MutArgs {
     uint32_t gen, child;
 };
 
-// A code's synonym word (J.syn6): codes of synonyms 0-4 in six-bit fields of
+// A code's synonym word (the 64 after J.lw6's log weights): codes of synonyms 0-4 in six-bit fields of
 // the low half, of synonym 5 in bits 0-5 of the high half, their number in
 // bits 8-10 and the code's own index in bits 12-14 of it.
 struct SynWord {

@@ -22,8 +22,8 @@ namespace {
 // to level, so most of the time goes into small sets: they need no allocation,
 // each level has one coordinate less, three coordinates are swept, and the
 // number of coordinates is a constant of the code.  400 points in six
-// dimensions: 115-144 ms with a vector per point and every level in all six
-// dimensions, 7 ms so.
+// dimensions, a run's final pool: 51 ms with a vector per point and every level in
+// all six dimensions, 3.7 ms so; 100 points on a sphere 34.8 and 1.8 ms.
 
 // Points of one level of the recursion, and the order they are taken in.
 struct Level {
